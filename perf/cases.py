@@ -182,7 +182,8 @@ def tolerance(case):
         # F32 arithmetic, but the attention rows are rounded to bf16: a last bit of F32 can be a
         # bf16 step of one value
         return dict(rel=1e-3, max=8e-3)
-    return dict(rel=1e-2, max=4e-2)
+    # seen against 64 bits: 0.3 % in the 2-norm, two bf16 steps of single values
+    return dict(rel=1e-2, max=6e-2)
 
 
 # ---------------------------------------------------------------------------------- program --
