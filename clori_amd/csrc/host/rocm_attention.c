@@ -35,7 +35,6 @@ enum {
     ROCM_TEAM_TILES_WIDE = 4,
     ROCM_TEAMS_MAX = 32,       /* teams per (session, kv head): two load trips of the last team's merge */
     ROCM_TEAM_GROUP_MAX = 8,   /* query heads per kv head a team's LDS holds */
-    ROCM_PREFILL_ROWS = YVEX_ROCM_PREFILL_ROWS, /* query rows per prefill workgroup */
     ROCM_WORK_ALIGNMENT = 256    /* src/backend/cuda/transformer.c:17 */
 };
 
@@ -452,7 +451,10 @@ static int rocm_attention_workspace_required(const yvex_transformer_attention_re
                     : balanced_workspace_bytes(waves, group, r->head_dimension, 1ull, &acc, &ml, &total)))
             return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");
         *bytes = total;
-    } else if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_EXACT_F32) {
+    } else if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_BF16_F32_ACCUMULATE) {
+        if (!yvex_rocm_prefill_workspace(r, bytes))
+            return refuse(err, YVEX_ERR_BOUNDS, where, "prefill workspace geometry overflowed");
+    } else {
         unsigned long long per_run;
         const unsigned long long runs = exact_split_runs(r, &per_run);
         if (runs) {
@@ -512,17 +514,10 @@ static int exact_tile_function(const yvex_transformer_attention_requirement *r,
     return 1;
 }
 
-/* What attention_execute_common has worked out of a request before it picks a kernel. */
-typedef struct attention_geometry {
-    unsigned long long q_stride, k_stride, v_stride; /* elements between tokens */
-    unsigned long long rows;                         /* query tokens x query heads */
-    int causal;
-} attention_geometry;
-
 /* The EXACT_F32 contract: the tile kernel on the fp32 matrix cores for prefill-shaped requests,
  * runs of keys for single rows over long histories, the row kernel for the rest. */
 static int attention_execute_exact(yvex_backend *backend, const yvex_transformer_attention_request *request,
-                                   yvex_device_tensor *lse, const attention_geometry *g,
+                                   yvex_device_tensor *lse, const yvex_rocm_attention_geometry *g,
                                    yvex_backend_operation_facts *facts, yvex_error *err)
 {
     yvex_rocm_backend_state *state = yvex_rocm_state(backend);
@@ -645,64 +640,6 @@ static int attention_execute_exact(yvex_backend *backend, const yvex_transformer
     return rc;
 }
 
-/* The BF16 contract over more than one query row (or a geometry the decode teams do not take):
- * the MFMA prefill kernel, 128 query rows of one head per workgroup. */
-static int attention_execute_prefill(yvex_backend *backend, const yvex_transformer_attention_request *request,
-                                     yvex_device_tensor *lse, const yvex_device_tensor *gate,
-                                     const attention_geometry *g, yvex_backend_operation_facts *facts,
-                                     yvex_error *err)
-{
-    static const char where[] = "rocm.transformer.attention";
-    yvex_rocm_backend_state *state = yvex_rocm_state(backend);
-    const yvex_transformer_attention_requirement *r = &request->requirement;
-    int rc;
-    yvex_rocm_prefill_params params;
-    const unsigned long long q_tiles = (r->query_tokens + ROCM_PREFILL_ROWS - 1ull) /
-                                       ROCM_PREFILL_ROWS;
-    memset(&params, 0, sizeof(params));
-    params.q = (const uint16_t *)request->query->data;
-    params.k = (const uint16_t *)request->key->data;
-    params.v = (const uint16_t *)request->value->data;
-    params.out = (uint16_t *)request->output->data;
-    params.lse = lse ? (float *)lse->data : NULL;
-    params.gate = gate ? (const uint16_t *)gate->data : NULL;
-    params.status = state->device_status;
-    params.q_stride = g->q_stride;
-    params.k_stride = g->k_stride;
-    params.v_stride = g->v_stride;
-    params.query_tokens = (uint32_t)r->query_tokens;
-    params.kv_tokens = (uint32_t)r->key_value_tokens;
-    params.query_start = (uint32_t)r->query_start;
-    params.query_heads = (uint32_t)r->query_heads;
-    params.kv_heads = (uint32_t)r->key_value_heads;
-    params.head_dim = (uint32_t)r->head_dimension;
-    params.causal = (uint32_t)g->causal;
-    params.scale_log2 = (1.0f / sqrtf((float)r->head_dimension)) * 1.4426950408889634f;
-    backend_workspace_reset(backend);
-    /* the kernel addresses K and V through 32-bit buffer offsets */
-    if (r->query_heads > 65535ull || q_tiles > 65535ull ||
-        r->query_heads * q_tiles > 0x7fffffffull ||
-        r->key_value_tokens * g->k_stride * 2ull >= 0xffffffffull ||
-        r->key_value_tokens * g->v_stride * 2ull >= 0xffffffffull)
-        return refuse(err, YVEX_ERR_BOUNDS, where,
-                      "prefill geometry exceeds admitted launch range");
-    rc = yvex_rocm_launch(backend,
-                          r->head_dimension == 64ull    ? YVEX_ROCM_FN_PREFILL_BF16_64
-                          : r->head_dimension == 256ull ? YVEX_ROCM_FN_PREFILL_BF16_256
-                                                        : YVEX_ROCM_FN_PREFILL_BF16,
-                          YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16,
-                          (unsigned int)(r->query_heads * q_tiles), 1u, 1u, 256u, 0u,
-                          &params, "rocm.transformer.gqa.prefill", err);
-    if (rc == YVEX_OK) {
-        facts->kernel_launches = 1ull;
-        facts->accelerated_matrix_launches = 1ull;
-        facts->compulsory_memory_facts_available = 1;
-        rc = yvex_rocm_complete(backend, YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16,
-                                "rocm.transformer.gqa.prefill", facts, err);
-    }
-    return rc;
-}
-
 static int attention_execute_common(yvex_backend *backend,
                                     const yvex_transformer_attention_request *request,
                                     yvex_device_tensor *lse, const yvex_device_tensor *gate,
@@ -713,7 +650,7 @@ static int attention_execute_common(yvex_backend *backend,
     const yvex_transformer_attention_requirement *r;
     unsigned long long q_width, kv_width, q_stride, k_stride, v_stride;
     unsigned long long q_elements, k_elements, v_elements, o_elements, rows;
-    attention_geometry geometry;
+    yvex_rocm_attention_geometry geometry;
     int exact, rc, causal;
     if (!request || !request->query || !request->key || !request->value || !request->output ||
         !facts)
@@ -784,7 +721,7 @@ static int attention_execute_common(yvex_backend *backend,
         job.scale = 1.0f / sqrtf((float)r->head_dimension);
         rc = decode_run(backend, &job, "rocm.transformer.gqa.decode", facts, err);
     } else {
-        rc = attention_execute_prefill(backend, request, lse, gate, &geometry, facts, err);
+        rc = yvex_rocm_prefill_execute(backend, request, lse, gate, &geometry, facts, err);
     }
     if (rc != YVEX_OK) return rc;
     request->output->is_written = 1;

@@ -1,0 +1,179 @@
+/* Multi-token bf16 attention of the ROCm arm: how the work of a launch is cut, and the launch.
+ *
+ * The query heads of a kv head are packed into the rows of its query tiles (kernel_params.h), so
+ * the number of items is kv_heads * ceil(query_tokens * group / 128), and an item walks the keys
+ * its last token sees in steps of 64.  (A single query token is not packed and not cut: one item
+ * per query head.)  Up to a multiple of the compute units the items are walked
+ * whole, one workgroup each, the longest first; when what is left over would keep a fraction of
+ * the units busy for long, its walks are cut into runs of keys, one workgroup each, and a second
+ * launch merges the runs.  Nine tokens of 40/8 heads of 128 behind 12001: one tile per query head
+ * walked 188 steps on 40 units, 160 us; packed and cut into 256 runs, 20 us.  2000 tokens of 24/4
+ * heads of 256 behind 13333: 376 items took two turns of 256 units with half of the second empty,
+ * 1182 us; with its tail cut, 873.  A prompt of 2048 tokens without a history is not cut and gains
+ * from the packing only that a tile spans 26 tokens instead of 128 (50.6 -> 50.2 us).  The cut is a function of the request's geometry only (256 units, never
+ * the device), so that the planner's workspace_required and the execution agree. */
+#include "rocm_state.h"
+
+#include <math.h>
+#include <string.h>
+
+enum { PREFILL_UNITS = 256, PREFILL_STEP_KEYS = 64, PREFILL_SPLITS_MAX = 64, PREFILL_RUN_STEPS_MIN = 2 };
+
+typedef struct prefill_plan {
+    unsigned long long pack, row_heads, rows, query_tiles, whole_items, tail_items, splits;
+    unsigned long long acc_bytes, ml_bytes; /* partials of the tail */
+} prefill_plan;
+
+/* Steps of an item of query tile `q_tile`. */
+static unsigned long long item_steps(const yvex_transformer_attention_requirement *r,
+                                     const prefill_plan *plan, unsigned long long q_tile)
+{
+    unsigned long long last = (q_tile + 1ull) * YVEX_ROCM_PREFILL_ROWS, keys = r->key_value_tokens;
+    if (last > plan->rows) last = plan->rows;
+    if (r->mask == YVEX_TRANSFORMER_ATTENTION_MASK_CAUSAL) keys = r->query_start + (last - 1ull) / plan->pack + 1ull;
+    return (keys + PREFILL_STEP_KEYS - 1ull) / PREFILL_STEP_KEYS;
+}
+
+/* What the tail costs in nanoseconds when each of its walks is cut into `splits` runs: every unit
+ * takes its share of the runs one after the other, each with the start and end of a workgroup;
+ * a cut tail also writes its partials, reads them back and pays a launch. */
+static unsigned long long tail_cost(const yvex_transformer_attention_requirement *r, const prefill_plan *plan,
+                                    unsigned long long steps, unsigned long long splits)
+{
+    const unsigned long long step_ns = 7ull * r->head_dimension; /* 0.9 us for a 128-row step at 128 */
+    const unsigned long long turns = (plan->tail_items * splits + PREFILL_UNITS - 1ull) / PREFILL_UNITS;
+    const unsigned long long live = plan->rows < YVEX_ROCM_PREFILL_ROWS ? plan->rows : YVEX_ROCM_PREFILL_ROWS;
+    unsigned long long cost = turns * ((steps + splits - 1ull) / splits * step_ns + 3500ull);
+    if (splits > 1ull) /* F32 rows written and read at about 4 TB/s, and the second launch */
+        cost += 5000ull + plan->tail_items * splits * live * r->head_dimension * 8ull / 4000ull;
+    return cost;
+}
+
+/* Returns 0 when a product overflows. */
+static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
+{
+    unsigned long long items, steps, splits, best, slots;
+    memset(plan, 0, sizeof(*plan));
+    plan->pack = r->query_tokens > 1ull ? r->query_heads / r->key_value_heads : 1ull;
+    plan->row_heads = r->query_heads / plan->pack;
+    if (!yvex_core_u64_mul(r->query_tokens, plan->pack, &plan->rows) || plan->rows > 0x7fffffffull) return 0;
+    plan->query_tiles = (plan->rows + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
+    if (!yvex_core_u64_mul(plan->query_tiles, plan->row_heads, &items) || items > 0x7fffffffull) return 0;
+    plan->whole_items = items;
+    plan->splits = 1ull;
+    if (!may_split || r->query_tokens == 1ull || items % PREFILL_UNITS == 0ull) return 1;
+    plan->whole_items = items / PREFILL_UNITS * PREFILL_UNITS;
+    plan->tail_items = items - plan->whole_items;
+    steps = item_steps(r, plan, plan->query_tiles - 1ull - plan->whole_items / plan->row_heads);
+    best = tail_cost(r, plan, steps, 1ull);
+    for (splits = 2ull; splits <= PREFILL_SPLITS_MAX && splits * PREFILL_RUN_STEPS_MIN <= steps; ++splits) {
+        const unsigned long long cost = tail_cost(r, plan, steps, splits);
+        if (cost < best) {
+            best = cost;
+            plan->splits = splits;
+        }
+    }
+    if (plan->splits == 1ull) {
+        plan->whole_items = items;
+        plan->tail_items = 0ull;
+        return 1;
+    }
+    slots = plan->tail_items * plan->splits * YVEX_ROCM_PREFILL_ROWS;
+    plan->acc_bytes = slots * r->head_dimension * sizeof(float);
+    plan->ml_bytes = slots * 2ull * sizeof(float);
+    return 1;
+}
+
+/* Bytes of the partials of a request (0: its walks are not cut). */
+int yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r, unsigned long long *bytes)
+{
+    prefill_plan plan;
+    if (!prefill_plan_make(r, 1, &plan)) return 0;
+    *bytes = plan.acc_bytes + plan.ml_bytes; /* both multiples of the 1 KB that 128 rows take */
+    return 1;
+}
+
+static yvex_rocm_function_id by_head_dimension(unsigned long long d, yvex_rocm_function_id at_64,
+                                               yvex_rocm_function_id at_128, yvex_rocm_function_id at_256)
+{
+    return d == 64ull ? at_64 : d == 256ull ? at_256 : at_128;
+}
+
+int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_attention_request *request,
+                              yvex_device_tensor *lse, const yvex_device_tensor *gate,
+                              const yvex_rocm_attention_geometry *g, yvex_backend_operation_facts *facts,
+                              yvex_error *err)
+{
+    static const char where[] = "rocm.transformer.gqa.prefill";
+    const yvex_backend_operation_variant variant = YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16;
+    yvex_rocm_backend_state *state = yvex_rocm_state(backend);
+    const yvex_transformer_attention_requirement *r = &request->requirement;
+    unsigned long long work = 0ull;
+    yvex_rocm_prefill_params params;
+    prefill_plan plan;
+    int rc;
+    /* the kernel addresses K and V through 32-bit buffer offsets */
+    if (r->query_heads > 65535ull || r->key_value_tokens * g->k_stride * 2ull >= 0xffffffffull ||
+        r->key_value_tokens * g->v_stride * 2ull >= 0xffffffffull || !prefill_plan_make(r, 1, &plan)) {
+        yvex_error_set(err, YVEX_ERR_BOUNDS, "rocm.transformer.attention",
+                       "prefill geometry exceeds admitted launch range");
+        return YVEX_ERR_BOUNDS;
+    }
+    backend_workspace_reset(backend);
+    /* Without an attached workspace that holds the partials the walks stay whole: allocating and
+     * freeing them around the call costs more than the cut saves, and waits for the stream. */
+    if (plan.splits > 1ull &&
+        yvex_backend_workspace_acquire(backend, plan.acc_bytes + plan.ml_bytes, 256ull, &work) !=
+            YVEX_BACKEND_RESIDENT_HIT) {
+        work = 0ull;
+        (void)prefill_plan_make(r, 0, &plan);
+    }
+    memset(&params, 0, sizeof(params));
+    params.q = (const uint16_t *)request->query->data;
+    params.k = (const uint16_t *)request->key->data;
+    params.v = (const uint16_t *)request->value->data;
+    params.out = (uint16_t *)request->output->data;
+    params.lse = lse ? (float *)lse->data : NULL;
+    params.gate = gate ? (const uint16_t *)gate->data : NULL;
+    params.status = state->device_status;
+    params.q_stride = g->q_stride;
+    params.k_stride = g->k_stride;
+    params.v_stride = g->v_stride;
+    params.query_tokens = (uint32_t)r->query_tokens;
+    params.kv_tokens = (uint32_t)r->key_value_tokens;
+    params.query_start = (uint32_t)r->query_start;
+    params.query_heads = (uint32_t)r->query_heads;
+    params.kv_heads = (uint32_t)r->key_value_heads;
+    params.pack = (uint32_t)plan.pack;
+    params.row_heads = (uint32_t)plan.row_heads;
+    params.causal = (uint32_t)g->causal;
+    params.rows = (uint32_t)plan.rows;
+    params.query_tiles = (uint32_t)plan.query_tiles;
+    params.scale_log2 = (1.0f / sqrtf((float)r->head_dimension)) * 1.4426950408889634f;
+    params.whole_items = (uint32_t)plan.whole_items;
+    params.tail_items = (uint32_t)plan.tail_items;
+    params.splits = (uint32_t)plan.splits;
+    params.part_acc = (float *)(uintptr_t)work;
+    params.part_ml = (float *)(uintptr_t)(work + plan.acc_bytes);
+    rc = yvex_rocm_launch(backend,
+                          by_head_dimension(r->head_dimension, YVEX_ROCM_FN_PREFILL_BF16_64,
+                                            YVEX_ROCM_FN_PREFILL_BF16, YVEX_ROCM_FN_PREFILL_BF16_256),
+                          variant, (unsigned int)(plan.whole_items + plan.tail_items * plan.splits), 1u, 1u, 256u,
+                          0u, &params, where, err);
+    if (rc == YVEX_OK && plan.splits > 1ull)
+        rc = yvex_rocm_launch(backend,
+                              by_head_dimension(r->head_dimension, YVEX_ROCM_FN_PREFILL_MERGE_64,
+                                                YVEX_ROCM_FN_PREFILL_MERGE, YVEX_ROCM_FN_PREFILL_MERGE_256),
+                              variant,
+                              (unsigned int)(plan.tail_items * YVEX_ROCM_PREFILL_ROWS * r->head_dimension / 1024ull),
+                              1u, 1u, 256u, 0u, &params, where, err);
+    if (rc == YVEX_OK) {
+        facts->kernel_launches = plan.splits > 1ull ? 2ull : 1ull;
+        facts->accelerated_matrix_launches = 1ull;
+        facts->temporary_bytes = plan.acc_bytes + plan.ml_bytes;
+        facts->compulsory_memory_facts_available = 1;
+        rc = yvex_rocm_complete(backend, variant, where, facts, err);
+    }
+    backend_workspace_reset(backend);
+    return rc;
+}

@@ -37,6 +37,9 @@ typedef enum {
     YVEX_ROCM_FN_PREFILL_BF16,
     YVEX_ROCM_FN_PREFILL_BF16_64,
     YVEX_ROCM_FN_PREFILL_BF16_256,
+    YVEX_ROCM_FN_PREFILL_MERGE,
+    YVEX_ROCM_FN_PREFILL_MERGE_64,
+    YVEX_ROCM_FN_PREFILL_MERGE_256,
     YVEX_ROCM_FN_MLA_DECODE_BF16,
     YVEX_ROCM_FN_MLA_DECODE_512_BF16,
     YVEX_ROCM_FN_KV_APPEND_BF16,
@@ -245,6 +248,19 @@ int yvex_rocm_op_attention(yvex_backend *backend, const yvex_device_tensor *quer
                            int causal, yvex_device_tensor *score_scratch,
                            yvex_device_tensor *probability_scratch, yvex_device_tensor *out,
                            yvex_error *err);
+/* What the attention entry points have worked out of a request before they pick a kernel. */
+typedef struct {
+    unsigned long long q_stride, k_stride, v_stride; /* elements between tokens */
+    unsigned long long rows;                         /* query tokens x query heads */
+    int causal;
+} yvex_rocm_attention_geometry;
+/* rocm_prefill.c: the BF16 contract over more than one query row (or a geometry the decode teams
+ * do not take), on the MFMA prefill kernels */
+int yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r, unsigned long long *bytes);
+int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_attention_request *request,
+                              yvex_device_tensor *lse, const yvex_device_tensor *gate,
+                              const yvex_rocm_attention_geometry *g, yvex_backend_operation_facts *facts,
+                              yvex_error *err);
 /* rocm_elementwise.c: the element-wise slots of the transformer operations table */
 int yvex_rocm_rotary_half_f32(yvex_backend *backend, yvex_device_tensor *values,
                               const yvex_device_tensor *cosines, const yvex_device_tensor *sines,

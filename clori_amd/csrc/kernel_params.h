@@ -188,8 +188,18 @@ typedef struct {
     uint64_t count, heads, head_dim, rotary_dim;
 } yvex_rocm_elementwise_params;
 
-/* Causal / full GQA prefill on bf16 token-major tensors.  The grid is one-dimensional:
- * query_heads * ceil(query_tokens / YVEX_ROCM_PREFILL_ROWS) workgroups of 256 threads. */
+/* Causal / full GQA prefill on bf16 token-major tensors.  `pack` query heads that share a kv head
+ * (all of its group, or one) are packed into the rows of one head's query tiles: row r of row
+ * head h is token r / pack of query head h * pack + r % pack, so a tile of YVEX_ROCM_PREFILL_ROWS
+ * rows spans few tokens, and few query tokens still share each key they read.  An item is one
+ * (row head, query tile); items are numbered heaviest first (item / row_heads counts the query
+ * tiles down from the last).  Workgroups
+ * 0 .. whole_items - 1 walk one item each; the tail_items behind them are walked by `splits`
+ * workgroups each, one run of 64-key steps per workgroup (workgroup whole_items + split *
+ * tail_items + i), which leave partials that yvex_rocm_prefill_merge* reads:
+ * part_acc [tail_items * splits][YVEX_ROCM_PREFILL_ROWS][head_dim] F32 (unnormalised), part_ml
+ * [tail_items * splits][YVEX_ROCM_PREFILL_ROWS][2] F32 = (running maximum in log2 units, sum).  The
+ * accumulator rows of a run that saw no key (maximum -inf) are not written. */
 #define YVEX_ROCM_PREFILL_ROWS 128
 typedef struct {
     const uint16_t *q, *k, *v;
@@ -197,11 +207,13 @@ typedef struct {
     float *lse; /* optional F32 [Tq][Hq] */
     int32_t *status;
     uint64_t q_stride, k_stride, v_stride; /* elements per token */
-    uint32_t query_tokens, kv_tokens, query_start, query_heads, kv_heads, head_dim;
-    uint32_t causal, reserved;
+    uint32_t query_tokens, kv_tokens, query_start, query_heads, kv_heads, pack;
+    uint32_t causal, rows; /* rows of a row head: query_tokens * pack */
     float scale_log2;
-    float reserved_f;
+    uint32_t query_tiles;
     const uint16_t *gate; /* optional bf16 [Tq][Hq][head_dim] sigmoid output gate */
+    float *part_acc, *part_ml;
+    uint32_t whole_items, tail_items, splits, row_heads;
 } yvex_rocm_prefill_params;
 
 /* Absorbed-latent MLA decode, split over the context.  A chunk spans at most

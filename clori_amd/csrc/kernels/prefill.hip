@@ -110,7 +110,9 @@ struct Prefill {
     const yvex_rocm_prefill_params &p;
     unsigned char *const lds;
     const int lane, wave, n, g;
-    uint32_t head, kv_head, row0;
+    uint32_t row_head, kv_head, row0;  // row0: first packed row of this wave
+    int32_t first_key, key_count;  // keys are numbered from the first one of this workgroup's run
+    int32_t visible;               // last key the lane's row sees
     // staging
     i32x4 k_rsrc, v_rsrc;
     uint32_t k_row_bytes, v_row_bytes, lds_base, k_off[kLoads], v_off[kLoads];
@@ -166,14 +168,13 @@ struct Prefill {
     // the tensor).
     __device__ inline void mask_tile(floatx16 (&s)[2], uint32_t tile) const
     {
-        const uint32_t key0 = tile * kKeyTile, row = row0 + n;
-        const uint32_t vis = p.causal ? min(p.query_start + row, p.kv_tokens - 1u) : p.kv_tokens - 1u;
+        const int32_t key0 = (int32_t)(tile * kKeyTile);
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const uint32_t key = key0 + mb * 32 + (i >> 2) * 8 + g * 4 + (i & 3);
-                if (key > vis) s[mb][i] = -INFINITY;
+                const int32_t key = key0 + mb * 32 + (i >> 2) * 8 + g * 4 + (i & 3);
+                if (key > visible) s[mb][i] = -INFINITY;
             }
     }
 
@@ -206,27 +207,42 @@ struct Prefill {
 
     __device__ inline void run()
     {
-        // heavier (later) query tiles are dispatched first; id % kv_heads picks the kv head
-        const uint32_t q_tiles = (p.query_tokens + kRowsPerBlock - 1) / kRowsPerBlock;
-        const uint32_t q_tile = q_tiles - 1u - blockIdx.x / p.query_heads;
-        const uint32_t in_tile = blockIdx.x % p.query_heads;
-        kv_head = in_tile % p.kv_heads;
-        head = kv_head * (p.query_heads / p.kv_heads) + in_tile / p.kv_heads;
-        row0 = q_tile * kRowsPerBlock + wave * kRowsPerWave;  // first row of this wave
+        // heavier (later) query tiles are dispatched first; item % row_heads picks the row head
+        uint32_t item = blockIdx.x, split = 0u;
+        const bool partial = item >= p.whole_items;
+        if (partial) {
+            split = (item - p.whole_items) / p.tail_items;
+            item = p.whole_items + (item - p.whole_items) % p.tail_items;
+        }
+        const uint32_t q_tile = p.query_tiles - 1u - item / p.row_heads;
+        row_head = item % p.row_heads;
+        kv_head = row_head * p.kv_heads / p.row_heads;
+        row0 = q_tile * kRowsPerBlock + wave * kRowsPerWave;
 
         // keys visible to the last row of the workgroup bound the walk
-        const uint32_t block_last_row = min(p.query_tokens, (q_tile + 1u) * kRowsPerBlock) - 1u;
-        const uint32_t kv_end = p.causal ? min(p.kv_tokens, p.query_start + block_last_row + 1u)
+        const uint32_t block_last_row = min(p.rows, (q_tile + 1u) * kRowsPerBlock) - 1u;
+        const uint32_t kv_end = p.causal ? min(p.kv_tokens, p.query_start + block_last_row / p.pack + 1u)
                                          : p.kv_tokens;
-        const uint32_t all_tiles = (kv_end + kKeyTile - 1) / kKeyTile;
-        const uint32_t tiles = all_tiles;
+        uint32_t tiles = (kv_end + kKeyTile - 1) / kKeyTile;
+        first_key = 0;
+        if (partial) {
+            const uint32_t per_split = (tiles + p.splits - 1u) / p.splits;
+            const uint32_t begin = min(tiles, split * per_split);
+            tiles = min(per_split, tiles - begin);
+            // (a run without steps keeps its addresses inside the tensors)
+            first_key = tiles != 0u ? (int32_t)(begin * kKeyTile) : 0;
+        }
+        key_count = (int32_t)p.kv_tokens - first_key;
 
         // ---- Q fragments: B operand, lane (n, g) holds Q[row n][16*kk + 8g .. +7] ----
         {
-            const uint32_t row = min(row0 + n, p.query_tokens - 1u);
-            const uint16_t *src = p.q + (uint64_t)row * p.q_stride + (uint64_t)head * kHeadDim + g * 8;
+            const uint32_t row = min(row0 + n, p.rows - 1u), token = row / p.pack;
+            const uint32_t head = row_head * p.pack + (row - token * p.pack);
+            const uint16_t *src = p.q + (uint64_t)token * p.q_stride + (uint64_t)head * kHeadDim + g * 8;
 #pragma unroll
             for (int kk = 0; kk < kSteps; ++kk) q[kk] = as_bf16x8(load_b128(src + kk * 16));
+            visible = (p.causal ? min((int32_t)(p.query_start + token), (int32_t)p.kv_tokens - 1)
+                                : (int32_t)p.kv_tokens - 1) - first_key;
         }
 
         // ---- tile staging: buffer loads that write LDS directly -----------------------
@@ -235,10 +251,10 @@ struct Prefill {
         // (rows of 128 bytes: eight rows per load, of 512 bytes: two).
         k_row_bytes = (uint32_t)p.k_stride * 2u;
         v_row_bytes = (uint32_t)p.v_stride * 2u;
-        k_rsrc = raw_buffer(p.k + (uint64_t)kv_head * kHeadDim,
-                            p.kv_tokens * k_row_bytes - kv_head * kRowBytes);
-        v_rsrc = raw_buffer(p.v + (uint64_t)kv_head * kHeadDim,
-                            p.kv_tokens * v_row_bytes - kv_head * kRowBytes);
+        k_rsrc = raw_buffer(p.k + (uint64_t)(uint32_t)first_key * p.k_stride + (uint64_t)kv_head * kHeadDim,
+                            (uint32_t)key_count * k_row_bytes - kv_head * kRowBytes);
+        v_rsrc = raw_buffer(p.v + (uint64_t)(uint32_t)first_key * p.v_stride + (uint64_t)kv_head * kHeadDim,
+                            (uint32_t)key_count * v_row_bytes - kv_head * kRowBytes);
         lds_base = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address_of(lds));
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) {
@@ -276,16 +292,20 @@ struct Prefill {
         neg_m = 0.f;
         l_run = 0.f;
 
-        // rows of this wave at or past query_tokens do no work but still help staging
-        const bool wave_active = row0 < p.query_tokens;
-        // last key visible to the wave's first / last row (causal)
-        const uint32_t wave_first_vis = p.causal ? p.query_start + row0 : p.kv_tokens - 1u;
-        const uint32_t wave_last_vis =
-            p.causal ? p.query_start + min(row0 + kRowsPerWave, p.query_tokens) - 1u : p.kv_tokens - 1u;
+        // a wave whose rows are all past the end does no work but still helps staging
+        const bool wave_active = row0 < p.rows;
+        // last key visible to the wave's first / last row
+        const int32_t wave_first_vis =
+            p.causal ? (int32_t)(p.query_start + row0 / p.pack) - first_key : key_count - 1;
+        const int32_t wave_last_vis =
+            p.causal ? (int32_t)(p.query_start + (min(row0 + kRowsPerWave, p.rows) - 1u) / p.pack) - first_key
+                     : key_count - 1;
         // tiles this wave computes with: those that hold a key one of its rows sees
-        const uint32_t my_tiles = wave_active ? min(tiles, wave_last_vis / kKeyTile + 1u) : 0u;
+        const uint32_t my_tiles =
+            wave_active && wave_last_vis >= 0 ? min(tiles, (uint32_t)wave_last_vis / kKeyTile + 1u) : 0u;
         auto needs_mask = [&](uint32_t tile) {
-            return tile * kKeyTile + kKeyTile - 1u > wave_first_vis || (tile + 1u) * kKeyTile > p.kv_tokens;
+            return (int32_t)(tile * kKeyTile + kKeyTile - 1u) > wave_first_vis ||
+                   (int32_t)((tile + 1u) * kKeyTile) > key_count;
         };
 
         // ---- prologue: K(0) and V(0) land, K(1) starts, S^T of tile 0 --------------------
@@ -411,15 +431,22 @@ struct Prefill {
         // nothing may still be in flight into LDS when the workgroup ends
         __builtin_amdgcn_s_waitcnt(0x0f70);
 
-        // ---- epilogue: normalise, publish bf16 rows and LSE -------------------------
         if (!wave_active) return;
-        const uint32_t row = row0 + n;
         float l = l_run;
         l += other_half(l);
-        const bool live = row < p.query_tokens;
+        if (partial) leave_partial((item - p.whole_items) * p.splits + split, l);
+        else publish(l);
+    }
+
+    // Normalises and publishes the bf16 rows and their LSE.
+    __device__ inline void publish(float l) const
+    {
+        const uint32_t row = row0 + n;
+        if (row >= p.rows) return;
+        const uint32_t token = row / p.pack, head = row_head * p.pack + (row - token * p.pack);
         const float inv = 1.0f / l;
         bool bad = false;
-        uint16_t *dst = p.out + ((uint64_t)row * p.query_heads + head) * kHeadDim;
+        uint16_t *dst = p.out + ((uint64_t)token * p.query_heads + head) * kHeadDim;
 #pragma unroll
         for (int db = 0; db < kDimBlocks; ++db)
 #pragma unroll
@@ -430,24 +457,43 @@ struct Prefill {
                 u32x2 w;
                 w.x = pack_bf16x2(a0, a1);
                 w.y = pack_bf16x2(a2, a3);
-                if (p.gate && live) {
+                if (p.gate) {
                     w = gate_four(w, p.gate + (dst - p.out) + db * 32 + grp * 8 + g * 4);
                     bad |= pair_not_finite(w.x) || pair_not_finite(w.y);
                 }
-                if (live) *reinterpret_cast<u32x2 *>(dst + db * 32 + grp * 8 + g * 4) = w;
+                *reinterpret_cast<u32x2 *>(dst + db * 32 + grp * 8 + g * 4) = w;
             }
-        if (live && bad) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
-        if (live && p.lse && g == 0)
-            p.lse[(uint64_t)row * p.query_heads + head] = (m_run + fast_log2(l)) * YVEX_LN2;
+        if (bad) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
+        if (p.lse && g == 0)
+            p.lse[(uint64_t)token * p.query_heads + head] = (m_run + fast_log2(l)) * YVEX_LN2;
+    }
+
+    // Leaves what this run of keys contributes to the wave's rows.
+    __device__ inline void leave_partial(uint32_t slot, float l) const
+    {
+        if (row0 + n >= p.rows) return;
+        const uint64_t at = (uint64_t)slot * kRowsPerBlock + wave * kRowsPerWave + n;
+        if (g == 0) {
+            p.part_ml[at * 2u] = m_run;
+            p.part_ml[at * 2u + 1u] = l;
+        }
+        if (m_run == -INFINITY) return;
+        float *acc = p.part_acc + at * kHeadDim + g * 4;
+#pragma unroll
+        for (int db = 0; db < kDimBlocks; ++db)
+#pragma unroll
+            for (int grp = 0; grp < 4; ++grp)
+                *reinterpret_cast<floatx4 *>(acc + db * 32 + grp * 8) =
+                    (floatx4){o[db][grp * 4], o[db][grp * 4 + 1], o[db][grp * 4 + 2], o[db][grp * 4 + 3]};
     }
 };
 
 }  // namespace
 
-// grid = query heads x query tiles of YVEX_ROCM_PREFILL_ROWS rows, block 256,
-// LDS 2 x (K + V) tiles.  `waves`: waves per SIMD the register budget is sized for: two
-// workgroups per CU for head_dim 64 and 128; head_dim 256 keeps 128 accumulator, 64 query and
-// 64 score registers per lane and its tiles fill 128 KB of LDS: one workgroup per CU.
+// grid = whole_items + tail_items * splits, block 256, LDS 2 x (K + V) tiles.  `waves`: waves per
+// SIMD the register budget is sized for: two workgroups per CU for head_dim 64 and 128; head_dim
+// 256 keeps 128 accumulator, 64 query and 64 score registers per lane and its tiles fill 128 KB
+// of LDS: one workgroup per CU.
 #define YVEX_PREFILL_KERNEL(name, head_dim, waves)                                                        \
     extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves, waves)))  \
     name(const yvex_rocm_prefill_params p)                                                                \
@@ -460,3 +506,73 @@ struct Prefill {
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128, 2)
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64, 2)
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_256, 256, 1)
+
+// Log-sum-exp merge of the runs of the split items and publication of their rows, in the order of
+// the runs.  head_dim / 4 threads per row, four lanes of the row each; grid = tail_items *
+// YVEX_ROCM_PREFILL_ROWS * head_dim / 4 / 256, block = 256.
+template <int kHeadDim>
+__device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p)
+{
+    constexpr uint32_t kThreads = kHeadDim / 4, kRows = 256u / kThreads;
+    constexpr int kWidth = 8;  // runs in flight per trip
+    const uint32_t packed = blockIdx.x * kRows + threadIdx.x / kThreads, d = (threadIdx.x % kThreads) * 4u;
+    const uint32_t tail = packed / kRowsPerBlock, in_tile = packed % kRowsPerBlock;
+    const uint32_t item = p.whole_items + tail;
+    const uint32_t row = (p.query_tiles - 1u - item / p.row_heads) * kRowsPerBlock + in_tile;
+    if (row >= p.rows) return;
+    const uint32_t token = row / p.pack, head = (item % p.row_heads) * p.pack + (row - token * p.pack);
+    const uint64_t first = (uint64_t)tail * p.splits * kRowsPerBlock + in_tile;
+    float top = -INFINITY, sum = 0.f;
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (uint32_t s0 = 0u; s0 < p.splits; s0 += (uint32_t)kWidth) {
+        float m[kWidth], l[kWidth];
+        floatx4 part[kWidth];
+#pragma unroll
+        for (int i = 0; i < kWidth; ++i) {
+            // runs past the end alias the last one, with weight zero
+            const uint64_t at = first + (uint64_t)min(s0 + (uint32_t)i, p.splits - 1u) * kRowsPerBlock;
+            m[i] = p.part_ml[at * 2u];
+            l[i] = p.part_ml[at * 2u + 1u];
+            part[i] = *reinterpret_cast<const floatx4 *>(p.part_acc + at * kHeadDim + d);
+        }
+        float m_new = top;
+#pragma unroll
+        for (int i = 0; i < kWidth; ++i) {
+            if (s0 + (uint32_t)i >= p.splits) m[i] = -INFINITY;
+            m_new = fmaxf(m_new, m[i]);
+        }
+        if (m_new == -INFINITY) continue;
+        const float keep = fast_exp2(top - m_new);
+        sum *= keep;
+        acc *= keep;
+#pragma unroll
+        for (int i = 0; i < kWidth; ++i) {
+            if (m[i] == -INFINITY) continue;  // nothing was left there
+            const float w = fast_exp2(m[i] - m_new);
+            sum += w * l[i];
+            acc += w * part[i];
+        }
+        top = m_new;
+    }
+    const uint64_t at = ((uint64_t)token * p.query_heads + head) * kHeadDim + d;
+    const float inv = 1.0f / sum;
+    bool bad = !(isfinite(acc[0] * inv) && isfinite(acc[1] * inv) && isfinite(acc[2] * inv) && isfinite(acc[3] * inv));
+    u32x2 w = {pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv)};
+    if (p.gate) {
+        w = gate_four(w, p.gate + at);
+        bad |= pair_not_finite(w.x) || pair_not_finite(w.y);
+    }
+    *reinterpret_cast<u32x2 *>(p.out + at) = w;
+    if (bad) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
+    if (p.lse && d == 0u) p.lse[(uint64_t)token * p.query_heads + head] = (top + fast_log2(sum)) * YVEX_LN2;
+}
+
+#define YVEX_PREFILL_MERGE_KERNEL(name, head_dim)                                                         \
+    extern "C" __global__ void __launch_bounds__(256) name(const yvex_rocm_prefill_params p)              \
+    {                                                                                                     \
+        prefill_merge<head_dim>(p);                                                                       \
+    }
+
+YVEX_PREFILL_MERGE_KERNEL(yvex_rocm_prefill_merge, 128)
+YVEX_PREFILL_MERGE_KERNEL(yvex_rocm_prefill_merge_64, 64)
+YVEX_PREFILL_MERGE_KERNEL(yvex_rocm_prefill_merge_256, 256)

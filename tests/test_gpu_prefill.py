@@ -176,3 +176,42 @@ def test_prefill_reference_qwen_patterns(backend, t, hq, hkv, d):
     assert_lse(lse, ref_lse, "qwen pattern d=%d" % d)
     again, lse2, _ = run_prefill(backend, q, k, v)
     assert np.array_equal(got, again) and np.array_equal(lse, lse2)
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("tq,tk,start,hq,hkv,causal,gated", [
+    (2, 700, 690, 8, 1, True, False),     # 16 packed rows: one wave of the tile has rows
+    (9, 4000, 3991, 10, 2, True, True),   # 45 rows, runs that end inside a tile
+    (33, 3001, 2960, 16, 4, False, False),
+    (26, 1500, 0, 5, 1, True, False),     # nothing to cut: the launch stays whole
+    (300, 5000, 4700, 6, 1, True, True),  # 15 items of 128 rows
+    (1300, 2600, 1300, 26, 2, True, False),  # 264 items: 256 walked whole, 8 cut
+])
+def test_prefill_packed_heads_and_cut_walks(backend, d, tq, tk, start, hq, hkv, causal, gated):
+    """The query heads of a kv head share the rows of a tile, and with a workspace attached the
+    walks that would leave compute units idle are cut into runs merged by a second launch: tails
+    of rows and keys, groups from 1 to 13, runs no row of a wave sees, gate, LSE."""
+    rng = np.random.default_rng(d + tq)
+    q, k, v = (bf16_normal(rng, shape) for shape in ((tq, hq, d), (tk, hkv, d), (tk, hkv, d)))
+    gate = bf16_normal(rng, q.shape) if gated else None
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, causal=causal, query_start=start, dtype=B.DTYPE_BF16,
+                                        contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+    need = backend.attention_workspace_required(req)
+    out, lse = backend.tensor("o", B.DTYPE_BF16, q.shape), backend.tensor("lse", B.DTYPE_F32, (tq, hq))
+    tensors = [backend.tensor(n, B.DTYPE_BF16, x.shape, x) for n, x in (("q", q), ("k", k), ("v", v))]
+    tg = backend.tensor("g", B.DTYPE_BF16, gate.shape, gate) if gated else None
+    work = backend.tensor("w", B.DTYPE_I8, (max(need, 256),))
+    backend.workspace_attach(work)
+    try:
+        facts = backend.attention_execute(req, *tensors, out, lse=lse, gate=tg)
+    finally:
+        backend.workspace_detach()
+    assert facts.kernel_launches == (2 if need else 1) and facts.temporary_bytes == need
+    assert need > 0 or tk <= 1500
+    rc, ref, _, ref_lse = ORACLE.gqa_bf16(q, k, v, query_start=start, causal=causal)
+    assert rc == 0
+    label = "cut d=%d tq=%d tk=%d" % (d, tq, tk)
+    if gated:
+        ref = ref / (1.0 + np.exp(-ORACLE.bf16_decode(gate).astype(np.float64)))
+    assert_close_bf16(out.read(), ref, label)
+    assert_lse(lse.read(), ref_lse, label)
