@@ -10,8 +10,9 @@
  * walked 188 steps on 40 units, 160 us; packed and cut into 256 runs, 20 us.  2000 tokens of 24/4
  * heads of 256 behind 13333: 376 items took two turns of 256 units with half of the second empty,
  * 1182 us; with its tail cut, 873.  A prompt of 2048 tokens without a history is not cut and gains
- * from the packing only that a tile spans 26 tokens instead of 128 (50.6 -> 50.2 us).  The cut is a function of the request's geometry only (256 units, never
- * the device), so that the planner's workspace_required and the execution agree. */
+ * from the packing only that a tile spans 26 tokens instead of 128 (50.6 -> 50.2 us).
+ * The cut is a function of the request's geometry only (256 units, never the device), so that the
+ * planner's workspace_required and the execution agree. */
 #include "rocm_state.h"
 
 #include <math.h>
