@@ -9,8 +9,9 @@
  * launch merges the runs.  Nine tokens of 40/8 heads of 128 behind 12001: one tile per query head
  * walked 188 steps on 40 units, 160 us; packed and cut into 256 runs, 20 us.  2000 tokens of 24/4
  * heads of 256 behind 13333: 376 items took two turns of 256 units with half of the second empty,
- * 1182 us; with its tail cut, 873.  A prompt of 2048 tokens without a history is not cut and gains
- * from the packing only that a tile spans 26 tokens instead of 128 (50.6 -> 50.2 us).
+ * 1182 us; with its tail cut, 873 (both with the kernel that prefill_pair.hip has replaced).  A
+ * prompt of 2048 tokens without a history is not cut and gains from the packing only that a tile
+ * spans 26 tokens instead of 128 (50.6 -> 50.2 us).
  * The cut is a function of the request's geometry only (256 units, never the device), so that the
  * planner's workspace_required and the execution agree. */
 #include "rocm_state.h"
@@ -55,7 +56,8 @@ static int prefill_plan_make(const yvex_transformer_attention_requirement *r, in
 {
     unsigned long long items, steps, splits, best, slots;
     memset(plan, 0, sizeof(*plan));
-    plan->pack = r->query_tokens > 1ull ? r->query_heads / r->key_value_heads : 1ull;
+    plan->pack = r->query_heads / r->key_value_heads;
+    if (r->query_tokens == 1ull || r->query_tokens * plan->pack >= YVEX_ROCM_PREFILL_PACKED_ROWS_MAX) plan->pack = 1ull;
     plan->row_heads = r->query_heads / plan->pack;
     if (!yvex_core_u64_mul(r->query_tokens, plan->pack, &plan->rows) || plan->rows > 0x7fffffffull) return 0;
     plan->query_tiles = (plan->rows + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
@@ -147,6 +149,7 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
     params.kv_heads = (uint32_t)r->key_value_heads;
     params.pack = (uint32_t)plan.pack;
     params.row_heads = (uint32_t)plan.row_heads;
+    params.pack_inverse = (uint32_t)((0xffffffffull + plan.pack) / plan.pack);
     params.causal = (uint32_t)g->causal;
     params.rows = (uint32_t)plan.rows;
     params.query_tiles = (uint32_t)plan.query_tiles;

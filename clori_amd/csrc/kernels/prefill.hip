@@ -1,7 +1,8 @@
 // Causal / full grouped-query attention prefill for gfx950 (wave64), bf16 in and out,
 // fp32 scores, online softmax and accumulation.  Token-major tensors ([token][head][dim],
-// per-token strides in elements); head_dim 128 is the tuned build, 64 and 256 are the same
-// code with other counts (the numbers in this comment are those of 128).
+// per-token strides in elements); head_dim 128 is the tuned build, 64 is the same code with other
+// counts (the numbers in this comment are those of 128), 256 has a kernel of its own
+// (prefill_pair.hip), merged by the merge at the end of this file.
 //
 // A workgroup of 4 waves owns one (query head, 128-row query tile): each wave owns
 // 32 query rows and walks the key/value tokens in tiles of 64 that the workgroup
@@ -50,6 +51,7 @@
 // kv head count is a multiple of the 8 XCDs, all users of one kv head share an L2.
 //
 #include "mfma.h"
+#include "prefill_rows.h"
 
 #include "../kernel_params.h"
 
@@ -64,7 +66,7 @@ constexpr int kDepth = 4;  // operand fetches in flight ahead of the MFMA that c
 typedef __attribute__((address_space(3))) short4v lds_short4;
 
 // Chunk swizzle of tile row r: the 16-byte chunk c of the row sits at chunk position c ^ x(r).
-// Rows of 256 and of 512 bytes all start in the same bank, x(r) permutes the 16 chunk
+// Rows of 256 bytes all start in the same bank, x(r) permutes the 16 chunk
 // positions of a 256-byte bank span by the row's low four bits (rows r..r+3 go four chunks
 // apart, which is what the transposed read needs; 16 consecutive rows take 16 different
 // positions, which is what the row read needs).  Rows of 128 bytes (head_dim 64) alternate
@@ -105,7 +107,7 @@ struct Prefill {
     static constexpr int kLoadRows = 64 / kRowChunks;         // tile rows one 1 KB load covers
     static constexpr int kSoftmaxSlots = 3 * kSlots / 4;      // the exponentials ride behind these slots
     static constexpr int kMaxPerSlot = 32 / (kSlots - kSoftmaxSlots);
-    static_assert(kHeadDim == 64 || kHeadDim == 128 || kHeadDim == 256, "head_dim 64, 128 or 256");
+    static_assert(kHeadDim == 64 || kHeadDim == 128, "head_dim 64 or 128");
 
     const yvex_rocm_prefill_params &p;
     unsigned char *const lds;
@@ -214,14 +216,14 @@ struct Prefill {
             split = (item - p.whole_items) / p.tail_items;
             item = p.whole_items + (item - p.whole_items) % p.tail_items;
         }
-        const uint32_t q_tile = p.query_tiles - 1u - item / p.row_heads;
-        row_head = item % p.row_heads;
-        kv_head = row_head * p.kv_heads / p.row_heads;
+        const uint32_t level = item / p.row_heads, q_tile = p.query_tiles - 1u - level;
+        row_head = item - level * p.row_heads;
+        kv_head = kv_head_of(p, row_head);
         row0 = q_tile * kRowsPerBlock + wave * kRowsPerWave;
 
         // keys visible to the last row of the workgroup bound the walk
         const uint32_t block_last_row = min(p.rows, (q_tile + 1u) * kRowsPerBlock) - 1u;
-        const uint32_t kv_end = p.causal ? min(p.kv_tokens, p.query_start + block_last_row / p.pack + 1u)
+        const uint32_t kv_end = p.causal ? min(p.kv_tokens, p.query_start + token_of(p, block_last_row) + 1u)
                                          : p.kv_tokens;
         uint32_t tiles = (kv_end + kKeyTile - 1) / kKeyTile;
         first_key = 0;
@@ -236,7 +238,7 @@ struct Prefill {
 
         // ---- Q fragments: B operand, lane (n, g) holds Q[row n][16*kk + 8g .. +7] ----
         {
-            const uint32_t row = min(row0 + n, p.rows - 1u), token = row / p.pack;
+            const uint32_t row = min(row0 + n, p.rows - 1u), token = token_of(p, row);
             const uint32_t head = row_head * p.pack + (row - token * p.pack);
             const uint16_t *src = p.q + (uint64_t)token * p.q_stride + (uint64_t)head * kHeadDim + g * 8;
 #pragma unroll
@@ -248,7 +250,7 @@ struct Prefill {
         // ---- tile staging: buffer loads that write LDS directly -----------------------
         // 1 KB load j of wave w fills rows 16w + 4j .. +3 of the tile; lane L owns chunk
         // position L % 16 of row 16w + 4j + L / 16 and fetches chunk (L % 16) ^ x(row)
-        // (rows of 128 bytes: eight rows per load, of 512 bytes: two).
+        // (rows of 128 bytes: eight rows per load).
         k_row_bytes = (uint32_t)p.k_stride * 2u;
         v_row_bytes = (uint32_t)p.v_stride * 2u;
         k_rsrc = raw_buffer(p.k + (uint64_t)(uint32_t)first_key * p.k_stride + (uint64_t)kv_head * kHeadDim,
@@ -296,9 +298,9 @@ struct Prefill {
         const bool wave_active = row0 < p.rows;
         // last key visible to the wave's first / last row
         const int32_t wave_first_vis =
-            p.causal ? (int32_t)(p.query_start + row0 / p.pack) - first_key : key_count - 1;
+            p.causal ? (int32_t)(p.query_start + token_of(p, row0)) - first_key : key_count - 1;
         const int32_t wave_last_vis =
-            p.causal ? (int32_t)(p.query_start + (min(row0 + kRowsPerWave, p.rows) - 1u) / p.pack) - first_key
+            p.causal ? (int32_t)(p.query_start + token_of(p, min(row0 + kRowsPerWave, p.rows) - 1u)) - first_key
                      : key_count - 1;
         // tiles this wave computes with: those that hold a key one of its rows sees
         const uint32_t my_tiles =
@@ -402,11 +404,8 @@ struct Prefill {
 #pragma unroll
                     for (int k4 = first; k4 < first + kMaxPerSlot; k4 += 4) {
                         const int mb = k4 >> 4, r = k4 & 15;
-                        if (kMaxPerSlot >= 4)
-                            mloc = fmaxf(fmaxf(mloc, s_next[mb][r]),
-                                         fmaxf(fmaxf(s_next[mb][r + 1], s_next[mb][r + 2]), s_next[mb][r + 3]));
-                        else
-                            mloc = fmaxf(mloc, fmaxf(s_next[mb][r], s_next[mb][r + 1]));
+                        mloc = fmaxf(fmaxf(mloc, s_next[mb][r]),
+                                     fmaxf(fmaxf(s_next[mb][r + 1], s_next[mb][r + 2]), s_next[mb][r + 3]));
                     }
                     asm volatile("" : "+v"(mloc));  // keeps this slice in its slot
                 }
@@ -443,7 +442,7 @@ struct Prefill {
     {
         const uint32_t row = row0 + n;
         if (row >= p.rows) return;
-        const uint32_t token = row / p.pack, head = row_head * p.pack + (row - token * p.pack);
+        const uint32_t token = token_of(p, row), head = row_head * p.pack + (row - token * p.pack);
         const float inv = 1.0f / l;
         bool bad = false;
         uint16_t *dst = p.out + ((uint64_t)token * p.query_heads + head) * kHeadDim;
@@ -490,12 +489,9 @@ struct Prefill {
 
 }  // namespace
 
-// grid = whole_items + tail_items * splits, block 256, LDS 2 x (K + V) tiles.  `waves`: waves per
-// SIMD the register budget is sized for: two workgroups per CU for head_dim 64 and 128; head_dim
-// 256 keeps 128 accumulator, 64 query and 64 score registers per lane and its tiles fill 128 KB
-// of LDS: one workgroup per CU.
-#define YVEX_PREFILL_KERNEL(name, head_dim, waves)                                                        \
-    extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves, waves)))  \
+// grid = whole_items + tail_items * splits, block 256, LDS 2 x (K + V) tiles; two workgroups per CU.
+#define YVEX_PREFILL_KERNEL(name, head_dim)                                                               \
+    extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))          \
     name(const yvex_rocm_prefill_params p)                                                                \
     {                                                                                                     \
         static_assert(YVEX_ROCM_PREFILL_ROWS == kRowsPerBlock, "host and kernel agree on the query tile"); \
@@ -503,9 +499,8 @@ struct Prefill {
         Prefill<head_dim>(p, lds).run();                                                                  \
     }
 
-YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128, 2)
-YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64, 2)
-YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_256, 256, 1)
+YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128)
+YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64)
 
 // Log-sum-exp merge of the runs of the split items and publication of their rows, in the order of
 // the runs.  head_dim / 4 threads per row, four lanes of the row each; grid = tail_items *
@@ -520,7 +515,7 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p)
     const uint32_t item = p.whole_items + tail;
     const uint32_t row = (p.query_tiles - 1u - item / p.row_heads) * kRowsPerBlock + in_tile;
     if (row >= p.rows) return;
-    const uint32_t token = row / p.pack, head = (item % p.row_heads) * p.pack + (row - token * p.pack);
+    const uint32_t token = token_of(p, row), head = (item % p.row_heads) * p.pack + (row - token * p.pack);
     const uint64_t first = (uint64_t)tail * p.splits * kRowsPerBlock + in_tile;
     float top = -INFINITY, sum = 0.f;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};

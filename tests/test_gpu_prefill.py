@@ -215,3 +215,40 @@ def test_prefill_packed_heads_and_cut_walks(backend, d, tq, tk, start, hq, hkv, 
         ref = ref / (1.0 + np.exp(-ORACLE.bf16_decode(gate).astype(np.float64)))
     assert_close_bf16(out.read(), ref, label)
     assert_lse(lse.read(), ref_lse, label)
+
+
+@pytest.mark.parametrize("tq,tk,start,hq,hkv,cut", [(70, 70, 0, 2, 1, False), (5, 1500, 1495, 12, 2, True),
+                                                    (200, 1000, 800, 4, 2, False)])
+def test_prefill_scores_far_above_the_first_tiles(backend, tq, tk, start, hq, hkv, cut):
+    """Scores whose weight exceeds the first 64 keys' by more than a float holds: the walk relative to
+    the first tile overflows and is done again with rescaling (head dimension 256).  Values of
+    half size: the softmax picks single rows, one bf16 step of which stays below the bar."""
+    rng = np.random.default_rng(tq)
+    d = 256
+    q = bf16_normal(rng, (tq, hq, d))
+    k = ORACLE.bf16_encode(rng.standard_normal((tk, hkv, d)).astype(np.float32) *
+                           np.where(np.arange(tk) < 64, 0.5, 48.0).astype(np.float32)[:, None, None])
+    v = bf16_normal(rng, (tk, hkv, d), 0.5)
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, causal=True, query_start=start, dtype=B.DTYPE_BF16,
+                                        contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+    out, lse = backend.tensor("o", B.DTYPE_BF16, q.shape), backend.tensor("lse", B.DTYPE_F32, (tq, hq))
+    tensors = [backend.tensor(n, B.DTYPE_BF16, x.shape, x) for n, x in (("q", q), ("k", k), ("v", v))]
+    work = backend.tensor("w", B.DTYPE_I8, (max(backend.attention_workspace_required(req), 256),))
+    if cut:
+        backend.workspace_attach(work)
+    try:
+        facts = backend.attention_execute(req, *tensors, out, lse=lse)
+    finally:
+        backend.workspace_detach()
+    assert facts.kernel_launches == (2 if cut else 1)
+    rc, ref, _, ref_lse = ORACLE.gqa_bf16(q, k, v, query_start=start, causal=True)
+    assert rc == 0 and ref_lse.max() > 100.0  # e^88.8 is the first weight a float does not hold
+    assert_close_bf16(out.read(), ref, "far above %d" % tq)
+    # an LSE of some hundreds: its float spacing is 3e-5, the scores' own rounding (256 products) more
+    assert np.abs(lse.read().astype(np.float64) - ref_lse).max() <= 1e-3
+    # what is not finite in the inputs is reported, not walked into silence
+    q[tq - 1, 0, 3] = 0x7F80
+    tensors[0].write(q)
+    with pytest.raises(YvexError) as e:
+        backend.attention_execute(req, *tensors, out)
+    assert e.value.code == B.YVEX_ERR_FORMAT
