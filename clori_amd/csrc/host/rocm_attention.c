@@ -1234,8 +1234,10 @@ static int rocm_mla_decode_execute(yvex_backend *backend,
             gp.row_elements = kp.key_dim;
             gp.max_rows = (uint32_t)r->max_compressed_tokens;
             rc = yvex_rocm_launch(backend, YVEX_ROCM_FN_GATHER_ROWS, variant,
-                                  (unsigned int)r->compressed_selected_stride, (unsigned int)r->batch,
-                                  1u, 128u, 0u, &gp, where, err);
+                                  (unsigned int)((r->compressed_selected_stride +
+                                                  YVEX_ROCM_GATHER_ENTRIES - 1ull) /
+                                                 YVEX_ROCM_GATHER_ENTRIES),
+                                  (unsigned int)r->batch, 1u, 256u, 0u, &gp, where, err);
             cp.pool = gp.rows;
             cp.page_table = gp.table;
             cp.pool_pages = (uint32_t)(r->batch * gather_pages);

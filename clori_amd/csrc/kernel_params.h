@@ -243,7 +243,9 @@ typedef struct {
 
 /* Gathers the selected compressed rows of every batch element into a contiguous paged pool
  * (batch * pages_each pages of page_tokens rows) and writes the identity page table for it.
- * grid = (selected_stride, batch), block = 128. */
+ * grid = (ceil(selected_stride / YVEX_ROCM_GATHER_ENTRIES), batch), block = 256; row_elements is
+ * 512 or 576. */
+#define YVEX_ROCM_GATHER_ENTRIES 16
 typedef struct {
     const uint16_t *pool;         /* [pool_pages][page_tokens][row_elements] */
     const int32_t *page_table;    /* [batch][table_stride] */

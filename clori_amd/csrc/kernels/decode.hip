@@ -1019,62 +1019,84 @@ yvex_rocm_decode_finish_256(const yvex_rocm_decode_params p)
 
 // Log-sum-exp merge of the chunk partials of one (session, query head): one wave per head,
 // eight output dims per lane (one 16-byte load of bf16 partials per chunk), four heads per
-// workgroup.  grid = (ceil(query_heads / 4), sessions), block = 256; head_dim = 512.
+// workgroup.  grid = (ceil(query_heads / 4), sessions), block = 256; head_dim = 512 (eight dims
+// in every lane).
 // kRope: the build that also turns the rope lanes of the published row back (its double
 // precision sine and cosine double the register use, so rows without a rotation keep their
-// own build).
+// own build).  Lane i takes the sine and cosine of pair i while the partials are on their way;
+// when each of the lanes that turn dims took those of its own four pairs after the merge, eight
+// evaluations stood at the end of every wave (32 x 64 rows over 11 chunks: 10.6 us, now 7.9 us).
 template <bool kRope>
 __device__ __forceinline__ void decode_merge_rows(const yvex_rocm_decode_merge_params &p)
 {
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t head = blockIdx.x * 4u + (threadIdx.x >> 6), session = blockIdx.y;
-    const uint32_t ctx = p.context ? (uint32_t)p.context[session] : p.fixed_context;
-    if (ctx == 0u || head >= p.query_heads || lane * 8u >= p.head_dim) return;
+    const uint32_t lane = threadIdx.x & 63u, session = blockIdx.y;
+    // one head per wave: its rows, statistics and sink are read through scalar addresses
+    const uint32_t head = blockIdx.x * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    if (head >= p.query_heads) return;
+    // Everything the wave needs beside the partials is asked for before anything is waited for
+    // (an absent tensor's load goes to one that is there): each was a trip to memory of its own,
+    // the sink's behind the merge.
+    const int32_t *extra_at = p.extra_context ? p.extra_context : p.context;
+    const float *sink_at = p.sinks ? p.sinks + head : p.part_ml;
+    const int64_t *position_at = p.positions ? p.positions + session : (const int64_t *)p.part_ml;
+    const uint32_t ctx = (uint32_t)p.context[session];
+    const uint32_t extra_loaded = (uint32_t)extra_at[session];
+    const float sink = *sink_at;
+    const uint64_t given = kRope ? (uint64_t)*position_at : 0u;
+    double frequency = kRope ? p.rope_frequency[lane] : 0.0;
+    const uint32_t extra_ctx = p.extra_context ? extra_loaded : 0u;
+    if (ctx == 0u) return;
     const uint32_t first_visible = p.window != 0u && ctx > p.window ? ctx - p.window : 0u;
     const uint32_t live = ctx - (first_visible & ~(p.window_align - 1u));
     const uint32_t own = min(p.max_chunks, (live + p.chunk_tokens - 1u) / p.chunk_tokens);
     // the chunks of a second candidate set follow the max_chunks slots of the first
-    const uint32_t extra_ctx = p.extra_context ? (uint32_t)p.extra_context[session] : 0u;
     const uint32_t extra = p.extra_context
         ? min(p.extra_max_chunks, (extra_ctx + p.extra_chunk_tokens - 1u) / p.extra_chunk_tokens) : 0u;
     const uint32_t chunks = own + extra, skip = p.max_chunks - own;
     const uint64_t base =
         ((uint64_t)session * (p.max_chunks + (p.extra_context ? p.extra_max_chunks : 0u))) * p.query_heads + head;
+    // Inverse rotation of the rope lanes (src/graph/core.c:499-507): the row is rounded to
+    // bf16, its last rope_dims lanes are turned back by the token position in adjacent pairs,
+    // in double as the reference does it (src/graph/numeric.c:935-947), and rounded again.  A
+    // lane's eight dims hold four whole pairs; rope_dims and head_dim are multiples of 8.
+    const uint64_t position = p.positions ? given : (uint64_t)(ctx - 1u);
+    double pair_cosine = 1.0, pair_sine = 0.0;
+    auto pair_angles = [&]() {
+        if (!kRope || lane * 2u >= p.rope_dims) return;
+        asm volatile("" : "+v"(frequency));  // here, behind the loads, and not ahead of them
+        const double angle = (double)position * frequency;
+        pair_cosine = cos(angle);
+        pair_sine = -sin(angle);
+    };
     float top, total, acc[8];
     merge_chunk_rows(
-        chunks,
-        [&](uint32_t c, float &m, float &l) {
+        chunks, lane,
+        [&](uint32_t c) {
             const uint64_t slot = base + (uint64_t)(c < own ? c : c + skip) * p.query_heads;
-            m = p.part_ml[slot * 2];
-            l = p.part_ml[slot * 2 + 1];
+            return load_b64(p.part_ml + slot * 2u);
         },
         [&](uint32_t c) {
             const uint64_t slot = base + (uint64_t)(c < own ? c : c + skip) * p.query_heads;
             return load_b128(p.part_acc + slot * p.head_dim + lane * 8u);
         },
-        top, total, acc);
+        pair_angles, top, total, acc);
     bool bad = false;
-    if (p.sinks) bad |= !merge_sink(p.sinks[head], top, total, acc);
+    if (p.sinks) bad |= !merge_sink(sink, top, total, acc);
     const float inv = 1.0f / total;
-    // Inverse rotation of the rope lanes (src/graph/core.c:499-507): the row is rounded to
-    // bf16, its last rope_dims lanes are turned back by the token position in adjacent pairs,
-    // in double as the reference does it (src/graph/numeric.c:935-947), and rounded again.  A
-    // lane's eight dims hold four whole pairs; rope_dims and head_dim are multiples of 8.
     const uint32_t rope_start = p.head_dim - p.rope_dims;
     const bool turn = kRope && p.rope_dims != 0u && lane * 8u >= rope_start;
-    const double position =
-        turn ? (p.positions ? (double)(uint64_t)p.positions[session] : (double)(ctx - 1u)) : 0.0;
     u32x4 out;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         float a = acc[2 * i] * inv, b = acc[2 * i + 1] * inv;
         bad |= !(isfinite(a) && isfinite(b));
+        // from the lane that holds the pair (any, where nothing turns: every lane takes part)
+        const int pair = (int)((lane * 8u - rope_start) / 2u) + i;
+        const double c = kRope ? __shfl(pair_cosine, pair, 64) : 1.0, s = kRope ? __shfl(pair_sine, pair, 64) : 0.0;
         if (kRope && turn) {
             // products and sums rounded one by one, as the C reference computes them
             // (src/graph/numeric.c:935-947 is built without contraction)
 #pragma clang fp contract(off)
-            const double angle = position * p.rope_frequency[(lane * 8u - rope_start) / 2u + (uint32_t)i];
-            const double c = cos(angle), s = -sin(angle);
             const double x = (double)bf16_to_f32(bf16_bits(a)), y = (double)bf16_to_f32(bf16_bits(b));
             a = (float)(x * c - y * s);
             b = (float)(x * s + y * c);
