@@ -44,7 +44,8 @@ constexpr int kHeadDim = 128;
 constexpr int kPageTokens = 16;
 constexpr int kWaves = YVEX_ROCM_KV_APPEND_HEADS;
 constexpr int kRowPitch = kHeadDim + 8;       // bf16 elements per LDS row (272 bytes)
-constexpr int kCodePitch = kHeadDim + 16;     // bytes per LDS row of value codes
+
+typedef __attribute__((address_space(4))) const int32_t constant_i32;
 
 __device__ inline void flag(int32_t *status, int code) { atomicCAS(status, 0, code); }
 
@@ -105,8 +106,10 @@ __device__ inline Span locate(const yvex_rocm_kv_append_params &p)
     }
     const uint32_t page = first_page + slot;
     if (page > last_page) return s;
-    // `page` counts 16-token blocks; a pool page holds 1 << page_shift of them
-    const int32_t id = p.page_table[(uint64_t)session * p.table_stride + (page >> p.page_shift)];
+    // `page` counts 16-token blocks; a pool page holds 1 << page_shift of them.  Nothing writes the
+    // table while the kernel runs, and the address is the same in all lanes: a scalar load.
+    constant_i32 *table = (constant_i32 *)(p.page_table + (uint64_t)session * p.table_stride);
+    const int32_t id = table[page >> p.page_shift];
     if (id < 0 || (uint32_t)id >= p.pool_pages) {
         if (threadIdx.x == 0) flag(p.status, YVEX_ROCM_DEVICE_CONTRACT);
         return s;
@@ -302,51 +305,96 @@ YVEX_KV_APPEND_BF16_KERNEL(yvex_rocm_kv_append_bf16_256, 256)
 
 namespace {
 
-// Q8_0 block of 32 values: f16 scale bits and 32 codes packed four to a word.
-__device__ inline bool quantise(const float (&x)[32], uint16_t &scale_bits, uint32_t (&codes)[8])
+typedef unsigned short ushort2v __attribute__((ext_vector_type(2)));
+
+// Q8_0 block of 32 bf16 values (16 packed words): f16 scale bits and 32 codes packed four to a
+// word.  Works on magnitudes: the sign of a code is put on four at a time at the end, and the
+// largest magnitude is that of the bf16 bits as integers, two per instruction, which also finds
+// infinities and NaN (their bits are the largest).  Returns false when a value is not finite or
+// f16 cannot hold the scale.
+__device__ inline bool quantise(const u32x4 (&x)[4], uint16_t &scale_bits, uint32_t (&codes)[8])
 {
 #pragma clang fp contract(off)   // the product is rounded before the rounding add, as in the reference
-    float maximum = 0.f;
+    ushort2v most = {0, 0};
 #pragma unroll
-    for (int e = 0; e < 32; ++e) maximum = fmaxf(maximum, fabsf(x[e]));
+    for (int w = 0; w < 16; ++w)
+        most = __builtin_elementwise_max(most, __builtin_bit_cast(ushort2v, x[w >> 2][w & 3] & 0x7fff7fffu));
+    const uint32_t largest = max((uint32_t)most.x, (uint32_t)most.y);
+    const float maximum = __builtin_bit_cast(float, largest << 16);
     const _Float16 half = (_Float16)(maximum / 127.0f);
     const float scale = (float)half;
     const float inverse = scale != 0.f ? 1.0f / scale : 0.f;
     scale_bits = __builtin_bit_cast(uint16_t, half);
-    // roundf (half away from zero) as a truncating convert of x + copysign(0.5 - 2^-25, x):
-    // exact for |x| < 2^23 (ties land on or above the next integer, the value just below a
-    // tie stays below it), then the clamp on the integer
+    // roundf (half away from zero) of a magnitude as a truncating convert of x + (0.5 - 2^-25):
+    // exact for x < 2^23 (ties land on or above the next integer, the value just below a tie
+    // stays below it); the clamp may come first, as 127 is whole
     const float nudge = __builtin_bit_cast(float, 0x3effffffu);
 #pragma unroll
     for (int w = 0; w < 8; ++w) {
+        const uint32_t pair[2] = {x[w >> 1][(2 * w) & 3], x[w >> 1][(2 * w + 1) & 3]};
         uint32_t word = 0u;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            const float scaled = x[4 * w + e] * inverse;
-            const int code = min(max((int)(scaled + copysignf(nudge, scaled)), -127), 127);
-            word |= ((uint32_t)code & 0xffu) << (8 * e);
+            const float value = (e & 1) ? high_half(pair[e >> 1]) : low_half(pair[e >> 1]);
+            const float scaled = fabsf(value * inverse);
+            word |= (uint32_t)fminf(scaled + nudge, 127.0f) << (8 * e);
         }
-        codes[w] = word;
+        // bytes 1 and 3 of either word hold the signs: all ones where a value is negative
+        const uint32_t negative = __builtin_amdgcn_perm(pair[1], pair[0], 0x0b0a0908u);
+        // 256 - code per byte, without borrows: 128 - code is at least 1
+        const uint32_t opposite = (0x80808080u - word) ^ 0x80808080u;
+        codes[w] = (word & ~negative) | (opposite & negative);
     }
-    return isfinite(scale) && !(maximum > 0.f && scale == 0.f);
+    return largest < 0x7f80u && isfinite(scale) && !(maximum > 0.f && scale == 0.f);
 }
+
+// The four lanes of a quad hold four bytes each; lane r is left with byte r of all four, the
+// byte of lane q in position q.
+__device__ inline uint32_t transposed_quad(uint32_t v, uint32_t select1, uint32_t select2)
+{
+    const uint32_t next = (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, true);  // quad_perm 1,0,3,2
+    const uint32_t pairs = __builtin_amdgcn_perm(next, v, select1);
+    const uint32_t other = (uint32_t)__builtin_amdgcn_mov_dpp((int)pairs, 0x4e, 0xf, 0xf, true);  // 2,3,0,1
+    return __builtin_amdgcn_perm(other, pairs, select2);
+}
+
+// What one wave of the Q8_0 writer keeps in LDS: bf16 rows on the way in (272-byte pitch), then,
+// over the value rows, the value codes as the block holds them with 64 bytes behind every 256.
+struct Q8Scratch {
+    uint16_t k_rows[kPageTokens][kRowPitch];
+    uint16_t v_rows[kPageTokens][kRowPitch];
+};
+constexpr uint32_t kCodeGroupPitch = 256 + 64, kCodeHalfPitch = 4 * kCodeGroupPitch;
+static_assert(2 * kCodeHalfPitch <= sizeof(uint16_t) * kPageTokens * kRowPitch, "codes fit the value rows");
+
+// A wave reads what its own lanes wrote: LDS takes a wave's instructions in order, so nothing has
+// to be waited for, but the compiler must keep the order.
+__device__ inline void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 
 }  // namespace
 
-// grid and waves as above.  After the rotary, lane (t = lane / 4, j = lane % 4) owns the 32
-// dims of Q8_0 block j of token t.
+// grid and waves as above; waves share nothing.  Lane (tg = lane / 16, j = lane / 4 % 4, r = lane
+// % 4) owns the 32 dims of Q8_0 block j of token 4 tg + r, so that a quad holds four tokens of
+// the same dims, which are one word of the value codes.
+//
+// Bound by memory: 16 sessions, 34000 new tokens of 8 heads at unaligned starts, 46.6 us for the
+// 215 MB (4.6 TB/s; a copy reaches 5.1).  It took 63.3 us when what a wave issues (1180 vector
+// instructions, half the time) and its three trips to memory at three waves per SIMD were the
+// bound: loads of pieces from 16 or 64 different rows at a time, where now whole 128- and 256-byte
+// stretches are fetched and re-laid in LDS; value codes gathered byte by byte from LDS, where now
+// the lanes of a quad transpose them and leave two 16-byte stores each; codes rounded, clamped and
+// packed with their signs one by one.  104 registers and 34 KB per workgroup: four waves per SIMD.
 extern "C" __global__ void __launch_bounds__(64 * kWaves)
 yvex_rocm_kv_append_q8_0(const yvex_rocm_kv_append_params p)
 {
-    __shared__ __attribute__((aligned(16))) uint16_t k_rows_all[kWaves][kPageTokens][kRowPitch];
-    __shared__ __attribute__((aligned(16))) unsigned char v_codes_all[kWaves][kPageTokens][kCodePitch];
+    __shared__ __attribute__((aligned(16))) Q8Scratch scratch[kWaves];
     const Span s = locate(p);
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t head = blockIdx.y * kWaves + wave;
-    const bool active = s.valid && head < p.kv_heads;
-    uint16_t (*k_rows)[kRowPitch] = k_rows_all[wave];
-    unsigned char (*v_codes)[kCodePitch] = v_codes_all[wave];
-    const uint32_t t = lane >> 2, j = lane & 3u;
+    if (!s.valid || head >= p.kv_heads) return;
+    uint16_t (*k_rows)[kRowPitch] = scratch[wave].k_rows, (*v_rows)[kRowPitch] = scratch[wave].v_rows;
+    unsigned char *image = (unsigned char *)v_rows;
+    const uint32_t r = lane & 3u, j = (lane >> 2) & 3u, tg = lane >> 4, t = 4u * tg + r;
     constexpr uint32_t kCodeBytes = kPageTokens * kHeadDim;
     constexpr uint32_t kBlockBytes = kCodeBytes + kPageTokens * 4 * 2;
     const uint64_t block = ((((uint64_t)s.page_id * p.kv_heads + head) << p.page_shift) + s.sub) *
@@ -354,97 +402,120 @@ yvex_rocm_kv_append_q8_0(const yvex_rocm_kv_append_params p)
     unsigned char *kdst = (unsigned char *)p.k_pool + block, *vdst = (unsigned char *)p.v_pool + block;
     const bool partial = s.lo != 0u || s.hi != (uint32_t)kPageTokens;
     const bool mine = t >= s.lo && t < s.hi;
-    const uint32_t pairs = p.rotary_dim / 16u;
-    bool ok = true, representable = true;
-    KeyChunk k[4];
-    u32x4 v[4];
-    uint32_t old[8] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
-    if (active) {
+
+    // Every load of the wave.  Keys: the chunks of the lower rotary halves in row order, each with
+    // its partner, then the chunks behind the rotary lanes.
+    const uint32_t pairs = p.rotary_dim / 16u, rest = 16u - 2u * pairs;
+    const uint32_t lower_chunks = kPageTokens * pairs, plain_chunks = kPageTokens * rest;
+    const uint32_t row_stride = p.kv_heads * kHeadDim;
+    const uint16_t *keys = p.key + ((uint64_t)s.row * p.kv_heads + head) * kHeadDim;
+    const uint16_t *values = p.value + ((uint64_t)s.row * p.kv_heads + head) * kHeadDim;
+    // rows of the span: outside tokens read the nearest one (loaded and dropped)
+    auto span_row = [&](uint32_t token) { return min(max(token, s.lo), s.hi - 1u) - s.lo; };
+    // quotients of piece numbers (below 256) by the chunks of a row, as a multiplication
+    const uint32_t pairs_inverse = pairs != 0u ? 65536u / pairs + 1u : 0u;
+    KeyChunk k[2];
+    u32x4 v[4], old[2] = {};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) key_issue(p, s, head, lane + 64u * i, k[i]);
-        {
-            const uint16_t *src = p.value + ((uint64_t)row_of(s, t) * p.kv_heads + head) * kHeadDim + 32u * j;
+    for (int i = 0; i < 2; ++i) {
+        if (64u * i >= lower_chunks) continue;
+        // lanes past the end repeat the last chunk
+        const uint32_t id = min(lane + 64u * i, lower_chunks - 1u);
+        k[i].t = id * pairs_inverse >> 16;
+        k[i].c8 = id - k[i].t * pairs;
+        k[i].role = kLower;
+        const uint32_t row = span_row(k[i].t);
+        const uint16_t *base = keys + (uint64_t)row * row_stride + k[i].c8 * 8u;
+        const uint64_t at = (uint64_t)(s.row + row) * p.rotary_dim + k[i].c8 * 8u;
+        k[i].own = load_b128(base);
+        k[i].other = load_b128(base + p.rotary_dim / 2u);
+        k[i].cs[0] = load_b128(p.cosine + at);
+        k[i].cs[1] = load_b128(p.cosine + at + 4);
+        k[i].sn[0] = load_b128(p.sine + at);
+        k[i].sn[1] = load_b128(p.sine + at + 4);
+    }
 #pragma unroll
-            for (int g = 0; g < 4; ++g) v[g] = load_b128(src + 8 * g);
-        }
-        if (partial) {
+    for (int i = 0; i < 4; ++i)
+        v[i] = load_b128(values + (uint64_t)span_row(4u * i + tg) * row_stride + (lane & 15u) * 8u);
+    if (partial) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i)
-                old[i] = *reinterpret_cast<const uint32_t *>(vdst + YVEX_ROCM_Q8_CODE_OFFSET((lane + 64u * i) * 4u));
-        }
-        // rotated key rows into LDS
+        for (int i = 0; i < 2; ++i) old[i] = load_b128(vdst + 1024u * i + 16u * lane);
+    }
+
+    if (plain_chunks != 0u) {
+        const uint32_t rest_inverse = 65536u / rest + 1u;
+        u32x4 plain[4];
+        uint32_t at[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            u32x4 lower, upper;
-            ok &= key_finish(k[i], lower, upper, p.rotary_mode != 0u) || k[i].t < s.lo || k[i].t >= s.hi;
-            if (k[i].role != kUpper)
-                *reinterpret_cast<u32x4 *>(&k_rows[k[i].t][k[i].c8 * 8u]) = lower;
-            if (k[i].role == kLower)
-                *reinterpret_cast<u32x4 *>(&k_rows[k[i].t][(k[i].c8 + pairs) * 8u]) = upper;
+            const uint32_t id = min(lane + 64u * i, plain_chunks - 1u), token = id * rest_inverse >> 16;
+            const uint32_t c8 = 2u * pairs + id - token * rest;
+            at[i] = token * kRowPitch + c8 * 8u;
+            plain[i] = load_b128(keys + (uint64_t)span_row(token) * row_stride + c8 * 8u);
         }
-        // values: quantise this lane's block, codes into LDS, scale straight to the pool
-        if (mine) {
-            float x[32];
-            uint32_t codes[8];
-            uint16_t scale_bits;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                ok &= finite_bits(v[g]);
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4 *>(&k_rows[0][0] + at[i]) = plain[i];
+    }
+    // rows into LDS, the keys rotated
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[8 * g + e] = bf16_of(v[g], e);
-            }
-            representable &= quantise(x, scale_bits, codes);
-            *reinterpret_cast<uint16_t *>(vdst + kCodeBytes + (t * 4u + j) * 2u) = scale_bits;
+    for (int i = 0; i < 2; ++i) {
+        if (64u * i >= lower_chunks) continue;
+        u32x4 lower, upper;
+        key_finish(k[i], lower, upper, p.rotary_mode != 0u);
+        *reinterpret_cast<u32x4 *>(&k_rows[k[i].t][k[i].c8 * 8u]) = lower;
+        *reinterpret_cast<u32x4 *>(&k_rows[k[i].t][(k[i].c8 + pairs) * 8u]) = upper;
+    }
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x2 w = {codes[2 * g], codes[2 * g + 1]};
-                *reinterpret_cast<u32x2 *>(&v_codes[t][32u * j + 8u * g]) = w;
-            }
+    for (int i = 0; i < 4; ++i) *reinterpret_cast<u32x4 *>(&v_rows[4u * i + tg][(lane & 15u) * 8u]) = v[i];
+    wave_lds_order();
+
+    bool ok = true;  // of the new tokens: finite, with a scale that f16 holds (src/gguf/quant_block.c:172-174)
+    u32x4 x[4];
+    uint32_t codes[8];
+    uint16_t scale_bits;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) x[g] = *reinterpret_cast<const u32x4 *>(&k_rows[t][32u * j + 8u * g]);
+    ok &= quantise(x, scale_bits, codes) || !mine;
+    if (mine) {
+        *reinterpret_cast<uint16_t *>(kdst + kCodeBytes + (t * 4u + j) * 2u) = scale_bits;
+        // key codes: 8-byte groups, bytes 8j .. 8j+7 of the 32 that lane 16g + t of a reading
+        // wave consumes (dims 32j + 8g + e)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const u32x2 w = {codes[2 * g], codes[2 * g + 1]};
+            *reinterpret_cast<u32x2 *>(kdst + YVEX_ROCM_Q8_CODE_OFFSET(((g * 16u + t) * 4u + j) * 8u)) = w;
         }
     }
-    __syncthreads();
-    if (active) {
-        if (mine) {
-            float x[32];
-            uint32_t codes[8];
-            uint16_t scale_bits;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x4 w = *reinterpret_cast<const u32x4 *>(&k_rows[t][32u * j + 8u * g]);
+    for (int g = 0; g < 4; ++g) x[g] = *reinterpret_cast<const u32x4 *>(&v_rows[t][32u * j + 8u * g]);
+    ok &= quantise(x, scale_bits, codes) || !mine;
+    if (mine) *reinterpret_cast<uint16_t *>(vdst + kCodeBytes + (t * 4u + j) * 2u) = scale_bits;
+    wave_lds_order();  // the codes go where the value rows were
+    // value codes: word (tg, m, b) holds 4 tokens of dim 16b + m, bytes 4b .. 4b+3 of the 32 that
+    // lane 16 tg + m of a reading wave consumes; lane r of a quad has dim 32j + 4w + r of them
+    const uint32_t select1 = (r & 1u) ? 0x03070105u : 0x06020400u, select2 = (r & 2u) ? 0x03020706u : 0x05040100u;
+    unsigned char *corner = image + (j >> 1) * kCodeHalfPitch + tg * kCodeGroupPitch + r * 16u + (j & 1u) * 8u;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) x[8 * g + e] = bf16_of(w, e);
-            }
-            representable &= quantise(x, scale_bits, codes);
-            *reinterpret_cast<uint16_t *>(kdst + kCodeBytes + (t * 4u + j) * 2u) = scale_bits;
-            // key codes: 8-byte groups, bytes 8j .. 8j+7 of the 32 that lane 16g + t of a reading
-            // wave consumes (dims 32j + 8g + e)
+    for (int w = 0; w < 8; ++w)
+        *reinterpret_cast<uint32_t *>(corner + (w & 3) * 64 + (w >> 2) * 4) =
+            transposed_quad(codes[w], select1, select2);
+    wave_lds_order();
+    if (4u * tg < s.hi && 4u * tg + 4u > s.lo) {
+        uint32_t fresh = 0xffffffffu;  // bytes of the new tokens among the four of the group
+        if (partial) {
+            fresh = 0u;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const u32x2 w = {codes[2 * g], codes[2 * g + 1]};
-                *reinterpret_cast<u32x2 *>(kdst + YVEX_ROCM_Q8_CODE_OFFSET(((g * 16u + t) * 4u + j) * 8u)) = w;
-            }
+            for (uint32_t q = 0; q < 4u; ++q)
+                if (4u * tg + q >= s.lo && 4u * tg + q < s.hi) fresh |= 0xffu << (8u * q);
         }
-        // value codes: 4-byte groups (4 tokens of one dim), bytes 4b .. 4b+3 of the 32 that lane
-        // 16 tg + m of a reading wave consumes, c = 16b + m
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const uint32_t id = lane + 64u * i;  // 512 groups = tg (4) x m (16) x b (8)
-            const uint32_t b = id & 7u, m = (id >> 3) & 15u, tg = id >> 7, c = 16u * b + m;
-            if (4u * tg + 4u <= s.lo || 4u * tg >= s.hi) continue;
-            uint32_t w = 0u;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t tt = 4u * tg + q;
-                const bool fresh = tt >= s.lo && tt < s.hi;
-                const uint32_t byte = fresh ? (uint32_t)v_codes[tt][c] : (old[i] >> (8 * q)) & 0xffu;
-                w |= byte << (8 * q);
-            }
-            *reinterpret_cast<uint32_t *>(vdst + YVEX_ROCM_Q8_CODE_OFFSET(id * 4u)) = w;
+        for (int i = 0; i < 2; ++i) {
+            const u32x4 now = *reinterpret_cast<const u32x4 *>(
+                image + i * kCodeHalfPitch + tg * kCodeGroupPitch + (lane & 15u) * 16u);
+            *reinterpret_cast<u32x4 *>(vdst + 1024u * i + 16u * lane) = (now & fresh) | (old[i] & ~fresh);
         }
-        // a block whose scale f16 cannot hold is refused like a non-finite value, as the
-        // reference encoder refuses it (src/gguf/quant_block.c:172-174)
-        if (!ok || !representable) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
     }
+    if (!ok) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
 }
 
 // Token-major history writer: the reference appends the new tokens to a layer's history with

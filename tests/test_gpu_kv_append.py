@@ -348,3 +348,47 @@ def test_append_bf16_pages_at_other_head_dimensions(backend, d, rotary_dim, rota
     assert_lse(lse.read(), ref_lse, "decode over appended pages d=%d" % d)
     for x in list(t.values()) + [tq, tc, out, lse]:
         x.release()
+
+
+@pytest.mark.parametrize("rotary_dim", [16, 48, 80, 96, 112])
+def test_q8_append_at_every_number_of_rotary_chunks(backend, rotary_dim):
+    """The Q8_0 writer deals rows to lanes by the chunks of the rotary halves and of the lanes
+    behind them: counts that do not divide 64, in both rotary orders, partly covered pages."""
+    for mode in (B.ROTARY_BF16_STAGED, B.ROTARY_F32_ROUNDED):
+        rng = np.random.default_rng(41 + rotary_dim)
+        t, got, want, _, _ = run_case(backend, rng, [0, 13, 30, 18], [16, 9, 5, 61], B.KV_Q8_0, rotary_dim,
+                                      "filled", rotary_mode=mode)
+        assert np.array_equal(got[0].reshape(want[0].shape), want[0])
+        assert np.array_equal(got[1].reshape(want[1].shape), want[1])
+        for x in t.values():
+            x.release()
+
+
+def test_q8_append_over_the_range_of_scales(backend):
+    """Blocks from the smallest scales f16 holds (subnormal, where codes reach the clamp at 127)
+    to the largest, both signs: byte-exact against the host encoder."""
+    rng = np.random.default_rng(47)
+    tokens = 200
+    exponents = rng.uniform(-16.5, 22.5, (tokens, HKV, D // 32, 1))
+    rows = (rng.uniform(-1.0, 1.0, (tokens, HKV, D // 32, 32)) * 2.0 ** exponents).astype(np.float32)
+    rows[rng.random(rows.shape[:3]) < 0.1] = -0.0
+    new = ORACLE.bf16_encode(rows.reshape(tokens, HKV, D))
+    pages = (tokens + 7 + PAGE - 1) // PAGE
+    table = rng.permutation(pages).astype(np.int32)[None]
+    tensors = [backend.tensor("k", B.DTYPE_BF16, new.shape, new),
+               backend.tensor("v", B.DTYPE_BF16, new.shape, new[::-1].copy()),
+               backend.tensor("r", B.DTYPE_I32, (1,), np.array([0], np.int32)),
+               backend.tensor("s", B.DTYPE_I32, (1,), np.array([7], np.int32)),
+               backend.tensor("c", B.DTYPE_I32, (1,), np.array([tokens], np.int32)),
+               backend.tensor("t", B.DTYPE_I32, table.shape, table)]
+    pools = [backend.tensor(n, B.DTYPE_I8, (pages * HKV * 2176,)) for n in ("kp", "vp")]
+    for pool in pools:
+        pool.zero()
+    backend.kv_append_execute(*tensors, *pools, HKV, pages, tokens, storage=B.KV_Q8_0)
+    encoded = q8_0_encode_rows(ORACLE.bf16_decode(new)).reshape(tokens, HKV, -1)
+    for pool, transposed, want in ((pools[0], False, encoded), (pools[1], True, encoded[::-1])):
+        got = kv_unpack_pages(pool.read(np.uint8, (-1,)), B.KV_Q8_0, transposed, pages, HKV)
+        got = got.reshape(pages, PAGE, HKV, -1)[table[0]].reshape(pages * PAGE, HKV, -1)
+        assert np.array_equal(got[7:7 + tokens], want)
+    for x in tensors + pools:
+        x.release()
