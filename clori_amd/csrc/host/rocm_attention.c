@@ -137,7 +137,11 @@ static int decode_workspace_bytes(unsigned long long slots, unsigned long long h
 
 /* A launch that fills the device merges its split segments with a second kernel; a smaller
  * one is bound by launch latency and merges inside the decode kernel (arrival counters). */
-static int decode_merges_in_kernel(unsigned int waves) { return waves < ROCM_DECODE_WAVES; }
+static int decode_merges_in_kernel(unsigned int waves, unsigned long long head_dim)
+{
+    /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
+    return waves < ROCM_DECODE_WAVES && head_dim == ROCM_MFMA_HEAD_DIM;
+}
 
 /* Waves of a team: eight, two per SIMD; four at head dimension 256, whose tiles and
  * accumulators take twice the registers. */
@@ -179,7 +183,7 @@ static int balanced_workspace_bytes(unsigned long long waves, unsigned long long
 {
     unsigned long long parts = 0ull, offsets;
     if (!decode_workspace_bytes(2ull * waves, group, head_dim, sizeof(float), acc_bytes, &parts)) return 0;
-    offsets = decode_merges_in_kernel((unsigned int)waves)
+    offsets = decode_merges_in_kernel((unsigned int)waves, head_dim)
                   ? 0ull : align_up((sessions + 1ull) * sizeof(uint32_t), ROCM_WORK_ALIGNMENT);
     *ml_bytes = parts - *acc_bytes;
     return yvex_core_u64_add(parts, offsets, total);
@@ -200,7 +204,6 @@ typedef struct {
     /* when set, the partials live here (nothing is acquired or released) */
     void *fixed_work;
     unsigned long long fixed_work_bytes;
-    int two_launches; /* the function has no build that merges in the kernel */
 } decode_job;
 
 /* Launches the decode kernel, the finish (merge) kernel when the launch fills the device, and
@@ -215,7 +218,7 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
     const unsigned int waves = decode_wave_count(job->sessions, job->kv_heads, job->max_context);
     const unsigned int teams = decode_team_count(job->page_table != NULL, group, job->head_dim,
                                                  job->max_context);
-    const int in_kernel = !job->two_launches && (teams || decode_merges_in_kernel(waves));
+    const int in_kernel = teams || decode_merges_in_kernel(waves, job->head_dim);
     void *work = NULL;
     yvex_error cleanup;
     int owned = 0, rc, cleanup_rc;
@@ -853,10 +856,8 @@ static int paged_decode_execute_common(yvex_backend *backend,
                       "tensors of this backend with the declared geometry");
     memset(&job, 0, sizeof(job));
     if (r->kv_storage == YVEX_ROCM_KV_BF16 && r->head_dimension != ROCM_MFMA_HEAD_DIM) {
-        /* the other head dimensions have the two-launch form only */
         job.function = r->head_dimension == 64ull ? YVEX_ROCM_FN_DECODE_PAGED_BF16_64
                                                   : YVEX_ROCM_FN_DECODE_PAGED_BF16_256;
-        job.two_launches = 1;
         job.variant = YVEX_BACKEND_VARIANT_ROCM_ATTENTION_PAGED_BF16;
     } else if (r->kv_storage == YVEX_ROCM_KV_BF16) {
         job.function = YVEX_ROCM_FN_DECODE_PAGED_BF16;
