@@ -7,7 +7,7 @@
  * whole, one workgroup each, the longest first; when what is left over would keep a fraction of
  * the units busy for long, its walks are cut into runs of keys, one workgroup each, and a second
  * launch merges the runs.  Nine tokens of 40/8 heads of 128 behind 12001: one tile per query head
- * walked 188 steps on 40 units, 160 us; packed and cut into 256 runs, 20 us.  2000 tokens of 24/4
+ * walked 188 steps on 40 units, 160 us; packed and cut into 256 runs, 17.4 us. 2000 tokens of 24/4
  * heads of 256 behind 13333: 376 items took two turns of 256 units with half of the second empty,
  * 1182 us; with its tail cut, 873 (both with the kernel that prefill_pair.hip has replaced).  A
  * prompt of 2048 tokens without a history is not cut and gains from the packing only that a tile
@@ -157,6 +157,8 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
     params.whole_items = (uint32_t)plan.whole_items;
     params.tail_items = (uint32_t)plan.tail_items;
     params.splits = (uint32_t)plan.splits;
+    /* one trip of the merge takes eight runs; more go to four groups of threads side by side */
+    params.merge_groups = plan.splits > 8ull ? 4u : 1u;
     params.part_acc = (float *)(uintptr_t)work;
     params.part_ml = (float *)(uintptr_t)(work + plan.acc_bytes);
     rc = yvex_rocm_launch(backend,
@@ -169,7 +171,8 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
                               by_head_dimension(r->head_dimension, YVEX_ROCM_FN_PREFILL_MERGE_64,
                                                 YVEX_ROCM_FN_PREFILL_MERGE, YVEX_ROCM_FN_PREFILL_MERGE_256),
                               variant,
-                              (unsigned int)(plan.tail_items * YVEX_ROCM_PREFILL_ROWS * r->head_dimension / 1024ull),
+                              (unsigned int)(plan.tail_items * YVEX_ROCM_PREFILL_ROWS * r->head_dimension *
+                                             params.merge_groups / 1024ull),
                               1u, 1u, 256u, 0u, &params, where, err);
     if (rc == YVEX_OK) {
         facts->kernel_launches = plan.splits > 1ull ? 2ull : 1ull;

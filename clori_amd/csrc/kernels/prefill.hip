@@ -502,30 +502,38 @@ struct Prefill {
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128)
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64)
 
-// Log-sum-exp merge of the runs of the split items and publication of their rows, in the order of
-// the runs.  head_dim / 4 threads per row, four lanes of the row each; grid = tail_items *
-// YVEX_ROCM_PREFILL_ROWS * head_dim / 4 / 256, block = 256.
+// Log-sum-exp merge of the runs of the split items and publication of their rows.  head_dim / 4
+// threads per row and group, four lanes of the row each; the runs of a row are dealt to
+// merge_groups (1 or 4) groups of threads, merged within each in the order of the runs and then
+// group by group.  grid = tail_items * YVEX_ROCM_PREFILL_ROWS * head_dim / 4 * merge_groups / 256,
+// block = 256.
+// A trip of eight runs is a trip to memory, and few tokens leave few rows to hide it: 9 tokens of
+// 40/8 heads of 128 in 32 runs took 6.5 us with one group (four trips one after the other): the call
+// 20.1 us, now 17.4 us.
 template <int kHeadDim>
-__device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p)
+__device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p, floatx4 *acc_of, float2 *ml_of)
 {
-    constexpr uint32_t kThreads = kHeadDim / 4, kRows = 256u / kThreads;
+    constexpr uint32_t kThreads = kHeadDim / 4;
     constexpr int kWidth = 8;  // runs in flight per trip
-    const uint32_t packed = blockIdx.x * kRows + threadIdx.x / kThreads, d = (threadIdx.x % kThreads) * 4u;
+    const uint32_t groups = p.merge_groups, member = threadIdx.x / kThreads, d = (threadIdx.x % kThreads) * 4u;
+    const uint32_t group = member & (groups - 1u);
+    const uint32_t packed = blockIdx.x * (256u / kThreads / groups) + member / groups;
     const uint32_t tail = packed / kRowsPerBlock, in_tile = packed % kRowsPerBlock;
     const uint32_t item = p.whole_items + tail;
     const uint32_t row = (p.query_tiles - 1u - item / p.row_heads) * kRowsPerBlock + in_tile;
-    if (row >= p.rows) return;
-    const uint32_t token = token_of(p, row), head = (item % p.row_heads) * p.pack + (row - token * p.pack);
+    const bool live = row < p.rows;
     const uint64_t first = (uint64_t)tail * p.splits * kRowsPerBlock + in_tile;
+    const uint32_t each = (p.splits + groups - 1u) / groups;
+    const uint32_t begin = min(group * each, p.splits), end = live ? min(begin + each, p.splits) : begin;
     float top = -INFINITY, sum = 0.f;
     floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s0 = 0u; s0 < p.splits; s0 += (uint32_t)kWidth) {
+    for (uint32_t s0 = begin; s0 < end; s0 += (uint32_t)kWidth) {
         float m[kWidth], l[kWidth];
         floatx4 part[kWidth];
 #pragma unroll
         for (int i = 0; i < kWidth; ++i) {
             // runs past the end alias the last one, with weight zero
-            const uint64_t at = first + (uint64_t)min(s0 + (uint32_t)i, p.splits - 1u) * kRowsPerBlock;
+            const uint64_t at = first + (uint64_t)min(s0 + (uint32_t)i, end - 1u) * kRowsPerBlock;
             m[i] = p.part_ml[at * 2u];
             l[i] = p.part_ml[at * 2u + 1u];
             part[i] = *reinterpret_cast<const floatx4 *>(p.part_acc + at * kHeadDim + d);
@@ -533,7 +541,7 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p)
         float m_new = top;
 #pragma unroll
         for (int i = 0; i < kWidth; ++i) {
-            if (s0 + (uint32_t)i >= p.splits) m[i] = -INFINITY;
+            if (s0 + (uint32_t)i >= end) m[i] = -INFINITY;
             m_new = fmaxf(m_new, m[i]);
         }
         if (m_new == -INFINITY) continue;
@@ -549,6 +557,22 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p)
         }
         top = m_new;
     }
+    if (groups != 1u) {
+        acc_of[threadIdx.x] = acc;
+        ml_of[threadIdx.x] = make_float2(top, sum);
+        __syncthreads();
+        if (group != 0u || !live) return;
+        for (uint32_t other = 1u; other < groups; ++other) {
+            const float2 ml = ml_of[threadIdx.x + other * kThreads];
+            if (ml.x == -INFINITY) continue;  // no run of that group saw a key
+            const float m_new = fmaxf(top, ml.x), keep = fast_exp2(top - m_new), w = fast_exp2(ml.x - m_new);
+            sum = sum * keep + w * ml.y;
+            acc = acc * keep + w * acc_of[threadIdx.x + other * kThreads];
+            top = m_new;
+        }
+    }
+    if (!live) return;
+    const uint32_t token = token_of(p, row), head = (item % p.row_heads) * p.pack + (row - token * p.pack);
     const uint64_t at = ((uint64_t)token * p.query_heads + head) * kHeadDim + d;
     const float inv = 1.0f / sum;
     bool bad = !(isfinite(acc[0] * inv) && isfinite(acc[1] * inv) && isfinite(acc[2] * inv) && isfinite(acc[3] * inv));
@@ -565,7 +589,9 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p)
 #define YVEX_PREFILL_MERGE_KERNEL(name, head_dim)                                                         \
     extern "C" __global__ void __launch_bounds__(256) name(const yvex_rocm_prefill_params p)              \
     {                                                                                                     \
-        prefill_merge<head_dim>(p);                                                                       \
+        __shared__ floatx4 acc_of[256];                                                                   \
+        __shared__ float2 ml_of[256];                                                                     \
+        prefill_merge<head_dim>(p, acc_of, ml_of);                                                        \
     }
 
 YVEX_PREFILL_MERGE_KERNEL(yvex_rocm_prefill_merge, 128)
