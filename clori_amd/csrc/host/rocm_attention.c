@@ -25,6 +25,7 @@ enum {
     ROCM_PAGE_TOKENS = 16,
     ROCM_GROUP_MAX = 16,
     ROCM_DECODE_WAVES = 2048,
+    ROCM_DECODE_PARTS_IN_KERNEL = 32,
     ROCM_DECODE_MIN_TILES = 8, /* 8 and 16 measure alike on a 4096-token context; 4 and 32 are a third slower */
     ROCM_TEAM_WAVES = 8,       /* waves of a decode team (one workgroup) */
     /* tiles a wave of a team is given when the history is short enough (context 4096: 10.3 us;
@@ -136,11 +137,16 @@ static int decode_workspace_bytes(unsigned long long slots, unsigned long long h
 }
 
 /* A launch that fills the device merges its split segments with a second kernel; a smaller
- * one is bound by launch latency and merges inside the decode kernel (arrival counters). */
-static int decode_merges_in_kernel(unsigned int waves, unsigned long long head_dim)
+ * one is bound by launch latency and merges inside the decode kernel (arrival counters), unless
+ * the longest session may be cut into so many parts that the one wave which completes a segment
+ * is busy merging them for longer than a launch takes (a session of 16384 tokens, 32/8 heads of
+ * 128, in 128 parts: 43.8 -> 20.2 us with the second launch; 32 parts: 15.3 us in the kernel). */
+static int decode_merges_in_kernel(unsigned int waves, unsigned long long head_dim, int paged,
+                                   unsigned long long max_context)
 {
     /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
-    return waves < ROCM_DECODE_WAVES && head_dim == ROCM_MFMA_HEAD_DIM;
+    if (waves >= ROCM_DECODE_WAVES || head_dim != ROCM_MFMA_HEAD_DIM) return 0;
+    return !paged || max_context <= ROCM_DECODE_PARTS_IN_KERNEL * ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
 }
 
 /* Waves of a team: eight, two per SIMD; four at head dimension 256, whose tiles and
@@ -178,12 +184,13 @@ static int decode_rows_geometry(const yvex_transformer_attention_requirement *r)
  * table. */
 static int balanced_workspace_bytes(unsigned long long waves, unsigned long long group,
                                     unsigned long long head_dim, unsigned long long sessions,
+                                    int paged, unsigned long long max_context,
                                     unsigned long long *acc_bytes, unsigned long long *ml_bytes,
                                     unsigned long long *total)
 {
     unsigned long long parts = 0ull, offsets;
     if (!decode_workspace_bytes(2ull * waves, group, head_dim, sizeof(float), acc_bytes, &parts)) return 0;
-    offsets = decode_merges_in_kernel((unsigned int)waves, head_dim)
+    offsets = decode_merges_in_kernel((unsigned int)waves, head_dim, paged, max_context)
                   ? 0ull : align_up((sessions + 1ull) * sizeof(uint32_t), ROCM_WORK_ALIGNMENT);
     *ml_bytes = parts - *acc_bytes;
     return yvex_core_u64_add(parts, offsets, total);
@@ -213,12 +220,13 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
 {
     yvex_rocm_backend_state *state = yvex_rocm_state(backend);
     yvex_rocm_decode_params dp;
-    unsigned long long acc_bytes = 0ull, ml_bytes = 0ull, total = 0ull, items;
+    unsigned long long acc_bytes = 0ull, ml_bytes = 0ull, total = 0ull, items, tiles, per_wave;
     const unsigned long long group = job->query_heads / job->kv_heads;
     const unsigned int waves = decode_wave_count(job->sessions, job->kv_heads, job->max_context);
     const unsigned int teams = decode_team_count(job->page_table != NULL, group, job->head_dim,
                                                  job->max_context);
-    const int in_kernel = teams || decode_merges_in_kernel(waves, job->head_dim);
+    int in_kernel =
+        teams || decode_merges_in_kernel(waves, job->head_dim, job->page_table != NULL, job->max_context);
     void *work = NULL;
     yvex_error cleanup;
     int owned = 0, rc, cleanup_rc;
@@ -228,11 +236,17 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
         (in_kernel && job->sessions * job->kv_heads > YVEX_ROCM_DECODE_SEGMENTS_MAX) ||
         !(teams ? decode_workspace_bytes(job->sessions * job->kv_heads * teams, group, job->head_dim,
                                          sizeof(float), &acc_bytes, &total)
-                : balanced_workspace_bytes(waves, group, job->head_dim, job->sessions, &acc_bytes,
+                : balanced_workspace_bytes(waves, group, job->head_dim, job->sessions,
+                                           job->page_table != NULL, job->max_context, &acc_bytes,
                                            &ml_bytes, &total)))
         return refuse(err, YVEX_ERR_BOUNDS, where, "decode geometry exceeds admitted integer range");
     backend_workspace_reset(backend);
     if (job->fixed_work) {
+        if (total > job->fixed_work_bytes && !in_kernel && waves < ROCM_DECODE_WAVES &&
+            job->head_dim == ROCM_MFMA_HEAD_DIM) {
+            in_kernel = 1; /* only the offsets do not fit, which the one-launch form does without */
+            total = acc_bytes + ml_bytes;
+        }
         if (total > job->fixed_work_bytes)
             return refuse(err, YVEX_ERR_BOUNDS, where,
                           "decode partials exceed the fixed device scratch "
@@ -268,6 +282,14 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
     dp.min_tiles = ROCM_DECODE_MIN_TILES;
     dp.fixed_context = (uint32_t)job->fixed_context;
     dp.waves = waves;
+    /* Parts of the longest session if the others are half as long on average.  One trip of the
+     * merge takes 24 parts; more go to four groups of threads side by side (2 sessions of 4096, 16/4
+     * heads of 64, 32 parts: 13.9 -> 12.2 us; head dimension 256, whose four groups are a workgroup
+     * of 1024, from the third trip on: 32 parts 18.5 -> 19.5 us, 128 parts 30.8 -> 27.6 us). */
+    tiles = (job->max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS;
+    per_wave = job->sessions * job->kv_heads * tiles / 2ull / waves;
+    if (per_wave < ROCM_DECODE_MIN_TILES) per_wave = ROCM_DECODE_MIN_TILES;
+    dp.finish_groups = tiles / per_wave > (job->head_dim > ROCM_MFMA_HEAD_DIM ? 48ull : 24ull) ? 4u : 1u;
     dp.scale_log2 = job->scale * 1.4426950408889634f;
     if (teams) /* teams of waves, merged through LDS and then between the teams */
         rc = yvex_rocm_launch(backend,
@@ -281,10 +303,11 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
                               waves, 1u, 1u, 64u, 0u, &dp, where, err);
     if (rc == YVEX_OK && !in_kernel)
         rc = yvex_rocm_launch(backend,
-                              job->head_dim > 128ull ? YVEX_ROCM_FN_DECODE_FINISH_256
-                                                     : YVEX_ROCM_FN_DECODE_FINISH,
+                              job->head_dim <= ROCM_MFMA_HEAD_DIM ? YVEX_ROCM_FN_DECODE_FINISH
+                              : dp.finish_groups == 1u            ? YVEX_ROCM_FN_DECODE_FINISH_256
+                                                                  : YVEX_ROCM_FN_DECODE_FINISH_256_GROUPED,
                               job->variant, (unsigned int)job->query_heads, (unsigned int)job->sessions, 1u,
-                              (unsigned int)job->head_dim, 0u, &dp, where, err);
+                              (unsigned int)job->head_dim * dp.finish_groups, 0u, &dp, where, err);
     if (rc == YVEX_OK) {
         facts->kernel_launches = in_kernel ? 1ull : 2ull;
         facts->accelerated_matrix_launches = 1ull;
@@ -451,7 +474,8 @@ static int rocm_attention_workspace_required(const yvex_transformer_attention_re
         const unsigned int teams = decode_team_count(0, group, r->head_dimension, visible_tokens(r));
         if (!(teams ? decode_workspace_bytes(r->key_value_heads * teams, group, r->head_dimension,
                                              sizeof(float), &acc, &total)
-                    : balanced_workspace_bytes(waves, group, r->head_dimension, 1ull, &acc, &ml, &total)))
+                    : balanced_workspace_bytes(waves, group, r->head_dimension, 1ull, 0, visible_tokens(r),
+                                               &acc, &ml, &total)))
             return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");
         *bytes = total;
     } else if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_BF16_F32_ACCUMULATE) {
@@ -805,7 +829,7 @@ static int rocm_paged_decode_workspace_required(const yvex_rocm_paged_decode_req
     if (!bytes) return refuse(err, YVEX_ERR_INVALID_ARG, where, "workspace byte output is required");
     waves = decode_wave_count(r->sessions, r->key_value_heads, r->max_context_tokens);
     if (!balanced_workspace_bytes(waves, r->query_heads / r->key_value_heads, r->head_dimension,
-                                  r->sessions, &acc, &ml, &total))
+                                  r->sessions, 1, r->max_context_tokens, &acc, &ml, &total))
         return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");
     *bytes = total;
     yvex_error_clear(err);

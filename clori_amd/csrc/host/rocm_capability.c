@@ -64,6 +64,8 @@ static const rocm_kernel_binding rocm_kernel_bindings[] = {
      YVEX_ROCM_FN_DECODE_PAGED_BF16_256},
     {"yvex_rocm_decode_finish_256", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_PAGED_BF16,
      YVEX_ROCM_FN_DECODE_FINISH_256},
+    {"yvex_rocm_decode_finish_256_grouped", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_PAGED_BF16,
+     YVEX_ROCM_FN_DECODE_FINISH_256_GROUPED},
     {"yvex_rocm_decode_merge", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_PAGED_BF16,
      YVEX_ROCM_FN_DECODE_MERGE},
     {"yvex_rocm_decode_merge_rope", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_MLA_BF16,

@@ -27,6 +27,7 @@ typedef enum {
     YVEX_ROCM_FN_DECODE_MERGE_ROPE,
     YVEX_ROCM_FN_DECODE_FINISH,
     YVEX_ROCM_FN_DECODE_FINISH_256,
+    YVEX_ROCM_FN_DECODE_FINISH_256_GROUPED,
     YVEX_ROCM_FN_DECODE_PAGED_Q8_0,
     YVEX_ROCM_FN_DECODE_PAGED_BF16_MERGED,
     YVEX_ROCM_FN_DECODE_PAGED_Q8_0_MERGED,

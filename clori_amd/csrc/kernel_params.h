@@ -95,7 +95,8 @@ typedef struct {
     uint32_t waves;
     uint32_t page_shift; /* a page is 16 << page_shift tokens: that many consecutive 16-token blocks */
     float scale_log2; /* softmax scale * log2(e) */
-    float reserved_f;
+    uint32_t finish_groups; /* groups of head_dim threads that the second launch deals a segment's
+                               parts to: 1 or 4 */
     const uint16_t *gate; /* optional bf16 [sessions][query_heads][head_dim] sigmoid output gate */
 } yvex_rocm_decode_params;
 

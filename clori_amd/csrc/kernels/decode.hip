@@ -933,70 +933,91 @@ YVEX_DECODE_TEAM_KERNEL(yvex_rocm_decode_rows_bf16_team_64, 64, 512, 2)
 YVEX_DECODE_TEAM_KERNEL(yvex_rocm_decode_rows_bf16_team_256, 256, 256, 1)
 
 // Merge of the split segments of the balanced decode when the decode kernel was launched
-// without arrival counters (large launches).  grid = (query_heads, sessions), block =
-// head_dim threads (one per output lane).  A segment that one wave covered was already
-// published by that wave and is skipped.
-__device__ __forceinline__ void decode_finish(const yvex_rocm_decode_params &p)
+// without arrival counters.  grid = (query_heads, sessions), block = head_dim * finish_groups
+// threads (1 or 4 groups): one per output lane and group, the parts of a segment dealt to the groups in runs and
+// the groups merged through LDS.  A segment that one wave covered was already published by that
+// wave and is skipped.
+// kGrouped: the build that can take four groups.
+template <bool kGrouped>
+__device__ __forceinline__ void decode_finish(const yvex_rocm_decode_params &p, float *group_acc, float2 *group_ml)
 {
-    const uint32_t head = blockIdx.x, session = blockIdx.y, d = threadIdx.x;
+    const uint32_t head = blockIdx.x, session = blockIdx.y;
+    // heads have 64, 128 or 256 lanes
+    const uint32_t team = kGrouped ? threadIdx.x >> (31 - __builtin_clz(p.head_dim)) : 0u;
+    const uint32_t d = kGrouped ? threadIdx.x & (p.head_dim - 1u) : threadIdx.x;
     const uint32_t group = p.query_heads / p.kv_heads;
     const uint32_t offset = p.offsets[session], next = p.offsets[session + 1u];
     const uint32_t total = p.offsets[p.sessions];
     const uint32_t tiles = (next - offset) / p.kv_heads;
-    if (tiles == 0u || d >= p.head_dim) return;
+    if (tiles == 0u) return;
     const uint32_t per_wave = max((total + p.waves - 1u) / p.waves, p.min_tiles);
     const uint32_t kv_head = head / group, hh = head % group;
     const uint32_t seg_begin = offset + kv_head * tiles, seg_end = seg_begin + tiles;
     const uint32_t w_first = seg_begin / per_wave, w_last = (seg_end - 1u) / per_wave;
+    const uint64_t at = ((uint64_t)session * p.query_heads + head) * p.head_dim + d;
     if (w_first == w_last) {
         // published by the decode kernel itself; only the output gate is left to apply
-        if (p.gate) {
-            const uint64_t at = ((uint64_t)session * p.query_heads + head) * p.head_dim + d;
+        if (p.gate && team == 0u) {
             const float o = bf16_to_f32(p.out[at]) * sigmoid(bf16_to_f32(p.gate[at]));
             if (!isfinite(o)) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
             p.out[at] = bf16_bits(o);
         }
         return;
     }
-    auto slot_of = [&](uint32_t j) -> uint64_t {
-        return ((uint64_t)j * 2u + (seg_begin >= j * per_wave ? 1u : 0u)) * group + hh;
-    };
+    // A wave leaves a segment's first part in its odd slot, other parts in its even one.  Slots and
+    // the offsets of their rows fit 32 bits (2048 waves, groups of 16, heads of 256: 67 MB).
+    auto slot_of = [&](uint32_t j) -> uint32_t { return (2u * j + (j == w_first ? 1u : 0u)) * group + hh; };
     // kWidth parts at a time: all loads of a trip are independent and in flight together
     // (indices past the end alias the last part with weight zero).  A 16384-token context is
     // cut into at most 17 parts when 2048 waves share the work of 32 such sessions, so one
     // trip, one memory round trip, covers every segment of the full-size launches (widths 8
-    // and 16 take three and two trips there and measure 1.4 and 4 us slower per step).
+    // and 16 take three and two trips there and measure 1.4 and 4 us slower per step).  A lone
+    // session of that length is cut into 128 parts, six trips one after the other: four groups take
+    // two (16/4 heads of 64: 22.2 -> 13.8 us the whole step).  The statistics of a trip are one load,
+    // a part per lane, and its weights one exponential; loaded and weighed by every lane for itself
+    // they were most of what a wave issued (64 sessions of 100 to 700 tokens, 24/4 heads of 256:
+    // 32.4 -> 28.4 us the step; 32 sessions to 16384, 32/8 of 128: 167.5 -> 165.7 us).
     constexpr int kWidth = 24;
+    const bool grouped = kGrouped && p.finish_groups != 1u;
+    const uint32_t each = !grouped ? w_last - w_first + 1u : (w_last - w_first + 4u) / 4u;
+    const uint32_t j_first = w_first + team * each, j_end = min(j_first + each, w_last + 1u);
+    const uint32_t lane = threadIdx.x & 63u;
     float top = -INFINITY, sum = 0.f, acc = 0.f;
-    for (uint32_t j0 = w_first; j0 <= w_last; j0 += (uint32_t)kWidth) {
-        float m[kWidth], l[kWidth], v[kWidth];
+    for (uint32_t j0 = j_first; j0 < j_end; j0 += (uint32_t)kWidth) {
+        const u32x2 ml = load_b64(p.part_ml + slot_of(min(j0 + min(lane, (uint32_t)kWidth - 1u), j_end - 1u)) * 2u);
+        float v[kWidth];
 #pragma unroll
-        for (int i = 0; i < kWidth; ++i) {
-            const uint64_t slot = slot_of(min(j0 + (uint32_t)i, w_last));
-            m[i] = p.part_ml[slot * 2u];
-            l[i] = p.part_ml[slot * 2u + 1u];
-            v[i] = p.part_acc[slot * p.head_dim + d];
-        }
-        float trip = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < kWidth; ++i) {
-            if (j0 + (uint32_t)i > w_last) m[i] = -INFINITY;
-            trip = fmaxf(trip, m[i]);
-        }
-        const float m_new = fmaxf(top, trip);
+        for (int i = 0; i < kWidth; ++i)
+            v[i] = p.part_acc[slot_of(min(j0 + (uint32_t)i, j_end - 1u)) * p.head_dim + d];
+        __builtin_amdgcn_sched_barrier(0);  // every load is on its way
+        const uint32_t mx = ml.x, lx = ml.y;
+        const bool holds = lane < (uint32_t)kWidth && j0 + lane < j_end;
+        const float m = holds ? __builtin_bit_cast(float, mx) : -INFINITY;
+        const float m_new = fmaxf(top, wave_max(m));
         const float keep = fast_exp2(top - m_new);
-        sum *= keep;
+        const float weight = fast_exp2(m - m_new);
+        sum = sum * keep + wave_sum(holds ? weight * __builtin_bit_cast(float, lx) : 0.f);
         acc *= keep;
 #pragma unroll
-        for (int i = 0; i < kWidth; ++i) {
-            const float w = fast_exp2(m[i] - m_new);
-            sum += w * l[i];
-            acc += w * v[i];
-        }
+        for (int i = 0; i < kWidth; ++i)
+            acc += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, weight), i)) * v[i];
         top = m_new;
     }
+    if (grouped) {
+        group_acc[threadIdx.x] = acc;
+        group_ml[threadIdx.x] = make_float2(top, sum);
+        __syncthreads();
+        if (team != 0u) return;
+        for (uint32_t other = 1u; other < 4u; ++other) {
+            const float2 ml = group_ml[threadIdx.x + other * p.head_dim];
+            if (ml.y == 0.f) continue;  // a group without parts
+            const float m_new = fmaxf(top, ml.x), keep = fast_exp2(top - m_new), w = fast_exp2(ml.x - m_new);
+            sum = sum * keep + w * ml.y;
+            acc = acc * keep + w * group_acc[threadIdx.x + other * p.head_dim];
+            top = m_new;
+        }
+    }
     float o = acc / sum;
-    const uint64_t at = ((uint64_t)session * p.query_heads + head) * p.head_dim + d;
     if (p.gate) o = bf16_to_f32(bf16_bits(o)) * sigmoid(bf16_to_f32(p.gate[at]));
     if (!isfinite(o)) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
     p.out[at] = bf16_bits(o);
@@ -1004,17 +1025,25 @@ __device__ __forceinline__ void decode_finish(const yvex_rocm_decode_params &p)
         p.lse[(uint64_t)session * p.query_heads + head] = (top + fast_log2(sum)) * YVEX_LN2;
 }
 
-extern "C" __global__ void __launch_bounds__(128)
-yvex_rocm_decode_finish(const yvex_rocm_decode_params p)
-{
-    decode_finish(p);
-}
+#define YVEX_DECODE_FINISH_KERNEL(name, THREADS)                                                      \
+    extern "C" __global__ void __launch_bounds__(THREADS) name(const yvex_rocm_decode_params p)      \
+    {                                                                                                \
+        __shared__ float group_acc[THREADS];                                                         \
+        __shared__ float2 group_ml[THREADS];                                                         \
+        decode_finish<true>(p, group_acc, group_ml);                                                 \
+    }
 
-// head dimension 256: a block of 256 threads
+// head dimensions 64 and 128
+YVEX_DECODE_FINISH_KERNEL(yvex_rocm_decode_finish, 512)
+// head dimension 256, four groups
+YVEX_DECODE_FINISH_KERNEL(yvex_rocm_decode_finish_256_grouped, 1024)
+
+// head dimension 256, one group: a build of its own (in the one above, whose bounds are 1024
+// threads, 64 sessions of 100 to 700 tokens and 24/4 heads take 33.2 instead of 32.4 us)
 extern "C" __global__ void __launch_bounds__(256)
 yvex_rocm_decode_finish_256(const yvex_rocm_decode_params p)
 {
-    decode_finish(p);
+    decode_finish<false>(p, nullptr, nullptr);
 }
 
 // Log-sum-exp merge of the chunk partials of one (session, query head): one wave per head,

@@ -441,3 +441,23 @@ def test_paged_decode_other_head_dimensions_refusals(backend):
         with pytest.raises(YvexError) as e:
             backend.paged_decode_workspace_required(req)
         assert e.value.code == B.YVEX_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("d,hq,hkv,contexts,launches", [
+    (128, 32, 8, [4096], 1),            # 32 parts: merged in the kernel
+    (128, 32, 8, [4097], 2),            # 33 parts: four groups of the second launch, 9 + 9 + 9 + 6
+    (128, 12, 1, [13000, 20], 2),       # several trips per group, and a session that is not cut
+    (64, 16, 4, [3201, 1], 2),          # 26 parts
+    (256, 24, 4, [6400, 700], 2),       # 50 parts: the grouped build at head dimension 256
+    (256, 6, 1, [6100], 2),             # 48 parts: two trips of the other
+])
+def test_paged_decode_few_long_sessions(backend, d, hq, hkv, contexts, launches):
+    """A lone session is cut into a part per eight tiles; who merges them follows their number."""
+    rng = np.random.default_rng(77 + d + hq)
+    q, k_rows, v_rows, table, ctx, pool_pages = make_paged_case(rng, contexts, hq, hkv, d=d)
+    got, lse, facts = run_paged(backend, q, k_rows, v_rows, table, ctx, hkv, pool_pages, max_context=max(contexts))
+    rc, ref, _, ref_lse = ORACLE.paged_decode(q, k_rows, v_rows, table, ctx, hkv, 16)
+    assert rc == 0
+    assert_close_bf16(got, ref, "long paged d=%d %s" % (d, contexts))
+    assert_lse(lse, ref_lse, "long paged d=%d %s" % (d, contexts))
+    assert facts.kernel_launches == launches
