@@ -38,6 +38,53 @@ __device__ inline floatx16 mfma_32x32x2(float a, float b, floatx16 c)
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
 
+// Last key a query may see (the rows of 2^32 keys are more than any memory holds).
+__device__ inline uint32_t last_visible(const yvex_rocm_gqa_f32_params &p, uint64_t own)
+{
+    return (uint32_t)(p.causal ? min(p.kv_tokens - 1u, own) : p.kv_tokens - 1u);
+}
+
+// Scores of one tile -> weights, with the running statistics and the accumulators brought to the
+// new maximum.  A lane holds keys 8 * (i / 4) + 4 * half + i % 4 of the tile for its query.
+//   masked  some query of the wave does not see every key of the tile (the same in all lanes)
+//   last    the last visible key of this lane's query, counted from the tile's first
+// The vector work of a tile is not all hidden behind the other wave's matrix work, and most of it
+// is for cases that most tiles are not: keys to mask (the diagonal and the last tile), a maximum
+// that moves (rare after the first tiles; a factor of one leaves every accumulator as it is).  Both
+// are behind branches: 1777 tokens, 40/8 heads of 128: 322.5 -> 315.0 us (103 TFLOP/s); 2048 tokens,
+// 16/4 of 64: 190 -> 169 us; 1024 tokens, 24/4 of 256: 308 -> 297 us.
+template <int kBlocks>
+__device__ __forceinline__ void weigh(floatx16 &s, bool masked, int last, float scale, int half, float &top,
+                                      float &sum, floatx16 (&out)[kBlocks])
+{
+    float peak = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] *= scale;
+    if (masked) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 8 * (i / 4) + 4 * half + i % 4 <= last ? s[i] : -INFINITY;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) peak = fmaxf(peak, s[i]);
+    peak = max_xor32(peak);
+    const float top_new = fmaxf(top, peak);
+    // key 0 is visible to every query, so top_new is finite from the first tile on
+    const float keep = fast_exp2((top - top_new) * YVEX_LOG2E);
+    if (__builtin_amdgcn_ballot_w64(keep != 1.0f) != 0ull) {
+        sum *= keep;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) out[b][i] *= keep;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        s[i] = fast_exp2((s[i] - top_new) * YVEX_LOG2E);
+        sum += s[i];
+    }
+    top = top_new;
+}
+
 // kBlocks: head_dim / 32.
 template <int kBlocks>
 struct GqaTile {
@@ -55,8 +102,9 @@ struct GqaTile {
     const int tid, lane, wave, column, half;
 
     __device__ GqaTile(const yvex_rocm_gqa_f32_params &params, float *shared)
-        : p(params), lds(shared), tid(threadIdx.x), lane(threadIdx.x & 63), wave(threadIdx.x >> 6),
-          column(threadIdx.x & 31), half((threadIdx.x >> 5) & 1)
+        : p(params), lds(shared), tid(threadIdx.x), lane(threadIdx.x & 63),
+          wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), column(threadIdx.x & 31),
+          half((threadIdx.x >> 5) & 1)
     {
     }
 
@@ -130,7 +178,9 @@ struct GqaTile {
         const uint64_t q0 = q_tile * kQueries + (uint64_t)wave * 32u;
         // rows past the last query repeat it: they compute, they are not stored
         const uint64_t token = min(q0 + (uint64_t)column, p.query_tokens - 1);
-        const uint64_t own = p.query_start + token;  // absolute position of this lane's query
+        // last key of this lane's query, and the keys that every query of the wave sees
+        const uint32_t last = last_visible(p, p.query_start + token);
+        const uint32_t seen_by_all = last_visible(p, p.query_start + min(q0, p.query_tokens - 1)) + 1u;
         // last key any query of the workgroup, and of this wave, may see
         const uint64_t group_last = p.causal
             ? min(p.kv_tokens, p.query_start + min((q_tile + 1) * kQueries, p.query_tokens))
@@ -199,30 +249,8 @@ struct GqaTile {
             }
             if (active) {
                 const float *vt = lds + (int)(t & 1) * kStageFloats + kKeys * kKStride;
-                // lane holds keys 8 * (i / 4) + 4 * half + i % 4 of the tile for its query
-                float peak = -INFINITY;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint64_t key = t * kKeys + (uint64_t)(8 * (i / 4) + 4 * half + i % 4);
-                    const bool visible = key < p.kv_tokens && (!p.causal || key <= own);
-                    s[i] = visible ? s[i] * p.scale : -INFINITY;
-                    peak = fmaxf(peak, s[i]);
-                }
-                peak = max_xor32(peak);
-                const float top_new = fmaxf(top, peak);
-                // key 0 is visible to every query, so top_new is finite from the first tile on
-                const float keep = fast_exp2((top - top_new) * YVEX_LOG2E);
-                sum *= keep;
-#pragma unroll
-                for (int b = 0; b < kBlocks; ++b)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) out[b][i] *= keep;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[i] = fast_exp2((s[i] - top_new) * YVEX_LOG2E);
-                    sum += s[i];
-                }
-                top = top_new;
+                const uint32_t key0 = (uint32_t)t * kKeys;
+                weigh(s, key0 + kKeys > seen_by_all, (int)(last - key0), p.scale, half, top, sum, out);
                 // O^T (head dims x queries) += V^T P^T over this lane half's 16 keys
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
@@ -286,9 +314,9 @@ struct GqaTilePair {
     const int tid, lane, wave, column, half, quarter, part;
 
     __device__ GqaTilePair(const yvex_rocm_gqa_f32_params &params, float *shared)
-        : p(params), lds(shared), tid(threadIdx.x), lane(threadIdx.x & 63), wave(threadIdx.x >> 6),
-          column(threadIdx.x & 31), half((threadIdx.x >> 5) & 1), quarter((threadIdx.x >> 6) & 3),
-          part(threadIdx.x >> 8)
+        : p(params), lds(shared), tid(threadIdx.x), lane(threadIdx.x & 63),
+          wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), column(threadIdx.x & 31),
+          half((threadIdx.x >> 5) & 1), quarter(wave & 3), part(wave >> 2)
     {
     }
 
@@ -343,7 +371,8 @@ struct GqaTilePair {
         const uint64_t kv_head = head / (p.query_heads / p.kv_heads);
         const uint64_t q0 = q_tile * kQueries + (uint64_t)quarter * 32u;
         const uint64_t token = min(q0 + (uint64_t)column, p.query_tokens - 1);
-        const uint64_t own = p.query_start + token;
+        const uint32_t last = last_visible(p, p.query_start + token);
+        const uint32_t seen_by_all = last_visible(p, p.query_start + min(q0, p.query_tokens - 1)) + 1u;
         const uint64_t group_last = p.causal
             ? min(p.kv_tokens, p.query_start + min((q_tile + 1) * kQueries, p.query_tokens))
             : p.kv_tokens;
@@ -427,28 +456,8 @@ struct GqaTilePair {
             }
             if (active) {
                 const float *vt = here + kKeys * kKStride + dim0;
-                float peak = -INFINITY;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint64_t key = t * kKeys + (uint64_t)(8 * (i / 4) + 4 * half + i % 4);
-                    const bool visible = key < p.kv_tokens && (!p.causal || key <= own);
-                    s[i] = visible ? s[i] * p.scale : -INFINITY;
-                    peak = fmaxf(peak, s[i]);
-                }
-                peak = max_xor32(peak);
-                const float top_new = fmaxf(top, peak);
-                const float keep = fast_exp2((top - top_new) * YVEX_LOG2E);
-                sum *= keep;
-#pragma unroll
-                for (int b = 0; b < kBlocks; ++b)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) out[b][i] *= keep;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    s[i] = fast_exp2((s[i] - top_new) * YVEX_LOG2E);
-                    sum += s[i];
-                }
-                top = top_new;
+                const uint32_t key0 = (uint32_t)t * kKeys;
+                weigh(s, key0 + kKeys > seen_by_all, (int)(last - key0), p.scale, half, top, sum, out);
 #pragma unroll
                 for (int i = 0; i < 16; ++i) {
                     const float *vrow = vt + (8 * (i / 4) + 4 * half + i % 4) * kVStride + column;
