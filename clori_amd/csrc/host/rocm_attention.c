@@ -25,7 +25,9 @@ enum {
     ROCM_PAGE_TOKENS = 16,
     ROCM_GROUP_MAX = 16,
     ROCM_DECODE_WAVES = 2048,
-    ROCM_DECODE_PARTS_IN_KERNEL = 32,
+    ROCM_DECODE_PARTS_IN_KERNEL = 8,
+    ROCM_DECODE_PARTS_FEW_WAVES = 17,
+    ROCM_DECODE_FEW_WAVES = 640,
     ROCM_DECODE_MIN_TILES = 8, /* 8 and 16 measure alike on a 4096-token context; 4 and 32 are a third slower */
     ROCM_TEAM_WAVES = 8,       /* waves of a decode team (one workgroup) */
     /* tiles a wave of a team is given when the history is short enough (context 4096: 10.3 us;
@@ -137,16 +139,21 @@ static int decode_workspace_bytes(unsigned long long slots, unsigned long long h
 }
 
 /* A launch that fills the device merges its split segments with a second kernel; a smaller
- * one is bound by launch latency and merges inside the decode kernel (arrival counters), unless
- * the longest session may be cut into so many parts that the one wave which completes a segment
- * is busy merging them for longer than a launch takes (a session of 16384 tokens, 32/8 heads of
- * 128, in 128 parts: 43.8 -> 20.2 us with the second launch; 32 parts: 15.3 us in the kernel). */
+ * one is bound by launch latency and merges inside the decode kernel (arrival counters), where the
+ * one wave that completes a segment merges its parts, eight per trip to memory.  That is worth
+ * the launch it saves up to eight parts of the longest session (32/8 heads of 128, bf16 pages, in
+ * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3)
+ * and costs little up to seventeen while few waves are in flight (1 x 1536 10.5 / 9.8, 1 x 2048
+ * 11.0 / 10.0); beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6
+ * / 13.1, 1 x 4096 16.0 / 12.0, 1 x 16384 43.8 / 20.2). */
 static int decode_merges_in_kernel(unsigned int waves, unsigned long long head_dim, int paged,
                                    unsigned long long max_context)
 {
+    const unsigned long long part_tokens = ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
     /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
     if (waves >= ROCM_DECODE_WAVES || head_dim != ROCM_MFMA_HEAD_DIM) return 0;
-    return !paged || max_context <= ROCM_DECODE_PARTS_IN_KERNEL * ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
+    return !paged || max_context <= ROCM_DECODE_PARTS_IN_KERNEL * part_tokens ||
+           (max_context <= ROCM_DECODE_PARTS_FEW_WAVES * part_tokens && waves <= ROCM_DECODE_FEW_WAVES);
 }
 
 /* Waves of a team: eight, two per SIMD; four at head dimension 256, whose tiles and

@@ -444,8 +444,10 @@ def test_paged_decode_other_head_dimensions_refusals(backend):
 
 
 @pytest.mark.parametrize("d,hq,hkv,contexts,launches", [
-    (128, 32, 8, [4096], 1),            # 32 parts: merged in the kernel
-    (128, 32, 8, [4097], 2),            # 33 parts: four groups of the second launch, 9 + 9 + 9 + 6
+    (128, 32, 8, [2176], 1),            # 17 parts, few waves: merged in the kernel
+    (128, 32, 8, [2177], 2),            # 18 parts: one group of the second launch
+    (128, 32, 8, [1025] * 10, 2),       # 9 parts, 650 waves
+    (128, 32, 8, [4097], 2),            # 33 parts: four groups, 9 + 9 + 9 + 6
     (128, 12, 1, [13000, 20], 2),       # several trips per group, and a session that is not cut
     (64, 16, 4, [3201, 1], 2),          # 26 parts
     (256, 24, 4, [6400, 700], 2),       # 50 parts: the grouped build at head dimension 256
