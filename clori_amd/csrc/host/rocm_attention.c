@@ -28,7 +28,7 @@ enum {
     ROCM_DECODE_PARTS_IN_KERNEL = 8,
     ROCM_DECODE_PARTS_FEW_WAVES = 17,
     ROCM_DECODE_FEW_WAVES = 640,
-    ROCM_DECODE_MIN_TILES = 8, /* 8 and 16 measure alike on a 4096-token context; 4 and 32 are a third slower */
+    ROCM_DECODE_MIN_TILES = 8, /* where a launch does not take fewer, see decode_cut_for */
     ROCM_TEAM_WAVES = 8,       /* waves of a decode team (one workgroup) */
     /* tiles a wave of a team is given when the history is short enough (context 4096: 10.3 us;
      * 1: 11.6, 4: 11.9, 8: 15.9) */
@@ -108,18 +108,61 @@ int yvex_rocm_op_attention(yvex_backend *backend, const yvex_device_tensor *quer
 
 /* ------------------------------------------------ split-K decode core ---- */
 
-/* Wave count and workspace of the balanced split-K decode are pure functions of the
- * request geometry (never of the device) so the planner's workspace_required and the
- * execution always agree: 2048 waves = 2 per SIMD of a 256-CU part, fewer when the
- * worst-case work cannot give each wave ROCM_DECODE_MIN_TILES tiles. */
-static unsigned int decode_wave_count(unsigned long long sessions, unsigned long long kv_heads,
-                                      unsigned long long max_context)
+/* How the balanced split-K decode cuts a request: a pure function of its geometry (never of the
+ * device), so that the planner's workspace_required and the execution always agree. */
+typedef struct {
+    unsigned int waves;     /* 2048 = 2 per SIMD of a 256-CU part, fewer when the work is too little */
+    unsigned int min_tiles; /* 16-token tiles a wave takes at least */
+    int in_kernel;          /* the parts of a segment are merged by the wave that completes it */
+} decode_cut;
+
+static unsigned int decode_wave_count(unsigned long long tiles, unsigned long long min_tiles)
 {
-    unsigned long long tiles = sessions * kv_heads *
-                               ((max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS);
-    unsigned long long waves = (tiles + ROCM_DECODE_MIN_TILES - 1ull) / ROCM_DECODE_MIN_TILES;
-    if (waves > ROCM_DECODE_WAVES) waves = ROCM_DECODE_WAVES;
+    const unsigned long long waves = (tiles + min_tiles - 1ull) / min_tiles;
+    if (waves > ROCM_DECODE_WAVES) return ROCM_DECODE_WAVES;
     return (unsigned int)(waves ? waves : 1ull);
+}
+
+/* A launch that fills the device merges its split segments with a second kernel; a smaller
+ * one is bound by launch latency and merges inside the decode kernel (arrival counters), where the
+ * one wave that completes a segment merges its parts, eight per trip to memory.  That is worth
+ * the launch it saves up to eight parts of the longest session (32/8 heads of 128, bf16 pages, in
+ * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3)
+ * and costs little up to seventeen while few waves are in flight (1 x 1536 10.5 / 9.8, 1 x 2048
+ * 11.0 / 10.0); beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6
+ * / 13.1, 1 x 4096 16.0 / 12.0, 1 x 16384 43.8 / 20.2).
+ *
+ * With the second launch, waves of a paged decode take as few as two tiles where that leaves every
+ * wave a place of its own on the device and no segment more parts than the second launch takes in a
+ * few trips: a wave's tiles come one after the other.  Waves of two or four tiles against eight, us:
+ * 24/4 heads of 256, 1 x 512 10.1 / 13.9, 1 x 2048 12.0 / 14.3, 5 x 3000 14.1 / 15.9, 24 x 600 16.4 / 18.4;
+ * 16/4 of 64, 1 x 2048 8.9 / 10.2, 24 x 600 10.6 / 11.5; 32/8 of 128, 2 x 4096 10.8 / 12.6, Q8_0 11.6 /
+ * 14.2.  Past the lines four tiles lose: 64 x 700 at 256 35.5 / 28.4 (more waves than places), 1 x 16384
+ * at 256 26.1 / 23.1 (256 parts), 8 x 2000 at 128 14.5 / 13.4 (2000 waves).
+ * `coarse`: the cut with the smallest workspace. */
+static decode_cut decode_cut_for(int paged, int coarse, unsigned long long sessions, unsigned long long kv_heads,
+                                 unsigned long long head_dim, unsigned long long max_context)
+{
+    const unsigned long long session_tiles = (max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS;
+    const unsigned long long tiles = sessions * kv_heads * session_tiles;
+    const unsigned long long part_tokens = ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
+    const unsigned long long places = head_dim == 64ull    ? ROCM_DECODE_WAVES
+                                      : head_dim == 128ull ? ROCM_DECODE_WAVES / 4 * 3
+                                                           : ROCM_DECODE_WAVES / 2;
+    const unsigned long long parts = head_dim == 64ull ? 128ull : 64ull;
+    decode_cut cut = {decode_wave_count(tiles, ROCM_DECODE_MIN_TILES), ROCM_DECODE_MIN_TILES, 0};
+    unsigned int fine;
+    /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
+    if (head_dim == ROCM_MFMA_HEAD_DIM && cut.waves < ROCM_DECODE_WAVES)
+        cut.in_kernel = !paged || coarse || max_context <= ROCM_DECODE_PARTS_IN_KERNEL * part_tokens ||
+                        (max_context <= ROCM_DECODE_PARTS_FEW_WAVES * part_tokens &&
+                         cut.waves <= ROCM_DECODE_FEW_WAVES);
+    for (fine = 2u; paged && !coarse && !cut.in_kernel && fine < cut.min_tiles; fine *= 2u)
+        if ((tiles + fine - 1ull) / fine <= places && (session_tiles + fine - 1ull) / fine <= parts) {
+            cut.min_tiles = fine;
+            cut.waves = decode_wave_count(tiles, fine);
+        }
+    return cut;
 }
 
 static int decode_workspace_bytes(unsigned long long slots, unsigned long long heads,
@@ -136,24 +179,6 @@ static int decode_workspace_bytes(unsigned long long slots, unsigned long long h
     if (!yvex_core_u64_add(acc, ml, total)) return 0;
     *acc_bytes = acc;
     return 1;
-}
-
-/* A launch that fills the device merges its split segments with a second kernel; a smaller
- * one is bound by launch latency and merges inside the decode kernel (arrival counters), where the
- * one wave that completes a segment merges its parts, eight per trip to memory.  That is worth
- * the launch it saves up to eight parts of the longest session (32/8 heads of 128, bf16 pages, in
- * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3)
- * and costs little up to seventeen while few waves are in flight (1 x 1536 10.5 / 9.8, 1 x 2048
- * 11.0 / 10.0); beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6
- * / 13.1, 1 x 4096 16.0 / 12.0, 1 x 16384 43.8 / 20.2). */
-static int decode_merges_in_kernel(unsigned int waves, unsigned long long head_dim, int paged,
-                                   unsigned long long max_context)
-{
-    const unsigned long long part_tokens = ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
-    /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
-    if (waves >= ROCM_DECODE_WAVES || head_dim != ROCM_MFMA_HEAD_DIM) return 0;
-    return !paged || max_context <= ROCM_DECODE_PARTS_IN_KERNEL * part_tokens ||
-           (max_context <= ROCM_DECODE_PARTS_FEW_WAVES * part_tokens && waves <= ROCM_DECODE_FEW_WAVES);
 }
 
 /* Waves of a team: eight, two per SIMD; four at head dimension 256, whose tiles and
@@ -189,16 +214,14 @@ static int decode_rows_geometry(const yvex_transformer_attention_requirement *r)
 
 /* Balanced decode: two partial slots per wave, then (two-kernel form) the per-session offset
  * table. */
-static int balanced_workspace_bytes(unsigned long long waves, unsigned long long group,
+static int balanced_workspace_bytes(const decode_cut *cut, unsigned long long group,
                                     unsigned long long head_dim, unsigned long long sessions,
-                                    int paged, unsigned long long max_context,
                                     unsigned long long *acc_bytes, unsigned long long *ml_bytes,
                                     unsigned long long *total)
 {
     unsigned long long parts = 0ull, offsets;
-    if (!decode_workspace_bytes(2ull * waves, group, head_dim, sizeof(float), acc_bytes, &parts)) return 0;
-    offsets = decode_merges_in_kernel((unsigned int)waves, head_dim, paged, max_context)
-                  ? 0ull : align_up((sessions + 1ull) * sizeof(uint32_t), ROCM_WORK_ALIGNMENT);
+    if (!decode_workspace_bytes(2ull * cut->waves, group, head_dim, sizeof(float), acc_bytes, &parts)) return 0;
+    offsets = cut->in_kernel ? 0ull : align_up((sessions + 1ull) * sizeof(uint32_t), ROCM_WORK_ALIGNMENT);
     *ml_bytes = parts - *acc_bytes;
     return yvex_core_u64_add(parts, offsets, total);
 }
@@ -229,30 +252,28 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
     yvex_rocm_decode_params dp;
     unsigned long long acc_bytes = 0ull, ml_bytes = 0ull, total = 0ull, items, tiles, per_wave;
     const unsigned long long group = job->query_heads / job->kv_heads;
-    const unsigned int waves = decode_wave_count(job->sessions, job->kv_heads, job->max_context);
-    const unsigned int teams = decode_team_count(job->page_table != NULL, group, job->head_dim,
-                                                 job->max_context);
-    int in_kernel =
-        teams || decode_merges_in_kernel(waves, job->head_dim, job->page_table != NULL, job->max_context);
+    const int paged = job->page_table != NULL;
+    const unsigned int teams = decode_team_count(paged, group, job->head_dim, job->max_context);
+    decode_cut cut = decode_cut_for(paged, 0, job->sessions, job->kv_heads, job->head_dim, job->max_context);
+    int in_kernel;
     void *work = NULL;
     yvex_error cleanup;
     int owned = 0, rc, cleanup_rc;
     if (!yvex_core_u64_mul(job->sessions * job->kv_heads,
                            (job->max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS, &items) ||
         items > 0x7fffffffull || job->sessions > 65535ull || job->query_heads > 65535ull ||
-        (in_kernel && job->sessions * job->kv_heads > YVEX_ROCM_DECODE_SEGMENTS_MAX) ||
+        ((teams || cut.in_kernel) && job->sessions * job->kv_heads > YVEX_ROCM_DECODE_SEGMENTS_MAX) ||
         !(teams ? decode_workspace_bytes(job->sessions * job->kv_heads * teams, group, job->head_dim,
                                          sizeof(float), &acc_bytes, &total)
-                : balanced_workspace_bytes(waves, group, job->head_dim, job->sessions,
-                                           job->page_table != NULL, job->max_context, &acc_bytes,
+                : balanced_workspace_bytes(&cut, group, job->head_dim, job->sessions, &acc_bytes,
                                            &ml_bytes, &total)))
         return refuse(err, YVEX_ERR_BOUNDS, where, "decode geometry exceeds admitted integer range");
     backend_workspace_reset(backend);
     if (job->fixed_work) {
-        if (total > job->fixed_work_bytes && !in_kernel && waves < ROCM_DECODE_WAVES &&
-            job->head_dim == ROCM_MFMA_HEAD_DIM) {
-            in_kernel = 1; /* only the offsets do not fit, which the one-launch form does without */
-            total = acc_bytes + ml_bytes;
+        if (total > job->fixed_work_bytes && !teams) {
+            cut = decode_cut_for(paged, 1, job->sessions, job->kv_heads, job->head_dim, job->max_context);
+            (void)balanced_workspace_bytes(&cut, group, job->head_dim, job->sessions, &acc_bytes, &ml_bytes,
+                                           &total);
         }
         if (total > job->fixed_work_bytes)
             return refuse(err, YVEX_ERR_BOUNDS, where,
@@ -263,6 +284,7 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
         rc = yvex_rocm_temporary_acquire(backend, total, &work, &owned, where, err);
         if (rc != YVEX_OK) return rc;
     }
+    in_kernel = teams || cut.in_kernel;
     memset(&dp, 0, sizeof(dp));
     dp.q = (const uint16_t *)job->q;
     dp.k_pool = job->k;
@@ -286,16 +308,16 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
     dp.pool_pages = (uint32_t)job->pool_pages;
     dp.page_shift = job->page_shift;
     dp.table_stride = (uint32_t)job->table_stride;
-    dp.min_tiles = ROCM_DECODE_MIN_TILES;
+    dp.min_tiles = cut.min_tiles;
     dp.fixed_context = (uint32_t)job->fixed_context;
-    dp.waves = waves;
+    dp.waves = cut.waves;
     /* Parts of the longest session if the others are half as long on average.  One trip of the
      * merge takes 24 parts; more go to four groups of threads side by side (2 sessions of 4096, 16/4
      * heads of 64, 32 parts: 13.9 -> 12.2 us; head dimension 256, whose four groups are a workgroup
      * of 1024, from the third trip on: 32 parts 18.5 -> 19.5 us, 128 parts 30.8 -> 27.6 us). */
     tiles = (job->max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS;
-    per_wave = job->sessions * job->kv_heads * tiles / 2ull / waves;
-    if (per_wave < ROCM_DECODE_MIN_TILES) per_wave = ROCM_DECODE_MIN_TILES;
+    per_wave = job->sessions * job->kv_heads * tiles / 2ull / cut.waves;
+    if (per_wave < cut.min_tiles) per_wave = cut.min_tiles;
     dp.finish_groups = tiles / per_wave > (job->head_dim > ROCM_MFMA_HEAD_DIM ? 48ull : 24ull) ? 4u : 1u;
     dp.scale_log2 = job->scale * 1.4426950408889634f;
     if (teams) /* teams of waves, merged through LDS and then between the teams */
@@ -307,7 +329,7 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
                               64u * decode_team_waves(job->head_dim), 0u, &dp, where, err);
     else
         rc = yvex_rocm_launch(backend, in_kernel ? job->merged_function : job->function, job->variant,
-                              waves, 1u, 1u, 64u, 0u, &dp, where, err);
+                              cut.waves, 1u, 1u, 64u, 0u, &dp, where, err);
     if (rc == YVEX_OK && !in_kernel)
         rc = yvex_rocm_launch(backend,
                               job->head_dim <= ROCM_MFMA_HEAD_DIM ? YVEX_ROCM_FN_DECODE_FINISH
@@ -476,13 +498,13 @@ static int rocm_attention_workspace_required(const yvex_transformer_attention_re
     if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_BF16_F32_ACCUMULATE &&
         decode_rows_geometry(r)) {
         /* split-K decode partials; geometry must match decode_run */
-        const unsigned int waves = decode_wave_count(1ull, r->key_value_heads, visible_tokens(r));
+        const decode_cut cut =
+            decode_cut_for(0, 0, 1ull, r->key_value_heads, r->head_dimension, visible_tokens(r));
         const unsigned long long group = r->query_heads / r->key_value_heads;
         const unsigned int teams = decode_team_count(0, group, r->head_dimension, visible_tokens(r));
         if (!(teams ? decode_workspace_bytes(r->key_value_heads * teams, group, r->head_dimension,
                                              sizeof(float), &acc, &total)
-                    : balanced_workspace_bytes(waves, group, r->head_dimension, 1ull, 0, visible_tokens(r),
-                                               &acc, &ml, &total)))
+                    : balanced_workspace_bytes(&cut, group, r->head_dimension, 1ull, &acc, &ml, &total)))
             return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");
         *bytes = total;
     } else if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_BF16_F32_ACCUMULATE) {
@@ -828,15 +850,15 @@ static int rocm_paged_decode_workspace_required(const yvex_rocm_paged_decode_req
 {
     static const char where[] = "rocm.attention.paged.workspace";
     unsigned long long acc = 0ull, ml = 0ull, total = 0ull;
-    unsigned int waves;
+    decode_cut cut;
     int rc;
     if (bytes) *bytes = 0ull;
     rc = paged_validate(r, where, err);
     if (rc != YVEX_OK) return rc;
     if (!bytes) return refuse(err, YVEX_ERR_INVALID_ARG, where, "workspace byte output is required");
-    waves = decode_wave_count(r->sessions, r->key_value_heads, r->max_context_tokens);
-    if (!balanced_workspace_bytes(waves, r->query_heads / r->key_value_heads, r->head_dimension,
-                                  r->sessions, 1, r->max_context_tokens, &acc, &ml, &total))
+    cut = decode_cut_for(1, 0, r->sessions, r->key_value_heads, r->head_dimension, r->max_context_tokens);
+    if (!balanced_workspace_bytes(&cut, r->query_heads / r->key_value_heads, r->head_dimension, r->sessions,
+                                  &acc, &ml, &total))
         return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");
     *bytes = total;
     yvex_error_clear(err);

@@ -449,12 +449,16 @@ def test_paged_decode_other_head_dimensions_refusals(backend):
     (128, 32, 8, [1025] * 10, 2),       # 9 parts, 650 waves
     (128, 32, 8, [4097], 2),            # 33 parts: four groups, 9 + 9 + 9 + 6
     (128, 12, 1, [13000, 20], 2),       # several trips per group, and a session that is not cut
-    (64, 16, 4, [3201, 1], 2),          # 26 parts
-    (256, 24, 4, [6400, 700], 2),       # 50 parts: the grouped build at head dimension 256
-    (256, 6, 1, [6100], 2),             # 48 parts: two trips of the other
+    (128, 16, 4, [4096, 77, 1500], 2),  # waves of four tiles: 64 parts
+    (64, 16, 4, [4096, 1], 2),          # waves of two tiles: 128 parts
+    (64, 16, 4, [4097], 2),             # of four: 65 parts
+    (64, 16, 4, [33, 16, 1], 2),        # of two, fewer tiles than waves
+    (256, 24, 4, [8193, 700], 2),       # of eight: 65 parts, the grouped build at head dimension 256
+    (256, 6, 1, [4096], 2),             # of four: 64 parts
+    (256, 24, 4, [800, 31, 2048], 2),   # of two: 64 parts
 ])
 def test_paged_decode_few_long_sessions(backend, d, hq, hkv, contexts, launches):
-    """A lone session is cut into a part per eight tiles; who merges them follows their number."""
+    """How many tiles a wave takes and who merges the parts follow the number of both."""
     rng = np.random.default_rng(77 + d + hq)
     q, k_rows, v_rows, table, ctx, pool_pages = make_paged_case(rng, contexts, hq, hkv, d=d)
     got, lse, facts = run_paged(backend, q, k_rows, v_rows, table, ctx, hkv, pool_pages, max_context=max(contexts))
