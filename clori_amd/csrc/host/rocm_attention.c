@@ -108,63 +108,6 @@ int yvex_rocm_op_attention(yvex_backend *backend, const yvex_device_tensor *quer
 
 /* ------------------------------------------------ split-K decode core ---- */
 
-/* How the balanced split-K decode cuts a request: a pure function of its geometry (never of the
- * device), so that the planner's workspace_required and the execution always agree. */
-typedef struct {
-    unsigned int waves;     /* 2048 = 2 per SIMD of a 256-CU part, fewer when the work is too little */
-    unsigned int min_tiles; /* 16-token tiles a wave takes at least */
-    int in_kernel;          /* the parts of a segment are merged by the wave that completes it */
-} decode_cut;
-
-static unsigned int decode_wave_count(unsigned long long tiles, unsigned long long min_tiles)
-{
-    const unsigned long long waves = (tiles + min_tiles - 1ull) / min_tiles;
-    if (waves > ROCM_DECODE_WAVES) return ROCM_DECODE_WAVES;
-    return (unsigned int)(waves ? waves : 1ull);
-}
-
-/* A launch that fills the device merges its split segments with a second kernel; a smaller
- * one is bound by launch latency and merges inside the decode kernel (arrival counters), where the
- * one wave that completes a segment merges its parts, eight per trip to memory.  That is worth
- * the launch it saves up to eight parts of the longest session (32/8 heads of 128, bf16 pages, in
- * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3)
- * and costs little up to seventeen while few waves are in flight (1 x 1536 10.5 / 9.8, 1 x 2048
- * 11.0 / 10.0); beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6
- * / 13.1, 1 x 4096 16.0 / 12.0, 1 x 16384 43.8 / 20.2).
- *
- * With the second launch, waves of a paged decode take as few as two tiles where that leaves every
- * wave a place of its own on the device and no segment more parts than the second launch takes in a
- * few trips: a wave's tiles come one after the other.  Waves of two or four tiles against eight, us:
- * 24/4 heads of 256, 1 x 512 10.1 / 13.9, 1 x 2048 12.0 / 14.3, 5 x 3000 14.1 / 15.9, 24 x 600 16.4 / 18.4;
- * 16/4 of 64, 1 x 2048 8.9 / 10.2, 24 x 600 10.6 / 11.5; 32/8 of 128, 2 x 4096 10.8 / 12.6, Q8_0 11.6 /
- * 14.2.  Past the lines four tiles lose: 64 x 700 at 256 35.5 / 28.4 (more waves than places), 1 x 16384
- * at 256 26.1 / 23.1 (256 parts), 8 x 2000 at 128 14.5 / 13.4 (2000 waves).
- * `coarse`: the cut with the smallest workspace. */
-static decode_cut decode_cut_for(int paged, int coarse, unsigned long long sessions, unsigned long long kv_heads,
-                                 unsigned long long head_dim, unsigned long long max_context)
-{
-    const unsigned long long session_tiles = (max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS;
-    const unsigned long long tiles = sessions * kv_heads * session_tiles;
-    const unsigned long long part_tokens = ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
-    const unsigned long long places = head_dim == 64ull    ? ROCM_DECODE_WAVES
-                                      : head_dim == 128ull ? ROCM_DECODE_WAVES / 4 * 3
-                                                           : ROCM_DECODE_WAVES / 2;
-    const unsigned long long parts = head_dim == 64ull ? 128ull : 64ull;
-    decode_cut cut = {decode_wave_count(tiles, ROCM_DECODE_MIN_TILES), ROCM_DECODE_MIN_TILES, 0};
-    unsigned int fine;
-    /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
-    if (head_dim == ROCM_MFMA_HEAD_DIM && cut.waves < ROCM_DECODE_WAVES)
-        cut.in_kernel = !paged || coarse || max_context <= ROCM_DECODE_PARTS_IN_KERNEL * part_tokens ||
-                        (max_context <= ROCM_DECODE_PARTS_FEW_WAVES * part_tokens &&
-                         cut.waves <= ROCM_DECODE_FEW_WAVES);
-    for (fine = 2u; paged && !coarse && !cut.in_kernel && fine < cut.min_tiles; fine *= 2u)
-        if ((tiles + fine - 1ull) / fine <= places && (session_tiles + fine - 1ull) / fine <= parts) {
-            cut.min_tiles = fine;
-            cut.waves = decode_wave_count(tiles, fine);
-        }
-    return cut;
-}
-
 static int decode_workspace_bytes(unsigned long long slots, unsigned long long heads,
                                   unsigned long long head_dim, unsigned long long element_bytes,
                                   unsigned long long *acc_bytes, unsigned long long *total)
@@ -212,6 +155,21 @@ static int decode_rows_geometry(const yvex_transformer_attention_requirement *r)
             r->query_heads / r->key_value_heads <= ROCM_TEAM_GROUP_MAX);
 }
 
+/* How the balanced split-K decode cuts a request: a pure function of its geometry (never of the
+ * device), so that the planner's workspace_required and the execution always agree. */
+typedef struct {
+    unsigned int waves;     /* 2048 = 2 per SIMD of a 256-CU part, fewer when the work is too little */
+    unsigned int min_tiles; /* 16-token tiles a wave takes at least */
+    int in_kernel;          /* the parts of a segment are merged by the wave that completes it */
+} decode_cut;
+
+static unsigned int decode_wave_count(unsigned long long tiles, unsigned long long min_tiles)
+{
+    const unsigned long long waves = (tiles + min_tiles - 1ull) / min_tiles;
+    if (waves > ROCM_DECODE_WAVES) return ROCM_DECODE_WAVES;
+    return (unsigned int)(waves ? waves : 1ull);
+}
+
 /* Balanced decode: two partial slots per wave, then (two-kernel form) the per-session offset
  * table. */
 static int balanced_workspace_bytes(const decode_cut *cut, unsigned long long group,
@@ -224,6 +182,74 @@ static int balanced_workspace_bytes(const decode_cut *cut, unsigned long long gr
     offsets = cut->in_kernel ? 0ull : align_up((sessions + 1ull) * sizeof(uint32_t), ROCM_WORK_ALIGNMENT);
     *ml_bytes = parts - *acc_bytes;
     return yvex_core_u64_add(parts, offsets, total);
+}
+
+static int cut_fits_scratch(const decode_cut *cut, unsigned long long group, unsigned long long head_dim,
+                            unsigned long long sessions)
+{
+    unsigned long long acc, ml, total;
+    return balanced_workspace_bytes(cut, group, head_dim, sessions, &acc, &ml, &total) &&
+           total <= YVEX_ROCM_STATIC_SCRATCH_BYTES;
+}
+
+/* A launch that fills the device merges its split segments with a second kernel; a smaller
+ * one is bound by launch latency and merges inside the decode kernel (arrival counters), where the
+ * one wave that completes a segment merges its parts, eight per trip to memory.  That is worth
+ * the launch it saves up to eight parts of the longest session (32/8 heads of 128, bf16 pages, in
+ * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3)
+ * and costs little up to seventeen while few waves are in flight (1 x 1536 10.5 / 9.8, 1 x 2048
+ * 11.0 / 10.0); beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6
+ * / 13.1, 1 x 4096 16.0 / 12.0, 1 x 16384 43.8 / 20.2).
+ *
+ * With the second launch, waves of a paged decode take as few as two tiles where that leaves every
+ * wave a place of its own on the device and no segment more parts than the second launch takes in a
+ * few trips: a wave's tiles come one after the other.  Waves of two or four tiles against eight, us:
+ * 24/4 heads of 256, 1 x 512 10.1 / 13.9, 1 x 2048 12.0 / 14.3, 5 x 3000 14.1 / 15.9, 24 x 600 16.4 / 18.4;
+ * 16/4 of 64, 1 x 2048 8.9 / 10.2, 24 x 600 10.6 / 11.5; 32/8 of 128, 2 x 4096 10.8 / 12.6, Q8_0 11.6 /
+ * 14.2.  Past the lines four tiles lose: 64 x 700 at 256 35.5 / 28.4 (more waves than places), 1 x 16384
+ * at 256 26.1 / 23.1 (256 parts), 8 x 2000 at 128 14.5 / 13.4 (2000 waves).
+ *
+ * The entry that allocates nothing has the same cut, bit for bit: forms that need more than its
+ * fixed scratch where the plain one (eight tiles, merged in the kernel) does not are left out. */
+static decode_cut decode_cut_for(int paged, unsigned long long sessions, unsigned long long kv_heads,
+                                 unsigned long long group, unsigned long long head_dim,
+                                 unsigned long long max_context)
+{
+    const unsigned long long session_tiles = (max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS;
+    const unsigned long long tiles = sessions * kv_heads * session_tiles;
+    const unsigned long long part_tokens = ROCM_DECODE_MIN_TILES * ROCM_PAGE_TOKENS;
+    const unsigned long long places = head_dim == 64ull    ? ROCM_DECODE_WAVES
+                                      : head_dim == 128ull ? ROCM_DECODE_WAVES / 4 * 3
+                                                           : ROCM_DECODE_WAVES / 2;
+    const unsigned long long parts = head_dim == 64ull ? 128ull : 64ull;
+    decode_cut cut = {decode_wave_count(tiles, ROCM_DECODE_MIN_TILES), ROCM_DECODE_MIN_TILES, 0}, other;
+    unsigned int fine;
+    if (!paged) {
+        cut.in_kernel = cut.waves < ROCM_DECODE_WAVES;
+        return cut;
+    }
+    /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
+    if (head_dim == ROCM_MFMA_HEAD_DIM && cut.waves < ROCM_DECODE_WAVES)
+        cut.in_kernel = max_context <= ROCM_DECODE_PARTS_IN_KERNEL * part_tokens ||
+                        (max_context <= ROCM_DECODE_PARTS_FEW_WAVES * part_tokens &&
+                         cut.waves <= ROCM_DECODE_FEW_WAVES) ||
+                        !cut_fits_scratch(&cut, group, head_dim, sessions);
+    for (fine = 2u; !cut.in_kernel && fine < cut.min_tiles; fine *= 2u) {
+        other = cut;
+        other.min_tiles = fine;
+        other.waves = decode_wave_count(tiles, fine);
+        if ((tiles + fine - 1ull) / fine <= places && (session_tiles + fine - 1ull) / fine <= parts &&
+            cut_fits_scratch(&other, group, head_dim, sessions))
+            cut = other;
+    }
+    /* partials that fit the scratch make room for the offsets behind them (the kernels cut the
+     * work by whatever number of waves there is) */
+    other = cut;
+    other.in_kernel = 1;
+    if (cut.waves < ROCM_DECODE_WAVES && head_dim != ROCM_MFMA_HEAD_DIM &&
+        cut_fits_scratch(&other, group, head_dim, sessions))
+        while (cut.waves > 1u && !cut_fits_scratch(&cut, group, head_dim, sessions)) --cut.waves;
+    return cut;
 }
 
 typedef struct {
@@ -254,15 +280,16 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
     const unsigned long long group = job->query_heads / job->kv_heads;
     const int paged = job->page_table != NULL;
     const unsigned int teams = decode_team_count(paged, group, job->head_dim, job->max_context);
-    decode_cut cut = decode_cut_for(paged, 0, job->sessions, job->kv_heads, job->head_dim, job->max_context);
-    int in_kernel;
+    const decode_cut cut =
+        decode_cut_for(paged, job->sessions, job->kv_heads, group, job->head_dim, job->max_context);
+    const int in_kernel = teams || cut.in_kernel;
     void *work = NULL;
     yvex_error cleanup;
     int owned = 0, rc, cleanup_rc;
     if (!yvex_core_u64_mul(job->sessions * job->kv_heads,
                            (job->max_context + ROCM_PAGE_TOKENS - 1ull) / ROCM_PAGE_TOKENS, &items) ||
         items > 0x7fffffffull || job->sessions > 65535ull || job->query_heads > 65535ull ||
-        ((teams || cut.in_kernel) && job->sessions * job->kv_heads > YVEX_ROCM_DECODE_SEGMENTS_MAX) ||
+        (in_kernel && job->sessions * job->kv_heads > YVEX_ROCM_DECODE_SEGMENTS_MAX) ||
         !(teams ? decode_workspace_bytes(job->sessions * job->kv_heads * teams, group, job->head_dim,
                                          sizeof(float), &acc_bytes, &total)
                 : balanced_workspace_bytes(&cut, group, job->head_dim, job->sessions, &acc_bytes,
@@ -270,11 +297,6 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
         return refuse(err, YVEX_ERR_BOUNDS, where, "decode geometry exceeds admitted integer range");
     backend_workspace_reset(backend);
     if (job->fixed_work) {
-        if (total > job->fixed_work_bytes && !teams) {
-            cut = decode_cut_for(paged, 1, job->sessions, job->kv_heads, job->head_dim, job->max_context);
-            (void)balanced_workspace_bytes(&cut, group, job->head_dim, job->sessions, &acc_bytes, &ml_bytes,
-                                           &total);
-        }
         if (total > job->fixed_work_bytes)
             return refuse(err, YVEX_ERR_BOUNDS, where,
                           "decode partials exceed the fixed device scratch "
@@ -284,7 +306,6 @@ static int decode_run(yvex_backend *backend, const decode_job *job, const char *
         rc = yvex_rocm_temporary_acquire(backend, total, &work, &owned, where, err);
         if (rc != YVEX_OK) return rc;
     }
-    in_kernel = teams || cut.in_kernel;
     memset(&dp, 0, sizeof(dp));
     dp.q = (const uint16_t *)job->q;
     dp.k_pool = job->k;
@@ -498,9 +519,9 @@ static int rocm_attention_workspace_required(const yvex_transformer_attention_re
     if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_BF16_F32_ACCUMULATE &&
         decode_rows_geometry(r)) {
         /* split-K decode partials; geometry must match decode_run */
-        const decode_cut cut =
-            decode_cut_for(0, 0, 1ull, r->key_value_heads, r->head_dimension, visible_tokens(r));
         const unsigned long long group = r->query_heads / r->key_value_heads;
+        const decode_cut cut =
+            decode_cut_for(0, 1ull, r->key_value_heads, group, r->head_dimension, visible_tokens(r));
         const unsigned int teams = decode_team_count(0, group, r->head_dimension, visible_tokens(r));
         if (!(teams ? decode_workspace_bytes(r->key_value_heads * teams, group, r->head_dimension,
                                              sizeof(float), &acc, &total)
@@ -856,7 +877,8 @@ static int rocm_paged_decode_workspace_required(const yvex_rocm_paged_decode_req
     rc = paged_validate(r, where, err);
     if (rc != YVEX_OK) return rc;
     if (!bytes) return refuse(err, YVEX_ERR_INVALID_ARG, where, "workspace byte output is required");
-    cut = decode_cut_for(1, 0, r->sessions, r->key_value_heads, r->head_dimension, r->max_context_tokens);
+    cut = decode_cut_for(1, r->sessions, r->key_value_heads, r->query_heads / r->key_value_heads,
+                         r->head_dimension, r->max_context_tokens);
     if (!balanced_workspace_bytes(&cut, r->query_heads / r->key_value_heads, r->head_dimension, r->sessions,
                                   &acc, &ml, &total))
         return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");

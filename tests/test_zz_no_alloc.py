@@ -68,6 +68,16 @@ def test_static_entry_at_other_head_dimensions(backend, d, hq, hkv):
     run_both(backend, [40, 700, 129], hq, hkv, B.KV_BF16, seed=15, d=d)
 
 
+@pytest.mark.parametrize("contexts,hq,hkv,d", [
+    ([4000, 3000, 900, 2500, 2], 32, 2, 128),      # 16 heads a group: the partials of waves of four tiles fit,
+    ([4096] * 3 + [5] * 2, 64, 4, 128),            # with more kv heads they would not
+    ([600, 1500, 40, 1333], 128, 8, 256),
+    ([16, 1] + [9] * 2707, 8, 1, 256),             # the partials fit, but not with their offsets
+])
+def test_static_entry_takes_the_same_cut(backend, contexts, hq, hkv, d):
+    run_both(backend, contexts, hq, hkv, B.KV_BF16, seed=16, d=d)
+
+
 def test_static_entry_refuses_what_does_not_fit(backend):
     # a query group of 16 at the full wave count needs 2*2048*16*(128+2)*4 B > 16 MiB
     rng = np.random.default_rng(13)
