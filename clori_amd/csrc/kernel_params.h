@@ -199,8 +199,9 @@ typedef struct {
  * workgroups each, one run of 64-key steps per workgroup (workgroup whole_items + split *
  * tail_items + i), which leave partials that yvex_rocm_prefill_merge* reads:
  * part_acc [tail_items * splits][YVEX_ROCM_PREFILL_ROWS][head_dim] F32 (unnormalised), part_ml
- * [tail_items * splits][YVEX_ROCM_PREFILL_ROWS][2] F32 = (running maximum in log2 units, sum).  The
- * accumulator rows of a run that saw no key (maximum -inf) are not written. */
+ * [tail_items * splits][YVEX_ROCM_PREFILL_ROWS][2] F32 = (running maximum in log2 units, sum).  Where
+ * the maximum is -inf the accumulator rows need not be written: the run saw no key of the row (its
+ * sum is 0), or only scores that are NaN (its sum is NaN, and so is the row). */
 #define YVEX_ROCM_PREFILL_ROWS 128
 typedef struct {
     const uint16_t *q, *k, *v;

@@ -541,16 +541,18 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p,
         float m_new = top;
 #pragma unroll
         for (int i = 0; i < kWidth; ++i) {
-            if (s0 + (uint32_t)i >= end) m[i] = -INFINITY;
+            if (s0 + (uint32_t)i >= end) m[i] = -INFINITY, l[i] = 0.f;
             m_new = fmaxf(m_new, m[i]);
         }
-        if (m_new == -INFINITY) continue;
-        const float keep = fast_exp2(top - m_new);
+        const float keep = m_new == -INFINITY ? 1.f : fast_exp2(top - m_new);
         sum *= keep;
         acc *= keep;
 #pragma unroll
         for (int i = 0; i < kWidth; ++i) {
-            if (m[i] == -INFINITY) continue;  // nothing was left there
+            if (m[i] == -INFINITY) {  // no rows were left: no key was seen, or only scores that are NaN
+                sum += l[i];
+                continue;
+            }
             const float w = fast_exp2(m[i] - m_new);
             sum += w * l[i];
             acc += w * part[i];
@@ -564,7 +566,10 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p,
         if (group != 0u || !live) return;
         for (uint32_t other = 1u; other < groups; ++other) {
             const float2 ml = ml_of[threadIdx.x + other * kThreads];
-            if (ml.x == -INFINITY) continue;  // no run of that group saw a key
+            if (ml.x == -INFINITY) {
+                sum += ml.y;
+                continue;
+            }
             const float m_new = fmaxf(top, ml.x), keep = fast_exp2(top - m_new), w = fast_exp2(ml.x - m_new);
             sum = sum * keep + w * ml.y;
             acc = acc * keep + w * acc_of[threadIdx.x + other * kThreads];

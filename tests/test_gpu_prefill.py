@@ -252,3 +252,46 @@ def test_prefill_scores_far_above_the_first_tiles(backend, tq, tk, start, hq, hk
     with pytest.raises(YvexError) as e:
         backend.attention_execute(req, *tensors, out)
     assert e.value.code == B.YVEX_ERR_FORMAT
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("tq,tk,hq,hkv,groups", [
+    (5, 4000, 10, 2, 4),  # many runs, merged by four groups of threads
+    (5, 1000, 10, 2, 1),  # few runs, one group
+])
+def test_prefill_reports_a_run_of_keys_that_are_not_numbers(backend, d, tq, tk, hq, hkv, groups):
+    """A cut walk one of whose runs sees nothing but NaN scores fails as the whole walk does, wherever
+    the run lies: the first, one in the middle, the last, and as many as a group of the merge takes."""
+    rng = np.random.default_rng(d + tk)
+    q, k, v = (bf16_normal(rng, shape) for shape in ((tq, hq, d), (tk, hkv, d), (tk, hkv, d)))
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, causal=True, query_start=tk - tq, dtype=B.DTYPE_BF16,
+                                        contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+    need = backend.attention_workspace_required(req)
+    items = -(-tq * (hq // hkv) // 128) * hkv
+    runs = need // (items * 128 * (d + 2) * 4)
+    steps = -(-tk // 64)
+    run_keys = -(-steps // runs) * 64
+    assert runs >= 3 and (runs > 8) == (groups == 4)
+    out, lse = backend.tensor("o", B.DTYPE_BF16, q.shape), backend.tensor("lse", B.DTYPE_F32, (tq, hq))
+    tq_, tk_, tv_ = (backend.tensor(n, B.DTYPE_BF16, x.shape, x) for n, x in (("q", q), ("k", k), ("v", v)))
+    work = backend.tensor("w", B.DTYPE_I8, (need,))
+    group_keys = -(-runs // groups) * run_keys
+    last = (steps - 1) // -(-steps // runs) * run_keys  # first key of the last run that has any
+    try:
+        for first, end in ((0, run_keys), (run_keys, 2 * run_keys), (last, tk), (0, group_keys), (run_keys, tk)):
+            poisoned = k.copy()
+            poisoned[first:end] = 0x7FC0
+            tk_.write(poisoned)
+            for attached in (False, True):
+                if attached:
+                    backend.workspace_attach(work)
+                try:
+                    with pytest.raises(YvexError) as e:
+                        backend.attention_execute(req, tq_, tk_, tv_, out, lse=lse)
+                finally:
+                    if attached:
+                        backend.workspace_detach()
+                assert e.value.code == B.YVEX_ERR_FORMAT, (first, end, attached)
+    finally:
+        for t in (out, lse, tq_, tk_, tv_, work):
+            t.release()
