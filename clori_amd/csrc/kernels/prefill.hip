@@ -580,7 +580,8 @@ __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p,
     const uint32_t token = token_of(p, row), head = (item % p.row_heads) * p.pack + (row - token * p.pack);
     const uint64_t at = ((uint64_t)token * p.query_heads + head) * kHeadDim + d;
     const float inv = 1.0f / sum;
-    bool bad = !(isfinite(acc[0] * inv) && isfinite(acc[1] * inv) && isfinite(acc[2] * inv) && isfinite(acc[3] * inv));
+    bool bad = !isfinite(sum);  // (an infinite sum would publish zeros)
+    bad |= !(isfinite(acc[0] * inv) && isfinite(acc[1] * inv) && isfinite(acc[2] * inv) && isfinite(acc[3] * inv));
     u32x2 w = {pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv)};
     if (p.gate) {
         w = gate_four(w, p.gate + at);

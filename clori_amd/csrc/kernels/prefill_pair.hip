@@ -414,11 +414,14 @@ struct PrefillPair {
         } else {
             step<false, true>(t, tiles, s_even, s_odd, first_visible);
         }
-        if (any_row_overflowed()) walk_rescaling(tiles);
 
         // ---- the pair's row sums, then partials or rows ----
         float l[2];
         pair_sum(l);
+        if (any_row_overflowed(l)) {
+            walk_rescaling(tiles);
+            pair_sum(l);
+        }
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb) {
             if (row0 + rb * 32 + n >= p.rows) continue;
@@ -445,18 +448,18 @@ struct PrefillPair {
         }
     }
 
-    // Whether a row of the workgroup is not finite (the same answer in every wave).
-    __device__ inline bool any_row_overflowed() const
+    // Whether a row of the workgroup is not finite (the same answer in every wave).  `l`: the complete
+    // row sums; each is the sum of four parts (two lane halves, two waves) that may be finite when it is not.
+    __device__ inline bool any_row_overflowed(const float (&l)[2]) const
     {
-        // a sum of magnitudes is finite only if every term is
-        float bad = l_run[0] + l_run[1];
+        bool bad = !(isfinite(l[0]) && isfinite(l[1]));
 #pragma unroll
         for (int rb = 0; rb < 2; ++rb)
 #pragma unroll
             for (int db = 0; db < kDimBlocks; ++db)
 #pragma unroll
-                for (int i = 0; i < 16; ++i) bad = fmaxf(bad, isfinite(o[rb][db][i]) ? 0.f : INFINITY);
-        const bool wave_bad = __builtin_amdgcn_ballot_w64(!isfinite(bad)) != 0ull;
+                for (int i = 0; i < 16; ++i) bad |= !isfinite(o[rb][db][i]);
+        const bool wave_bad = __builtin_amdgcn_ballot_w64(bad) != 0ull;
         __syncthreads();  // the area has been read
         if (lane == 0) *reinterpret_cast<uint32_t *>(lds + kStatArea + wave * 4) = wave_bad ? 1u : 0u;
         __syncthreads();
@@ -518,7 +521,7 @@ struct PrefillPair {
         const uint32_t head = row_head * p.pack + (row - token * p.pack);
         const float inv = 1.0f / l;
         const uint64_t at = ((uint64_t)token * p.query_heads + head) * kDim + half * 128 + g * 4;
-        bool bad = false;
+        bool bad = !isfinite(l);  // (an infinite sum would publish zeros)
 #pragma unroll
         for (int db = 0; db < kDimBlocks; ++db)
 #pragma unroll

@@ -295,3 +295,46 @@ def test_prefill_reports_a_run_of_keys_that_are_not_numbers(backend, d, tq, tk, 
     finally:
         for t in (out, lse, tq_, tk_, tv_, work):
             t.release()
+
+
+def far_above_first_tile(backend, cut, keys_of_the_sum, log2_sum):
+    """Rows whose later keys all have the same score, so far above the first 64 (score 0) that the
+    weights of `keys_of_the_sum` of them add up to 2^log2_sum relative to the first tile."""
+    rng = np.random.default_rng(5)
+    tq, tk, hq, hkv, d = 5, 1500, 12, 2, 256
+    # score = (64 q0 + q1) / 16: a step of q1 is 0.09 in log2 units; all of it whole bf16 numbers
+    units = round((log2_sum - np.log2(keys_of_the_sum)) * 16.0 * np.log(2.0))
+    q, k = np.zeros((tq, hq, d), np.float32), np.zeros((tk, hkv, d), np.float32)
+    q[:, :, 0], q[:, :, 1] = units // 64, units % 64
+    k[64:, :, 0], k[64:, :, 1] = 64.0, 1.0
+    # small signed values: the accumulators stay finite where the row sum does not
+    v = 0.02 * rng.standard_normal((tk, hkv, d)) + np.where(np.arange(tk) < 192, 0.06, -0.04)[:, None, None]
+    q, k, v = (ORACLE.bf16_encode(x.astype(np.float32)) for x in (q, k, v))
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, causal=True, query_start=tk - tq, dtype=B.DTYPE_BF16,
+                                        contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+    need = backend.attention_workspace_required(req)
+    out, lse = backend.tensor("o", B.DTYPE_BF16, q.shape), backend.tensor("lse", B.DTYPE_F32, (tq, hq))
+    tensors = [backend.tensor(n, B.DTYPE_BF16, x.shape, x) for n, x in (("q", q), ("k", k), ("v", v))]
+    work = backend.tensor("w", B.DTYPE_I8, (need,))
+    if cut:
+        backend.workspace_attach(work)
+    try:
+        facts = backend.attention_execute(req, *tensors, out, lse=lse)
+    finally:
+        if cut:
+            backend.workspace_detach()
+    assert facts.kernel_launches == (2 if cut else 1)
+    rc, ref, _, ref_lse = ORACLE.gqa_bf16(q, k, v, query_start=tk - tq, causal=True)
+    assert rc == 0
+    label = "2^%.1f %s" % (log2_sum, "cut" if cut else "whole")
+    assert_close_bf16(out.read(), ref, label)
+    assert_lse(lse.read(), ref_lse, label)
+    for t in [out, lse, work] + tensors:
+        t.release()
+
+
+@pytest.mark.parametrize("log2_sum", [float(x) for x in np.arange(125.0, 131.5, 0.5)])
+def test_prefill_row_sums_about_the_largest_float(backend, log2_sum):
+    """Sums that a float just holds and just does not, spread over the lanes and waves that share a
+    row (each holds a quarter, which is finite up to 2^130)."""
+    far_above_first_tile(backend, False, 1500 - 5 - 64, log2_sum)
