@@ -552,10 +552,12 @@ struct PrefillPair {
     }
     __device__ inline void leave_partial(uint32_t slot, int rb, float l) const
     {
-        // the sum is brought into [1, 2) by a whole power of two, so that the merge's weights are
-        // relative to the row's own magnitude
+        // the sum is brought into [1, 2) (the largest into [2, 4)) by a whole power of two, so that the
+        // merge's weights are relative to the row's own magnitude; fast_exp2 has no subnormal results:
+        // 2^-126 is the least factor
         const bool none = !(l > 0.f);
-        const float shift = none || !isfinite(l) ? 0.f : __builtin_floorf(fast_log2(l)), factor = fast_exp2(-shift);
+        const float shift = none || !isfinite(l) ? 0.f : fminf(__builtin_floorf(fast_log2(l)), 126.f);
+        const float factor = fast_exp2(-shift);
         if (g == 0 && half == 0) leave_statistics(slot, rb, l * factor, none && l == 0.f ? -INFINITY : ref[rb] + shift);
         const uint64_t at = (uint64_t)slot * kRowsPerBlock + pair * 64 + rb * 32 + n;
         float *acc = p.part_acc + at * kDim + half * 128 + g * 4;

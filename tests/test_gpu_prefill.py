@@ -338,3 +338,10 @@ def test_prefill_row_sums_about_the_largest_float(backend, log2_sum):
     """Sums that a float just holds and just does not, spread over the lanes and waves that share a
     row (each holds a quarter, which is finite up to 2^130)."""
     far_above_first_tile(backend, False, 1500 - 5 - 64, log2_sum)
+
+
+@pytest.mark.parametrize("log2_sum", [float(x) for x in np.arange(125.0, 131.5, 0.5)])
+def test_prefill_run_sums_about_the_largest_float(backend, log2_sum):
+    """The same in one run of a cut walk (the first, which alone starts below the other keys): its
+    partial is scaled by a power of two, and its share of the weights is a few per cent."""
+    far_above_first_tile(backend, True, 64, log2_sum)
