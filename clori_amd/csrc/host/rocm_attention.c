@@ -529,8 +529,7 @@ static int rocm_attention_workspace_required(const yvex_transformer_attention_re
             return refuse(err, YVEX_ERR_BOUNDS, where, "decode workspace geometry overflowed");
         *bytes = total;
     } else if (r->numeric_contract == YVEX_TRANSFORMER_ATTENTION_NUMERIC_BF16_F32_ACCUMULATE) {
-        if (!yvex_rocm_prefill_workspace(r, bytes))
-            return refuse(err, YVEX_ERR_BOUNDS, where, "prefill workspace geometry overflowed");
+        *bytes = yvex_rocm_prefill_workspace(r);
     } else {
         unsigned long long per_run;
         const unsigned long long runs = exact_split_runs(r, &per_run);

@@ -51,17 +51,19 @@ static unsigned long long tail_cost(const yvex_transformer_attention_requirement
     return cost;
 }
 
-/* Returns 0 when a product overflows. */
+/* Returns 0 when the request is past the launch range: 65535 query heads or tiles of 128 tokens,
+ * 2^31 - 1 (head, tile) pairs (so that rows stay below 2^27). */
 static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
 {
+    const unsigned long long token_tiles = (r->query_tokens + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
     unsigned long long items, steps, splits, best, slots;
     memset(plan, 0, sizeof(*plan));
-    plan->pack = r->query_heads / r->key_value_heads;
-    if (r->query_tokens == 1ull || r->query_tokens * plan->pack >= YVEX_ROCM_PREFILL_PACKED_ROWS_MAX) plan->pack = 1ull;
+    if (r->query_heads > 65535ull || token_tiles > 65535ull || r->query_heads * token_tiles > 0x7fffffffull) return 0;
+    plan->pack = r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads;
     plan->row_heads = r->query_heads / plan->pack;
-    if (!yvex_core_u64_mul(r->query_tokens, plan->pack, &plan->rows) || plan->rows > 0x7fffffffull) return 0;
+    plan->rows = r->query_tokens * plan->pack;
     plan->query_tiles = (plan->rows + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
-    if (!yvex_core_u64_mul(plan->query_tiles, plan->row_heads, &items) || items > 0x7fffffffull) return 0;
+    items = plan->query_tiles * plan->row_heads;
     plan->whole_items = items;
     plan->splits = 1ull;
     if (!may_split || r->query_tokens == 1ull || items % PREFILL_UNITS == 0ull) return 1;
@@ -87,13 +89,12 @@ static int prefill_plan_make(const yvex_transformer_attention_requirement *r, in
     return 1;
 }
 
-/* Bytes of the partials of a request (0: its walks are not cut). */
-int yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r, unsigned long long *bytes)
+/* Bytes of the partials of a request (0: its walks are not cut, or the execution will refuse it). */
+unsigned long long yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r)
 {
     prefill_plan plan;
-    if (!prefill_plan_make(r, 1, &plan)) return 0;
-    *bytes = plan.acc_bytes + plan.ml_bytes; /* both multiples of the 1 KB that 128 rows take */
-    return 1;
+    /* both multiples of the 1 KB that 128 rows take */
+    return prefill_plan_make(r, 1, &plan) ? plan.acc_bytes + plan.ml_bytes : 0ull;
 }
 
 static yvex_rocm_function_id by_head_dimension(unsigned long long d, yvex_rocm_function_id at_64,
@@ -116,7 +117,7 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
     prefill_plan plan;
     int rc;
     /* the kernel addresses K and V through 32-bit buffer offsets */
-    if (r->query_heads > 65535ull || r->key_value_tokens * g->k_stride * 2ull >= 0xffffffffull ||
+    if (r->key_value_tokens * g->k_stride * 2ull >= 0xffffffffull ||
         r->key_value_tokens * g->v_stride * 2ull >= 0xffffffffull || !prefill_plan_make(r, 1, &plan)) {
         yvex_error_set(err, YVEX_ERR_BOUNDS, "rocm.transformer.attention",
                        "prefill geometry exceeds admitted launch range");

@@ -257,7 +257,7 @@ typedef struct {
 } yvex_rocm_attention_geometry;
 /* rocm_prefill.c: the BF16 contract over more than one query row (or a geometry the decode teams
  * do not take), on the MFMA prefill kernels */
-int yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r, unsigned long long *bytes);
+unsigned long long yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r);
 int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_attention_request *request,
                               yvex_device_tensor *lse, const yvex_device_tensor *gate,
                               const yvex_rocm_attention_geometry *g, yvex_backend_operation_facts *facts,

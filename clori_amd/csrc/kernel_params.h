@@ -216,11 +216,9 @@ typedef struct {
     const uint16_t *gate; /* optional bf16 [Tq][Hq][head_dim] sigmoid output gate */
     float *part_acc, *part_ml;
     uint32_t whole_items, tail_items, splits, row_heads;
-    uint32_t pack_inverse; /* ceil(2^32 / pack); unused when pack = 1, rows < 2^28 otherwise */
+    uint32_t pack_inverse; /* ceil(2^32 / pack); unused when pack = 1, rows < 2^27 otherwise */
     uint32_t merge_groups; /* groups of threads that the merge deals a row's runs to: 1 or 4 */
 } yvex_rocm_prefill_params;
-
-#define YVEX_ROCM_PREFILL_PACKED_ROWS_MAX (1u << 28)
 
 /* Absorbed-latent MLA decode, split over the context.  A chunk spans at most
  * YVEX_ROCM_MLA_MAX_CHUNK_PAGES pages (a bound of the host's partition; the kernel reads the

@@ -814,6 +814,25 @@ def test_paged_and_mla_admission():
         assert e.value.code == B.YVEX_ERR_UNSUPPORTED
 
 
+def test_prefill_past_the_launch_range_is_refused():
+    """65535 tiles of 128 query tokens are the most a bf16 prefill takes; the workspace query of a
+    request that its execution refuses answers 0."""
+    tokens = 65535 * 128 + 1
+    with Backend() as b:
+        rows = b.tensor("rows", B.DTYPE_BF16, (tokens, 1, 64))
+        rows.handle.contents.is_written = 1  # a gigabyte that nothing touches
+        out = b.tensor("o", B.DTYPE_BF16, (tokens, 1, 64))
+        req = b.attention_requirement(tokens, tokens, 1, 1, 64, causal=False, dtype=B.DTYPE_BF16,
+                                      contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+        assert b.attention_workspace_required(req) == 0
+        with pytest.raises(YvexError) as e:
+            b.attention_execute(req, rows, rows, rows, out)
+        assert e.value.code == B.YVEX_ERR_BOUNDS and not out.is_written
+        wide = b.attention_requirement(2**31 - 1, 2**31 - 1, 1024, 1024, 64, dtype=B.DTYPE_BF16,
+                                       contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+        assert b.attention_workspace_required(wide) == 0
+
+
 def test_paged_decode_workspace_holds_the_offsets_of_the_second_launch():
     """Partials and statistics of two slots per wave, and wherever a second launch merges them (head
     dimensions 64 and 256 always) the offsets of every session behind them."""
