@@ -19,7 +19,19 @@
 #include <math.h>
 #include <string.h>
 
-enum { PREFILL_UNITS = 256, PREFILL_STEP_KEYS = 64, PREFILL_SPLITS_MAX = 64, PREFILL_RUN_STEPS_MIN = 2 };
+enum {
+    PREFILL_UNITS = 256,
+    PREFILL_STEP_KEYS = 64,
+    PREFILL_SPLITS_MAX = 64,
+    PREFILL_RUN_STEPS_MIN = 2,
+    /* Bytes of partial rows a request may ask for.  Runs past it are many runs of many items, whose
+     * predicted gain is small and whose partials cost more than predicted (24/4 heads of 256, before
+     * with 32, 16 and 7 runs / now: 1316 tokens behind 803329 21.8 / 20.9 ms, 2631 behind 342689 18.4 /
+     * 18.1, 736 behind 25193 476 / 461 us; 686 behind 346068, 23 runs in 401 MB, 5.2 / 5.6 ms).  A
+     * threshold on the predicted gain would be wrong: 17 tokens of 16/4 heads of 64 behind 867 are to
+     * gain 1.4 % and take 8.9 us instead of 13.1. */
+    PREFILL_PARTIALS_MAX = 96 << 20
+};
 
 typedef struct prefill_plan {
     unsigned long long pack, row_heads, rows, query_tiles, whole_items, tail_items, splits;
@@ -56,7 +68,7 @@ static unsigned long long tail_cost(const yvex_transformer_attention_requirement
 static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
 {
     const unsigned long long token_tiles = (r->query_tokens + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
-    unsigned long long items, steps, splits, best, slots;
+    unsigned long long items, steps, splits, best, slots, run_bytes;
     memset(plan, 0, sizeof(*plan));
     if (r->query_heads > 65535ull || token_tiles > 65535ull || r->query_heads * token_tiles > 0x7fffffffull) return 0;
     plan->pack = r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads;
@@ -70,8 +82,10 @@ static int prefill_plan_make(const yvex_transformer_attention_requirement *r, in
     plan->whole_items = items / PREFILL_UNITS * PREFILL_UNITS;
     plan->tail_items = items - plan->whole_items;
     steps = item_steps(r, plan, plan->query_tiles - 1ull - plan->whole_items / plan->row_heads);
+    run_bytes = plan->tail_items * YVEX_ROCM_PREFILL_ROWS * r->head_dimension * sizeof(float);
     best = tail_cost(r, plan, steps, 1ull);
-    for (splits = 2ull; splits <= PREFILL_SPLITS_MAX && splits * PREFILL_RUN_STEPS_MIN <= steps; ++splits) {
+    for (splits = 2ull; splits <= PREFILL_SPLITS_MAX && splits * PREFILL_RUN_STEPS_MIN <= steps &&
+                        splits * run_bytes <= PREFILL_PARTIALS_MAX; ++splits) {
         const unsigned long long cost = tail_cost(r, plan, steps, splits);
         if (cost < best) {
             best = cost;

@@ -833,6 +833,25 @@ def test_prefill_past_the_launch_range_is_refused():
         assert b.attention_workspace_required(wide) == 0
 
 
+@pytest.mark.parametrize("tokens,start,hq,hkv,d,runs", [
+    (9, 12001, 40, 8, 128, 32),      # one item per kv head
+    (2000, 13333, 24, 4, 256, 2),    # 120 items behind a whole turn
+    (736, 25193, 24, 4, 256, 5),     # seven runs would take 123 MB
+    (1316, 803329, 24, 4, 256, 1),   # 32 runs: a gigabyte for 0.3 %, three runs nothing
+    (2631, 342689, 24, 4, 256, 1),   # 16 runs: 507 MB for 3 %
+    (686, 346068, 24, 4, 256, 5),    # 23 runs: 401 MB
+    (17, 867, 16, 4, 64, 7),         # 0.9 MB
+])
+def test_prefill_workspace_is_bounded(tokens, start, hq, hkv, d, runs):
+    """The partial rows of a cut prefill stay within 96 MiB."""
+    with Backend() as b:
+        r = b.attention_requirement(tokens, start + tokens, hq, hkv, d, query_start=start, dtype=B.DTYPE_BF16,
+                                    contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+        items = -(-tokens * (hq // hkv) // 128) * hkv % 256
+        need = items * runs * 128 * (d + 2) * 4 if runs > 1 else 0
+        assert b.attention_workspace_required(r) == need <= (96 << 20) * (d + 2) // d
+
+
 def test_paged_decode_workspace_holds_the_offsets_of_the_second_launch():
     """Partials and statistics of two slots per wave, and wherever a second launch merges them (head
     dimensions 64 and 256 always) the offsets of every session behind them."""
