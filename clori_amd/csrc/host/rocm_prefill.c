@@ -9,9 +9,12 @@
  * launch merges the runs.  Nine tokens of 40/8 heads of 128 behind 12001: one tile per query head
  * walked 188 steps on 40 units, 160 us; packed and cut into 256 runs, 17.4 us. 2000 tokens of 24/4
  * heads of 256 behind 13333: 376 items took two turns of 256 units with half of the second empty,
- * 1182 us; with its tail cut, 873 (both with the kernel that prefill_pair.hip has replaced).  A
+ * 1182 us; with its tail cut, 873 (both with one wave per 32 rows; prefill_pair.hip has 634).  A
  * prompt of 2048 tokens without a history is not cut and gains from the packing only that a tile
- * spans 26 tokens instead of 128 (50.6 -> 50.2 us).
+ * spans 26 tokens instead of 128 (50.6 -> 50.2 us).  Walks that are not cut and all start at once are
+ * packed only where that does not put them into fewer workgroups: packed / one query head to a tile,
+ * us, 40 tokens of 40/8 heads of 128 7.5 / 6.5, 300 11.4 / 10.7, 20 behind 200 9.7 / 8.9;
+ * with as many workgroups either way 500 behind 500 of 16/4 of 64 15.9 / 16.1.
  * The cut is a function of the request's geometry only (256 units, never the device), so that the
  * planner's workspace_required and the execution agree. */
 #include "rocm_state.h"
@@ -63,22 +66,24 @@ static unsigned long long tail_cost(const yvex_transformer_attention_requirement
     return cost;
 }
 
-/* Returns 0 when the request is past the launch range: 65535 query heads or tiles of 128 tokens,
- * 2^31 - 1 (head, tile) pairs (so that rows stay below 2^27). */
-static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
+/* Every walk whole, `pack` query heads to a row head. */
+static void plan_whole(const yvex_transformer_attention_requirement *r, unsigned long long pack, prefill_plan *plan)
 {
-    const unsigned long long token_tiles = (r->query_tokens + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
-    unsigned long long items, steps, splits, best, slots, run_bytes;
     memset(plan, 0, sizeof(*plan));
-    if (r->query_heads > 65535ull || token_tiles > 65535ull || r->query_heads * token_tiles > 0x7fffffffull) return 0;
-    plan->pack = r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads;
-    plan->row_heads = r->query_heads / plan->pack;
-    plan->rows = r->query_tokens * plan->pack;
+    plan->pack = pack;
+    plan->row_heads = r->query_heads / pack;
+    plan->rows = r->query_tokens * pack;
     plan->query_tiles = (plan->rows + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
-    items = plan->query_tiles * plan->row_heads;
-    plan->whole_items = items;
+    plan->whole_items = plan->query_tiles * plan->row_heads;
     plan->splits = 1ull;
-    if (!may_split || r->query_tokens == 1ull || items % PREFILL_UNITS == 0ull) return 1;
+}
+
+/* Cuts the walks of the items past a multiple of the units where that is predicted to take less time. */
+static void plan_cut(const yvex_transformer_attention_requirement *r, prefill_plan *plan)
+{
+    const unsigned long long items = plan->whole_items;
+    unsigned long long steps, splits, best, slots, run_bytes;
+    if (items % PREFILL_UNITS == 0ull) return;
     plan->whole_items = items / PREFILL_UNITS * PREFILL_UNITS;
     plan->tail_items = items - plan->whole_items;
     steps = item_steps(r, plan, plan->query_tiles - 1ull - plan->whole_items / plan->row_heads);
@@ -95,11 +100,27 @@ static int prefill_plan_make(const yvex_transformer_attention_requirement *r, in
     if (plan->splits == 1ull) {
         plan->whole_items = items;
         plan->tail_items = 0ull;
-        return 1;
+        return;
     }
     slots = plan->tail_items * plan->splits * YVEX_ROCM_PREFILL_ROWS;
     plan->acc_bytes = slots * r->head_dimension * sizeof(float);
     plan->ml_bytes = slots * 2ull * sizeof(float);
+}
+
+/* Returns 0 when the request is past the launch range: 65535 query heads or tiles of 128 tokens,
+ * 2^31 - 1 (head, tile) pairs (so that rows stay below 2^27). */
+static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
+{
+    const unsigned long long token_tiles = (r->query_tokens + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
+    if (r->query_heads > 65535ull || token_tiles > 65535ull || r->query_heads * token_tiles > 0x7fffffffull) return 0;
+    plan_whole(r, r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads, plan);
+    if (may_split && r->query_tokens > 1ull) plan_cut(r, plan);
+    if (plan->splits == 1ull && r->query_tokens > 1ull && r->query_heads * token_tiles <= PREFILL_UNITS) {
+        /* Every walk has a unit of its own either way; one query head to a tile then means as many
+         * steps in more workgroups of fewer live waves. */
+        if (r->head_dimension != 256ull && r->query_heads * token_tiles > plan->whole_items)
+            plan_whole(r, 1ull, plan);
+    }
     return 1;
 }
 
@@ -177,8 +198,8 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
     params.part_acc = (float *)(uintptr_t)work;
     params.part_ml = (float *)(uintptr_t)(work + plan.acc_bytes);
     rc = yvex_rocm_launch(backend,
-                          by_head_dimension(r->head_dimension, YVEX_ROCM_FN_PREFILL_BF16_64,
-                                            YVEX_ROCM_FN_PREFILL_BF16, YVEX_ROCM_FN_PREFILL_BF16_256),
+                          by_head_dimension(r->head_dimension, YVEX_ROCM_FN_PREFILL_BF16_64, YVEX_ROCM_FN_PREFILL_BF16,
+                                            YVEX_ROCM_FN_PREFILL_BF16_256),
                           variant, (unsigned int)(plan.whole_items + plan.tail_items * plan.splits), 1u, 1u, 256u,
                           0u, &params, where, err);
     if (rc == YVEX_OK && plan.splits > 1ull)

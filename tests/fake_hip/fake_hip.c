@@ -22,6 +22,7 @@ static int capturing;                       /* a stream capture is open */
 static unsigned long long captured_launches;
 
 static unsigned int last_grid_x;
+static const char *last_function;
 static unsigned char last_params[512];
 unsigned long long fake_hip_launches(void) { return launches; }
 /* launches that carried a batch of queued copies, and copies handed to the runtime one by one */
@@ -32,6 +33,7 @@ unsigned long long fake_hip_small_transfers(void) { return small_transfers; }
 /* status words handed to the host through its mailbox */
 unsigned long long fake_hip_status_forwards(void) { return forwards; }
 unsigned int fake_hip_last_grid_x(void) { return last_grid_x; }
+const char *fake_hip_last_function(void) { return last_function; }
 /* the bytes kept of the last launch's parameter struct */
 const unsigned char *fake_hip_last_params(void) { return last_params; }
 unsigned long long fake_hip_live_allocations(void) { return allocations - frees; }
@@ -227,6 +229,7 @@ hipError_t hipModuleLaunchKernel(hipFunction_t f, unsigned int gx, unsigned int 
     /* the last launch's grid width and the head of its one by-value parameter, for tests that
      * look at what the host handed to a kernel */
     last_grid_x = gx;
+    last_function = (const char *)f;
     {
         /* FAKE_HIP_PARAM_BYTES: how many bytes of the parameter struct the test wants kept (it
          * knows the struct it expects; nothing is read unless it asks) */

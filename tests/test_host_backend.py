@@ -833,6 +833,29 @@ def test_prefill_past_the_launch_range_is_refused():
         assert b.attention_workspace_required(wide) == 0
 
 
+@pytest.mark.parametrize("tokens,start,hq,hkv,d,pack,grid", [
+    (40, 0, 40, 8, 128, 1, 40),     # packed: 16 workgroups
+    (300, 0, 40, 8, 128, 1, 120),   # 96
+    (20, 20, 16, 4, 64, 1, 16),     # 4
+    (512, 0, 32, 8, 128, 4, 128),   # as many either way
+    (700, 0, 48, 8, 128, 6, 264),   # 288 would not all start at once
+    (40, 0, 24, 4, 256, 6, 8),      # pairs of waves take whole tiles
+])
+def test_prefill_whole_walks_are_spread_over_the_units(fake_runtime, env, tokens, start, hq, hkv, d, pack, grid):
+    """Whole walks that all start at once have one query head to a tile where that makes more
+    workgroups of them."""
+    fake_runtime.fake_hip_last_grid_x.restype = C.c_uint
+    fake_runtime.fake_hip_last_params.restype = C.POINTER(C.c_ubyte)
+    env("FAKE_HIP_PARAM_BYTES", "96")
+    with Backend() as b:
+        req = b.attention_requirement(tokens, start + tokens, hq, hkv, d, query_start=start, dtype=B.DTYPE_BF16,
+                                      contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+        q, k = written(b, "q", B.DTYPE_BF16, (tokens, hq, d)), written(b, "k", B.DTYPE_BF16, (start + tokens, hkv, d))
+        b.attention_execute(req, q, k, k, b.tensor("o", B.DTYPE_BF16, (tokens, hq, d)))
+        assert fake_runtime.fake_hip_last_grid_x() == grid
+        assert int.from_bytes(bytes(fake_runtime.fake_hip_last_params()[92:96]), "little") == pack
+
+
 @pytest.mark.parametrize("tokens,start,hq,hkv,d,runs", [
     (9, 12001, 40, 8, 128, 32),      # one item per kv head
     (2000, 13333, 24, 4, 256, 2),    # 120 items behind a whole turn
