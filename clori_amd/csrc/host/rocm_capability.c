@@ -80,6 +80,8 @@ static const rocm_kernel_binding rocm_kernel_bindings[] = {
      YVEX_ROCM_FN_PREFILL_BF16_64},
     {"yvex_rocm_prefill_bf16_256", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16,
      YVEX_ROCM_FN_PREFILL_BF16_256},
+    {"yvex_rocm_prefill_bf16_256_short", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16,
+     YVEX_ROCM_FN_PREFILL_BF16_256_SHORT},
     {"yvex_rocm_prefill_merge", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16, YVEX_ROCM_FN_PREFILL_MERGE},
     {"yvex_rocm_prefill_merge_64", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_BF16,
      YVEX_ROCM_FN_PREFILL_MERGE_64},

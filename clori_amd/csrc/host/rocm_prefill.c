@@ -13,8 +13,8 @@
  * prompt of 2048 tokens without a history is not cut and gains from the packing only that a tile
  * spans 26 tokens instead of 128 (50.6 -> 50.2 us).  Walks that are not cut and all start at once are
  * packed only where that does not put them into fewer workgroups: packed / one query head to a tile,
- * us, 40 tokens of 40/8 heads of 128 7.5 / 6.5, 300 11.4 / 10.7, 20 behind 200 9.7 / 8.9;
- * with as many workgroups either way 500 behind 500 of 16/4 of 64 15.9 / 16.1.
+ * us, 40 tokens of 40/8 heads of 128 7.5 / 6.5, 300 11.4 / 10.7, 20 behind 200 9.7 / 8.9, 21 of 24/4 of
+ * 256 11.6 / 9.7; with as many workgroups either way 500 behind 500 of 16/4 of 64 15.9 / 16.1.
  * The cut is a function of the request's geometry only (256 units, never the device), so that the
  * planner's workspace_required and the execution agree. */
 #include "rocm_state.h"
@@ -39,6 +39,7 @@ enum {
 typedef struct prefill_plan {
     unsigned long long pack, row_heads, rows, query_tiles, whole_items, tail_items, splits;
     unsigned long long acc_bytes, ml_bytes; /* partials of the tail */
+    int short_walks; /* head dimension 256: on the kernel for those */
 } prefill_plan;
 
 /* Steps of an item of query tile `q_tile`. */
@@ -107,6 +108,16 @@ static void plan_cut(const yvex_transformer_attention_requirement *r, prefill_pl
     plan->ml_bytes = slots * 2ull * sizeof(float);
 }
 
+/* Whole walks of so few steps, at head dimension 256, that the pairs of prefill_pair.hip cost more to
+ * start and end than they save per step: up to seven steps, four where few tokens leave the other
+ * kernel's waves without rows.  One wave per 32 rows / pairs, us, 24/4 heads: 128 tokens 15.0 / 19.2,
+ * 256 19.7 / 22.7, 448 24.7 / 26.8, 513 (nine steps) 29.3 / 29.8, 700 36.5 / 33.6; 60 behind 150 18.1 /
+ * 22.2, 120 behind 260 23.8 / 25.1, 128 behind 380 (eight) 28.5 / 28.0, 10 behind 200 17.4 / 17.1. */
+static int walks_are_short(const yvex_transformer_attention_requirement *r, const prefill_plan *plan)
+{
+    return item_steps(r, plan, plan->query_tiles - 1ull) <= (r->query_tokens >= 64ull ? 7ull : 4ull);
+}
+
 /* Returns 0 when the request is past the launch range: 65535 query heads or tiles of 128 tokens,
  * 2^31 - 1 (head, tile) pairs (so that rows stay below 2^27). */
 static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
@@ -116,10 +127,12 @@ static int prefill_plan_make(const yvex_transformer_attention_requirement *r, in
     plan_whole(r, r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads, plan);
     if (may_split && r->query_tokens > 1ull) plan_cut(r, plan);
     if (plan->splits == 1ull && r->query_tokens > 1ull && r->query_heads * token_tiles <= PREFILL_UNITS) {
+        const int short_walks = r->head_dimension == 256ull && walks_are_short(r, plan);
         /* Every walk has a unit of its own either way; one query head to a tile then means as many
          * steps in more workgroups of fewer live waves. */
-        if (r->head_dimension != 256ull && r->query_heads * token_tiles > plan->whole_items)
+        if ((r->head_dimension != 256ull || short_walks) && r->query_heads * token_tiles > plan->whole_items)
             plan_whole(r, 1ull, plan);
+        plan->short_walks = short_walks;
     }
     return 1;
 }
@@ -199,7 +212,8 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
     params.part_ml = (float *)(uintptr_t)(work + plan.acc_bytes);
     rc = yvex_rocm_launch(backend,
                           by_head_dimension(r->head_dimension, YVEX_ROCM_FN_PREFILL_BF16_64, YVEX_ROCM_FN_PREFILL_BF16,
-                                            YVEX_ROCM_FN_PREFILL_BF16_256),
+                                            plan.short_walks ? YVEX_ROCM_FN_PREFILL_BF16_256_SHORT
+                                                             : YVEX_ROCM_FN_PREFILL_BF16_256),
                           variant, (unsigned int)(plan.whole_items + plan.tail_items * plan.splits), 1u, 1u, 256u,
                           0u, &params, where, err);
     if (rc == YVEX_OK && plan.splits > 1ull)

@@ -38,6 +38,7 @@ typedef enum {
     YVEX_ROCM_FN_PREFILL_BF16,
     YVEX_ROCM_FN_PREFILL_BF16_64,
     YVEX_ROCM_FN_PREFILL_BF16_256,
+    YVEX_ROCM_FN_PREFILL_BF16_256_SHORT,
     YVEX_ROCM_FN_PREFILL_MERGE,
     YVEX_ROCM_FN_PREFILL_MERGE_64,
     YVEX_ROCM_FN_PREFILL_MERGE_256,

@@ -1,8 +1,8 @@
 // Causal / full grouped-query attention prefill for gfx950 (wave64), bf16 in and out,
 // fp32 scores, online softmax and accumulation.  Token-major tensors ([token][head][dim],
-// per-token strides in elements); head_dim 128 is the tuned build, 64 is the same code with other
-// counts (the numbers in this comment are those of 128), 256 has a kernel of its own
-// (prefill_pair.hip), merged by the merge at the end of this file.
+// per-token strides in elements); head_dim 128 is the tuned build, 64 and 256 are the same code with
+// other counts (the numbers in this comment are those of 128).  256 has a kernel of its own
+// (prefill_pair.hip) for all but short walks; its runs are merged by the merge at the end of this file.
 //
 // A workgroup of 4 waves owns one (query head, 128-row query tile): each wave owns
 // 32 query rows and walks the key/value tokens in tiles of 64 that the workgroup
@@ -66,7 +66,7 @@ constexpr int kDepth = 4;  // operand fetches in flight ahead of the MFMA that c
 typedef __attribute__((address_space(3))) short4v lds_short4;
 
 // Chunk swizzle of tile row r: the 16-byte chunk c of the row sits at chunk position c ^ x(r).
-// Rows of 256 bytes all start in the same bank, x(r) permutes the 16 chunk
+// Rows of 256 and of 512 bytes all start in the same bank, x(r) permutes the 16 chunk
 // positions of a 256-byte bank span by the row's low four bits (rows r..r+3 go four chunks
 // apart, which is what the transposed read needs; 16 consecutive rows take 16 different
 // positions, which is what the row read needs).  Rows of 128 bytes (head_dim 64) alternate
@@ -107,7 +107,7 @@ struct Prefill {
     static constexpr int kLoadRows = 64 / kRowChunks;         // tile rows one 1 KB load covers
     static constexpr int kSoftmaxSlots = 3 * kSlots / 4;      // the exponentials ride behind these slots
     static constexpr int kMaxPerSlot = 32 / (kSlots - kSoftmaxSlots);
-    static_assert(kHeadDim == 64 || kHeadDim == 128, "head_dim 64 or 128");
+    static_assert(kHeadDim == 64 || kHeadDim == 128 || kHeadDim == 256, "head_dim 64, 128 or 256");
 
     const yvex_rocm_prefill_params &p;
     unsigned char *const lds;
@@ -250,7 +250,7 @@ struct Prefill {
         // ---- tile staging: buffer loads that write LDS directly -----------------------
         // 1 KB load j of wave w fills rows 16w + 4j .. +3 of the tile; lane L owns chunk
         // position L % 16 of row 16w + 4j + L / 16 and fetches chunk (L % 16) ^ x(row)
-        // (rows of 128 bytes: eight rows per load).
+        // (rows of 128 bytes: eight rows per load, of 512 bytes: two).
         k_row_bytes = (uint32_t)p.k_stride * 2u;
         v_row_bytes = (uint32_t)p.v_stride * 2u;
         k_rsrc = raw_buffer(p.k + (uint64_t)(uint32_t)first_key * p.k_stride + (uint64_t)kv_head * kHeadDim,
@@ -404,8 +404,11 @@ struct Prefill {
 #pragma unroll
                     for (int k4 = first; k4 < first + kMaxPerSlot; k4 += 4) {
                         const int mb = k4 >> 4, r = k4 & 15;
-                        mloc = fmaxf(fmaxf(mloc, s_next[mb][r]),
-                                     fmaxf(fmaxf(s_next[mb][r + 1], s_next[mb][r + 2]), s_next[mb][r + 3]));
+                        if (kMaxPerSlot >= 4)
+                            mloc = fmaxf(fmaxf(mloc, s_next[mb][r]),
+                                         fmaxf(fmaxf(s_next[mb][r + 1], s_next[mb][r + 2]), s_next[mb][r + 3]));
+                        else  // two at 256
+                            mloc = fmaxf(mloc, fmaxf(s_next[mb][r], s_next[mb][r + 1]));
                     }
                     asm volatile("" : "+v"(mloc));  // keeps this slice in its slot
                 }
@@ -489,9 +492,11 @@ struct Prefill {
 
 }  // namespace
 
-// grid = whole_items + tail_items * splits, block 256, LDS 2 x (K + V) tiles; two workgroups per CU.
-#define YVEX_PREFILL_KERNEL(name, head_dim)                                                               \
-    extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))          \
+// grid = whole_items + tail_items * splits, block 256, LDS 2 x (K + V) tiles.  `waves`: waves per SIMD
+// the register budget is sized for: two workgroups per CU for head_dim 64 and 128; head_dim 256 keeps
+// 128 accumulator, 64 query and 64 score registers per lane and its tiles fill 128 KB of LDS: one.
+#define YVEX_PREFILL_KERNEL(name, head_dim, waves)                                                        \
+    extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves, waves)))  \
     name(const yvex_rocm_prefill_params p)                                                                \
     {                                                                                                     \
         static_assert(YVEX_ROCM_PREFILL_ROWS == kRowsPerBlock, "host and kernel agree on the query tile"); \
@@ -499,8 +504,9 @@ struct Prefill {
         Prefill<head_dim>(p, lds).run();                                                                  \
     }
 
-YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128)
-YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64)
+YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128, 2)
+YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64, 2)
+YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_256_short, 256, 1)
 
 // Log-sum-exp merge of the runs of the split items and publication of their rows.  head_dim / 4
 // threads per row and group, four lanes of the row each; the runs of a row are dealt to

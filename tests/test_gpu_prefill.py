@@ -217,6 +217,24 @@ def test_prefill_packed_heads_and_cut_walks(backend, d, tq, tk, start, hq, hkv, 
     assert_lse(lse.read(), ref_lse, label)
 
 
+@pytest.mark.parametrize("tq,tk,start,hq,hkv,causal", [
+    (2, 3, 1, 12, 2, True),         # one step, two rows of one wave
+    (130, 130, 0, 6, 1, True),      # a second tile of two tokens
+    (63, 256, 193, 24, 4, True),    # four steps below 64 tokens
+    (200, 447, 247, 6, 3, False),   # seven, every row up to a ragged end
+    (448, 448, 0, 24, 4, True),     # seven
+    (449, 449, 0, 4, 4, True),      # eight: pairs of waves
+])
+def test_prefill_short_walks_at_head_dimension_256(backend, tq, tk, start, hq, hkv, causal):
+    rng = np.random.default_rng(tq + tk)
+    q, k, v = (bf16_normal(rng, shape) for shape in ((tq, hq, 256), (tk, hkv, 256), (tk, hkv, 256)))
+    got, lse, facts = run_prefill(backend, q, k, v, query_start=start, causal=causal)
+    rc, ref, _, ref_lse = ORACLE.gqa_bf16(q, k, v, query_start=start, causal=causal)
+    assert rc == 0 and facts.kernel_launches == 1
+    assert_close_bf16(got, ref, "short tq=%d tk=%d" % (tq, tk))
+    assert_lse(lse, ref_lse, "short tq=%d tk=%d" % (tq, tk))
+
+
 @pytest.mark.parametrize("tq,tk,start,hq,hkv,cut", [(70, 70, 0, 2, 1, False), (5, 1500, 1495, 12, 2, True),
                                                     (200, 1000, 800, 4, 2, False)])
 def test_prefill_scores_far_above_the_first_tiles(backend, tq, tk, start, hq, hkv, cut):

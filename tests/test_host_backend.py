@@ -839,7 +839,8 @@ def test_prefill_past_the_launch_range_is_refused():
     (20, 20, 16, 4, 64, 1, 16),     # 4
     (512, 0, 32, 8, 128, 4, 128),   # as many either way
     (700, 0, 48, 8, 128, 6, 264),   # 288 would not all start at once
-    (40, 0, 24, 4, 256, 6, 8),      # pairs of waves take whole tiles
+    (21, 0, 24, 4, 256, 1, 24),     # 4 of the kernel for short walks
+    (513, 0, 24, 4, 256, 6, 100),   # nine steps: pairs of waves take whole tiles
 ])
 def test_prefill_whole_walks_are_spread_over_the_units(fake_runtime, env, tokens, start, hq, hkv, d, pack, grid):
     """Whole walks that all start at once have one query head to a tile where that makes more
@@ -854,6 +855,24 @@ def test_prefill_whole_walks_are_spread_over_the_units(fake_runtime, env, tokens
         b.attention_execute(req, q, k, k, b.tensor("o", B.DTYPE_BF16, (tokens, hq, d)))
         assert fake_runtime.fake_hip_last_grid_x() == grid
         assert int.from_bytes(bytes(fake_runtime.fake_hip_last_params()[92:96]), "little") == pack
+
+
+@pytest.mark.parametrize("tokens,start,hq,hkv,d,name", [
+    (128, 0, 24, 4, 256, "256_short"), (448, 0, 24, 4, 256, "256_short"), (449, 0, 24, 4, 256, "256"),
+    (64, 384, 24, 4, 256, "256_short"), (63, 385, 24, 4, 256, "256"), (63, 193, 24, 4, 256, "256_short"),
+    (63, 194, 24, 4, 256, "256"), (500, 0, 96, 8, 256, "256"),
+    (1, 200, 32, 2, 256, "256"), (128, 0, 24, 4, 128, ""), (128, 0, 24, 4, 64, "64"),
+])
+def test_prefill_kernel_of_short_walks(fake_runtime, tokens, start, hq, hkv, d, name):
+    """Head dimension 256: whole walks of up to seven steps of 64 keys (four below 64 query tokens)
+    that all start at once have a kernel of their own."""
+    fake_runtime.fake_hip_last_function.restype = C.c_char_p
+    with Backend() as b:
+        req = b.attention_requirement(tokens, start + tokens, hq, hkv, d, query_start=start, dtype=B.DTYPE_BF16,
+                                      contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+        q, k = written(b, "q", B.DTYPE_BF16, (tokens, hq, d)), written(b, "k", B.DTYPE_BF16, (start + tokens, hkv, d))
+        assert b.attention_execute(req, q, k, k, b.tensor("o", B.DTYPE_BF16, (tokens, hq, d))).kernel_launches == 1
+        assert fake_runtime.fake_hip_last_function().decode() == "yvex_rocm_prefill_bf16" + (name and "_" + name)
 
 
 @pytest.mark.parametrize("tokens,start,hq,hkv,d,runs", [
