@@ -210,7 +210,11 @@ static int cut_fits_scratch(const decode_cut *cut, unsigned long long group, uns
  * at 256 26.1 / 23.1 (256 parts), 8 x 2000 at 128 14.5 / 13.4 (2000 waves).
  *
  * The entry that allocates nothing has the same cut, bit for bit: forms that need more than its
- * fixed scratch where the plain one (eight tiles, merged in the kernel) does not are left out. */
+ * fixed scratch where the plain one (eight tiles, merged in the kernel) does not are left out.  Where
+ * the plain one does not fit either, that entry refuses the request, and only the waves of fewer
+ * tiles are left out, whose partials cost more than they gain by then (16/1 heads of 256, 16 x 4096
+ * 24.7 / 22.0 with eight; 64/4 of 128 merged in the kernel / with a second launch, 1 x 32768 147.5 /
+ * 21.8, 12 x 4096 58.4 / 27.3, 8 x 8000 in Q8_0 86.6 / 24.8). */
 static decode_cut decode_cut_for(int paged, unsigned long long sessions, unsigned long long kv_heads,
                                  unsigned long long group, unsigned long long head_dim,
                                  unsigned long long max_context)
@@ -224,16 +228,20 @@ static decode_cut decode_cut_for(int paged, unsigned long long sessions, unsigne
     const unsigned long long parts = head_dim == 64ull ? 128ull : 64ull;
     decode_cut cut = {decode_wave_count(tiles, ROCM_DECODE_MIN_TILES), ROCM_DECODE_MIN_TILES, 0}, other;
     unsigned int fine;
+    int plain_fits;
     if (!paged) {
         cut.in_kernel = cut.waves < ROCM_DECODE_WAVES;
         return cut;
     }
+    other = cut;
+    other.in_kernel = 1;
+    plain_fits = cut_fits_scratch(&other, group, head_dim, sessions);
     /* the paged kernels of head dimensions 64 and 256 have the two-launch form only */
     if (head_dim == ROCM_MFMA_HEAD_DIM && cut.waves < ROCM_DECODE_WAVES)
         cut.in_kernel = max_context <= ROCM_DECODE_PARTS_IN_KERNEL * part_tokens ||
                         (max_context <= ROCM_DECODE_PARTS_FEW_WAVES * part_tokens &&
                          cut.waves <= ROCM_DECODE_FEW_WAVES) ||
-                        !cut_fits_scratch(&cut, group, head_dim, sessions);
+                        (plain_fits && !cut_fits_scratch(&cut, group, head_dim, sessions));
     for (fine = 2u; !cut.in_kernel && fine < cut.min_tiles; fine *= 2u) {
         other = cut;
         other.min_tiles = fine;
@@ -244,10 +252,7 @@ static decode_cut decode_cut_for(int paged, unsigned long long sessions, unsigne
     }
     /* partials that fit the scratch make room for the offsets behind them (the kernels cut the
      * work by whatever number of waves there is) */
-    other = cut;
-    other.in_kernel = 1;
-    if (cut.waves < ROCM_DECODE_WAVES && head_dim != ROCM_MFMA_HEAD_DIM &&
-        cut_fits_scratch(&other, group, head_dim, sessions))
+    if (cut.waves < ROCM_DECODE_WAVES && head_dim != ROCM_MFMA_HEAD_DIM && plain_fits)
         while (cut.waves > 1u && !cut_fits_scratch(&cut, group, head_dim, sessions)) --cut.waves;
     return cut;
 }

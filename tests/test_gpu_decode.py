@@ -467,3 +467,22 @@ def test_paged_decode_few_long_sessions(backend, d, hq, hkv, contexts, launches)
     assert_close_bf16(got, ref, "long paged d=%d %s" % (d, contexts))
     assert_lse(lse, ref_lse, "long paged d=%d %s" % (d, contexts))
     assert facts.kernel_launches == launches
+
+
+@pytest.mark.parametrize("d,hq,hkv,contexts", [
+    (128, 64, 4, [32000, 5]),        # 250 parts of a lone long session
+    (128, 64, 4, [4096, 2500] * 6),  # 1536 waves
+    (256, 16, 1, [4096, 700] * 8),   # 512 waves of eight tiles
+])
+def test_paged_decode_wide_groups_past_the_fixed_scratch(backend, d, hq, hkv, contexts):
+    """Sixteen query heads per kv head, more partials than the fixed scratch holds in any form: the
+    second launch merges them like any others."""
+    rng = np.random.default_rng(d + len(contexts))
+    q, k_rows, v_rows, table, ctx, pool_pages = make_paged_case(rng, contexts, hq, hkv, d=d)
+    got, lse, facts = run_paged(backend, q, k_rows, v_rows, table, ctx, hkv, pool_pages, max_context=max(contexts))
+    rc, ref, _, ref_lse = ORACLE.paged_decode(q, k_rows, v_rows, table, ctx, hkv, 16)
+    assert rc == 0
+    label = "wide group d=%d %d sessions" % (d, len(contexts))
+    assert_close_bf16(got, ref, label)
+    assert_lse(lse, ref_lse, label)
+    assert facts.kernel_launches == 2 and facts.temporary_bytes > 16 << 20

@@ -906,6 +906,24 @@ def test_paged_decode_workspace_holds_the_offsets_of_the_second_launch():
             assert b.paged_decode_workspace_required(r) >= partials + 4 * (sessions + 1)
 
 
+@pytest.mark.parametrize("sessions,hq,hkv,d,context,waves", [
+    (12, 64, 4, 128, 4096, 1536),  # neither form fits the fixed scratch
+    (1, 64, 4, 128, 32768, 1024),
+    (16, 16, 1, 256, 4096, 512),   # waves of four tiles do not fit it
+    (5, 32, 2, 128, 12800, 1000),  # both forms of eight tiles do
+    (2, 32, 2, 128, 4096, 256),    # waves of four tiles do
+])
+def test_paged_decode_cut_of_wide_groups(sessions, hq, hkv, d, context, waves):
+    """The merge inside the kernel is taken for the fixed scratch's sake only where that form fits it
+    and the other does not."""
+    with Backend() as b:
+        pages = sessions * (context // 16)
+        r = b.paged_requirement(sessions, hq, hkv, d, 16, pages, context // 16, context)
+        rows = 2 * waves * (hq // hkv)
+        need = -(-rows * d * 4 // 256) * 256 + -(-rows * 8 // 256) * 256 + -(-4 * (sessions + 1) // 256) * 256
+        assert b.paged_decode_workspace_required(r) == need
+
+
 def test_kv_append_admission():
     """Refusal order of the page writer: arguments, then geometry the kernels do not cover,
     then tensor views; one launch, both pools marked written."""
