@@ -196,10 +196,12 @@ static int cut_fits_scratch(const decode_cut *cut, unsigned long long group, uns
  * one is bound by launch latency and merges inside the decode kernel (arrival counters), where the
  * one wave that completes a segment merges its parts, eight per trip to memory.  That is worth
  * the launch it saves up to eight parts of the longest session (32/8 heads of 128, bf16 pages, in
- * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3)
- * and costs little up to seventeen while few waves are in flight (1 x 1536 10.5 / 9.8, 1 x 2048
- * 11.0 / 10.0); beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6
- * / 13.1, 1 x 4096 16.0 / 12.0, 1 x 16384 43.8 / 20.2).
+ * the kernel / with a second launch: 1 x 1024 tokens 9.3 / 10.0 us, 24 x 600 in Q8_0 14.7 / 16.3);
+ * beyond, it is the longest thing in the launch (16 x 1500 25.7 / 19.9, 8 x 2000 16.6 / 13.1, 1 x 4096
+ * 16.0 / 12.0, 1 x 16384 43.8 / 20.2).  Up to seventeen parts with few waves in flight it is kept as
+ * the form that such requests always had, one launch and no offsets, and not for its speed: with a
+ * second launch and waves of two tiles 1 x 1200 takes 9.0 instead of 12.5 us, 1 x 2048 10.1 / 13.6, 5 x
+ * 1600 12.7 / 15.0, 1 x 1536 of 64/4 heads 9.1 / 20.0.
  *
  * With the second launch, waves of a paged decode take as few as two tiles where that leaves every
  * wave a place of its own on the device and no segment more parts than the second launch takes in a
