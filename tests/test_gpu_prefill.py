@@ -217,6 +217,40 @@ def test_prefill_packed_heads_and_cut_walks(backend, d, tq, tk, start, hq, hkv, 
     assert_lse(lse.read(), ref_lse, label)
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_prefill_workspace_is_an_offer(backend, d):
+    """A request that would be cut walks whole, with the same bits, when the workspace is absent or one
+    byte short of what it asked for; cut and whole agree with the oracle, and either repeats itself."""
+    rng = np.random.default_rng(d)
+    tq, tk, hq, hkv = 7, 3000, 12, 2
+    q, k, v = (bf16_normal(rng, shape) for shape in ((tq, hq, d), (tk, hkv, d), (tk, hkv, d)))
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, query_start=tk - tq, dtype=B.DTYPE_BF16,
+                                        contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+    need = backend.attention_workspace_required(req)
+    rc, ref, _, ref_lse = ORACLE.gqa_bf16(q, k, v, query_start=tk - tq, causal=True)
+    assert rc == 0 and need > 0
+    tensors = [backend.tensor(n, B.DTYPE_BF16, x.shape, x) for n, x in (("q", q), ("k", k), ("v", v))]
+    out, lse = backend.tensor("o", B.DTYPE_BF16, q.shape), backend.tensor("lse", B.DTYPE_F32, (tq, hq))
+    results = {}
+    for size in (0, need - 1, need, need + 4096, 0):
+        work = backend.tensor("w", B.DTYPE_I8, (size,)) if size else None
+        if work:
+            backend.workspace_attach(work)
+        try:
+            facts = backend.attention_execute(req, *tensors, out, lse=lse)
+        finally:
+            if work:
+                backend.workspace_detach()
+                work.release()
+        cut = size >= need
+        assert facts.kernel_launches == (2 if cut else 1) and facts.temporary_bytes == (need if cut else 0)
+        got = out.read(), lse.read()
+        assert_close_bf16(got[0], ref, "workspace of %d" % size)
+        assert_lse(got[1], ref_lse, "workspace of %d" % size)
+        first = results.setdefault(cut, got)
+        assert np.array_equal(got[0], first[0]) and np.array_equal(got[1], first[1]), size
+
+
 @pytest.mark.parametrize("tq,tk,start,hq,hkv,causal", [
     (2, 3, 1, 12, 2, True),         # one step, two rows of one wave
     (130, 130, 0, 6, 1, True),      # a second tile of two tokens
