@@ -898,12 +898,14 @@ def test_paged_decode_workspace_holds_the_offsets_of_the_second_launch():
     """Partials and statistics of two slots per wave, and wherever a second launch merges them (head
     dimensions 64 and 256 always) the offsets of every session behind them."""
     with Backend() as b:
-        for sessions, hq, hkv, d, context in ((5, 24, 4, 256, 3000), (70, 16, 4, 64, 500), (64, 24, 4, 256, 16384)):
+        # waves of four tiles, of eight, and as many as there are
+        for sessions, hq, hkv, d, context, waves in ((5, 24, 4, 256, 3000, 940), (70, 16, 4, 64, 500, 1120),
+                                                     (64, 24, 4, 256, 16384, 2048)):
             r = b.paged_requirement(sessions, hq, hkv, d, 16, 70000, (context + 15) // 16, context)
-            waves = min(2048, -(-sessions * hkv * -(-context // 16) // 8))
             rows = 2 * waves * (hq // hkv)
             partials = -(-rows * d * 4 // 256) * 256 + -(-rows * 8 // 256) * 256
-            assert b.paged_decode_workspace_required(r) >= partials + 4 * (sessions + 1)
+            offsets = -(-4 * (sessions + 1) // 256) * 256
+            assert b.paged_decode_workspace_required(r) == partials + offsets
 
 
 @pytest.mark.parametrize("sessions,hq,hkv,d,context,waves", [
