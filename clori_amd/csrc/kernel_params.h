@@ -112,7 +112,7 @@ typedef struct {
     uint16_t *out; /* bf16 [sessions][query_heads][head_dim] */
     float *lse;    /* optional F32 [sessions][query_heads] */
     int32_t *status;
-    uint32_t sessions, query_heads, head_dim, chunk_tokens, max_chunks, fixed_context;
+    uint32_t sessions, query_heads, head_dim, chunk_tokens, max_chunks;
     const float *sinks; /* optional F32 [query_heads]: one extra logit per head with value 0 */
     uint32_t window;    /* sliding window of the producing kernel (sets its first chunk) */
     uint32_t window_align; /* the producer starts its chunks at first_visible rounded down to this */
