@@ -35,7 +35,8 @@ __device__ inline float wave_sum(float v)
 // come sixteen chunks per trip, every load of a trip independent of the others (chunks past the
 // end alias the last one with weight zero): one memory round trip per sixteen chunks.  With every
 // lane loading and weighing the statistics of every chunk for itself the merge of 16 x 128 rows of
-// 512 dims over up to 16 chunks took 9.8 us, this 6.2 us (33 MB of partials).
+// 512 dims over 3 to 16 chunks took 6.7 us, this 6.1 us; over 16 chunks each (33 MB of partials) both
+// take 8.0 us.
 //   stats(c):       (running maximum in log2 units, denominator) of chunk c
 //   piece(c):       the lane's 16 bytes of chunk c's row, c the same in all lanes
 //   meanwhile():    work of the caller that runs while the first loads are in flight

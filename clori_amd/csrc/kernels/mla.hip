@@ -529,7 +529,7 @@ __device__ __forceinline__ void copy_rows(const uint64_t *row, const uint16_t *p
 // Three dependent trips to memory (list, page table, rows) bound it, not the bytes.  One lane per
 // entry makes the first two, for the YVEX_ROCM_GATHER_ENTRIES entries of a workgroup at once, and
 // every thread has all its pieces in flight before it stores one.  32 lists of 512 rows of 1 KB:
-// 7.4 us, 33.5 MB moved at 4.5 TB/s (10.7 us with a workgroup of 128 threads per entry, 16384
+// 7.9 us, 33.5 MB moved at 4.2 TB/s (10.3 us with a workgroup of 128 threads per entry, 16384
 // workgroups, each its own chain).
 extern "C" __global__ void __launch_bounds__(256)
 yvex_rocm_gather_rows(const yvex_rocm_gather_rows_params p)

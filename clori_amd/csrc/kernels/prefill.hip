@@ -4,8 +4,9 @@
 // other counts (the numbers in this comment are those of 128).  256 has a kernel of its own
 // (prefill_pair.hip) for all but short walks; its runs are merged by the merge at the end of this file.
 //
-// A workgroup of 4 waves owns one (query head, 128-row query tile): each wave owns
-// 32 query rows and walks the key/value tokens in tiles of 64 that the workgroup
+// A workgroup of 4 waves owns one item, 128 packed rows of one row head (kernel_params.h: the query
+// heads that share a kv head, or one of them), or one run of keys of it: each wave owns
+// 32 rows and walks the key/value tokens in tiles of 64 that the workgroup
 // stages in LDS once and all four waves share.  Two workgroups are resident per CU; they
 // are not synchronised with each other, so the serial part of one trip (barrier, maximum
 // bookkeeping) of one overlaps the matrix work of the other.
@@ -47,8 +48,8 @@
 // 2^kLazyLog2, harmless in fp32 sums and in the bf16 operand of the second product.
 // Row sums are taken over the unrounded fp32 probabilities: with a handful of visible keys
 // the rounding of single bf16 terms would show in the log-sum-exp output.
-// Workgroups are numbered so that heavier (later) query tiles start first and, when the
-// kv head count is a multiple of the 8 XCDs, all users of one kv head share an L2.
+// Workgroups are numbered so that heavier (later) query tiles start first and, with packed heads
+// and a kv head count that is a multiple of the 8 XCDs, all users of one kv head share an L2.
 //
 #include "mfma.h"
 #include "prefill_rows.h"

@@ -25,14 +25,16 @@
 // tile of the walk, and it stays: fp32 sums and bf16 probabilities keep their relative precision
 // whatever their magnitude, so nothing is lost as long as nothing overflows (a later score would
 // have to be about 2^100 times the first tile's largest in weight).  The walk therefore carries no
-// maximum, no decision and no rescaling.  Rows that end up not finite are walked again by a loop
-// that rescales in every tile (walk_rescaling); what is still not finite then is the inputs' fault.
+// maximum, no decision and no rescaling.  Where a complete row sum or an accumulator is not finite in
+// the end, the workgroup walks again with a loop that rescales in every tile (walk_rescaling); what is
+// still not finite then is the inputs' fault.
 //
 // 2000 tokens of 24/4 heads behind 13333 (704 GFLOP): 873 us with one wave per 32 rows (a maximum, a
 // decision and 33 spilled registers in every step), 634 us here.  The main loop holds no spilled
 // register (256 + 256 registers: O^T and three quarters of the queries in accumulation registers) and
-// meets no bank conflict; its MFMAs are busy 58 % of the cycles, at a clock that the load has pulled
-// down to 1.7 GHz: 1.23 PFLOP/s inside the walk, where a large library GEMM reaches 1.32.
+// meets no bank conflict; its MFMAs are busy 59 % of the waves' cycles, 46 % of the device's (256 units
+// work on 496 workgroups), and the launch of 708 GFLOP with its masked keys takes 618 us: 1.15 PFLOP/s,
+// where a large library GEMM reaches 1.28.
 //
 // A workgroup spends some 20000 cycles before its first and after its last step, most of them on
 // instructions that it meets once (47 KB of code): whole walks of a few steps keep the kernel of
