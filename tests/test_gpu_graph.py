@@ -130,6 +130,44 @@ def test_recorded_decode_step_appends_then_attends(backend):
     backend.workspace_detach()
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("attached", [True, False])
+def test_recorded_prefill_replays_equal_eager(backend, d, attached):
+    """Drafted tokens behind a history: recorded with the workspace the walks are cut and merged by a
+    second launch, recorded without one they are whole and nothing is allocated."""
+    rng = np.random.default_rng(803 + d)
+    tq, tk, hq, hkv = 9, 3000, 12, 2
+    k, v = bf16_normal(rng, (tk, hkv, d)), bf16_normal(rng, (tk, hkv, d))
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, query_start=tk - tq, dtype=B.DTYPE_BF16,
+                                        contract=B.NUMERIC_BF16_F32_ACCUMULATE)
+    tensors = [backend.tensor("q", B.DTYPE_BF16, (tq, hq, d), bf16_normal(rng, (tq, hq, d))),
+               backend.tensor("k", B.DTYPE_BF16, k.shape, k), backend.tensor("v", B.DTYPE_BF16, v.shape, v)]
+    out, eager = (backend.tensor(n, B.DTYPE_BF16, (tq, hq, d)) for n in ("o", "e"))
+    work = backend.tensor("work", B.DTYPE_I8, (backend.attention_workspace_required(req),))
+    if attached:
+        backend.workspace_attach(work)
+    backend.graph_begin()
+    backend.attention_execute(req, *tensors, out)
+    graph = backend.graph_end()
+    for replay in range(4):
+        q = bf16_normal(rng, (tq, hq, d))
+        tensors[0].write(q)
+        out.zero()
+        assert backend.graph_launch(graph).kernel_launches == (2 if attached else 1)
+        got = out.read()
+        unrelated_eager_work(backend, rng)
+        backend.attention_execute(req, *tensors, eager)
+        assert np.array_equal(got, eager.read()), "replay %d" % replay
+        rc, ref, _, _ = ORACLE.gqa_bf16(q, k, v, query_start=tk - tq, causal=True)
+        assert rc == 0
+        assert_close_bf16(got, ref, "recorded prefill replay %d" % replay)
+    backend.graph_release(graph)
+    if attached:
+        backend.workspace_detach()
+    for x in tensors + [out, eager, work]:
+        x.release()
+
+
 def test_bandwidth_probe_on_the_device(backend):
     """The probe's record on a real part: a streaming read of 1 GiB sustains terabytes per
     second, below the published peak; the copy moves read plus write."""
