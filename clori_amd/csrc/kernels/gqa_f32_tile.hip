@@ -1,12 +1,16 @@
-// EXACT_F32 grouped-query attention on the fp32 matrix cores of gfx950 (wave64).
+// EXACT_F32 grouped-query attention on the matrix cores of gfx950 (wave64).
 //
-// F32 tensors in, F32 out, every product an F32 product: the numeric contract of the
+// An item (128 query tokens of one query head) is walked with every F32 product as three f16 products
+// (gqa_f32_halves.h), and once more by the fp32 walk below when that gives a result that is not finite
+// or meets values past its range: what such an item publishes or reports is the fp32 walk's.
+//
+// The fp32 walk: F32 tensors in, F32 out, every product an F32 product: the numeric contract of the
 // reference's only attention request (src/backend/cuda/exact_attention.c:35-49) and the
 // arithmetic of its own device kernel (float dot products, float online softmax,
 // src/backend/cuda/transformer_kernels.cu:136-208), here in 32x32 tiles on
 // v_mfma_f32_32x32x2_f32 instead of one row at a time.
 //
-// One workgroup = 128 consecutive query tokens of one query head, four waves of 32 queries.
+// One item = 128 consecutive query tokens of one query head, four waves of 32 queries.
 // Key and value rows of the head's KV group go through LDS in tiles of 32 tokens, shared by
 // the four waves, double buffered: the rows of tile t+1 are fetched into registers before
 // the matrix work of tile t and written to the other buffer after it.
@@ -24,6 +28,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../kernel_params.h"
+#include "gqa_f32_halves.h"
 #include "mfma.h"
 
 namespace {
@@ -36,12 +41,6 @@ __device__ inline void flag_status(int32_t *status, int code)
 __device__ inline floatx16 mfma_32x32x2(float a, float b, floatx16 c)
 {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// Last key a query may see (the rows of 2^32 keys are more than any memory holds).
-__device__ inline uint32_t last_visible(const yvex_rocm_gqa_f32_params &p, uint64_t own)
-{
-    return (uint32_t)(p.causal ? min(p.kv_tokens - 1u, own) : p.kv_tokens - 1u);
 }
 
 // Scores of one tile -> weights, with the running statistics and the accumulators brought to the
@@ -101,10 +100,9 @@ struct GqaTile {
     float *lds;
     const int tid, lane, wave, column, half;
 
-    __device__ GqaTile(const yvex_rocm_gqa_f32_params &params, float *shared)
-        : p(params), lds(shared), tid(threadIdx.x), lane(threadIdx.x & 63),
-          wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), column(threadIdx.x & 31),
-          half((threadIdx.x >> 5) & 1)
+    __device__ GqaTile(const yvex_rocm_gqa_f32_params &params, float *shared, int thread)
+        : p(params), lds(shared), tid(thread), lane(thread & 63),
+          wave(__builtin_amdgcn_readfirstlane(thread >> 6)), column(thread & 31), half((thread >> 5) & 1)
     {
     }
 
@@ -135,38 +133,6 @@ struct GqaTile {
             const int c = tid + 256 * j, row = c / (kDim / 4), piece = c % (kDim / 4);
             *reinterpret_cast<floatx4 *>(tile + row * row_stride + 4 * piece) = s.piece[j];
         }
-    }
-
-    // Items (one head, one tile of queries) are numbered heaviest first.  A scheduled launch
-    // hands every workgroup a row of items (the count, then the items, 16 bytes: one scalar
-    // load); otherwise the workgroup runs the one item its number stands for.
-    __device__ void run() const
-    {
-        uint32_t count = 1u;
-        u32x4 row = {0u, 0u, 0u, 0u};
-        if (p.lists != nullptr) {
-            typedef __attribute__((address_space(4))) const u32x4 constant_u32x4;
-            row = *(constant_u32x4 *)(uintptr_t)(p.lists + (uint64_t)blockIdx.x * 8u);
-            count = min(row.x & 0xffffu, 7u);
-        }
-        for (uint32_t j = 1u; j <= count; ++j) {
-            const uint32_t word = j >> 1 == 0u ? row.x : j >> 1 == 1u ? row.y : j >> 1 == 2u ? row.z : row.w;
-            item(p.lists != nullptr ? (word >> ((j & 1u) * 16u)) & 0xffffu : paired_item());
-            // every wave is done with the tiles in LDS before the next item stages its own
-            if (j < count) __syncthreads();
-        }
-    }
-
-    __device__ uint32_t paired_item() const
-    {
-        // Without lists: the hardware gives workgroup b of the first 2 * pair_units to compute
-        // unit b % pair_units, and the kernel is bound by the matrix cores, so a unit's time
-        // follows the key tiles it walks: the second workgroup of a unit takes the second tier of
-        // items in reverse, and the unit that got the heaviest item gets the lightest of them
-        // (equal sums for causal walks; 433 against 459 us for 40 heads x 16 tiles of 2048 tokens).
-        return blockIdx.x >= p.pair_units && blockIdx.x < 2u * p.pair_units
-                   ? 3u * p.pair_units - 1u - blockIdx.x
-                   : blockIdx.x;
     }
 
     __device__ void item(const uint64_t id) const
@@ -313,10 +279,10 @@ struct GqaTilePair {
     float *lds;
     const int tid, lane, wave, column, half, quarter, part;
 
-    __device__ GqaTilePair(const yvex_rocm_gqa_f32_params &params, float *shared)
-        : p(params), lds(shared), tid(threadIdx.x), lane(threadIdx.x & 63),
-          wave(__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6))), column(threadIdx.x & 31),
-          half((threadIdx.x >> 5) & 1), quarter(wave & 3), part(wave >> 2)
+    __device__ GqaTilePair(const yvex_rocm_gqa_f32_params &params, float *shared, int thread)
+        : p(params), lds(shared), tid(thread), lane(thread & 63),
+          wave(__builtin_amdgcn_readfirstlane(thread >> 6)), column(thread & 31), half((thread >> 5) & 1),
+          quarter(wave & 3), part(wave >> 2)
     {
     }
 
@@ -343,23 +309,6 @@ struct GqaTilePair {
         for (int j = 0; j < kChunks; ++j) {
             const int c = tid + kThreads * j, row = c / (kDim / 4), piece = c % (kDim / 4);
             *reinterpret_cast<floatx4 *>(tile + row * row_stride + 4 * piece) = s.piece[j];
-        }
-    }
-
-    // item lists as in GqaTile::run
-    __device__ void run() const
-    {
-        uint32_t count = 1u;
-        u32x4 row = {0u, 0u, 0u, 0u};
-        if (p.lists != nullptr) {
-            typedef __attribute__((address_space(4))) const u32x4 constant_u32x4;
-            row = *(constant_u32x4 *)(uintptr_t)(p.lists + (uint64_t)blockIdx.x * 8u);
-            count = min(row.x & 0xffffu, 7u);
-        }
-        for (uint32_t j = 1u; j <= count; ++j) {
-            const uint32_t word = j >> 1 == 0u ? row.x : j >> 1 == 1u ? row.y : j >> 1 == 2u ? row.z : row.w;
-            item(p.lists != nullptr ? (word >> ((j & 1u) * 16u)) & 0xffffu : blockIdx.x);
-            if (j < count) __syncthreads();
         }
     }
 
@@ -493,24 +442,60 @@ struct GqaTilePair {
     }
 };
 
+// Items (one head, one tile of queries) are numbered heaviest first.  A scheduled launch
+// hands every workgroup a row of items (the count, then the items, 16 bytes: one scalar
+// load); otherwise the workgroup runs the one item its number stands for.
+// Without lists the hardware gives workgroup b of the first 2 * pair_units to compute
+// unit b % pair_units, and a unit's time follows the key tiles it walks: the second workgroup
+// of a unit takes the second tier of items in reverse, and the unit that got the heaviest item
+// gets the lightest of them (equal sums for causal walks).
+// An item that `Halves` gives back is walked by `Walk`.
+template <typename Halves, typename Walk>
+__device__ void run_items(const yvex_rocm_gqa_f32_params &p, unsigned char *shared)
+{
+    uint32_t count = 1u;
+    u32x4 row = {0u, 0u, 0u, 0u};
+    if (p.lists != nullptr) {
+        typedef __attribute__((address_space(4))) const u32x4 constant_u32x4;
+        row = *(constant_u32x4 *)(uintptr_t)(p.lists + (uint64_t)blockIdx.x * 8u);
+        count = min(row.x & 0xffffu, 7u);
+    }
+    const uint32_t paired = blockIdx.x >= p.pair_units && blockIdx.x < 2u * p.pair_units
+                                ? 3u * p.pair_units - 1u - blockIdx.x
+                                : blockIdx.x;
+    for (uint32_t j = 1u; j <= count; ++j) {
+        const uint32_t word = j >> 1 == 0u ? row.x : j >> 1 == 1u ? row.y : j >> 1 == 2u ? row.z : row.w;
+        const uint32_t id = p.lists != nullptr ? (word >> ((j & 1u) * 16u)) & 0xffffu : paired;
+        // (opaque, so that what depends on the lane is not kept in registers from item to item)
+        int thread = (int)threadIdx.x;
+        __asm__ volatile("" : "+v"(thread));
+        if (!Halves(p, *reinterpret_cast<typename Halves::Shared *>(shared), thread).item(id)) {
+            __syncthreads();  // every wave has read the verdict
+            __asm__ volatile("" : "+v"(thread));
+            Walk(p, reinterpret_cast<float *>(shared), thread).item(id);
+        }
+        // every wave is done with the tiles in LDS before the next item stages its own
+        if (j < count) __syncthreads();
+    }
+}
+
+constexpr int larger(int a, int b) { return a > b ? a : b; }
+
 }  // namespace
 
 // `waves`: waves per SIMD the register budget is sized for.
-#define YVEX_GQA_F32_TILE_KERNEL(name, blocks, waves)                                                   \
-    extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(waves, waves))) \
-    name(const yvex_rocm_gqa_f32_params p)                                                                \
-    {                                                                                                     \
-        __shared__ __attribute__((aligned(16))) float lds[2 * GqaTile<blocks>::kStageFloats];             \
-        GqaTile<blocks>(p, lds).run();                                                                    \
+#define YVEX_GQA_F32_TILE_KERNEL(name, halves, walk, threads, waves)                                          \
+    extern "C" __global__ void __launch_bounds__(threads) __attribute__((amdgpu_waves_per_eu(waves, waves)))   \
+    name(const yvex_rocm_gqa_f32_params p)                                                                      \
+    {                                                                                                           \
+        typedef halves Halves;                                                                                  \
+        __shared__ __attribute__((aligned(16))) unsigned char                                                   \
+            lds[larger((int)sizeof(Halves::Shared), (int)sizeof(float) * 2 * walk::kStageFloats)];              \
+        run_items<Halves, walk>(p, lds);                                                                        \
     }
+#define YVEX_HALVES(part, parts) GqaHalves<part, parts>
 
-YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_64, 2, 2)
-YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_128, 4, 2)
-
-// head dimension 256: pairs of waves, see GqaTilePair
-extern "C" __global__ void __launch_bounds__(GqaTilePair::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-yvex_rocm_gqa_f32_tile_256(const yvex_rocm_gqa_f32_params p)
-{
-    __shared__ __attribute__((aligned(16))) float lds[2 * GqaTilePair::kStageFloats];
-    GqaTilePair(p, lds).run();
-}
+YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_64, YVEX_HALVES(64, 1), GqaTile<2>, 256, 2)
+YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_128, YVEX_HALVES(128, 1), GqaTile<4>, 256, 2)
+// pairs of waves split the head dimension
+YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_256, YVEX_HALVES(128, 2), GqaTilePair, 512, 2)

@@ -359,6 +359,81 @@ def test_gqa_matrix_core_kernel_scheduled_launch_equals_the_first(backend, tq, s
         t.release()
 
 
+def as_halves_cases():
+    """(name, q, k, v, tolerance relative to the largest visible value): rows whose magnitudes the split into
+    halves has to follow."""
+    def rows(seed, tq, tk, hq, hkv, d):
+        rng = np.random.default_rng(seed)
+        return (rng.standard_normal((tq, hq, d)).astype(np.float32),
+                rng.standard_normal((tk, hkv, d)).astype(np.float32),
+                rng.standard_normal((tk, hkv, d)).astype(np.float32))
+    for d, hq, hkv in ((64, 2, 1), (128, 2, 2), (256, 2, 1)):
+        q, k, v = rows(d, 65, 161, hq, hkv, d)
+        yield "powers-%d" % d, q * np.float32(2.0 ** -40), k * np.float32(2.0 ** 40), v * np.float32(2.0 ** -90)
+        yield "largest-%d" % d, q * np.float32(2.0 ** 45), k * np.float32(2.0 ** -45), v * np.float32(2.0 ** 45)
+        # value rows that grow along the history, and whole groups of keys and values that are zero
+        grown = v * np.exp2(np.linspace(-20, 12, v.shape[0])).astype(np.float32)[:, None, None]
+        grown[:8] = 0.0
+        grown[64:96] = 0.0
+        zeroed = k.copy()
+        zeroed[8:16] = 0.0
+        yield "grown-%d" % d, q, zeroed, grown
+        # past the range of the halves: the fp32 walk
+        past = v.copy()
+        past[100, 0, 3] = np.float32(2.0 ** 70)
+        yield "past-%d" % d, q, k, past
+        low = k.copy()
+        low[40] = np.float32(-2.0 ** 60) * np.sign(q[0, 0])
+        yield "far-key-%d" % d, np.abs(q) + np.float32(0.5), -np.abs(low), v
+
+
+@pytest.mark.parametrize("case", list(as_halves_cases()), ids=lambda c: c[0])
+@pytest.mark.parametrize("causal", [True, False])
+def test_gqa_matrix_core_kernel_follows_magnitudes(backend, case, causal):
+    """Scores keep the size that N(0,1) rows give (or saturate to a weight of zero), so the reference's bound
+    for its float device kernel, 2e-5 on N(0,1) values, holds relative to the largest value that a query sees."""
+    _, q, k, v = case
+    start = k.shape[0] - q.shape[0] - 7 if causal else 0
+    out, lse, facts = run_exact(backend, q, k, v, query_start=start, causal=causal)
+    assert facts.accelerated_matrix_launches == 1
+    rc, ref, ref_lse = ORACLE.gqa(q, k, v, query_start=start, causal=causal)
+    assert rc == 0
+    top = np.maximum.accumulate(np.abs(v).max(axis=2), axis=0)   # [key, kv head]
+    group = q.shape[1] // k.shape[1]
+    for token in range(q.shape[0]):
+        last = start + token if causal else k.shape[0] - 1
+        for head in range(q.shape[1]):
+            bound = 2e-5 * top[last, head // group]
+            assert np.abs(out[token, head].astype(np.float64) - ref[token, head]).max() <= bound
+    assert np.abs(lse - ref_lse).max() < 2e-5 * max(1.0, np.abs(ref_lse).max())
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(64, 2, 1), (128, 5, 1), (256, 2, 1)])
+def test_gqa_matrix_core_kernel_infinities(backend, d, hq, hkv):
+    """An infinite key that no query sees changes nothing; one that a query sees, with a product of one sign
+    that excludes the key, or an infinite value, ends as the fp32 walk ends it."""
+    rng = np.random.default_rng(d + 1)
+    q = (np.abs(rng.standard_normal((64, hq, d))) + 0.1).astype(np.float32)
+    k = rng.standard_normal((96, hkv, d)).astype(np.float32)
+    v = rng.standard_normal((96, hkv, d)).astype(np.float32)
+    good, _, _ = run_exact(backend, q, k, v, query_start=0)
+    bad = k.copy()
+    bad[64:] = np.inf
+    same, _, _ = run_exact(backend, q, bad, v, query_start=0)       # keys 64.. are past every query
+    assert np.abs(same - good).max() < 2e-5
+    bad = k.copy()
+    bad[5, 0, 2] = -np.inf                                         # a score of -inf: a weight of zero
+    out, _, _ = run_exact(backend, q, bad, v, query_start=0)
+    rc, ref, _ = ORACLE.gqa(q, np.where(np.isinf(bad), np.float32(-1e30), bad), v)
+    assert rc == 0 and np.abs(out - ref).max() < 2e-5
+    for value in (np.inf, np.nan):
+        bad = v.copy()
+        bad[9, 0, 1] = value
+        with pytest.raises(YvexError) as e:
+            run_exact(backend, q, k, bad, query_start=0)
+        assert e.value.code == B.YVEX_ERR_FORMAT
+
+
 # ------------------------------------------------ decode-shaped requests over long contexts ----
 
 @pytest.mark.parametrize("tq,tk,hq,hkv,d,causal", [
