@@ -1,0 +1,81 @@
+// F32 values as the sum of two f16 values, for products on the f16 matrix cores.
+#ifndef YVEX_ROCM_KERNELS_F16_SPLIT_H
+#define YVEX_ROCM_KERNELS_F16_SPLIT_H
+
+#include "mfma.h"
+
+namespace {
+
+typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ floatx16 mfma_32x32x16_f16(halfx8 a, halfx8 b, floatx16 c)
+{
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// Magnitudes compare as whole numbers; a NaN is larger than all of them.
+template <int kControl>
+__device__ __forceinline__ uint32_t dpp_max(uint32_t v)
+{
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kControl, 0xf, 0xf, true));
+}
+
+// The largest magnitude of three values (fmaxf also makes NaNs quiet, at an instruction a value).
+__device__ __forceinline__ uint32_t largest(float a, float b, float c)
+{
+    uint32_t r;
+    __asm__("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
+// Biased exponent that a group whose largest magnitude has these bits is scaled by: 2^(141 - e)
+// brings it to [2^14, 2^15).  Both that factor and its inverse 2^(e - 141) are normal numbers for
+// e in [kExponentLeast, kExponentMost]; a group below the range is scaled as its least, one above
+// it (2^51 and more, infinities) is left to the fp32 walk.
+constexpr uint32_t kExponentLeast = 15u, kExponentMost = 177u;
+
+__device__ __forceinline__ uint32_t group_exponent(uint32_t max_bits)
+{
+    return min(max(max_bits >> 23, kExponentLeast), kExponentMost);
+}
+
+__device__ __forceinline__ float power_of_two(uint32_t biased) { return __builtin_bit_cast(float, biased << 23); }
+
+__device__ __forceinline__ float down_factor(uint32_t e) { return power_of_two(268u - e); }
+__device__ __forceinline__ float up_factor(uint32_t e) { return power_of_two(e - 14u); }
+
+template <int kValue>
+struct Index {
+    static constexpr int value = kValue;
+};
+// f(Index<0>), f(Index<1>) ... f(Index<kCount - 1>): the slots of a trip are more than a loop is unrolled for
+template <int kCount, int kFrom = 0, typename F>
+__device__ __forceinline__ void for_each(const F &f)
+{
+    if constexpr (kFrom < kCount) {
+        f(Index<kFrom>());
+        for_each<kCount, kFrom + 1>(f);
+    }
+}
+
+// Two values times `factor` as pairs of halves: four instructions, one rounding each (the compiler takes
+// seven).  The compiler sees no instructions here and inserts no wait states: the values must not come
+// straight from a transcendental instruction (whose result the next but one may read first), and the
+// results not go straight into an MFMA or a lane exchange (two instructions in between).
+#define YVEX_SPLIT_PAIR(name, where)                                                                       \
+    __device__ __forceinline__ void name(float a, float b, float factor, uint32_t &hi, uint32_t &lo)       \
+    {                                                                                                      \
+        __asm__ volatile("v_fma_mixlo_f16 %0, %2, %4, 0\n\t"                                             \
+                         "v_fma_mixhi_f16 %0, %3, %4, 0\n\t"                                             \
+                         "v_fma_mixlo_f16 %1, %2, %4, -%0 op_sel_hi:[0,0,1]\n\t"                         \
+                         "v_fma_mixhi_f16 %1, %3, %4, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]"               \
+                         : "=&v"(hi), "=&v"(lo)                                                            \
+                         : "v"(a), "v"(b), where(factor));                                                 \
+    }
+YVEX_SPLIT_PAIR(split_pair, "s")          // a factor that is the same in all lanes
+YVEX_SPLIT_PAIR(split_pair_by_lane, "v")
+#undef YVEX_SPLIT_PAIR
+
+}  // namespace
+
+#endif  // YVEX_ROCM_KERNELS_F16_SPLIT_H
