@@ -442,11 +442,13 @@ static unsigned long long visible_tokens(const yvex_transformer_attention_requir
                                                              : r->key_value_tokens;
 }
 
-/* The EXACT_F32 request has three kernels; the choice is a function of the request geometry
- * (and of the 16-byte alignment of the views) only.
+/* The EXACT_F32 request has these kernels; the choice is a function of the request geometry
+ * (of the 16-byte alignment of the views, and of whether a workspace is attached that holds what the
+ * planner named) only.
  *   - Prefill-shaped requests (at least 32 query tokens, head dimension 64, 128 or 256) run in
- *     32 x 32 tiles on the fp32 matrix cores with float statistics, the arithmetic of the
- *     reference's own device kernel (src/backend/cuda/transformer_kernels.cu:136-208).
+ *     32 x 32 tiles on the matrix cores with float statistics, the arithmetic of the
+ *     reference's own device kernel (src/backend/cuda/transformer_kernels.cu:136-208): with the
+ *     workspace over keys and values split beforehand (rocm_halved.c), otherwise in one launch.
  *   - Other requests over 512 or more keys (the decode step of the session layer,
  *     src/runtime/stateful_attention.c:326-352) are cut into runs of keys, one wave per
  *     (token, head, run) with double-precision statistics, eight runs per workgroup; the
@@ -540,6 +542,7 @@ static int rocm_attention_workspace_required(const yvex_transformer_attention_re
     } else {
         unsigned long long per_run;
         const unsigned long long runs = exact_split_runs(r, &per_run);
+        if (exact_tile_geometry(r)) *bytes = yvex_rocm_halved_workspace(r);
         if (runs) {
             if (!exact_split_workspace(r, runs, &acc, &total))
                 return refuse(err, YVEX_ERR_BOUNDS, where, "attention workspace geometry overflowed");
@@ -597,7 +600,7 @@ static int exact_tile_function(const yvex_transformer_attention_requirement *r,
     return 1;
 }
 
-/* The EXACT_F32 contract: the tile kernel on the fp32 matrix cores for prefill-shaped requests,
+/* The EXACT_F32 contract: the tile kernels on the matrix cores for prefill-shaped requests,
  * runs of keys for single rows over long histories, the row kernel for the rest. */
 static int attention_execute_exact(yvex_backend *backend, const yvex_transformer_attention_request *request,
                                    yvex_device_tensor *lse, const yvex_rocm_attention_geometry *g,
@@ -610,7 +613,7 @@ static int attention_execute_exact(yvex_backend *backend, const yvex_transformer
     yvex_rocm_function_id tile_function = YVEX_ROCM_FN_GQA_F32;
     unsigned long long split_runs = 0ull, split_keys = 0ull, split_bytes = 0ull;
     void *split_work = NULL;
-    int tiled = 0, split_owned = 0;
+    int tiled, halved = 0, split_owned = 0;
     memset(&params, 0, sizeof(params));
     params.q = (const float *)request->query->data;
     params.k = (const float *)request->key->data;
@@ -630,8 +633,16 @@ static int attention_execute_exact(yvex_backend *backend, const yvex_transformer
     params.scale = 1.0f / sqrtf((float)r->head_dimension);
     params.causal = g->causal;
     backend_workspace_reset(backend);
-    if (exact_tile_function(r, g->q_stride, g->k_stride, g->v_stride, request, &tile_function)) {
-        /* 128 query tokens of one head per workgroup, on the fp32 matrix cores */
+    tiled = exact_tile_function(r, g->q_stride, g->k_stride, g->v_stride, request, &tile_function);
+    if (tiled) {
+        rc = yvex_rocm_halved_launch(backend, request, &params, facts, &halved, err);
+        split_bytes = facts->temporary_bytes;
+        if (rc != YVEX_OK) return rc;
+    }
+    if (halved) {
+        rc = YVEX_OK;
+    } else if (tiled) {
+        /* 128 query tokens of one head per workgroup */
         const unsigned long long groups =
             r->query_heads * ((r->query_tokens + ROCM_EXACT_TILE_QUERIES - 1ull) / ROCM_EXACT_TILE_QUERIES);
         if (groups > 0x7fffffffull)
@@ -666,7 +677,6 @@ static int attention_execute_exact(yvex_backend *backend, const yvex_transformer
                               /* at 256 pairs of waves split the head dimension: eight waves */
                               r->head_dimension == 256ull ? 512u : 256u, 0u,
                               &params, "rocm.transformer.gqa", err);
-        tiled = 1;
     } else if ((split_runs = exact_split_runs(r, &split_keys)) != 0ull &&
                !(((uintptr_t)request->query->data | (uintptr_t)request->key->data |
                   (uintptr_t)request->value->data) & 15u)) {
@@ -702,7 +712,7 @@ static int attention_execute_exact(yvex_backend *backend, const yvex_transformer
                               1u, 64u, 0u, &params, "rocm.transformer.gqa", err);
     }
     if (rc == YVEX_OK) {
-        facts->kernel_launches = 1ull;
+        if (!halved) facts->kernel_launches = 1ull;
         facts->accelerated_matrix_launches = tiled ? 1ull : 0ull;
         facts->temporary_bytes = split_bytes;
         facts->compulsory_memory_facts_available = 1;

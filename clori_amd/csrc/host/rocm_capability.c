@@ -47,6 +47,24 @@ static const rocm_kernel_binding rocm_kernel_bindings[] = {
      YVEX_ROCM_FN_GQA_F32_TILE_128},
     {"yvex_rocm_gqa_f32_tile_256", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
      YVEX_ROCM_FN_GQA_F32_TILE_256},
+    {"yvex_rocm_gqa_f32_halve_64", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_HALVE_64},
+    {"yvex_rocm_gqa_f32_halve_128", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_HALVE_128},
+    {"yvex_rocm_gqa_f32_halve_256", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_HALVE_256},
+    {"yvex_rocm_gqa_f32_halved_64", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_HALVED_64},
+    {"yvex_rocm_gqa_f32_halved_128", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_HALVED_128},
+    {"yvex_rocm_gqa_f32_halved_256", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_HALVED_256},
+    {"yvex_rocm_gqa_f32_merge_64", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_MERGE_64},
+    {"yvex_rocm_gqa_f32_merge_128", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_MERGE_128},
+    {"yvex_rocm_gqa_f32_merge_256", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,
+     YVEX_ROCM_FN_GQA_F32_MERGE_256},
     {"yvex_rocm_fill_u32", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32, YVEX_ROCM_FN_FILL_U32},
     {"yvex_rocm_stream_read", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32, YVEX_ROCM_FN_STREAM_READ},
     {"yvex_rocm_rotary_half_plain_f32", YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32,

@@ -1,0 +1,143 @@
+/* Prefill-shaped EXACT_F32 requests over keys and values split into halves beforehand: the plan of a
+ * request, the bytes it wants attached, and its launches.
+ *
+ * One launch splits the visible key and value rows (kernels/gqa_f32_halved.h), the second walks them
+ * with the query heads of a kv head packed into the rows of its tiles and, where the launch would leave
+ * units idle, in runs of keys (the plan of the bf16 prefill, rocm_prefill.c, with steps of 32 keys), and
+ * a third merges the runs.  Halves and partials live in the attached workspace; without one
+ * that holds them a request runs in one launch that splits as it goes (gqa_f32_halves.h).
+ * Everything here is a function of the request's geometry only, so that the planner's
+ * workspace_required and the execution agree. */
+#include "rocm_state.h"
+
+#include <math.h>
+#include <string.h>
+
+enum {
+    HALVED_STEP_KEYS = 32,
+    HALVED_FACTOR_WORDS = 8 /* of a tile */
+};
+#define HALVED_TILES_MAX (512ull << 20) /* bytes of halves a request may ask for */
+
+typedef struct {
+    yvex_rocm_walk_plan walk;
+    unsigned long long kv_tiles, tile_bytes, factor_bytes; /* of all kv heads */
+    unsigned long long total;
+} halved_plan;
+
+static unsigned long long visible_keys(const yvex_transformer_attention_requirement *r)
+{
+    return r->mask == YVEX_TRANSFORMER_ATTENTION_MASK_CAUSAL ? r->query_start + r->query_tokens
+                                                             : r->key_value_tokens;
+}
+
+/* Returns 0 when the request is not for these kernels.  Walks of fewer than 2 d + 128 keys stay with the one
+ * launch: the launch that splits, and a workgroup's longer start, cost more than they save.  With the
+ * workspace / without, us: 40/8 heads of 128, 200 tokens 24.6 / 23.7, 300 29.4 / 29.0, 450 36.7 / 39.7,
+ * 1777 118 / 142, 4096 461 / 640, 32 behind 200 25.3 / 23.6, 128 behind 300 33.0 / 37.4, 32 behind 4000 46 /
+ * 271, 300 behind 5000 125 / 316; 16/4 of 64, 64 11.2 / 9.6, 200 14.6 / 15.4, 1000 36.1 / 44.8; 24/4 of 256, 300
+ * 58 / 48, 32 behind 300 43.3 / 47.7, 500 75.3 / 74.3, 2000 204 / 231, 64 behind 20000 192 / 2003. */
+static int halved_plan_make(const yvex_transformer_attention_requirement *r, halved_plan *plan)
+{
+    const unsigned long long d = r->head_dimension, group = r->query_heads / r->key_value_heads;
+    memset(plan, 0, sizeof(*plan));
+    /* row counts below 2^27 (kernel_params.h), 32-bit offsets into a tile and into the tiles of a kv head */
+    if (r->query_tokens > (1ull << 27) / group || r->query_heads > 65535ull ||
+        r->key_value_tokens > (1ull << 30) || ((r->key_token_stride | r->value_token_stride) >> 24) != 0ull ||
+        (r->key_value_heads * d >> 24) != 0ull)
+        return 0;
+    if (visible_keys(r) < 2ull * d + 128ull) return 0;
+    plan->kv_tiles = (visible_keys(r) + HALVED_STEP_KEYS - 1ull) / HALVED_STEP_KEYS;
+    plan->tile_bytes = r->key_value_heads * plan->kv_tiles * 256ull * d;
+    plan->factor_bytes = r->key_value_heads * plan->kv_tiles * HALVED_FACTOR_WORDS * sizeof(uint32_t);
+    plan->factor_bytes = (plan->factor_bytes + 255ull) & ~255ull;
+    if (plan->tile_bytes > HALVED_TILES_MAX) return 0;
+    yvex_rocm_walk_plan_whole(r, group, HALVED_STEP_KEYS, &plan->walk);
+    if (plan->walk.whole_items > 0x7fffffffull) return 0;
+    yvex_rocm_walk_plan_cut(r, &plan->walk);
+    plan->total = plan->tile_bytes + plan->factor_bytes + plan->walk.acc_bytes + plan->walk.ml_bytes;
+    return 1;
+}
+
+unsigned long long yvex_rocm_halved_workspace(const yvex_transformer_attention_requirement *r)
+{
+    halved_plan plan;
+    return halved_plan_make(r, &plan) ? plan.total : 0ull;
+}
+
+static yvex_rocm_function_id by_head_dimension(unsigned long long d, yvex_rocm_function_id at_64)
+{
+    return d == 64ull ? at_64 : (yvex_rocm_function_id)(at_64 + (d == 128ull ? 1 : 2));
+}
+
+int yvex_rocm_halved_launch(yvex_backend *backend, const yvex_transformer_attention_request *request,
+                            const yvex_rocm_gqa_f32_params *f, yvex_backend_operation_facts *facts, int *taken,
+                            yvex_error *err)
+{
+    static const char where[] = "rocm.transformer.gqa";
+    const yvex_backend_operation_variant variant = YVEX_BACKEND_VARIANT_ROCM_ATTENTION_GQA_F32;
+    const yvex_transformer_attention_requirement *r = &request->requirement;
+    const yvex_rocm_backend_state *state = yvex_rocm_state(backend);
+    yvex_rocm_gqa_f32_halved_params params;
+    yvex_rocm_prefill_params *w = &params.walk;
+    unsigned long long work = 0ull;
+    halved_plan plan;
+    int rc;
+    *taken = 0;
+    if (!halved_plan_make(r, &plan) ||
+        yvex_backend_workspace_acquire(backend, plan.total, 256ull, &work) != YVEX_BACKEND_RESIDENT_HIT)
+        return YVEX_OK;
+    *taken = 1;
+    memset(&params, 0, sizeof(params));
+    w->q = (const uint16_t *)(const void *)f->q;
+    w->k = (const uint16_t *)(const void *)f->k;
+    w->v = (const uint16_t *)(const void *)f->v;
+    w->out = (uint16_t *)(void *)f->out;
+    w->lse = f->lse;
+    w->status = f->status;
+    w->q_stride = f->q_stride;
+    w->k_stride = f->k_stride;
+    w->v_stride = f->v_stride;
+    w->query_tokens = (uint32_t)f->query_tokens;
+    w->kv_tokens = (uint32_t)f->kv_tokens;
+    w->query_start = (uint32_t)f->query_start;
+    w->query_heads = (uint32_t)f->query_heads;
+    w->kv_heads = (uint32_t)f->kv_heads;
+    w->pack = (uint32_t)plan.walk.pack;
+    w->row_heads = (uint32_t)plan.walk.row_heads;
+    w->pack_inverse = (uint32_t)((0xffffffffull + plan.walk.pack) / plan.walk.pack);
+    w->causal = (uint32_t)f->causal;
+    w->rows = (uint32_t)plan.walk.rows;
+    w->query_tiles = (uint32_t)plan.walk.query_tiles;
+    w->whole_items = (uint32_t)plan.walk.whole_items;
+    w->tail_items = (uint32_t)plan.walk.tail_items;
+    w->splits = (uint32_t)plan.walk.splits;
+    w->merge_groups = plan.walk.splits > 8ull ? 4u : 1u;
+    params.tiles = (unsigned char *)(uintptr_t)work;
+    params.factors = (uint32_t *)(uintptr_t)(work + plan.tile_bytes);
+    w->part_acc = (float *)(uintptr_t)(work + plan.tile_bytes + plan.factor_bytes);
+    w->part_ml = (float *)(uintptr_t)(work + plan.tile_bytes + plan.factor_bytes + plan.walk.acc_bytes);
+    params.scale = f->scale;
+    params.kv_tiles = (uint32_t)plan.kv_tiles;
+    /* two workgroups of a unit: the second tier of items in reverse, equal sums for causal walks */
+    if (f->causal && r->head_dimension != 256ull && state->compute_units > 0 &&
+        plan.walk.whole_items >= 2ull * (unsigned long long)state->compute_units)
+        params.pair_units = (uint32_t)state->compute_units;
+    rc = yvex_rocm_launch(backend, by_head_dimension(r->head_dimension, YVEX_ROCM_FN_GQA_F32_HALVE_64), variant,
+                          (unsigned int)plan.kv_tiles, (unsigned int)r->key_value_heads, 1u, 256u, 0u, &params,
+                          where, err);
+    if (rc == YVEX_OK)
+        rc = yvex_rocm_launch(backend, by_head_dimension(r->head_dimension, YVEX_ROCM_FN_GQA_F32_HALVED_64), variant,
+                              (unsigned int)(plan.walk.whole_items + plan.walk.tail_items * plan.walk.splits), 1u,
+                              1u, 256u, 0u, &params, where, err);
+    if (rc == YVEX_OK && plan.walk.splits > 1ull)
+        rc = yvex_rocm_launch(backend, by_head_dimension(r->head_dimension, YVEX_ROCM_FN_GQA_F32_MERGE_64), variant,
+                              (unsigned int)(plan.walk.tail_items * YVEX_ROCM_PREFILL_ROWS * r->head_dimension *
+                                             w->merge_groups / 1024ull),
+                              1u, 1u, 256u, 0u, &params, where, err);
+    if (rc == YVEX_OK) {
+        facts->kernel_launches = plan.walk.splits > 1ull ? 3ull : 2ull;
+        facts->temporary_bytes = plan.total;
+    }
+    return rc;
+}

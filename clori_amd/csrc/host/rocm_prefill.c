@@ -24,7 +24,6 @@
 
 enum {
     PREFILL_UNITS = 256,
-    PREFILL_STEP_KEYS = 64,
     PREFILL_SPLITS_MAX = 64,
     PREFILL_RUN_STEPS_MIN = 2,
     /* Bytes of partial rows a request may ask for.  Runs past it are many runs of many items, whose
@@ -36,29 +35,24 @@ enum {
     PREFILL_PARTIALS_MAX = 96 << 20
 };
 
-typedef struct prefill_plan {
-    unsigned long long pack, row_heads, rows, query_tiles, whole_items, tail_items, splits;
-    unsigned long long acc_bytes, ml_bytes; /* partials of the tail */
-    int short_walks; /* head dimension 256: on the kernel for those */
-} prefill_plan;
-
 /* Steps of an item of query tile `q_tile`. */
 static unsigned long long item_steps(const yvex_transformer_attention_requirement *r,
-                                     const prefill_plan *plan, unsigned long long q_tile)
+                                     const yvex_rocm_walk_plan *plan, unsigned long long q_tile)
 {
     unsigned long long last = (q_tile + 1ull) * YVEX_ROCM_PREFILL_ROWS, keys = r->key_value_tokens;
     if (last > plan->rows) last = plan->rows;
     if (r->mask == YVEX_TRANSFORMER_ATTENTION_MASK_CAUSAL) keys = r->query_start + (last - 1ull) / plan->pack + 1ull;
-    return (keys + PREFILL_STEP_KEYS - 1ull) / PREFILL_STEP_KEYS;
+    return (keys + plan->step_keys - 1ull) / plan->step_keys;
 }
 
 /* What the tail costs in nanoseconds when each of its walks is cut into `splits` runs: every unit
  * takes its share of the runs one after the other, each with the start and end of a workgroup;
  * a cut tail also writes its partials, reads them back and pays a launch. */
-static unsigned long long tail_cost(const yvex_transformer_attention_requirement *r, const prefill_plan *plan,
+static unsigned long long tail_cost(const yvex_transformer_attention_requirement *r, const yvex_rocm_walk_plan *plan,
                                     unsigned long long steps, unsigned long long splits)
 {
-    const unsigned long long step_ns = 7ull * r->head_dimension; /* 0.9 us for a 128-row step at 128 */
+    /* 0.9 us for a 128-row step at 128, of 64 keys in bf16 and of 32 with F32 products as three */
+    const unsigned long long step_ns = 7ull * r->head_dimension;
     const unsigned long long turns = (plan->tail_items * splits + PREFILL_UNITS - 1ull) / PREFILL_UNITS;
     const unsigned long long live = plan->rows < YVEX_ROCM_PREFILL_ROWS ? plan->rows : YVEX_ROCM_PREFILL_ROWS;
     unsigned long long cost = turns * ((steps + splits - 1ull) / splits * step_ns + 3500ull);
@@ -68,9 +62,11 @@ static unsigned long long tail_cost(const yvex_transformer_attention_requirement
 }
 
 /* Every walk whole, `pack` query heads to a row head. */
-static void plan_whole(const yvex_transformer_attention_requirement *r, unsigned long long pack, prefill_plan *plan)
+void yvex_rocm_walk_plan_whole(const yvex_transformer_attention_requirement *r, unsigned long long pack,
+                               unsigned long long step_keys, yvex_rocm_walk_plan *plan)
 {
     memset(plan, 0, sizeof(*plan));
+    plan->step_keys = step_keys;
     plan->pack = pack;
     plan->row_heads = r->query_heads / pack;
     plan->rows = r->query_tokens * pack;
@@ -80,7 +76,7 @@ static void plan_whole(const yvex_transformer_attention_requirement *r, unsigned
 }
 
 /* Cuts the walks of the items past a multiple of the units where that is predicted to take less time. */
-static void plan_cut(const yvex_transformer_attention_requirement *r, prefill_plan *plan)
+void yvex_rocm_walk_plan_cut(const yvex_transformer_attention_requirement *r, yvex_rocm_walk_plan *plan)
 {
     const unsigned long long items = plan->whole_items;
     unsigned long long steps, splits, best, slots, run_bytes;
@@ -113,25 +109,25 @@ static void plan_cut(const yvex_transformer_attention_requirement *r, prefill_pl
  * kernel's waves without rows.  One wave per 32 rows / pairs, us, 24/4 heads: 128 tokens 15.0 / 19.2,
  * 256 19.7 / 22.7, 448 24.7 / 26.8, 513 (nine steps) 29.3 / 29.8, 700 36.5 / 33.6; 60 behind 150 18.1 /
  * 22.2, 120 behind 260 23.8 / 25.1, 128 behind 380 (eight) 28.5 / 28.0, 10 behind 200 17.4 / 17.1. */
-static int walks_are_short(const yvex_transformer_attention_requirement *r, const prefill_plan *plan)
+static int walks_are_short(const yvex_transformer_attention_requirement *r, const yvex_rocm_walk_plan *plan)
 {
     return item_steps(r, plan, plan->query_tiles - 1ull) <= (r->query_tokens >= 64ull ? 7ull : 4ull);
 }
 
 /* Returns 0 when the request is past the launch range: 65535 query heads or tiles of 128 tokens,
  * 2^31 - 1 (head, tile) pairs (so that rows stay below 2^27). */
-static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, prefill_plan *plan)
+static int prefill_plan_make(const yvex_transformer_attention_requirement *r, int may_split, yvex_rocm_walk_plan *plan)
 {
     const unsigned long long token_tiles = (r->query_tokens + YVEX_ROCM_PREFILL_ROWS - 1ull) / YVEX_ROCM_PREFILL_ROWS;
     if (r->query_heads > 65535ull || token_tiles > 65535ull || r->query_heads * token_tiles > 0x7fffffffull) return 0;
-    plan_whole(r, r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads, plan);
-    if (may_split && r->query_tokens > 1ull) plan_cut(r, plan);
+    yvex_rocm_walk_plan_whole(r, r->query_tokens == 1ull ? 1ull : r->query_heads / r->key_value_heads, 64ull, plan);
+    if (may_split && r->query_tokens > 1ull) yvex_rocm_walk_plan_cut(r, plan);
     if (plan->splits == 1ull && r->query_tokens > 1ull && r->query_heads * token_tiles <= PREFILL_UNITS) {
         const int short_walks = r->head_dimension == 256ull && walks_are_short(r, plan);
         /* Every walk has a unit of its own either way; one query head to a tile then means as many
          * steps in more workgroups of fewer live waves. */
         if ((r->head_dimension != 256ull || short_walks) && r->query_heads * token_tiles > plan->whole_items)
-            plan_whole(r, 1ull, plan);
+            yvex_rocm_walk_plan_whole(r, 1ull, 64ull, plan);
         plan->short_walks = short_walks;
     }
     return 1;
@@ -140,7 +136,7 @@ static int prefill_plan_make(const yvex_transformer_attention_requirement *r, in
 /* Bytes of the partials of a request (0: its walks are not cut, or the execution will refuse it). */
 unsigned long long yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r)
 {
-    prefill_plan plan;
+    yvex_rocm_walk_plan plan;
     /* both multiples of the 1 KB that 128 rows take */
     return prefill_plan_make(r, 1, &plan) ? plan.acc_bytes + plan.ml_bytes : 0ull;
 }
@@ -162,7 +158,7 @@ int yvex_rocm_prefill_execute(yvex_backend *backend, const yvex_transformer_atte
     const yvex_transformer_attention_requirement *r = &request->requirement;
     unsigned long long work = 0ull;
     yvex_rocm_prefill_params params;
-    prefill_plan plan;
+    yvex_rocm_walk_plan plan;
     int rc;
     /* the kernel addresses K and V through 32-bit buffer offsets */
     if (r->key_value_tokens * g->k_stride * 2ull >= 0xffffffffull ||

@@ -18,6 +18,15 @@ typedef enum {
     YVEX_ROCM_FN_GQA_F32_TILE_64,
     YVEX_ROCM_FN_GQA_F32_TILE_128,
     YVEX_ROCM_FN_GQA_F32_TILE_256,
+    YVEX_ROCM_FN_GQA_F32_HALVE_64,
+    YVEX_ROCM_FN_GQA_F32_HALVE_128,
+    YVEX_ROCM_FN_GQA_F32_HALVE_256,
+    YVEX_ROCM_FN_GQA_F32_HALVED_64,
+    YVEX_ROCM_FN_GQA_F32_HALVED_128,
+    YVEX_ROCM_FN_GQA_F32_HALVED_256,
+    YVEX_ROCM_FN_GQA_F32_MERGE_64,
+    YVEX_ROCM_FN_GQA_F32_MERGE_128,
+    YVEX_ROCM_FN_GQA_F32_MERGE_256,
     YVEX_ROCM_FN_FILL_U32,
     YVEX_ROCM_FN_DECODE_PAGED_BF16,
     YVEX_ROCM_FN_DECODE_PAGED_BF16_64,
@@ -256,6 +265,23 @@ typedef struct {
     unsigned long long rows;                         /* query tokens x query heads */
     int causal;
 } yvex_rocm_attention_geometry;
+/* How the walk of a request is cut (rocm_prefill.c): packed rows, items, runs of keys
+ * (kernel_params.h, yvex_rocm_prefill_params). */
+typedef struct {
+    unsigned long long pack, row_heads, rows, query_tiles, whole_items, tail_items, splits;
+    unsigned long long acc_bytes, ml_bytes; /* partials of the tail */
+    unsigned long long step_keys;           /* keys of a step of the walk */
+    int short_walks; /* bf16 at head dimension 256: on the kernel for those */
+} yvex_rocm_walk_plan;
+void yvex_rocm_walk_plan_whole(const yvex_transformer_attention_requirement *r, unsigned long long pack,
+                               unsigned long long step_keys, yvex_rocm_walk_plan *plan);
+void yvex_rocm_walk_plan_cut(const yvex_transformer_attention_requirement *r, yvex_rocm_walk_plan *plan);
+/* rocm_halved.c: prefill-shaped EXACT_F32 requests with an attached workspace; *taken 0: nothing was
+ * launched, the request is for the kernels that need none */
+unsigned long long yvex_rocm_halved_workspace(const yvex_transformer_attention_requirement *r);
+int yvex_rocm_halved_launch(yvex_backend *backend, const yvex_transformer_attention_request *request,
+                            const yvex_rocm_gqa_f32_params *f, yvex_backend_operation_facts *facts, int *taken,
+                            yvex_error *err);
 /* rocm_prefill.c: the BF16 contract over more than one query row (or a geometry the decode teams
  * do not take), on the MFMA prefill kernels */
 unsigned long long yvex_rocm_prefill_workspace(const yvex_transformer_attention_requirement *r);

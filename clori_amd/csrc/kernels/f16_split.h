@@ -7,6 +7,7 @@
 namespace {
 
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
+typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ floatx16 mfma_32x32x16_f16(halfx8 a, halfx8 b, floatx16 c)
 {
@@ -75,6 +76,29 @@ __device__ __forceinline__ void for_each(const F &f)
 YVEX_SPLIT_PAIR(split_pair, "s")          // a factor that is the same in all lanes
 YVEX_SPLIT_PAIR(split_pair_by_lane, "v")
 #undef YVEX_SPLIT_PAIR
+
+// The same in two steps.
+__device__ __forceinline__ void split_hi(float a, float b, float factor, uint32_t &hi)
+{
+    __asm__ volatile("v_fma_mixlo_f16 %0, %1, %3, 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0"
+                     : "=&v"(hi)
+                     : "v"(a), "v"(b), "s"(factor));
+}
+__device__ __forceinline__ void split_lo(float a, float b, float factor, uint32_t hi, uint32_t &lo)
+{
+    __asm__ volatile("v_fma_mixlo_f16 %0, %1, %3, -%4 op_sel_hi:[0,0,1]\n\t"
+                     "v_fma_mixhi_f16 %0, %2, %3, -%4 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+                     : "=&v"(lo)
+                     : "v"(a), "v"(b), "s"(factor), "v"(hi));
+}
+
+// x / y given r = 1 / y: one step of Newton's method from x r, which leaves the nearest value but for rare
+// halfway cases (a division takes four times as many instructions; a row has head_dim of them).
+__device__ __forceinline__ float quotient(float x, float y, float r)
+{
+    const float q = x * r;
+    return fmaf(fmaf(-q, y, x), r, q);
+}
 
 }  // namespace
 

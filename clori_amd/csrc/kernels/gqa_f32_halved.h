@@ -1,0 +1,547 @@
+// EXACT_F32 attention over keys and values that were split into halves beforehand.
+//
+// The products are those of gqa_f32_halves.h (an F32 product as three f16 products, the same powers of
+// two), but the splits, which took half of the vector work there, and which every workgroup made for
+// itself, are made once by a launch of their own (halve_rows) that leaves every tile of 32 keys as the walk wants
+// it in LDS: the walk's tiles are filled by loads that write LDS directly, its registers
+// hold no rows on their way, and a trip is bound by its MFMAs.  Items, packed rows and runs of keys are those of
+// the bf16 prefill (kernel_params.h), with steps of 32 keys.
+//
+// What bounds the walk is power: 4096 tokens of 40/8 heads of 128 run at 1.66 GHz with the matrix cores busy
+// 62 % of the cycles, 1.1 PFLOP/s of f16 products (a large bf16 product reaches 1.29 on this part), 373
+// TFLOP/s of F32 ones; 1777 tokens 112 of 118 us.  Trips that prefetch their first operands across the barrier, and
+// peaks without canonical forms, made no difference there (122 against 121 us), which is why no more is
+// hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us).
+#ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
+#define YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
+
+#include "../kernel_params.h"
+#include "f16_split.h"
+#include "gqa_f32_halve_rows.h"
+#include "gqa_f32_walk.h"
+#include "mfma.h"
+#include "prefill_rows.h"
+
+namespace {
+
+// The walk.  A workgroup of four waves of 32 packed rows owns one item or one run of its keys.  Products are
+// transposed (S^T = K Q^T, O^T += V^T P^T, 32x32x16), so a lane owns one row and 16 of a tile's 32
+// keys, and the weights are the operand of the second product where they are.
+//
+// The trip of tile t is one sequence of slots, an MFMA each: first S^T of tile t+1, then the update
+// with tile t; behind the MFMAs ride the loads of K(t+2) and V(t+1), the exponentials of tile t and their
+// split, and the maximum of tile t+1.  An MFMA leaves room for about 24 cycles of vector work (whole
+// instructions take 4 to 5, the exponential and the conversions 8 to 9), so a pair of weights is
+// four steps of less than that.
+template <int kDim>
+struct GqaHalved {
+    typedef HalvedTile<kDim> Tile;
+    static constexpr int kBlocks = kDim / 32, kSteps = kDim / 16, kKeys = Tile::kKeys;
+    static constexpr int kRows = YVEX_ROCM_PREFILL_ROWS, kPlane = Tile::kPlane, kTensor = Tile::kTensor;
+    static constexpr int kLoads = kTensor / 4096;  // 1 KB loads per wave and K or V tile
+    static constexpr int kHalfSlots = 3 * kSteps, kSlots = 2 * kHalfSlots;
+    // weights are at most 2^kLazy (a maximum is raised when it is exceeded by that), so times
+    // 2^kWeightShift they stay inside f16
+    static constexpr int kLazy = 6, kWeightShift = 15 - kLazy;
+
+    static constexpr int kKeyBuffers = 3;
+
+    struct Shared {
+        __attribute__((aligned(16))) unsigned char k[kKeyBuffers][kTensor];
+        __attribute__((aligned(16))) unsigned char v[2][kTensor];
+    };
+
+    const yvex_rocm_gqa_f32_halved_params &p;
+    Shared &lds;
+    const int lane, wave, column, half;
+    uint32_t first_tile, tiles;      // of this workgroup's run
+    int visible;                     // last key the lane's row sees, from the run's first on
+    i32x4 rsrc;                      // the kv head's tiles
+    const uint32_t *factors;         // and their factors
+    uint32_t lds_base, k_unit, v_unit[2];
+    halfx8 q_hi[kSteps], q_lo[kSteps];
+    float q_factor;
+    floatx16 out[kBlocks];
+    float top, neg_top, sum;         // the maximum that weights are relative to (log2 units), this half's denominator
+    int reference;                   // the exponent that the accumulators are relative to
+    floatx4 next_factor;             // of the keys of the tile after the next, on their way
+    u32x4 next_exponent;             // of the values of the next tile
+    uint32_t key_buffer;             // the K tile that the last trip left: free for the next load
+
+    __device__ GqaHalved(const yvex_rocm_gqa_f32_halved_params &params, Shared &shared, int thread)
+        : p(params), lds(shared), lane(thread & 63), wave(__builtin_amdgcn_readfirstlane(thread >> 6)),
+          column(thread & 31), half((thread >> 5) & 1)
+    {
+    }
+
+    // 1 KB load j of this wave for the K or V tile `tile` into buffer `buf`; tiles past the last are the
+    // last once more, so that a trip has no branches.
+    __device__ __forceinline__ void stage(uint32_t tile, uint32_t to, uint32_t at, int j) const
+    {
+        const uint32_t mine = (uint32_t)(wave * (kTensor / 4) + j * 1024);
+        lds_dma_b128(lds_base + to + mine, rsrc, (uint32_t)lane * 16u,
+                     (uint32_t)__builtin_amdgcn_readfirstlane(
+                         (int)((first_tile + min(tile, tiles - 1u)) * (uint32_t)Tile::kBytes + at + mine)));
+    }
+    __device__ __forceinline__ void stage_keys(uint32_t tile, uint32_t buf, int j) const
+    {
+        stage(tile, buf * (uint32_t)kTensor, 0u, j);
+    }
+    __device__ __forceinline__ void stage_values(uint32_t tile, int buf, int j) const
+    {
+        stage(tile, (uint32_t)((kKeyBuffers + buf) * kTensor), (uint32_t)kTensor, j);
+    }
+
+    __device__ __forceinline__ void fetch_factors(uint32_t k_tile, uint32_t v_tile)
+    {
+        // (through the vector memory path: a scalar load would make every LDS wait a full one)
+        uint32_t zero = 0u;
+        __asm__ volatile("" : "+v"(zero));
+        const uint32_t *at = factors + zero;
+        next_factor = *reinterpret_cast<const floatx4 *>(at + (first_tile + min(k_tile, tiles - 1u)) * 8u);
+        next_exponent = *reinterpret_cast<const u32x4 *>(at + (first_tile + min(v_tile, tiles - 1u)) * 8u + 4u);
+    }
+
+    // `unit`: of the lane, in the tile's buffer
+    __device__ __forceinline__ halfx8 key_operand(uint32_t unit, int step, int plane) const
+    {
+        return *reinterpret_cast<const halfx8 *>(lds.k[0] + unit + step * 1024 + plane * kPlane);
+    }
+    // operand m = u * kBlocks + block
+    __device__ __forceinline__ halfx8 value_operand(int buf, int m, int plane) const
+    {
+        const int u = m / kBlocks, b = m % kBlocks;
+        return *reinterpret_cast<const halfx8 *>(lds.v[buf] + v_unit[b & 1] + u * kDim * 32 + b * 512 +
+                                                 plane * kPlane);
+    }
+
+    __device__ __forceinline__ void mask(floatx16 &s, uint32_t tile) const
+    {
+        int seen = visible - (int)(tile * kKeys) - 4 * half;
+        __asm__ volatile("" : "+v"(seen));  // (the sixteen sums are not to be kept in registers)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 8 * (i / 4) + i % 4 <= seen ? s[i] : -INFINITY;
+    }
+
+    // the largest of four scores in log2 units, with what came before
+    __device__ static __forceinline__ float peak_of(const floatx16 &s, const floatx4 &factor, int g, float peak)
+    {
+        const float m = fmaxf(fmaxf(fmaxf(s[4 * g], s[4 * g + 1]), s[4 * g + 2]), s[4 * g + 3]);
+        return fmaxf(peak, m * factor[g]);
+    }
+    __device__ static __forceinline__ float peak_of(const floatx16 &s, const floatx4 &factor)
+    {
+        return peak_of(s, factor, 3, peak_of(s, factor, 2, peak_of(s, factor, 1, peak_of(s, factor, 0, -INFINITY))));
+    }
+    // The same without fmaxf's canonical forms.  The compiler sees no instructions here: the scores must
+    // have been complete for some MFMAs.
+    __device__ static __forceinline__ void peak_step(const floatx16 &s, const floatx4 &factor, int g, float &peak)
+    {
+        float m;
+        __asm__ volatile("v_max3_f32 %0, %2, %3, %4\n\t"
+                         "v_max_f32 %0, %0, %5\n\t"
+                         "v_mul_f32 %0, %0, %6\n\t"
+                         "v_max_f32 %1, %1, %0"
+                         : "=&v"(m), "+v"(peak)
+                         : "v"(s[4 * g]), "v"(s[4 * g + 1]), "v"(s[4 * g + 2]), "v"(s[4 * g + 3]), "v"(factor[g]));
+    }
+
+    // Brings the maximum to the peak of a tile (over both halves of a row) that exceeds it by more than
+    // 2^kLazy in some row, and what is accumulated to the exponents of the tile's values.
+    __device__ __forceinline__ void adjust(float peak, int most)
+    {
+        const float raised = fmaxf(top, peak);
+        // a row that has seen nothing yet keeps the maximum -inf
+        float keep = raised == -INFINITY ? 1.f : fast_exp2(top - raised);
+        sum *= keep;
+        if (most > reference) {
+            // one power of two of room, so that the accumulators seldom move
+            keep = __builtin_amdgcn_ldexpf(keep, reference - most - 1);
+            reference = most + 1;
+            if (most > (int)kExponentMost) sum = __builtin_nanf("");  // values past the range
+        }
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) out[b][i] *= keep;
+        top = raised;
+        neg_top = raised == -INFINITY ? 0.f : -raised;
+    }
+
+    // What goes from trip to trip beside the scores: the operands of the first slots, the peak of the
+    // tile in this lane's half of its row.
+    struct Carried {
+        halfx8 hi[2], lo[2];
+        float peak;
+    };
+
+    // The trip of tile t; kAt = t % 2.
+    template <int kAt>
+    __device__ __forceinline__ void trip(uint32_t t, uint32_t wave_tiles, uint32_t unmasked, floatx16 &s_cur,
+                                         floatx16 &s_next, floatx4 &f_cur, floatx4 &f_next, Carried &c)
+    {
+        constexpr int kNext = kAt ^ 1;
+        // K(t+2) and V(t) have landed (this wave's loads, then everybody's); every wave is done with
+        // K(t) and V(t-1)
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        __syncthreads();
+        f_next = next_factor * q_factor;
+        u32x4 exponents = next_exponent;
+        __asm__ volatile("" : "+v"(f_next), "+v"(exponents));
+        fetch_factors(t + 2u, t + 1u);
+        const uint32_t free_keys = key_buffer;
+        key_buffer = key_buffer == 2u ? 0u : key_buffer + 1u;  // of t+1, and after that of t+2
+        if (t >= wave_tiles) {
+            // nothing of this tile is visible to the wave: it only keeps staging
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j) stage_keys(t + 3u, free_keys, j);
+#pragma unroll
+            for (int j = 0; j < kLoads; ++j) stage_values(t + 1u, kNext, j);
+            return;
+        }
+        const uint32_t k_now = k_unit + key_buffer * (uint32_t)kTensor;
+        const uint32_t k_then = k_unit + (key_buffer == 2u ? 0u : key_buffer + 1u) * (uint32_t)kTensor;
+        halfx8(&hi)[2] = c.hi, (&lo)[2] = c.lo;
+        float weight_factor[4];
+        uint32_t p_hi[8], p_lo[8];
+        float part_sum = 0.f, peak = -INFINITY;
+        int e[4], most = 0;
+        bool raise = false;
+        // the maximum of this tile's rows and the exponents of its values
+        auto settle_step = [&](int k) __attribute__((always_inline)) {
+            if (k < 4) {
+                e[k] = __builtin_amdgcn_readfirstlane((int)exponents[k]);
+                most = max(most, e[k]);
+            }
+            if (k == 0) c.peak = max_xor32(c.peak);
+            if (k == 2) raise = __builtin_amdgcn_ballot_w64(c.peak > top + (float)kLazy) != 0ull;
+        };
+        // pair k / 4 of the weights: the two exponentials, then their hi and their lo halves
+        auto weigh_step = [&](int k) __attribute__((always_inline)) {
+            const int w = k / 4 * 2 + k % 4;
+            if (k % 4 < 2) {
+                s_cur[w] = fast_exp2(fmaf(s_cur[w], f_cur[w / 4], neg_top));
+                part_sum += s_cur[w];
+                // (behind the sum: the exponential's result has been read once)
+                __asm__ volatile("" : "+v"(s_cur[w]), "+v"(part_sum));
+            } else if (k % 4 == 2) {
+                split_hi(s_cur[w - 2], s_cur[w - 1], weight_factor[k / 8], p_hi[k / 4]);
+            } else {
+                split_lo(s_cur[w - 3], s_cur[w - 2], weight_factor[k / 8], p_hi[k / 4], p_lo[k / 4]);
+            }
+        };
+        constexpr int kSettled = 4;  // slots before the weights can be formed
+        auto slot = [&](auto index) __attribute__((always_inline)) {
+            constexpr int i = decltype(index)::value;
+            constexpr int m = (i % kHalfSlots) / 3, term = i % 3;
+            if constexpr (i < kHalfSlots) {
+                const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+                s_next = mfma_32x32x16_f16(term == 0 ? lo[m % 2] : hi[m % 2], term == 1 ? q_lo[m] : q_hi[m],
+                                           i == 0 ? zero : s_next);
+            } else {
+                constexpr int first = m / kBlocks * 4;
+                u32x4 words;
+                if constexpr (term == 1)
+                    words = (u32x4){p_lo[first], p_lo[first + 1], p_lo[first + 2], p_lo[first + 3]};
+                else
+                    words = (u32x4){p_hi[first], p_hi[first + 1], p_hi[first + 2], p_hi[first + 3]};
+                out[m % kBlocks] = mfma_32x32x16_f16(term == 0 ? lo[m % 2] : hi[m % 2],
+                                                     __builtin_bit_cast(halfx8, words), out[m % kBlocks]);
+            }
+            // the operands two steps on: of K(t+1), of V(t), and of K(t+2) for the next trip
+            if constexpr (term != 1) {
+                constexpr int n = m + 2 + (i < kHalfSlots ? 0 : kSteps);
+                halfx8 &into = (term == 0 ? lo : hi)[m % 2];
+                if constexpr (n < kSteps) into = key_operand(k_now, n, term == 0);
+                else if constexpr (n < 2 * kSteps) into = value_operand(kAt, n - kSteps, term == 0);
+                else into = key_operand(k_then, n - 2 * kSteps, term == 0);
+            }
+            if constexpr (i < kLoads) stage_keys(t + 3u, free_keys, i);
+            else if constexpr (i < 2 * kLoads) stage_values(t + 1u, kNext, i - kLoads);
+            ride<i, 4, 0, kSettled>(settle_step);
+            // the first eight weights before the update's first MFMA, the others before its second half, with
+            // two slots between a split and the MFMA that reads it
+            ride<i, 16, kSettled, kHalfSlots - 1>(weigh_step);
+            ride<i, 16, kHalfSlots - 1, 3 * kHalfSlots / 2 - 1>(
+                [&](int k) __attribute__((always_inline)) { weigh_step(16 + k); });
+            ride<i, 4, 3 * kHalfSlots / 2, kSlots>(
+                [&](int g) __attribute__((always_inline)) { peak_step(s_next, f_next, g, peak); });
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        __builtin_amdgcn_sched_barrier(0);
+        for_each<kSettled>(slot);
+        if (raise || most > reference) adjust(c.peak, most);
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            weight_factor[g] = power_of_two((uint32_t)max(127 + kWeightShift + e[g] - reference, 0));
+        __builtin_amdgcn_sched_barrier(0);
+        for_each<kSlots, kSettled>(slot);
+        sum += part_sum;
+        if (t + 1u >= unmasked && t + 1u < wave_tiles) {
+            mask(s_next, t + 1u);
+            peak = peak_of(s_next, f_next);
+        }
+        c.peak = peak;
+    }
+
+    // Steps of a kind, spread over slots [kFrom, kTo).
+    template <int kSlot, int kCount, int kFrom, int kTo, typename F>
+    __device__ static __forceinline__ void ride(const F &step)
+    {
+        for_each<kCount>([&](auto k) __attribute__((always_inline)) {
+            if constexpr (kFrom + decltype(k)::value * (kTo - kFrom) / kCount == kSlot) step(decltype(k)::value);
+        });
+    }
+
+    __device__ __forceinline__ void load_queries(const float *row)
+    {
+        float most = 0.f;
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            const floatx4 a = *reinterpret_cast<const floatx4 *>(row + 16 * s);
+            const floatx4 b = *reinterpret_cast<const floatx4 *>(row + 16 * s + 4);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) most = fmaxf(most, fmaxf(fabsf(a[j]), fabsf(b[j])));
+        }
+        const uint32_t bits = __builtin_bit_cast(uint32_t, max_xor32(most)), e = group_exponent(bits);
+        q_factor = bits >> 23 > kExponentMost ? __builtin_nanf("") : up_factor(e) * (p.scale * YVEX_LOG2E);
+        // (read a second time: the registers are short)
+        __asm__ volatile("" : "+v"(row));
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s) {
+            const floatx4 a = *reinterpret_cast<const floatx4 *>(row + 16 * s);
+            const floatx4 b = *reinterpret_cast<const floatx4 *>(row + 16 * s + 4);
+            uint32_t h[4], l[4];
+            split_pair_by_lane(a[0], a[1], down_factor(e), h[0], l[0]);
+            split_pair_by_lane(a[2], a[3], down_factor(e), h[1], l[1]);
+            split_pair_by_lane(b[0], b[1], down_factor(e), h[2], l[2]);
+            split_pair_by_lane(b[2], b[3], down_factor(e), h[3], l[3]);
+            const u32x4 hi = {h[0], h[1], h[2], h[3]}, lo = {l[0], l[1], l[2], l[3]};
+            q_hi[s] = __builtin_bit_cast(halfx8, hi);
+            q_lo[s] = __builtin_bit_cast(halfx8, lo);
+        }
+    }
+
+    __device__ __forceinline__ void run()
+    {
+        const yvex_rocm_prefill_params &w = p.walk;
+        uint32_t item = blockIdx.x, split = 0u;
+        const bool partial = item >= w.whole_items;
+        if (partial) {
+            split = (item - w.whole_items) / w.tail_items;
+            item = w.whole_items + (item - w.whole_items) % w.tail_items;
+        } else if (item >= p.pair_units && item < 2u * p.pair_units) {
+            // the second workgroup of a unit takes the second tier of items in reverse
+            item = 3u * p.pair_units - 1u - item;
+        }
+        const uint32_t level = item / w.row_heads, row_head = item - level * w.row_heads;
+        const uint32_t kv_head = kv_head_of(w, row_head);
+        const uint32_t tile_row = (w.query_tiles - 1u - level) * kRows, tile_end = min(w.rows, tile_row + kRows);
+        const uint32_t row0 = tile_row + (uint32_t)wave * 32u;
+        auto last_of = [&](uint32_t row) {
+            return w.causal ? min(w.kv_tokens, w.query_start + token_of(w, row) + 1u) : w.kv_tokens;
+        };
+        tiles = (last_of(tile_end - 1u) + kKeys - 1u) / kKeys;
+        first_tile = 0u;
+        if (partial) {
+            const uint32_t per_split = (tiles + w.splits - 1u) / w.splits;
+            first_tile = min(tiles, split * per_split);
+            tiles = min(per_split, tiles - first_tile);
+            if (tiles == 0u) first_tile = 0u;  // a run without steps
+        }
+        const int first_key = (int)(first_tile * kKeys);
+        const bool wave_active = row0 < w.rows && tiles != 0u;
+        const int wave_first_sees = (int)last_of(min(row0, w.rows - 1u)) - first_key;  // keys, as a count
+        const int wave_last_sees = (int)last_of(min(row0 + 32u, w.rows) - 1u) - first_key;
+        const uint32_t wave_tiles =
+            wave_active && wave_last_sees > 0 ? min(tiles, (uint32_t)(wave_last_sees + kKeys - 1) / kKeys) : 0u;
+        const uint32_t unmasked = wave_first_sees > 0 ? (uint32_t)wave_first_sees / kKeys : 0u;
+        const uint32_t row = min(row0 + (uint32_t)column, w.rows - 1u), token = token_of(w, row);
+        const uint32_t head = row_head * w.pack + (row - token * w.pack);
+        visible = (int)last_of(row) - 1 - first_key;
+
+        const uint64_t head_bytes = (uint64_t)p.kv_tiles * Tile::kBytes;
+        rsrc = raw_buffer(p.tiles + kv_head * head_bytes, (uint32_t)head_bytes);
+        factors = p.factors + (uint64_t)kv_head * p.kv_tiles * 8u;
+        lds_base = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address_of(lds.k[0]));
+        k_unit = (uint32_t)(half * 32 + column) * 16u;
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            v_unit[b] = (uint32_t)((half * kDim + Tile::value_unit(32 * b + column)) * 16 - b * 512);
+        reference = 0;
+        top = -INFINITY;
+        neg_top = 0.f;
+        sum = 0.f;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) out[b][i] = 0.f;
+
+        if (tiles != 0u) walk_tiles(wave_tiles, unmasked, (const float *)w.q + (uint64_t)token * w.q_stride +
+                                                              (uint64_t)head * kDim + 8 * half);
+
+        // the accumulators are relative to 2^(reference - 127), weights to 2^kWeightShift and values to 2^14
+        const bool own = row0 + (uint32_t)column < w.rows;
+        sum = sum_xor32(sum);
+        const float inverse = 1.0f / sum;
+        // (a run none of whose keys the row sees leaves a maximum of -inf and nothing)
+        bool good = isfinite(sum) && (partial && top == -INFINITY ? sum == 0.f : sum > 0.f && isfinite(top));
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                out[b][i] = __builtin_amdgcn_ldexpf(partial ? out[b][i] : quotient(out[b][i], sum, inverse),
+                                                    reference - (141 + kWeightShift));
+                good &= isfinite(out[b][i]);
+            }
+        // (the tiles in LDS are done with)
+        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.k[0]);
+        __syncthreads();
+        if (lane == 0 && wave == 0) *verdict = 0u;
+        __syncthreads();
+        if (own && !good) *verdict = 1u;
+        __syncthreads();
+        const bool failed = *verdict != 0u;
+        const uint32_t slot = partial ? (item - w.whole_items) * w.splits + split : 0u;
+        if (failed) {
+            __syncthreads();  // every wave has read the verdict
+            walk_again(partial, slot, row_head, tile_row, tile_end);
+            return;
+        }
+        if (!own) return;
+        if (partial)
+            leave_partial(slot, row - tile_row, out, top, sum);
+        else
+            publish(head, token, out, top * YVEX_LN2 + logf(sum));
+    }
+
+    __device__ __forceinline__ void walk_tiles(uint32_t wave_tiles, uint32_t unmasked, const float *query)
+    {
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) stage_keys(0u, 0u, j);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) stage_keys(1u, 1u, j);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) stage_values(0u, 0, j);
+        fetch_factors(0u, 0u);
+        load_queries(query);
+        floatx4 f_even = next_factor * q_factor, f_odd;
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        __syncthreads();
+        fetch_factors(1u, 0u);
+#pragma unroll
+        for (int j = 0; j < kLoads; ++j) stage_keys(2u, 2u, j);
+        floatx16 s_even, s_odd;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s_even[i] = 0.f;
+#pragma unroll
+        for (int m = 0; m < kSteps; ++m) {
+            const halfx8 lo = key_operand(k_unit, m, 1), hi = key_operand(k_unit, m, 0);
+            s_even = mfma_32x32x16_f16(lo, q_hi[m], s_even);
+            s_even = mfma_32x32x16_f16(hi, q_lo[m], s_even);
+            s_even = mfma_32x32x16_f16(hi, q_hi[m], s_even);
+        }
+        Carried c;
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            c.lo[k] = key_operand(k_unit + kTensor, k, 1);
+            c.hi[k] = key_operand(k_unit + kTensor, k, 0);
+        }
+        if (unmasked == 0u) mask(s_even, 0u);
+        c.peak = peak_of(s_even, f_even);
+        key_buffer = 0u;
+        // (two copies of a trip instead of three take less time to fetch: 1777 tokens 122 -> 118.5 us; at 256 the
+        // compiler moves more registers about in that form: 1000 tokens 112 -> 132)
+        uint32_t t = 0u;
+        if constexpr (kDim == 256) {
+            for (; t + 1u < tiles; t += 2u) {
+                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, f_even, f_odd, c);
+                trip<1>(t + 1u, wave_tiles, unmasked, s_odd, s_even, f_odd, f_even, c);
+            }
+            if (t < tiles) trip<0>(t, wave_tiles, unmasked, s_even, s_odd, f_even, f_odd, c);
+        } else {
+            for (;;) {
+                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, f_even, f_odd, c);
+                if (++t == tiles) break;
+                trip<1>(t, wave_tiles, unmasked, s_odd, s_even, f_odd, f_even, c);
+                if (++t == tiles) break;
+            }
+        }
+        // nothing may still be in flight into LDS
+        __builtin_amdgcn_s_waitcnt(0x0f70);
+    }
+
+    __device__ __forceinline__ void publish(uint32_t head, uint32_t token, const floatx16 (&o)[kBlocks],
+                                            float lse) const
+    {
+        const uint64_t at = (uint64_t)token * p.walk.query_heads + head;
+        float *row = (float *)p.walk.out + at * kDim;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<floatx4 *>(row + 32 * b + 8 * g + 4 * half) =
+                    (floatx4){o[b][4 * g], o[b][4 * g + 1], o[b][4 * g + 2], o[b][4 * g + 3]};
+        if (p.walk.lse && half == 0) p.walk.lse[at] = lse;
+    }
+
+    // What this run of keys contributes to row `row` of its tile (the maximum in log2 units).
+    __device__ __forceinline__ void leave_partial(uint32_t slot, uint32_t row, const floatx16 (&o)[kBlocks], float m,
+                                                  float l) const
+    {
+        const uint64_t at = (uint64_t)slot * kRows + row;
+        if (half == 0) {
+            p.walk.part_ml[at * 2u] = m;
+            p.walk.part_ml[at * 2u + 1u] = l;
+        }
+        float *acc = p.walk.part_acc + at * kDim + half * 4;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<floatx4 *>(acc + b * 32 + g * 8) =
+                    (floatx4){o[b][g * 4], o[b][g * 4 + 1], o[b][g * 4 + 2], o[b][g * 4 + 3]};
+    }
+
+    // The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.
+    __device__ __forceinline__ void walk_again(bool partial, uint32_t slot, uint32_t row_head,
+                                                         uint32_t tile_row, uint32_t tile_end) const
+    {
+        const yvex_rocm_prefill_params &w = p.walk;
+        yvex_rocm_gqa_f32_params f = {};
+        f.q = (const float *)w.q;
+        f.k = (const float *)w.k;
+        f.v = (const float *)w.v;
+        f.out = (float *)w.out;
+        f.lse = w.lse;
+        f.status = w.status;
+        f.query_tokens = w.query_tokens;
+        f.kv_tokens = w.kv_tokens;
+        f.query_start = w.query_start;
+        f.query_heads = w.query_heads;
+        f.kv_heads = w.kv_heads;
+        f.q_stride = w.q_stride;
+        f.k_stride = w.k_stride;
+        f.v_stride = w.v_stride;
+        f.scale = p.scale;
+        f.causal = (int32_t)w.causal;
+        const GqaTile<kBlocks> tile(f, reinterpret_cast<float *>(&lds), wave * 64 + lane);
+        for (uint32_t h = 0u; h < w.pack; ++h) {
+            // rows token * pack + h in [tile_row, tile_end)
+            const uint32_t first = (tile_row + w.pack - 1u - h) / w.pack, end = (tile_end + w.pack - 1u - h) / w.pack;
+            if (first >= end) continue;
+            tile.walk(row_head * w.pack + h, first, end, first_tile, partial ? first_tile + tiles : ~0ull >> 8,
+                      [&](uint64_t head, uint64_t token, floatx16(&o)[kBlocks], float m, float l) {
+                          if (partial)
+                              leave_partial(slot, (uint32_t)token * w.pack + h - tile_row, o, m * YVEX_LOG2E, l);
+                          else
+                              tile.publish(head, token, o, m, l);
+                      });
+            __syncthreads();  // every wave is done with the tiles in LDS
+        }
+    }
+};
+
+}  // namespace
+
+#endif  // YVEX_ROCM_KERNELS_GQA_F32_HALVED_H

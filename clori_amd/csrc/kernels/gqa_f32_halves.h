@@ -16,15 +16,10 @@
 
 #include "../kernel_params.h"
 #include "f16_split.h"
+#include "gqa_f32_walk.h"
 #include "mfma.h"
 
 namespace {
-
-// Last key a query may see (the rows of 2^32 keys are more than any memory holds).
-__device__ __forceinline__ uint32_t last_visible(const yvex_rocm_gqa_f32_params &p, uint64_t own)
-{
-    return (uint32_t)(p.causal ? min(p.kv_tokens - 1u, own) : p.kv_tokens - 1u);
-}
 
 // One workgroup = one item: 128 consecutive query tokens of one query head, a team of four waves of 32
 // queries (kParts = 1), or two teams that split the head dimension (kParts = 2, head dimension
@@ -569,12 +564,14 @@ struct GqaHalves {
         // the accumulators are relative to 2^(reference - 127), weights to 2^kWeightShift and values to 2^14
         const bool own = q0 + (uint64_t)column < p.query_tokens;
         sum = sum_xor32(sum);
+        const float inverse = 1.0f / sum;
         bool good = sum > 0.f && isfinite(sum) && isfinite(top);
 #pragma unroll
         for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                out[b][i] = __builtin_amdgcn_ldexpf(out[b][i] / sum, reference - (141 + kWeightShift));
+                out[b][i] = __builtin_amdgcn_ldexpf(quotient(out[b][i], sum, inverse),
+                                                    reference - (141 + kWeightShift));
                 good &= isfinite(out[b][i]);
             }
         if (extreme || (own && !good)) lds.failed = 1u;

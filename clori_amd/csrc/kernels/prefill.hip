@@ -53,6 +53,7 @@
 //
 #include "mfma.h"
 #include "prefill_rows.h"
+#include "run_merge.h"
 
 #include "../kernel_params.h"
 
@@ -509,94 +510,24 @@ YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16, 128, 2)
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_64, 64, 2)
 YVEX_PREFILL_KERNEL(yvex_rocm_prefill_bf16_256_short, 256, 1)
 
-// Log-sum-exp merge of the runs of the split items and publication of their rows.  head_dim / 4
-// threads per row and group, four lanes of the row each; the runs of a row are dealt to
-// merge_groups (1 or 4) groups of threads, merged within each in the order of the runs and then
-// group by group.  grid = tail_items * YVEX_ROCM_PREFILL_ROWS * head_dim / 4 * merge_groups / 256,
-// block = 256.
-// A trip of eight runs is a trip to memory, and few tokens leave few rows to hide it: 9 tokens of
-// 40/8 heads of 128 in 32 runs took 6.5 us with one group (four trips one after the other): the call
-// 20.1 us, now 17.4 us.
+// (run_merge.h: grid, groups)
 template <int kHeadDim>
 __device__ __forceinline__ void prefill_merge(const yvex_rocm_prefill_params &p, floatx4 *acc_of, float2 *ml_of)
 {
-    constexpr uint32_t kThreads = kHeadDim / 4;
-    constexpr int kWidth = 8;  // runs in flight per trip
-    const uint32_t groups = p.merge_groups, member = threadIdx.x / kThreads, d = (threadIdx.x % kThreads) * 4u;
-    const uint32_t group = member & (groups - 1u);
-    const uint32_t packed = blockIdx.x * (256u / kThreads / groups) + member / groups;
-    const uint32_t tail = packed / kRowsPerBlock, in_tile = packed % kRowsPerBlock;
-    const uint32_t item = p.whole_items + tail;
-    const uint32_t row = (p.query_tiles - 1u - item / p.row_heads) * kRowsPerBlock + in_tile;
-    const bool live = row < p.rows;
-    const uint64_t first = (uint64_t)tail * p.splits * kRowsPerBlock + in_tile;
-    const uint32_t each = (p.splits + groups - 1u) / groups;
-    const uint32_t begin = min(group * each, p.splits), end = live ? min(begin + each, p.splits) : begin;
-    float top = -INFINITY, sum = 0.f;
-    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-    for (uint32_t s0 = begin; s0 < end; s0 += (uint32_t)kWidth) {
-        float m[kWidth], l[kWidth];
-        floatx4 part[kWidth];
-#pragma unroll
-        for (int i = 0; i < kWidth; ++i) {
-            // runs past the end alias the last one, with weight zero
-            const uint64_t at = first + (uint64_t)min(s0 + (uint32_t)i, end - 1u) * kRowsPerBlock;
-            m[i] = p.part_ml[at * 2u];
-            l[i] = p.part_ml[at * 2u + 1u];
-            part[i] = *reinterpret_cast<const floatx4 *>(p.part_acc + at * kHeadDim + d);
+    merge_runs<kHeadDim>(p, acc_of, ml_of, [&](uint64_t row, uint32_t d, const floatx4 &acc, float top, float sum) {
+        const uint64_t at = row * kHeadDim + d;
+        const float inv = 1.0f / sum;
+        bool bad = !isfinite(sum);  // (an infinite sum would publish zeros)
+        bad |= !(isfinite(acc[0] * inv) && isfinite(acc[1] * inv) && isfinite(acc[2] * inv) && isfinite(acc[3] * inv));
+        u32x2 w = {pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv)};
+        if (p.gate) {
+            w = gate_four(w, p.gate + at);
+            bad |= pair_not_finite(w.x) || pair_not_finite(w.y);
         }
-        float m_new = top;
-#pragma unroll
-        for (int i = 0; i < kWidth; ++i) {
-            if (s0 + (uint32_t)i >= end) m[i] = -INFINITY, l[i] = 0.f;
-            m_new = fmaxf(m_new, m[i]);
-        }
-        const float keep = m_new == -INFINITY ? 1.f : fast_exp2(top - m_new);
-        sum *= keep;
-        acc *= keep;
-#pragma unroll
-        for (int i = 0; i < kWidth; ++i) {
-            if (m[i] == -INFINITY) {  // no rows were left: no key was seen, or only scores that are NaN
-                sum += l[i];
-                continue;
-            }
-            const float w = fast_exp2(m[i] - m_new);
-            sum += w * l[i];
-            acc += w * part[i];
-        }
-        top = m_new;
-    }
-    if (groups != 1u) {
-        acc_of[threadIdx.x] = acc;
-        ml_of[threadIdx.x] = make_float2(top, sum);
-        __syncthreads();
-        if (group != 0u || !live) return;
-        for (uint32_t other = 1u; other < groups; ++other) {
-            const float2 ml = ml_of[threadIdx.x + other * kThreads];
-            if (ml.x == -INFINITY) {
-                sum += ml.y;
-                continue;
-            }
-            const float m_new = fmaxf(top, ml.x), keep = fast_exp2(top - m_new), w = fast_exp2(ml.x - m_new);
-            sum = sum * keep + w * ml.y;
-            acc = acc * keep + w * acc_of[threadIdx.x + other * kThreads];
-            top = m_new;
-        }
-    }
-    if (!live) return;
-    const uint32_t token = token_of(p, row), head = (item % p.row_heads) * p.pack + (row - token * p.pack);
-    const uint64_t at = ((uint64_t)token * p.query_heads + head) * kHeadDim + d;
-    const float inv = 1.0f / sum;
-    bool bad = !isfinite(sum);  // (an infinite sum would publish zeros)
-    bad |= !(isfinite(acc[0] * inv) && isfinite(acc[1] * inv) && isfinite(acc[2] * inv) && isfinite(acc[3] * inv));
-    u32x2 w = {pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv)};
-    if (p.gate) {
-        w = gate_four(w, p.gate + at);
-        bad |= pair_not_finite(w.x) || pair_not_finite(w.y);
-    }
-    *reinterpret_cast<u32x2 *>(p.out + at) = w;
-    if (bad) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
-    if (p.lse && d == 0u) p.lse[(uint64_t)token * p.query_heads + head] = (top + fast_log2(sum)) * YVEX_LN2;
+        *reinterpret_cast<u32x2 *>(p.out + at) = w;
+        if (bad) flag(p.status, YVEX_ROCM_DEVICE_NUMERIC);
+        if (p.lse && d == 0u) p.lse[row] = (top + fast_log2(sum)) * YVEX_LN2;
+    });
 }
 
 #define YVEX_PREFILL_MERGE_KERNEL(name, head_dim)                                                         \

@@ -434,6 +434,105 @@ def test_gqa_matrix_core_kernel_infinities(backend, d, hq, hkv):
         assert e.value.code == B.YVEX_ERR_FORMAT
 
 
+def run_attached(backend, q, k, v, short=0, **kw):
+    """run_exact with the workspace that the request asks for attached (`short` bytes less of it)."""
+    tq, hq, d = q.shape
+    tk, hkv, _ = k.shape
+    need = backend.attention_workspace_required(backend.attention_requirement(tq, tk, hq, hkv, d, **kw))
+    work = backend.tensor("work", B.DTYPE_I8, (max(need - short, 256),))
+    backend.workspace_attach(work)
+    try:
+        return run_exact(backend, q, k, v, **kw) + (need,)
+    finally:
+        backend.workspace_detach()
+        work.release()
+
+
+@pytest.mark.parametrize("tq,tk,hq,hkv,d,start,causal", [
+    (33, 384, 4, 1, 128, 351, True), (129, 385, 10, 2, 128, 256, True), (1000, 1000, 5, 1, 128, 0, True),
+    (40, 3001, 10, 2, 128, 2950, True), (64, 799, 3, 3, 128, 0, False), (520, 1040, 40, 8, 128, 520, True),
+    (32, 257, 6, 2, 64, 224, True), (1300, 1300, 16, 4, 64, 0, True), (77, 9000, 7, 1, 64, 8923, True),
+    (100, 700, 4, 4, 64, 3, False), (32, 641, 6, 1, 256, 609, True), (700, 700, 6, 2, 256, 0, True),
+    (50, 4000, 24, 4, 256, 3950, True), (96, 900, 4, 4, 256, 0, False),
+])
+def test_gqa_split_beforehand_matches_cpu_operator(backend, tq, tk, hq, hkv, d, start, causal):
+    """With its workspace attached a prefill-shaped request splits keys and values beforehand, packs the query
+    heads of a kv head into the rows of a tile and cuts walks that would leave units idle: the same bound as
+    without, at the edges of tiles of 32 keys and 128 rows, from the shortest walk that takes this way."""
+    rng = np.random.default_rng(tq * 17 + tk + d)
+    q = rng.standard_normal((tq, hq, d)).astype(np.float32)
+    k = rng.standard_normal((tk, hkv, d)).astype(np.float32)
+    v = rng.standard_normal((tk, hkv, d)).astype(np.float32)
+    out, lse, facts, need = run_attached(backend, q, k, v, query_start=start, causal=causal)
+    assert need > 0 and facts.temporary_bytes == need
+    assert facts.kernel_launches in (2, 3) and facts.accelerated_matrix_launches == 1
+    rc, ref, ref_lse = ORACLE.gqa(q, k, v, query_start=start, causal=causal)
+    assert rc == 0
+    assert np.abs(out - ref).max() < 2e-5, np.abs(out - ref).max()
+    assert np.abs(lse - ref_lse).max() < 2e-5
+    again, lse_again, _, _ = run_attached(backend, q, k, v, query_start=start, causal=causal)
+    assert np.array_equal(out, again) and np.array_equal(lse, lse_again)
+    # one byte short of what it asked for: one launch, nothing allocated
+    whole, lse_whole, facts, _ = run_attached(backend, q, k, v, short=1, query_start=start, causal=causal)
+    assert facts.kernel_launches == 1 and facts.temporary_bytes == 0
+    assert np.abs(whole - ref).max() < 2e-5 and np.abs(lse_whole - ref_lse).max() < 2e-5
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_gqa_split_beforehand_follows_magnitudes_and_views(backend, d):
+    """Rows over many magnitudes, interleaved rows, values past the range of the halves in a cut walk (their
+    runs are walked in fp32), infinities and NaN."""
+    rng = np.random.default_rng(d + 5)
+    tq, tk, hq, hkv = 45, 1500, 6, 2
+    q, k, v = (rng.standard_normal(shape).astype(np.float32)
+               for shape in ((tq, hq, d), (tk, hkv, d), (tk, hkv, d)))
+    start = tk - tq
+    grown = v * np.exp2(np.linspace(-20, 12, tk)).astype(np.float32)[:, None, None]
+    grown[:8] = 0.0
+    past = v.copy()
+    past[777, 0, 3] = np.float32(2.0 ** 70)
+    for label, case in (("powers", (q * np.float32(2.0 ** -40), k * np.float32(2.0 ** 40), v * np.float32(2.0 ** -90))),
+                        ("grown", (q, k, grown)), ("past", (q, k, past))):
+        out, lse, facts, _ = run_attached(backend, *case, query_start=start)
+        assert facts.kernel_launches == 3
+        rc, ref, ref_lse = ORACLE.gqa(*case, query_start=start)
+        assert rc == 0
+        top = np.abs(case[2]).max(axis=(0, 2))
+        for head in range(hq):
+            assert np.abs(out[:, head] - ref[:, head]).max() <= 2e-5 * top[head // (hq // hkv)], label
+        assert np.abs(lse - ref_lse).max() < 2e-5 * max(1.0, np.abs(ref_lse).max())
+    # interleaved [K | V] rows: the same bits
+    packed, _, _, need = run_attached(backend, q, k, v, query_start=start)
+    rows = f32(backend, "rows", np.concatenate([k.reshape(tk, -1), v.reshape(tk, -1)], axis=1))
+    span, stride = (2 * tk - 1) * hkv * d, 2 * hkv * d
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, query_start=start, k_stride=stride, v_stride=stride)
+    work, out_t = backend.tensor("work", B.DTYPE_I8, (need,)), f32(backend, "out", shape=q.shape)
+    assert backend.attention_workspace_required(req) == need
+    backend.workspace_attach(work)
+    backend.attention_execute(req, f32(backend, "q", q), rows.view(0, B.DTYPE_F32, (span,)),
+                              rows.view(hkv * d * 4, B.DTYPE_F32, (span,)), out_t)
+    backend.workspace_detach()
+    assert np.array_equal(out_t.read(), packed)
+    # a key of -inf that every score excludes, infinities that no query sees, and values that are not finite
+    positive = np.abs(q) + np.float32(0.1)
+    excluded = k.copy()
+    excluded[5, 0, 2] = -np.inf
+    out, _, _, _ = run_attached(backend, positive, excluded, v, query_start=start)
+    rc, ref, _ = ORACLE.gqa(positive, np.where(np.isinf(excluded), np.float32(-1e30), excluded), v, query_start=start)
+    assert rc == 0 and np.abs(out - ref).max() < 2e-5
+    unseen = k.copy()
+    unseen[tk - 30:] = np.inf
+    out, _, _, _ = run_attached(backend, q, unseen, v, query_start=start - 30)
+    rc, ref, _ = ORACLE.gqa(q, k[:tk - 30], v[:tk - 30], query_start=start - 30)
+    assert rc == 0 and np.abs(out - ref).max() < 2e-5
+    for bad, at in ((np.inf, v), (np.nan, v), (np.nan, k)):
+        tensor = at.copy()
+        tensor[700, 1, 7] = bad
+        with pytest.raises(YvexError) as e:
+            run_attached(backend, q, k if at is v else tensor, tensor if at is v else v, query_start=start)
+        assert e.value.code == B.YVEX_ERR_FORMAT
+
+
 # ------------------------------------------------ decode-shaped requests over long contexts ----
 
 @pytest.mark.parametrize("tq,tk,hq,hkv,d,causal", [

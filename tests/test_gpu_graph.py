@@ -168,6 +168,42 @@ def test_recorded_prefill_replays_equal_eager(backend, d, attached):
         x.release()
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("attached", [True, False])
+def test_recorded_exact_prefill_replays_equal_eager(backend, d, attached):
+    """EXACT_F32 tokens behind a history: recorded with the workspace keys and values are split, walked in runs and
+    merged by three launches, recorded without one it is one launch and nothing is allocated."""
+    rng = np.random.default_rng(903 + d)
+    tq, tk, hq, hkv = 40, 2000, 6, 2
+    k, v = (rng.standard_normal((tk, hkv, d)).astype(np.float32) for _ in range(2))
+    req = backend.attention_requirement(tq, tk, hq, hkv, d, query_start=tk - tq)
+    tensors = [backend.tensor("q", B.DTYPE_F32, (tq, hq, d), rng.standard_normal((tq, hq, d)).astype(np.float32)),
+               backend.tensor("k", B.DTYPE_F32, k.shape, k), backend.tensor("v", B.DTYPE_F32, v.shape, v)]
+    out, eager = (backend.tensor(n, B.DTYPE_F32, (tq, hq, d)) for n in ("o", "e"))
+    work = backend.tensor("work", B.DTYPE_I8, (backend.attention_workspace_required(req),))
+    if attached:
+        backend.workspace_attach(work)
+    backend.graph_begin()
+    backend.attention_execute(req, *tensors, out)
+    graph = backend.graph_end()
+    for replay in range(4):
+        q = rng.standard_normal((tq, hq, d)).astype(np.float32)
+        tensors[0].write(q)
+        out.zero()
+        assert backend.graph_launch(graph).kernel_launches == (3 if attached else 1)
+        got = out.read()
+        unrelated_eager_work(backend, rng)
+        backend.attention_execute(req, *tensors, eager)
+        assert np.array_equal(got, eager.read()), "replay %d" % replay
+        rc, ref, _ = ORACLE.gqa(q, k, v, query_start=tk - tq)
+        assert rc == 0 and np.abs(got - ref).max() < 2e-5
+    backend.graph_release(graph)
+    if attached:
+        backend.workspace_detach()
+    for x in tensors + [out, eager, work]:
+        x.release()
+
+
 def test_bandwidth_probe_on_the_device(backend):
     """The probe's record on a real part: a streaming read of 1 GiB sustains terabytes per
     second, below the published peak; the copy moves read plus write."""

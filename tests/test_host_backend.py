@@ -670,6 +670,40 @@ def test_bounded_primitive_refusal_order_and_facts(fake_runtime):
         assert rc == B.YVEX_ERR_INVALID_ARG
 
 
+def test_exact_prefill_workspace_is_planned_and_offered(fake_runtime):
+    """Prefill-shaped EXACT_F32 requests name the bytes of their halves and partials; attached they run in two or
+    three launches, one byte short, or absent, in one that allocates nothing."""
+    with Backend() as b:
+        for d in (64, 128, 256):
+            shortest = 2 * d + 128
+            assert b.attention_workspace_required(
+                b.attention_requirement(32, shortest - 1, 4, 2, d, query_start=shortest - 33)) == 0
+            for tokens, keys, launches in ((32, shortest, None), (32, 6000, 3), (8192, 8192, 2)):
+                req = b.attention_requirement(tokens, keys, 4, 2, d, query_start=keys - tokens)
+                need = b.attention_workspace_required(req)
+                tiles = 2 * ((keys + 31) // 32)
+                halves = tiles * 256 * d + (tiles * 32 + 255) // 256 * 256
+                assert need >= halves
+                launches = launches or (3 if need > halves else 2)
+                assert (launches == 3) == (need > halves)
+                q, out = written(b, "q", B.DTYPE_F32, (tokens, 4, d)), b.tensor("o", B.DTYPE_F32, (tokens, 4, d))
+                k = written(b, "k", B.DTYPE_F32, (keys, 2, d))
+                for size in (need, need - 1):
+                    work = b.tensor("workspace", B.DTYPE_I8, (size,))
+                    b.workspace_attach(work)
+                    live = fake_runtime.fake_hip_live_allocations()
+                    facts = b.attention_execute(req, q, k, k, out)
+                    assert fake_runtime.fake_hip_live_allocations() == live
+                    assert (facts.kernel_launches, facts.temporary_bytes, facts.accelerated_matrix_launches) == (
+                        (launches, need, 1) if size == need else (1, 0, 1))
+                    b.workspace_detach()
+                    work.release()
+        # past the bytes that a request may ask for, and strides that 32-bit offsets do not reach
+        assert b.attention_workspace_required(b.attention_requirement(64, 600000, 8, 8, 128, query_start=599936)) == 0
+        wide = b.attention_requirement(64, 500, 8, 8, 128, query_start=436, k_stride=1 << 24, v_stride=1 << 24)
+        assert b.attention_workspace_required(wide) == 0
+
+
 def test_attention_execute_contracts_facts_and_workspace(fake_runtime):
     with Backend() as b:
         # exact F32: one launch, one synchronisation, a 4-byte status read-back
