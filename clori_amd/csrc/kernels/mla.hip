@@ -62,7 +62,11 @@ __device__ inline int swizzle(int r) { return (((r >> 1) & 1) << 2) | ((r >> 2) 
 // (tests/unit/deepseek_arch_ir.c:110-125: 64 heads, one 512-lane row per token with the rope
 // lanes inside, key and value the same row); rows are 1024 bytes in memory and keep the
 // 1152-byte pitch in LDS (so the bank analysis above holds unchanged), every wave stages
-// eight whole rows, one per load, and waves 2 and 3 only stage: they own no heads.
+// eight whole rows, one per load, and waves w and w + 2 share 32 heads: both compute their scores (as
+// many MFMAs as one wave's whole update takes), each accumulates and leaves half of the value
+// lanes.  A tile is 48 MFMAs of a wave instead of 64, and a partial row leaves from two waves (with the
+// other two waves only staging / now, the whole reduce: 32 lists of 512 rows 39.7 / 36.9 us, 1 26.2 / 22.9, 64
+// elements of 32768 tokens without lists 35.5 / 33.3).
 template <int kKeyDim, int kHeads>
 __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsigned char *lds)
 {
@@ -71,12 +75,14 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     constexpr bool kRowPerLoad = kSourceRowBytes == 1024;    // one 1 KB load is one row
     constexpr int kLoadsPerWave = kRowPerLoad ? kTile / 4 : kTileBytes / 1024 / 4;  // 8 or 9
     constexpr int kLoadPitch = kRowPerLoad ? kRowBytes : 1024;  // LDS distance between a wave's loads
-    constexpr int kActiveWaves = kHeads / kHeadsPerWave;
-    constexpr int kQueryRounds = kActiveWaves / 2;           // two head groups per round
+    constexpr int kHeadGroups = kHeads / kHeadsPerWave;
+    constexpr int kQueryRounds = kHeadGroups / 2;            // two head groups per round
+    constexpr int kValueParts = 4 / kHeadGroups;             // waves that share the value lanes of a head
+    constexpr int kBlocks = 16 / kValueParts;                // 32-dim blocks of O^T of a wave
     static_assert(kSteps % 4 == 0 && kSteps / 4 == kLoadsPerWave,
                   "the loads of a tile ride behind k-steps 1, 5, 9, ...");
     static_assert(kRowPerLoad || kSourceRowBytes == kRowBytes, "rows are 1024 or 1152 bytes");
-    static_assert(kActiveWaves == 2 || kActiveWaves == 4, "head groups come in pairs");
+    static_assert(kHeadGroups == 2 || kHeadGroups == 4, "head groups come in pairs");
     // at most one younger tile outstanding: vmcnt(kLoadsPerWave), lgkmcnt and expcnt untouched
     constexpr int kWaitTile = 0x0f70 | kLoadsPerWave;
     // at most two younger tiles outstanding
@@ -154,7 +160,9 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     }
     const uint32_t t1 = min(ctx, t0 + p.chunk_tokens);
     const uint32_t tiles = (t1 - t0 + kTile - 1) / kTile;
-    const uint32_t head = wave * kHeadsPerWave + n;
+    const int group = kValueParts == 1 ? wave : wave % kHeadGroups;
+    const int part = kValueParts == 1 ? 0 : wave / kHeadGroups;
+    const uint32_t head = group * kHeadsPerWave + n;
 
     // ---- tile staging --------------------------------------------------------------
     // Page ids come by scalar loads, one tile ahead of the staging that needs them; an id
@@ -217,7 +225,7 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
             for (int h = 0; h < 2; ++h) {
                 const int r = 8 * h + 4 * g + (a >> 2);
                 const int chunk16 = (par * 4 + 2 * b1 + ((a >> 1) & 1)) ^ swizzle(r);
-                v_addr[par][h] = (uint32_t)(r * kRowBytes + (chunk16 << 4) + 8 * (a & 1));
+                v_addr[par][h] = (uint32_t)(r * kRowBytes + (chunk16 << 4) + 8 * (a & 1) + part * kBlocks * 64);
             }
     }
 
@@ -233,7 +241,7 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     // round 0 has landed when only the two tiles behind it are outstanding
     __builtin_amdgcn_s_waitcnt(kWaitTwoTiles);
     __syncthreads();
-    if (wave < 2) take_queries();
+    if (kQueryRounds == 1 || wave < 2) take_queries();
     if (kQueryRounds == 2) {
         __syncthreads();  // buffers 2 and 3 are free again
         stage_queries(1);
@@ -242,23 +250,9 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
         if (wave >= 2) take_queries();
     }
     __syncthreads();  // buffers 2 and 3 are free for tiles once every wave holds its fragments
-    if (kActiveWaves < 4 && wave >= kActiveWaves) {
-        // a wave without heads: it stages its quarter of every tile and keeps the barriers of
-        // the computing waves (one per tile, one before their epilogue)
-        for (uint32_t t = 0; t < tiles; ++t) {
-            __builtin_amdgcn_s_waitcnt(kWaitTile);
-            __syncthreads();
-            stage_tile(t + 2u, page_checked(id_ahead));
-            id_ahead = page_fetch(t + 3u);
-        }
-        __builtin_amdgcn_s_waitcnt(0x0f70);
-        __syncthreads();
-        return;
-    }
-
-    floatx16 o[16];
+    floatx16 o[kBlocks];
 #pragma unroll
-    for (int db = 0; db < 16; ++db)
+    for (int db = 0; db < kBlocks; ++db)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
     float m_run = -INFINITY, neg_m = 0.f, l_run = 0.f;
@@ -316,7 +310,7 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
             l_run *= alpha;
             // one block at a time through the VALU; the accumulators live in AGPRs
 #pragma unroll
-            for (int db = 0; db < 16; ++db) {
+            for (int db = 0; db < kBlocks; ++db) {
                 asm volatile("" : "+a"(o[db]));
                 o[db] *= alpha;
                 asm volatile("" : "+a"(o[db]));
@@ -338,10 +332,11 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     uint32_t pk_prev[8], pk_cur[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) pk_prev[j] = 0u;
-    // O^T += C^T . P^T with the tile at `tile`, MFMAs [first, last) of the 32 (token half u =
-    // index / 16, dim block db = index % 16)
+    // O^T += C^T . P^T with the tile at `tile`, MFMAs [first, last) of the kUpdates (token half u =
+    // index / kBlocks, dim block db = index % kBlocks of the wave's part)
+    constexpr int kUpdates = 2 * kBlocks;
     auto value_operand = [&](const unsigned char *tile, int index) -> bf16x8 {
-        const int u = index >> 4, db = index & 15;
+        const int u = index / kBlocks, db = index % kBlocks;
         const int imm = (db & ~1) * 64 + u * 16 * kRowBytes;
         const short4v lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
             (lds_short4 *)(tile + v_addr[db & 1][0] + imm));
@@ -353,7 +348,7 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     auto accumulate = [&](const unsigned char *tile, const uint32_t (&pk)[8], int first, int last) {
 #pragma unroll
         for (int index = first; index < last; ++index) {
-            const int u = index >> 4, db = index & 15;
+            const int u = index / kBlocks, db = index % kBlocks;
             const u32x4 w = {pk[u * 4 + 0], pk[u * 4 + 1], pk[u * 4 + 2], pk[u * 4 + 3]};
             o[db] = mfma_32x32x16(value_operand(tile, index), as_bf16x8(w), o[db]);
         }
@@ -406,16 +401,17 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
         }
         l_run += lsum;
         if (decltype(with_update)::value) {
-            accumulate(prev_tile, pk_prev, kEarly, 32);
+            accumulate(prev_tile, pk_prev, kEarly, kUpdates);
             // three transposed operand pairs in flight ahead of the MFMAs that consume them,
-            // one exponential behind every second MFMA
+            // one exponential behind every second MFMA (every MFMA where they are half as many)
             __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
-            for (int i = 0; i < (32 - kEarly - 4) / 2; ++i) {
+            for (int i = 0; i < (kUpdates - kEarly - 4) / 2; ++i) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x400, kValueParts, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                if (kValueParts == 2) __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
             }
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -433,10 +429,10 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
         step(t, std::integral_constant<bool, true>());
     // the update with the last tile
     __builtin_amdgcn_sched_barrier(0);
-    accumulate(lds + ((tiles - 1u) % kBuffers) * kTileBytes, pk_prev, 0, 32);
+    accumulate(lds + ((tiles - 1u) % kBuffers) * kTileBytes, pk_prev, 0, kUpdates);
     __builtin_amdgcn_sched_group_barrier(0x100, 6, 0);
 #pragma unroll
-    for (int i = 0; i < 29; ++i) {
+    for (int i = 0; i < kUpdates - 3; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
@@ -447,14 +443,15 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     float l = l_run;
     l = sum_xor32(l);
     const uint64_t slot = ((uint64_t)batch * p.slot_stride + p.first_slot + chunk) * p.heads + head;
-    // The accumulators are lane = head, registers = dims; through LDS they become one
-    // contiguous 1 KB bf16 row per head, written by one 16-byte store per lane.
-    constexpr int kOutPitch = kValueDim * 2 + 16;  // 1040 B, keeps 16-byte alignment
+    // The accumulators are lane = head, registers = dims; through LDS they become contiguous bf16 rows
+    // (1 KB per head, or half of that), written by 16-byte stores.
+    constexpr int kOutDims = kValueDim / kValueParts, kOutPitch = kOutDims * 2 + 16;  // keeps 16-byte alignment
+    constexpr int kOutLanes = kOutDims / 8, kOutRows = 64 / kOutLanes;                // rows per store
     static_assert(4 * kHeadsPerWave * kOutPitch <= kBuffers * kTileBytes, "epilogue fits the tiles");
     __syncthreads();  // every wave is done with the tile buffers
     unsigned char *rows = lds + wave * (kHeadsPerWave * kOutPitch);
 #pragma unroll
-    for (int db = 0; db < 16; ++db)
+    for (int db = 0; db < kBlocks; ++db)
 #pragma unroll
         for (int grp = 0; grp < 4; ++grp) {
             u32x2 v;
@@ -466,20 +463,21 @@ __device__ __forceinline__ void mla_decode(const yvex_rocm_mla_params &p, unsign
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     {
         const uint64_t slot0 =
-            ((uint64_t)batch * p.slot_stride + p.first_slot + chunk) * p.heads + wave * kHeadsPerWave;
-        uint16_t *dst = p.part_acc + slot0 * kValueDim + lane * 8;
+            ((uint64_t)batch * p.slot_stride + p.first_slot + chunk) * p.heads + group * kHeadsPerWave;
+        const int at = lane % kOutLanes * 8;
+        uint16_t *dst = p.part_acc + slot0 * kValueDim + part * kOutDims + at;
         // every workgroup starts its 32 rows at another one: the rows of all workgroups are
         // 1 KB apart at the same offsets of 128 KB regions, and written in step they would all
         // be in the same memory channels at the same time
         const int skew = (int)((chunk * 5u + batch * 3u) & 31u);
 #pragma unroll 8
-        for (int i = 0; i < kHeadsPerWave; ++i) {
-            const int hh = (i + skew) & (kHeadsPerWave - 1);
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(rows + hh * kOutPitch + lane * 16);
+        for (int i = 0; i < kHeadsPerWave / kOutRows; ++i) {
+            const int hh = (i * kOutRows + lane / kOutLanes + skew) & (kHeadsPerWave - 1);
+            const u32x4 v = *reinterpret_cast<const u32x4 *>(rows + hh * kOutPitch + at * 2);
             *reinterpret_cast<u32x4 *>(dst + (uint64_t)hh * kValueDim) = v;
         }
     }
-    if (g == 0) {
+    if (g == 0 && part == 0) {
         p.part_ml[slot * 2 + 0] = m_run;
         p.part_ml[slot * 2 + 1] = l;
     }
