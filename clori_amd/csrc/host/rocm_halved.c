@@ -31,12 +31,13 @@ static unsigned long long visible_keys(const yvex_transformer_attention_requirem
                                                              : r->key_value_tokens;
 }
 
-/* Returns 0 when the request is not for these kernels.  Walks of fewer than 2 d + 128 keys stay with the one
+/* Returns 0 when the request is not for these kernels.  Walks of fewer than d + 192 keys stay with the one
  * launch: the launch that splits, and a workgroup's longer start, cost more than they save.  With the
- * workspace / without, us: 40/8 heads of 128, 200 tokens 24.6 / 23.7, 300 29.4 / 29.0, 450 36.7 / 39.7,
- * 1777 118 / 142, 4096 461 / 640, 32 behind 200 25.3 / 23.6, 128 behind 300 33.0 / 37.4, 32 behind 4000 46 /
- * 271, 300 behind 5000 125 / 316; 16/4 of 64, 64 11.2 / 9.6, 200 14.6 / 15.4, 1000 36.1 / 44.8; 24/4 of 256, 300
- * 58 / 48, 32 behind 300 43.3 / 47.7, 500 75.3 / 74.3, 2000 204 / 231, 64 behind 20000 192 / 2003. */
+ * workspace / without, us: 40/8 heads of 128, 200 tokens 24.2 / 23.7, 300 29.1 / 28.6, 350 31.1 / 31.6, 1777
+ * 118 / 142, 4096 461 / 640, 32 behind 200 24.9 / 23.8, 32 behind 300 24.9 / 28.7, 32 behind 4000 45 / 271, 300
+ * behind 5000 125 / 316; 16/4 of 64, 100 12.2 / 12.5, 200 14.7 / 15.6, 32 behind 100 13.6 / 12.2, 32 behind 200
+ * 16.1 / 16.0, 1000 35.4 / 44.8; 24/4 of 256, 300 53 / 47, 450 62 / 64, 500 66 / 74, 32 behind 420 38 / 60,
+ * 1000 104 / 130, 64 behind 20000 183 / 2003. */
 static int halved_plan_make(const yvex_transformer_attention_requirement *r, halved_plan *plan)
 {
     const unsigned long long d = r->head_dimension, group = r->query_heads / r->key_value_heads;
@@ -46,7 +47,7 @@ static int halved_plan_make(const yvex_transformer_attention_requirement *r, hal
         r->key_value_tokens > (1ull << 30) || ((r->key_token_stride | r->value_token_stride) >> 24) != 0ull ||
         (r->key_value_heads * d >> 24) != 0ull)
         return 0;
-    if (visible_keys(r) < 2ull * d + 128ull) return 0;
+    if (visible_keys(r) < d + 192ull) return 0;
     plan->kv_tiles = (visible_keys(r) + HALVED_STEP_KEYS - 1ull) / HALVED_STEP_KEYS;
     plan->tile_bytes = r->key_value_heads * plan->kv_tiles * 256ull * d;
     plan->factor_bytes = r->key_value_heads * plan->kv_tiles * HALVED_FACTOR_WORDS * sizeof(uint32_t);

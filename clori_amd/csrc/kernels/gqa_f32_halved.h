@@ -11,7 +11,7 @@
 // 62 % of the cycles, 1.1 PFLOP/s of f16 products (a large bf16 product reaches 1.29 on this part), 373
 // TFLOP/s of F32 ones; 1777 tokens 112 of 118 us.  Trips that prefetch their first operands across the barrier, and
 // peaks without canonical forms, made no difference there (122 against 121 us), which is why no more is
-// hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us).
+// hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us, now 104).
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 #define YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 
@@ -23,6 +23,87 @@
 #include "prefill_rows.h"
 
 namespace {
+
+// What a run of keys contributes to row `row` of its tile (the maximum in log2 units), scaled.
+template <int kBlocks, class Scale>
+__device__ __forceinline__ void leave_partial(float *part_acc, float *part_ml, uint32_t slot, uint32_t row, int half,
+                                              const floatx16 (&o)[kBlocks], float m, float l, const Scale &scale)
+{
+    const uint64_t at = (uint64_t)slot * YVEX_ROCM_PREFILL_ROWS + row;
+    if (half == 0) {
+        part_ml[at * 2u] = m;
+        part_ml[at * 2u + 1u] = l;
+    }
+    float *acc = part_acc + at * (32u * kBlocks) + half * 4;
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<floatx4 *>(acc + b * 32 + g * 8) =
+                (floatx4){scale(o[b][g * 4]), scale(o[b][g * 4 + 1]), scale(o[b][g * 4 + 2]), scale(o[b][g * 4 + 3])};
+}
+
+// The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  It takes
+// the kernel's arguments from where they lie; `arguments` is the kernel's to find, a function that is called
+// is not given the place.
+typedef __attribute__((address_space(3))) unsigned char local_bytes;
+typedef __attribute__((address_space(4))) const yvex_rocm_gqa_f32_halved_params constant_params;
+template <int kDim>
+__device__ __forceinline__ void walk_again(constant_params *arguments, local_bytes *shared, bool cut, uint32_t slot_,
+                                           uint32_t row_head_, uint32_t tile_row_, uint32_t tile_end_,
+                                           uint32_t first_tile_, uint32_t tiles_)
+{
+    auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+    const uint64_t at = (uint64_t)arguments;
+    constant_params &p = *(constant_params *)((uint64_t)uniform((uint32_t)(at >> 32)) << 32 | uniform((uint32_t)at));
+    const uint32_t slot = uniform(slot_), row_head = uniform(row_head_), tile_row = uniform(tile_row_);
+    const uint32_t tile_end = uniform(tile_end_), first_tile = uniform(first_tile_), tiles = uniform(tiles_);
+    const bool partial = uniform(cut) != 0u;
+    const uint32_t pack = p.walk.pack;
+    yvex_rocm_gqa_f32_params f = {};
+    f.q = (const float *)p.walk.q;
+    f.k = (const float *)p.walk.k;
+    f.v = (const float *)p.walk.v;
+    f.out = (float *)p.walk.out;
+    f.lse = p.walk.lse;
+    f.status = p.walk.status;
+    f.query_tokens = p.walk.query_tokens;
+    f.kv_tokens = p.walk.kv_tokens;
+    f.query_start = p.walk.query_start;
+    f.query_heads = p.walk.query_heads;
+    f.kv_heads = p.walk.kv_heads;
+    f.q_stride = p.walk.q_stride;
+    f.k_stride = p.walk.k_stride;
+    f.v_stride = p.walk.v_stride;
+    f.scale = p.scale;
+    f.causal = (int32_t)p.walk.causal;
+    float *const part_acc = p.walk.part_acc, *const part_ml = p.walk.part_ml;
+    const GqaTile<kDim / 32> tile(f, (float *)(unsigned char *)shared, (int)threadIdx.x);
+    for (uint32_t h = 0u; h < pack; ++h) {
+        // rows token * pack + h in [tile_row, tile_end)
+        const uint32_t first = (tile_row + pack - 1u - h) / pack, end = (tile_end + pack - 1u - h) / pack;
+        if (first >= end) continue;
+        tile.walk(row_head * pack + h, first, end, first_tile, partial ? first_tile + tiles : ~0ull >> 8,
+                  [&](uint64_t head, uint64_t token, floatx16(&o)[kDim / 32], float m, float l) {
+                      if (partial)
+                          leave_partial(part_acc, part_ml, slot, (uint32_t)token * pack + h - tile_row, tile.half, o,
+                                        m * YVEX_LOG2E, l, [](float x) { return x; });
+                      else
+                          tile.publish(head, token, o, m, l);
+                  });
+        __syncthreads();  // every wave is done with the tiles in LDS
+    }
+}
+
+// The same as a function of its own: inlined, its registers are found by spilling the walk's (24/4 heads of 256,
+// 700 tokens 100 -> 85 us, 1000 112 -> 108; at 64, where they are there, the call costs 2 %).
+template <int kDim>
+__device__ __attribute__((noinline)) void walk_again_apart(constant_params *arguments, local_bytes *shared, bool cut,
+                                                           uint32_t slot, uint32_t row_head, uint32_t tile_row,
+                                                           uint32_t tile_end, uint32_t first_tile, uint32_t tiles)
+{
+    walk_again<kDim>(arguments, shared, cut, slot, row_head, tile_row, tile_end, first_tile, tiles);
+}
 
 // The walk.  A workgroup of four waves of 32 packed rows owns one item or one run of its keys.  Products are
 // transposed (S^T = K Q^T, O^T += V^T P^T, 32x32x16), so a lane owns one row and 16 of a tile's 32
@@ -295,30 +376,27 @@ struct GqaHalved {
 
     __device__ __forceinline__ void load_queries(const float *row)
     {
+        floatx4 x[kSteps][2];
         float most = 0.f;
 #pragma unroll
-        for (int s = 0; s < kSteps; ++s) {
-            const floatx4 a = *reinterpret_cast<const floatx4 *>(row + 16 * s);
-            const floatx4 b = *reinterpret_cast<const floatx4 *>(row + 16 * s + 4);
+        for (int s = 0; s < kSteps; ++s)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) most = fmaxf(most, fmaxf(fabsf(a[j]), fabsf(b[j])));
-        }
+            for (int j = 0; j < 2; ++j) x[s][j] = *reinterpret_cast<const floatx4 *>(row + 16 * s + 4 * j);
+#pragma unroll
+        for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) most = fmaxf(most, fabsf(x[s][j / 4][j % 4]));
         const uint32_t bits = __builtin_bit_cast(uint32_t, max_xor32(most)), e = group_exponent(bits);
         q_factor = bits >> 23 > kExponentMost ? __builtin_nanf("") : up_factor(e) * (p.scale * YVEX_LOG2E);
-        // (read a second time: the registers are short)
-        __asm__ volatile("" : "+v"(row));
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) {
-            const floatx4 a = *reinterpret_cast<const floatx4 *>(row + 16 * s);
-            const floatx4 b = *reinterpret_cast<const floatx4 *>(row + 16 * s + 4);
-            uint32_t h[4], l[4];
-            split_pair_by_lane(a[0], a[1], down_factor(e), h[0], l[0]);
-            split_pair_by_lane(a[2], a[3], down_factor(e), h[1], l[1]);
-            split_pair_by_lane(b[0], b[1], down_factor(e), h[2], l[2]);
-            split_pair_by_lane(b[2], b[3], down_factor(e), h[3], l[3]);
-            const u32x4 hi = {h[0], h[1], h[2], h[3]}, lo = {l[0], l[1], l[2], l[3]};
-            q_hi[s] = __builtin_bit_cast(halfx8, hi);
-            q_lo[s] = __builtin_bit_cast(halfx8, lo);
+            uint32_t hi[4], lo[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                split_pair_by_lane(x[s][j / 2][2 * (j % 2)], x[s][j / 2][2 * (j % 2) + 1], down_factor(e), hi[j],
+                                   lo[j]);
+            q_hi[s] = __builtin_bit_cast(halfx8, (u32x4){hi[0], hi[1], hi[2], hi[3]});
+            q_lo[s] = __builtin_bit_cast(halfx8, (u32x4){lo[0], lo[1], lo[2], lo[3]});
         }
     }
 
@@ -380,18 +458,24 @@ struct GqaHalved {
         if (tiles != 0u) walk_tiles(wave_tiles, unmasked, (const float *)w.q + (uint64_t)token * w.q_stride +
                                                               (uint64_t)head * kDim + 8 * half);
 
-        // the accumulators are relative to 2^(reference - 127), weights to 2^kWeightShift and values to 2^14
         const bool own = row0 + (uint32_t)column < w.rows;
         sum = sum_xor32(sum);
-        const float inverse = 1.0f / sum;
         // (a run none of whose keys the row sees leaves a maximum of -inf and nothing)
         bool good = isfinite(sum) && (partial && top == -INFINITY ? sum == 0.f : sum > 0.f && isfinite(top));
+        // the accumulators are relative to 2^(reference - 127), weights to 2^kWeightShift and values to 2^14
+        const int shift = reference - (141 + kWeightShift);
+        const float inverse = 1.0f / sum;
+        if (!partial) {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) out[b][i] = quotient(out[b][i], sum, inverse);
+        }
 #pragma unroll
         for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                out[b][i] = __builtin_amdgcn_ldexpf(partial ? out[b][i] : quotient(out[b][i], sum, inverse),
-                                                    reference - (141 + kWeightShift));
+                out[b][i] = __builtin_amdgcn_ldexpf(out[b][i], shift);
                 good &= isfinite(out[b][i]);
             }
         // (the tiles in LDS are done with)
@@ -405,14 +489,29 @@ struct GqaHalved {
         const uint32_t slot = partial ? (item - w.whole_items) * w.splits + split : 0u;
         if (failed) {
             __syncthreads();  // every wave has read the verdict
-            walk_again(partial, slot, row_head, tile_row, tile_end);
+            local_bytes *shared = (local_bytes *)(void *)&lds;
+            constant_params *arguments = (constant_params *)__builtin_amdgcn_kernarg_segment_ptr();
+            if constexpr (kDim == 64)
+                walk_again<kDim>(arguments, shared, partial, slot, row_head, tile_row, tile_end, first_tile, tiles);
+            else
+                walk_again_apart<kDim>(arguments, shared, partial, slot, row_head, tile_row, tile_end, first_tile,
+                                       tiles);
             return;
         }
         if (!own) return;
-        if (partial)
-            leave_partial(slot, row - tile_row, out, top, sum);
-        else
-            publish(head, token, out, top * YVEX_LN2 + logf(sum));
+        if (partial) {
+            leave_partial(w.part_acc, w.part_ml, slot, row - tile_row, half, out, top, sum, [](float x) { return x; });
+            return;
+        }
+        const uint64_t at = (uint64_t)token * w.query_heads + head;
+        float *to = (float *)w.out + at * kDim;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                *reinterpret_cast<floatx4 *>(to + 32 * b + 8 * g + 4 * half) =
+                    (floatx4){out[b][4 * g], out[b][4 * g + 1], out[b][4 * g + 2], out[b][4 * g + 3]};
+        if (w.lse && half == 0) w.lse[at] = top * YVEX_LN2 + logf(sum);
     }
 
     __device__ __forceinline__ void walk_tiles(uint32_t wave_tiles, uint32_t unmasked, const float *query)
@@ -469,76 +568,6 @@ struct GqaHalved {
         }
         // nothing may still be in flight into LDS
         __builtin_amdgcn_s_waitcnt(0x0f70);
-    }
-
-    __device__ __forceinline__ void publish(uint32_t head, uint32_t token, const floatx16 (&o)[kBlocks],
-                                            float lse) const
-    {
-        const uint64_t at = (uint64_t)token * p.walk.query_heads + head;
-        float *row = (float *)p.walk.out + at * kDim;
-#pragma unroll
-        for (int b = 0; b < kBlocks; ++b)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<floatx4 *>(row + 32 * b + 8 * g + 4 * half) =
-                    (floatx4){o[b][4 * g], o[b][4 * g + 1], o[b][4 * g + 2], o[b][4 * g + 3]};
-        if (p.walk.lse && half == 0) p.walk.lse[at] = lse;
-    }
-
-    // What this run of keys contributes to row `row` of its tile (the maximum in log2 units).
-    __device__ __forceinline__ void leave_partial(uint32_t slot, uint32_t row, const floatx16 (&o)[kBlocks], float m,
-                                                  float l) const
-    {
-        const uint64_t at = (uint64_t)slot * kRows + row;
-        if (half == 0) {
-            p.walk.part_ml[at * 2u] = m;
-            p.walk.part_ml[at * 2u + 1u] = l;
-        }
-        float *acc = p.walk.part_acc + at * kDim + half * 4;
-#pragma unroll
-        for (int b = 0; b < kBlocks; ++b)
-#pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<floatx4 *>(acc + b * 32 + g * 8) =
-                    (floatx4){o[b][g * 4], o[b][g * 4 + 1], o[b][g * 4 + 2], o[b][g * 4 + 3]};
-    }
-
-    // The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.
-    __device__ __forceinline__ void walk_again(bool partial, uint32_t slot, uint32_t row_head,
-                                                         uint32_t tile_row, uint32_t tile_end) const
-    {
-        const yvex_rocm_prefill_params &w = p.walk;
-        yvex_rocm_gqa_f32_params f = {};
-        f.q = (const float *)w.q;
-        f.k = (const float *)w.k;
-        f.v = (const float *)w.v;
-        f.out = (float *)w.out;
-        f.lse = w.lse;
-        f.status = w.status;
-        f.query_tokens = w.query_tokens;
-        f.kv_tokens = w.kv_tokens;
-        f.query_start = w.query_start;
-        f.query_heads = w.query_heads;
-        f.kv_heads = w.kv_heads;
-        f.q_stride = w.q_stride;
-        f.k_stride = w.k_stride;
-        f.v_stride = w.v_stride;
-        f.scale = p.scale;
-        f.causal = (int32_t)w.causal;
-        const GqaTile<kBlocks> tile(f, reinterpret_cast<float *>(&lds), wave * 64 + lane);
-        for (uint32_t h = 0u; h < w.pack; ++h) {
-            // rows token * pack + h in [tile_row, tile_end)
-            const uint32_t first = (tile_row + w.pack - 1u - h) / w.pack, end = (tile_end + w.pack - 1u - h) / w.pack;
-            if (first >= end) continue;
-            tile.walk(row_head * w.pack + h, first, end, first_tile, partial ? first_tile + tiles : ~0ull >> 8,
-                      [&](uint64_t head, uint64_t token, floatx16(&o)[kBlocks], float m, float l) {
-                          if (partial)
-                              leave_partial(slot, (uint32_t)token * w.pack + h - tile_row, o, m * YVEX_LOG2E, l);
-                          else
-                              tile.publish(head, token, o, m, l);
-                      });
-            __syncthreads();  // every wave is done with the tiles in LDS
-        }
     }
 };
 

@@ -449,10 +449,10 @@ def run_attached(backend, q, k, v, short=0, **kw):
 
 
 @pytest.mark.parametrize("tq,tk,hq,hkv,d,start,causal", [
-    (33, 384, 4, 1, 128, 351, True), (129, 385, 10, 2, 128, 256, True), (1000, 1000, 5, 1, 128, 0, True),
+    (33, 320, 4, 1, 128, 287, True), (129, 385, 10, 2, 128, 256, True), (1000, 1000, 5, 1, 128, 0, True),
     (40, 3001, 10, 2, 128, 2950, True), (64, 799, 3, 3, 128, 0, False), (520, 1040, 40, 8, 128, 520, True),
-    (32, 257, 6, 2, 64, 224, True), (1300, 1300, 16, 4, 64, 0, True), (77, 9000, 7, 1, 64, 8923, True),
-    (100, 700, 4, 4, 64, 3, False), (32, 641, 6, 1, 256, 609, True), (700, 700, 6, 2, 256, 0, True),
+    (32, 256, 6, 2, 64, 224, True), (1300, 1300, 16, 4, 64, 0, True), (77, 9000, 7, 1, 64, 8923, True),
+    (100, 700, 4, 4, 64, 3, False), (32, 448, 6, 1, 256, 416, True), (700, 700, 6, 2, 256, 0, True),
     (50, 4000, 24, 4, 256, 3950, True), (96, 900, 4, 4, 256, 0, False),
 ])
 def test_gqa_split_beforehand_matches_cpu_operator(backend, tq, tk, hq, hkv, d, start, causal):
