@@ -33,11 +33,11 @@ static unsigned long long visible_keys(const yvex_transformer_attention_requirem
 
 /* Returns 0 when the request is not for these kernels.  Walks of fewer than d + 192 keys stay with the one
  * launch: the launch that splits, and a workgroup's longer start, cost more than they save.  With the
- * workspace / without, us: 40/8 heads of 128, 200 tokens 24.2 / 23.7, 300 29.1 / 28.6, 350 31.1 / 31.6, 1777
- * 118 / 142, 4096 461 / 640, 32 behind 200 24.9 / 23.8, 32 behind 300 24.9 / 28.7, 32 behind 4000 45 / 271, 300
- * behind 5000 125 / 316; 16/4 of 64, 100 12.2 / 12.5, 200 14.7 / 15.6, 32 behind 100 13.6 / 12.2, 32 behind 200
- * 16.1 / 16.0, 1000 35.4 / 44.8; 24/4 of 256, 300 53 / 47, 450 62 / 64, 500 66 / 74, 32 behind 420 38 / 60,
- * 1000 104 / 130, 64 behind 20000 183 / 2003. */
+ * workspace / without, us: 40/8 heads of 128, 200 tokens 24.2 / 23.7, 330 26.5 / 31.5, 400 28 / 35, 1777
+ * 116 / 142, 4096 461 / 640, 32 behind 200 24.9 / 23.8, 32 behind 290 20.8 / 28.6, 32 behind 4000 45 / 271, 300
+ * behind 5000 125 / 316; 16/4 of 64, 100 12.2 / 12.5, 200 14.7 / 15.6, 32 behind 100 13.6 / 12.2, 32 behind 230
+ * 16.1 / 17.0, 1000 35.4 / 44.8; 24/4 of 256, 300 53 / 47, 450 57 / 64, 500 61 / 74, 32 behind 420 33 / 60,
+ * 1000 101 / 130, 64 behind 20000 175 / 2003. */
 static int halved_plan_make(const yvex_transformer_attention_requirement *r, halved_plan *plan)
 {
     const unsigned long long d = r->head_dimension, group = r->query_heads / r->key_value_heads;

@@ -11,7 +11,7 @@
 // 62 % of the cycles, 1.1 PFLOP/s of f16 products (a large bf16 product reaches 1.29 on this part), 373
 // TFLOP/s of F32 ones; 1777 tokens 112 of 118 us.  Trips that prefetch their first operands across the barrier, and
 // peaks without canonical forms, made no difference there (122 against 121 us), which is why no more is
-// hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us, now 104).
+// hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us, now 101).
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 #define YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 
@@ -24,10 +24,10 @@
 
 namespace {
 
-// What a run of keys contributes to row `row` of its tile (the maximum in log2 units), scaled.
-template <int kBlocks, class Scale>
+// What a run of keys contributes to row `row` of its tile (the maximum in log2 units).
+template <int kBlocks>
 __device__ __forceinline__ void leave_partial(float *part_acc, float *part_ml, uint32_t slot, uint32_t row, int half,
-                                              const floatx16 (&o)[kBlocks], float m, float l, const Scale &scale)
+                                              const floatx16 (&o)[kBlocks], float m, float l)
 {
     const uint64_t at = (uint64_t)slot * YVEX_ROCM_PREFILL_ROWS + row;
     if (half == 0) {
@@ -40,7 +40,7 @@ __device__ __forceinline__ void leave_partial(float *part_acc, float *part_ml, u
 #pragma unroll
         for (int g = 0; g < 4; ++g)
             *reinterpret_cast<floatx4 *>(acc + b * 32 + g * 8) =
-                (floatx4){scale(o[b][g * 4]), scale(o[b][g * 4 + 1]), scale(o[b][g * 4 + 2]), scale(o[b][g * 4 + 3])};
+                (floatx4){o[b][g * 4], o[b][g * 4 + 1], o[b][g * 4 + 2], o[b][g * 4 + 3]};
 }
 
 // The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  It takes
@@ -87,7 +87,7 @@ __device__ __forceinline__ void walk_again(constant_params *arguments, local_byt
                   [&](uint64_t head, uint64_t token, floatx16(&o)[kDim / 32], float m, float l) {
                       if (partial)
                           leave_partial(part_acc, part_ml, slot, (uint32_t)token * pack + h - tile_row, tile.half, o,
-                                        m * YVEX_LOG2E, l, [](float x) { return x; });
+                                        m * YVEX_LOG2E, l);
                       else
                           tile.publish(head, token, o, m, l);
                   });
@@ -478,14 +478,14 @@ struct GqaHalved {
                 out[b][i] = __builtin_amdgcn_ldexpf(out[b][i], shift);
                 good &= isfinite(out[b][i]);
             }
-        // (the tiles in LDS are done with)
-        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.k[0]);
+        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.v[1]);  // a word of each wave, behind the rows
+        __syncthreads();  // the tiles in LDS are done with
+        lay_rows_down();
+        if (lane == 0) verdict[wave] = 0u;
+        if (own && !good) verdict[wave] = 1u;
         __syncthreads();
-        if (lane == 0 && wave == 0) *verdict = 0u;
-        __syncthreads();
-        if (own && !good) *verdict = 1u;
-        __syncthreads();
-        const bool failed = *verdict != 0u;
+        const u32x4 verdicts = *reinterpret_cast<u32x4 *>(verdict);
+        const bool failed = (verdicts[0] | verdicts[1] | verdicts[2] | verdicts[3]) != 0u;
         const uint32_t slot = partial ? (item - w.whole_items) * w.splits + split : 0u;
         if (failed) {
             __syncthreads();  // every wave has read the verdict
@@ -498,20 +498,56 @@ struct GqaHalved {
                                        tiles);
             return;
         }
-        if (!own) return;
+        if (row0 >= w.rows) return;
         if (partial) {
-            leave_partial(w.part_acc, w.part_ml, slot, row - tile_row, half, out, top, sum, [](float x) { return x; });
+            const uint64_t first = (uint64_t)slot * kRows + (row0 - tile_row);
+            publish_rows(row0, [&](uint32_t, uint32_t r) { return w.part_acc + (first + r) * kDim; });
+            if (own && half == 0) {
+                float *ml = w.part_ml + 2u * (first + (uint32_t)column);
+                ml[0] = top;
+                ml[1] = sum;
+            }
             return;
         }
-        const uint64_t at = (uint64_t)token * w.query_heads + head;
-        float *to = (float *)w.out + at * kDim;
+        publish_rows(row0, [&](uint32_t row_, uint32_t) {
+            const uint32_t token_ = token_of(w, row_);
+            return (float *)w.out +
+                   ((uint64_t)token_ * w.query_heads + (row_head * w.pack + (row_ - token_ * w.pack))) * kDim;
+        });
+        if (own && w.lse && half == 0)
+            w.lse[(uint64_t)token * w.query_heads + head] = top * YVEX_LN2 + logf(sum);
+    }
+
+    // The wave's 32 rows go through its part of LDS, 16-byte units of a row dealt by its number so that
+    // both sides spread over the banks.  They are laid down before the vote: kept in registers over it,
+    // which the call of the fallback takes, they were spilled and fetched back, 5.4 us at the end of a
+    // workgroup and 27 MB of scratch written (1777 tokens of 40 heads of 128).
+    static constexpr uint32_t kUnits = kDim / 4;
+    __device__ __forceinline__ floatx4 *laid_rows() const
+    {
+        static_assert(4 * 32 * kDim * 4 <= offsetof(Shared, v[1]), "rows end before the verdicts");
+        return reinterpret_cast<floatx4 *>(lds.k[0]) + (uint32_t)wave * 32u * kUnits;
+    }
+    __device__ __forceinline__ void lay_rows_down() const
+    {
+        floatx4 *rows = laid_rows();
 #pragma unroll
-        for (int b = 0; b < kBlocks; ++b)
+        for (uint32_t b = 0; b < (uint32_t)kBlocks; ++b)
 #pragma unroll
-            for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<floatx4 *>(to + 32 * b + 8 * g + 4 * half) =
+            for (uint32_t g = 0; g < 4; ++g)
+                rows[(uint32_t)column * kUnits + ((8u * b + 2u * g + (uint32_t)half) ^ ((uint32_t)column & 15u))] =
                     (floatx4){out[b][4 * g], out[b][4 * g + 1], out[b][4 * g + 2], out[b][4 * g + 3]};
-        if (w.lse && half == 0) w.lse[at] = top * YVEX_LN2 + logf(sum);
+    }
+    template <typename To>
+    __device__ __forceinline__ void publish_rows(uint32_t row0, const To &to) const
+    {
+        const floatx4 *rows = laid_rows();
+#pragma unroll
+        for (uint32_t i = 0; i < kUnits / 2u; ++i) {
+            const uint32_t r = (i * 64u + (uint32_t)lane) / kUnits, unit = (i * 64u + (uint32_t)lane) % kUnits;
+            const floatx4 x = rows[r * kUnits + (unit ^ (r & 15u))];
+            if (row0 + r < p.walk.rows) *reinterpret_cast<floatx4 *>(to(row0 + r, r) + 4u * unit) = x;
+        }
     }
 
     __device__ __forceinline__ void walk_tiles(uint32_t wave_tiles, uint32_t unmasked, const float *query)
