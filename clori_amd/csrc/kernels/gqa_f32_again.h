@@ -1,0 +1,96 @@
+// The fp32 walk of an item whose f16 halves left the range: what gqa_f32_halved.h falls back to.
+#ifndef YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
+#define YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
+
+#include <hip/hip_runtime.h>
+
+#include "../kernel_params.h"
+#include "gqa_f32_walk.h"
+#include "mfma.h"
+
+namespace {
+
+// What a run of keys contributes to row `row` of its tile (the maximum in log2 units).
+template <int kBlocks>
+__device__ __forceinline__ void leave_partial(float *part_acc, float *part_ml, uint32_t slot, uint32_t row, int half,
+                                              const floatx16 (&o)[kBlocks], float m, float l)
+{
+    const uint64_t at = (uint64_t)slot * YVEX_ROCM_PREFILL_ROWS + row;
+    if (half == 0) {
+        part_ml[at * 2u] = m;
+        part_ml[at * 2u + 1u] = l;
+    }
+    float *acc = part_acc + at * (32u * kBlocks) + half * 4;
+#pragma unroll
+    for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<floatx4 *>(acc + b * 32 + g * 8) =
+                (floatx4){o[b][g * 4], o[b][g * 4 + 1], o[b][g * 4 + 2], o[b][g * 4 + 3]};
+}
+
+// The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  It takes
+// the kernel's arguments from where they lie; `arguments` is the kernel's to find, a function that is called
+// is not given the place.
+typedef __attribute__((address_space(3))) unsigned char local_bytes;
+typedef __attribute__((address_space(4))) const yvex_rocm_gqa_f32_halved_params constant_params;
+template <int kDim>
+__device__ __forceinline__ void walk_again(constant_params *arguments, local_bytes *shared, bool cut, uint32_t slot_,
+                                           uint32_t row_head_, uint32_t tile_row_, uint32_t tile_end_,
+                                           uint32_t first_tile_, uint32_t tiles_)
+{
+    auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
+    const uint64_t at = (uint64_t)arguments;
+    constant_params &p = *(constant_params *)((uint64_t)uniform((uint32_t)(at >> 32)) << 32 | uniform((uint32_t)at));
+    const uint32_t slot = uniform(slot_), row_head = uniform(row_head_), tile_row = uniform(tile_row_);
+    const uint32_t tile_end = uniform(tile_end_), first_tile = uniform(first_tile_), tiles = uniform(tiles_);
+    const bool partial = uniform(cut) != 0u;
+    const uint32_t pack = p.walk.pack;
+    yvex_rocm_gqa_f32_params f = {};
+    f.q = (const float *)p.walk.q;
+    f.k = (const float *)p.walk.k;
+    f.v = (const float *)p.walk.v;
+    f.out = (float *)p.walk.out;
+    f.lse = p.walk.lse;
+    f.status = p.walk.status;
+    f.query_tokens = p.walk.query_tokens;
+    f.kv_tokens = p.walk.kv_tokens;
+    f.query_start = p.walk.query_start;
+    f.query_heads = p.walk.query_heads;
+    f.kv_heads = p.walk.kv_heads;
+    f.q_stride = p.walk.q_stride;
+    f.k_stride = p.walk.k_stride;
+    f.v_stride = p.walk.v_stride;
+    f.scale = p.scale;
+    f.causal = (int32_t)p.walk.causal;
+    float *const part_acc = p.walk.part_acc, *const part_ml = p.walk.part_ml;
+    const GqaTile<kDim / 32> tile(f, (float *)(unsigned char *)shared, (int)threadIdx.x);
+    for (uint32_t h = 0u; h < pack; ++h) {
+        // rows token * pack + h in [tile_row, tile_end)
+        const uint32_t first = (tile_row + pack - 1u - h) / pack, end = (tile_end + pack - 1u - h) / pack;
+        if (first >= end) continue;
+        tile.walk(row_head * pack + h, first, end, first_tile, partial ? first_tile + tiles : ~0ull >> 8,
+                  [&](uint64_t head, uint64_t token, floatx16(&o)[kDim / 32], float m, float l) {
+                      if (partial)
+                          leave_partial(part_acc, part_ml, slot, (uint32_t)token * pack + h - tile_row, tile.half, o,
+                                        m * YVEX_LOG2E, l);
+                      else
+                          tile.publish(head, token, o, m, l);
+                  });
+        __syncthreads();  // every wave is done with the tiles in LDS
+    }
+}
+
+// The same as a function of its own: inlined, its registers are found by spilling the walk's (24/4 heads of 256,
+// 700 tokens 100 -> 85 us, 1000 112 -> 108; at 64, where they are there, the call costs 2 %).
+template <int kDim>
+__device__ __attribute__((noinline)) void walk_again_apart(constant_params *arguments, local_bytes *shared, bool cut,
+                                                           uint32_t slot, uint32_t row_head, uint32_t tile_row,
+                                                           uint32_t tile_end, uint32_t first_tile, uint32_t tiles)
+{
+    walk_again<kDim>(arguments, shared, cut, slot, row_head, tile_row, tile_end, first_tile, tiles);
+}
+
+}  // namespace
+
+#endif  // YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
