@@ -9,7 +9,7 @@
 //
 // What bounds the walk is power: 4096 tokens of 40/8 heads of 128 run at 1.66 GHz with the matrix cores busy
 // 62 % of the cycles, 1.1 PFLOP/s of f16 products (a large bf16 product reaches 1.29 on this part), 373
-// TFLOP/s of F32 ones; 1777 tokens 112 of 118 us.  Trips that prefetch their first operands across the barrier, and
+// TFLOP/s of F32 ones; 1777 tokens 108 of 116 us.  Trips that prefetch their first operands across the barrier, and
 // peaks without canonical forms, made no difference there (122 against 121 us), which is why no more is
 // hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us, now 101).
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
@@ -506,7 +506,7 @@ struct GqaHalved {
         c.peak = peak_of(s_even, f_even);
         key_buffer = 0u;
         // (two copies of a trip instead of three take less time to fetch: 1777 tokens 122 -> 118.5 us; at 256 the
-        // compiler moves more registers about in that form: 1000 tokens 112 -> 132)
+        // compiler moves more registers about in that form: 1000 tokens 102 -> 116)
         uint32_t t = 0u;
         if constexpr (kDim == 256) {
             for (; t + 1u < tiles; t += 2u) {
