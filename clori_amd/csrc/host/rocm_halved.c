@@ -15,6 +15,7 @@
 
 enum {
     HALVED_STEP_KEYS = 32,
+    HALVED_GROUP_MAX = 16, /* query heads packed into the rows of a tile */
     HALVED_FACTOR_WORDS = 8 /* of a tile */
 };
 #define HALVED_TILES_MAX (512ull << 20) /* bytes of halves a request may ask for */
@@ -42,8 +43,9 @@ static int halved_plan_make(const yvex_transformer_attention_requirement *r, hal
 {
     const unsigned long long d = r->head_dimension, group = r->query_heads / r->key_value_heads;
     memset(plan, 0, sizeof(*plan));
-    /* row counts below 2^27 (kernel_params.h), 32-bit offsets into a tile and into the tiles of a kv head */
-    if (r->query_tokens > (1ull << 27) / group || r->query_heads > 65535ull ||
+    /* token_of (prefill_rows.h) is exact for row counts below 2^27 and at most 16 heads to a kv head (with 71 it is
+     * first wrong at token 975685, with 127 at 304672); 32-bit offsets into a tile and into the tiles of a kv head */
+    if (group > HALVED_GROUP_MAX || r->query_tokens > (1ull << 27) / group || r->query_heads > 65535ull ||
         r->key_value_tokens > (1ull << 30) || ((r->key_token_stride | r->value_token_stride) >> 24) != 0ull ||
         (r->key_value_heads * d >> 24) != 0ull)
         return 0;

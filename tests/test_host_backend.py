@@ -704,6 +704,27 @@ def test_exact_prefill_workspace_is_planned_and_offered(fake_runtime):
         assert b.attention_workspace_required(wide) == 0
 
 
+def test_exact_prefill_packs_only_groups_whose_tokens_are_found(fake_runtime):
+    """A packed row's token is the upper half of its product with a rounded-up inverse.  Restated here: exact below
+    2^27 rows for up to 16 heads to a kv head, wrong inside the other limits for wider groups, which therefore
+    name no workspace and run one head to a tile."""
+    def first_wrong_token(pack, rows):
+        # the last row of token t, t * pack + pack - 1, is the first to be carried past t + 1
+        inverse = (0xffffffff + pack) // pack
+        excess = pack * inverse - (1 << 32)
+        token = -(-(1 << 32) // excess) // pack if excess else rows
+        for t in range(max(token - 2, 0), min(token + 3, rows // pack)):
+            if (t * pack + pack - 1) * inverse >> 32 != t:
+                return t
+        return None
+    assert all(first_wrong_token(pack, 1 << 27) is None for pack in range(2, 17))
+    assert first_wrong_token(71, 1 << 27) == 975685 and first_wrong_token(127, 1 << 27) == 304672
+    with Backend() as b:
+        for group, packed in ((5, True), (16, True), (17, False), (71, False), (127, False)):
+            req = b.attention_requirement(64, 4000, group, 1, 64, query_start=3936)
+            assert (b.attention_workspace_required(req) > 0) == packed
+
+
 def test_attention_execute_contracts_facts_and_workspace(fake_runtime):
     with Backend() as b:
         # exact F32: one launch, one synchronisation, a 4-byte status read-back
