@@ -5,7 +5,7 @@
  * with the query heads of a kv head packed into the rows of its tiles and, where the launch would leave
  * units idle, in runs of keys (the plan of the bf16 prefill, rocm_prefill.c, with steps of 32 keys), and
  * a third merges the runs.  Halves and partials live in the attached workspace; without one
- * that holds them a request runs in one launch that splits as it goes (gqa_f32_halves.h).
+ * that holds them a request runs in one launch with fp32 products (kernels/gqa_f32_walk.h).
  * Everything here is a function of the request's geometry only, so that the planner's
  * workspace_required and the execution agree. */
 #include "rocm_state.h"

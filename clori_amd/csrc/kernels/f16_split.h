@@ -21,14 +21,6 @@ __device__ __forceinline__ uint32_t dpp_max(uint32_t v)
     return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kControl, 0xf, 0xf, true));
 }
 
-// The largest magnitude of three values (fmaxf also makes NaNs quiet, at an instruction a value).
-__device__ __forceinline__ uint32_t largest(float a, float b, float c)
-{
-    uint32_t r;
-    __asm__("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
-}
-
 // Biased exponent that a group whose largest magnitude has these bits is scaled by: 2^(141 - e)
 // brings it to [2^14, 2^15).  Both that factor and its inverse 2^(e - 141) are normal numbers for
 // e in [kExponentLeast, kExponentMost]; a group below the range is scaled as its least, one above
@@ -63,19 +55,15 @@ __device__ __forceinline__ void for_each(const F &f)
 // seven).  The compiler sees no instructions here and inserts no wait states: the values must not come
 // straight from a transcendental instruction (whose result the next but one may read first), and the
 // results not go straight into an MFMA or a lane exchange (two instructions in between).
-#define YVEX_SPLIT_PAIR(name, where)                                                                       \
-    __device__ __forceinline__ void name(float a, float b, float factor, uint32_t &hi, uint32_t &lo)       \
-    {                                                                                                      \
-        __asm__ volatile("v_fma_mixlo_f16 %0, %2, %4, 0\n\t"                                             \
-                         "v_fma_mixhi_f16 %0, %3, %4, 0\n\t"                                             \
-                         "v_fma_mixlo_f16 %1, %2, %4, -%0 op_sel_hi:[0,0,1]\n\t"                         \
-                         "v_fma_mixhi_f16 %1, %3, %4, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]"               \
-                         : "=&v"(hi), "=&v"(lo)                                                            \
-                         : "v"(a), "v"(b), where(factor));                                                 \
-    }
-YVEX_SPLIT_PAIR(split_pair, "s")          // a factor that is the same in all lanes
-YVEX_SPLIT_PAIR(split_pair_by_lane, "v")
-#undef YVEX_SPLIT_PAIR
+__device__ __forceinline__ void split_pair_by_lane(float a, float b, float factor, uint32_t &hi, uint32_t &lo)
+{
+    __asm__ volatile("v_fma_mixlo_f16 %0, %2, %4, 0\n\t"
+                     "v_fma_mixhi_f16 %0, %3, %4, 0\n\t"
+                     "v_fma_mixlo_f16 %1, %2, %4, -%0 op_sel_hi:[0,0,1]\n\t"
+                     "v_fma_mixhi_f16 %1, %3, %4, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+                     : "=&v"(hi), "=&v"(lo)
+                     : "v"(a), "v"(b), "v"(factor));
+}
 
 // The same in two steps.
 __device__ __forceinline__ void split_hi(float a, float b, float factor, uint32_t &hi)

@@ -1,8 +1,9 @@
 // EXACT_F32 attention over keys and values that were split into halves beforehand.
 //
-// The products are those of gqa_f32_halves.h (an F32 product as three f16 products, the same powers of
-// two), but the splits, which took half of the vector work there, and which every workgroup made for
-// itself, are made once by a launch of their own (halve_rows) that leaves every tile of 32 keys as the walk wants
+// An F32 value times a power of two is written as the sum of two f16 values, hi = its nearest and
+// lo = the nearest of what hi leaves, and a product as hi hi + hi lo + lo hi.  The f16 matrix
+// instruction does 16 times the fp32 one's work per cycle, so three of them take 3/16 of its time.
+// The splits are made once by a launch of their own (halve_rows) that leaves every tile of 32 keys as the walk wants
 // it in LDS: the walk's tiles are filled by loads that write LDS directly, its registers
 // hold no rows on their way, and a trip is bound by its MFMAs.  Items, packed rows and runs of keys are those of
 // the bf16 prefill (kernel_params.h), with steps of 32 keys.

@@ -1,16 +1,17 @@
-// EXACT_F32 grouped-query attention on the matrix cores of gfx950 (wave64).
+// EXACT_F32 grouped-query attention on the matrix cores of gfx950 (wave64): the fp32 walk of items of 128 query
+// tokens of one query head (gqa_f32_walk.h), which needs no workspace, and the walk over keys and values split
+// beforehand (gqa_f32_halved.h).
 //
-// An item (128 query tokens of one query head) is walked with every F32 product as three f16 products
-// (gqa_f32_halves.h), and once more by the fp32 walk (gqa_f32_walk.h) when that gives a result that is not finite
-// or meets values past its range: what such an item publishes or reports is the fp32 walk's.
+// The one-launch form stays with fp32 products.  Split products in it take 150 us instead of 314 (1777 tokens of
+// 40/8 heads of 128), but with one power of two to eight rows they lost what lay 2^20 and more below the largest of
+// the eight, and split as the walk over halves splits them every workgroup would make the splits for itself again.
 //
 // grid = query_heads * ceil(query_tokens / 128), the longest (last) query tiles first;
-// block = 256.
+// block = 256 (512 at head dimension 256).
 #include <hip/hip_runtime.h>
 
 #include "../kernel_params.h"
 #include "gqa_f32_halved.h"
-#include "gqa_f32_halves.h"
 #include "gqa_f32_walk.h"
 #include "run_merge.h"
 
@@ -23,9 +24,8 @@ namespace {
 // unit b % pair_units, and a unit's time follows the key tiles it walks: the second workgroup
 // of a unit takes the second tier of items in reverse, and the unit that got the heaviest item
 // gets the lightest of them (equal sums for causal walks).
-// An item that `Halves` gives back is walked by `Walk`.
-template <typename Halves, typename Walk>
-__device__ void run_items(const yvex_rocm_gqa_f32_params &p, unsigned char *shared)
+template <typename Walk>
+__device__ void run_items(const yvex_rocm_gqa_f32_params &p, float *shared)
 {
     uint32_t count = 1u;
     u32x4 row = {0u, 0u, 0u, 0u};
@@ -43,11 +43,7 @@ __device__ void run_items(const yvex_rocm_gqa_f32_params &p, unsigned char *shar
         // (opaque, so that what depends on the lane is not kept in registers from item to item)
         int thread = (int)threadIdx.x;
         __asm__ volatile("" : "+v"(thread));
-        if (!Halves(p, *reinterpret_cast<typename Halves::Shared *>(shared), thread).item(id)) {
-            __syncthreads();  // every wave has read the verdict
-            __asm__ volatile("" : "+v"(thread));
-            Walk(p, reinterpret_cast<float *>(shared), thread).item(id);
-        }
+        Walk(p, shared, thread).item(id);
         // every wave is done with the tiles in LDS before the next item stages its own
         if (j < count) __syncthreads();
     }
@@ -77,21 +73,18 @@ constexpr int larger(int a, int b) { return a > b ? a : b; }
 }  // namespace
 
 // `waves`: waves per SIMD the register budget is sized for.
-#define YVEX_GQA_F32_TILE_KERNEL(name, halves, walk, threads, waves)                                          \
+#define YVEX_GQA_F32_TILE_KERNEL(name, walk, threads, waves)                                                  \
     extern "C" __global__ void __launch_bounds__(threads) __attribute__((amdgpu_waves_per_eu(waves, waves)))   \
     name(const yvex_rocm_gqa_f32_params p)                                                                      \
     {                                                                                                           \
-        typedef halves Halves;                                                                                  \
-        __shared__ __attribute__((aligned(16))) unsigned char                                                   \
-            lds[larger((int)sizeof(Halves::Shared), (int)sizeof(float) * 2 * walk::kStageFloats)];              \
-        run_items<Halves, walk>(p, lds);                                                                        \
+        __shared__ __attribute__((aligned(16))) float lds[2 * walk::kStageFloats];                              \
+        run_items<walk>(p, lds);                                                                                \
     }
-#define YVEX_HALVES(part, parts) GqaHalves<part, parts>
 
-YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_64, YVEX_HALVES(64, 1), GqaTile<2>, 256, 2)
-YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_128, YVEX_HALVES(128, 1), GqaTile<4>, 256, 2)
+YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_64, GqaTile<2>, 256, 2)
+YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_128, GqaTile<4>, 256, 2)
 // pairs of waves split the head dimension
-YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_256, YVEX_HALVES(128, 2), GqaTilePair, 512, 2)
+YVEX_GQA_F32_TILE_KERNEL(yvex_rocm_gqa_f32_tile_256, GqaTilePair, 512, 2)
 
 #define YVEX_GQA_F32_HALVED_KERNELS(dim, waves)                                                                   \
     extern "C" __global__ void __launch_bounds__(256)                                                             \

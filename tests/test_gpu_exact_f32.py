@@ -408,6 +408,84 @@ def test_gqa_matrix_core_kernel_follows_magnitudes(backend, case, causal):
     assert np.abs(lse - ref_lse).max() < 2e-5 * max(1.0, np.abs(ref_lse).max())
 
 
+def spread_cases(d, power, tq=64, tk=500, hq=4, hkv=2):
+    """(label, q, k, v, query_start): N(0,1) rows, and one row, channel or component that is 2^power of that while
+    scores stay moderate (or exclude a key altogether).  Dimension 0 of the queries is positive, so that a key can be
+    excluded through it; the last keys are seen by no query."""
+    rng = np.random.default_rng(power * 1000 + d + tk)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((tq, hq, d), (tk, hkv, d), (tk, hkv, d)))
+    q[..., 0] = np.abs(q[..., 0]) + np.float32(1.0)
+    big = np.float32(2.0 ** power)
+    start = tk - tq - 21
+    last = start + tq                       # the first key that no query sees
+
+    def changed(array, where, by):
+        array = array.copy()
+        array[where] = by(array[where])
+        return array
+
+    def grow(x):
+        return x * big
+
+    for label, key in (("octet", last), ("tile", last + 8), ("later", last - 1), ("later-tile", last - 30)):
+        yield "key-" + label, q, changed(k, np.s_[key, :, 1:], grow), v, start
+        yield "value-" + label, q, k, changed(v, key, grow), start
+    for label, key in (("early", 3), ("late", start - 5)):
+        excluded = changed(k, np.s_[key, :, 0], lambda x: -big * np.float32(d))
+        yield "excluded-" + label, q, excluded, v, start
+        yield "excluded-value-" + label, q, excluded, changed(v, key, grow), start
+        yield "excluded-component-" + label, q, excluded, changed(v, np.s_[key, :, 5], grow), start
+        yield "component-" + label, q, k, changed(v, np.s_[key, :, 5], grow), start
+    yield "value-channel", q, k, changed(v, np.s_[:, :, 7], grow), start
+    yield "value-row-small", q, k, changed(v, np.s_[40:48], lambda x: x / big), start
+    quiet_k, quiet_q = changed(k, np.s_[..., 9], np.zeros_like), changed(q, np.s_[..., 9], np.zeros_like)
+    yield "query-channel", changed(q, np.s_[..., 9], grow), quiet_k, v, start
+    yield "key-channel", quiet_q, changed(k, np.s_[..., 9], grow), v, start
+    # a first key that takes all but 2^-5 to 2^-17 of the weight, with a value near zero, or zero
+    for label, extra, factor in (("", 8.0, 1e-4), ("-deep", 16.0, 1e-6), ("-zero", 16.0, 0.0)):
+        sink = changed(k, np.s_[0, :, 0], lambda x: np.float32(extra * math.sqrt(d)))
+        yield "sink" + label, changed(q, np.s_[..., 0], lambda x: np.ones_like(x)), sink, \
+            changed(v, 0, lambda x: x * np.float32(factor)), start
+
+
+def relative_to_weighted_magnitudes(out, q, k, v, start):
+    """The largest error of an output element against 64 bits, relative to sum w |v| of that element."""
+    tq, hq, d = q.shape
+    worst = 0.0
+    for head in range(hq):
+        kv = head // (hq // k.shape[1])
+        scores = q[:, head].astype(np.float64) @ k[:, kv].astype(np.float64).T / math.sqrt(d)
+        scores[np.arange(k.shape[0])[None, :] > (start + np.arange(tq))[:, None]] = -np.inf
+        weights = np.exp(scores - scores.max(axis=1, keepdims=True))
+        weights /= weights.sum(axis=1, keepdims=True)
+        values = v[:, kv].astype(np.float64)
+        size = weights @ np.abs(values)
+        error = np.abs(out[:, head].astype(np.float64) - weights @ values)
+        worst = max(worst, float((error / np.where(size > 0.0, size, 1.0)).max()))
+    return worst
+
+
+# A score is a sum of d products, rounded d / 2 times on the way (two lane halves): a random walk of
+# sqrt(d / 2) 2^-25 sum |q k| / sqrt(d), with |q k| of 0.64 on average 0.6e-7 d, 1.5e-6 at 256 where all of it goes
+# one way; weights carry it into the sum, which adds a few 2^-24 of its own (seen: 2.6e-6).  An exponent of x log2
+# units below the maximum is rounded to 2^-24 x, twice, and the maximum itself as a score: 3e-6 more at 23 of them,
+# which is what the deep sinks have (seen: 5.5e-6).
+def spread_bound(label):
+    return 8e-6 if label.startswith("sink-") else 4e-6
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("power", [16, 24, 32, 40, 50])
+def test_gqa_matrix_core_kernel_holds_the_spread(backend, d, power):
+    """One row, channel or component of 2^16 to 2^50 among N(0,1) ones, seen, unseen or of weight zero, and sinks:
+    every output element keeps its bits relative to sum w |v| of that element."""
+    for label, q, k, v, start in spread_cases(d, power):
+        out, lse, facts = run_exact(backend, q, k, v, query_start=start)
+        assert facts.accelerated_matrix_launches == 1 and facts.kernel_launches == 1
+        worst = relative_to_weighted_magnitudes(out, q, k, v, start)
+        assert worst < spread_bound(label), (label, worst)
+
+
 @pytest.mark.parametrize("d,hq,hkv", [(64, 2, 1), (128, 5, 1), (256, 2, 1)])
 def test_gqa_matrix_core_kernel_infinities(backend, d, hq, hkv):
     """An infinite key that no query sees changes nothing; one that a query sees, with a product of one sign
