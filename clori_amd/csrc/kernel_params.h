@@ -227,8 +227,7 @@ typedef struct {
  *   walk:    the request as for the bf16 prefill, but q, k, v and out are F32, gate is unused, and a step
  *            is 32 keys
  *   tiles:   [kv_heads][kv_tiles][256 * head_dim] bytes
- *   factors: [kv_heads][kv_tiles][8]: per eight keys the F32 factor of their scores, then per eight
- *            values their exponent
+ *   factors: [kv_heads][kv_tiles][8]: four words unused, then per eight values their exponent
  *   pair_units: as in yvex_rocm_gqa_f32_params */
 typedef struct {
     yvex_rocm_prefill_params walk;

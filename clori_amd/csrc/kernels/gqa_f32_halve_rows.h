@@ -15,6 +15,7 @@ namespace {
 template <int kDim>
 struct HalvedTile {
     static constexpr int kKeys = 32;
+    static constexpr float kKeyFactor = 128.f;  // of every key value (gqa_f32_halved.h)
     static constexpr int kPlane = kKeys * kDim * 2, kTensor = 2 * kPlane, kBytes = 2 * kTensor;
 
     // Where the unit of `dim` lies among those of its keys: lanes that write units four dims apart,
@@ -23,9 +24,7 @@ struct HalvedTile {
 };
 
 // Splits the rows of one tile of one kv head: a workgroup of four waves, eight rows of K and eight of V each.
-// Beside the tile it leaves the factor that each eight keys' scores take (NaN where a key lies past the
-// range: the scores are then not finite, and neither is any row that sees them) and the exponent of
-// each eight values (past kExponentMost there).
+// Beside the tile it leaves the exponent of each eight values (past kExponentMost where one lies past the range).
 // Bound by memory: 14.6 MB of rows in and as much out, 1777 tokens of 8 kv heads of 128.
 template <int kDim>
 struct HalveRows {
@@ -85,24 +84,18 @@ struct HalveRows {
         for (int j = 0; j < kPieces; ++j) k[j] = load(keys, k_offset + 256 * (j / 2) + 16 * (j % 2));
 #pragma unroll
         for (int j = 0; j < kPieces; ++j) v[j] = load(values, v_offset + (uint32_t)j * v_row);
-        uint32_t k_most = 0u, v_most = 0u;
+        uint32_t v_most = 0u;
 #pragma unroll
         for (int j = 0; j < kPieces; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                k_most = max(k_most, bits_of(k[j][i]));
-                v_most = max(v_most, bits_of(v[j][i]));
-            }
-        k_most = wave_max(k_most);
+            for (int i = 0; i < 4; ++i) v_most = max(v_most, bits_of(v[j][i]));
         v_most = wave_max(v_most);
-        const uint32_t k_exponent = group_exponent(k_most), v_exponent = group_exponent(v_most);
+        const uint32_t v_exponent = group_exponent(v_most);
         if (lane == 0) {
             uint32_t *words = p.factors + ((uint64_t)kv_head * p.kv_tiles + tile) * 8u;
-            words[quarter] = k_most >> 23 > kExponentMost ? 0x7fc00000u
-                                                          : __builtin_bit_cast(uint32_t, up_factor(k_exponent));
             words[4 + quarter] = v_most >> 23 > kExponentMost ? kExponentMost + 1u : v_exponent;
         }
-        const float k_factor = down_factor(k_exponent), v_factor = down_factor(v_exponent);
+        const float v_factor = down_factor(v_exponent);
         unsigned char *k_unit = lds + ((lane >> 3) * 32 + 8 * quarter + (lane & 7)) * 16;
 #pragma unroll
         for (int r = 0; r < kOctets; ++r) {
@@ -110,7 +103,7 @@ struct HalveRows {
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 _Float16 h, l;
-                halves(k[2 * r + j / 4][j % 4], k_factor, h, l);
+                halves(k[2 * r + j / 4][j % 4], Tile::kKeyFactor, h, l);
                 hi[j] = h;
                 lo[j] = l;
             }

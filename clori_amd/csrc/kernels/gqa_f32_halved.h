@@ -3,6 +3,16 @@
 // An F32 value times a power of two is written as the sum of two f16 values, hi = its nearest and
 // lo = the nearest of what hi leaves, and a product as hi hi + hi lo + lo hi.  The f16 matrix
 // instruction does 16 times the fp32 one's work per cycle, so three of them take 3/16 of its time.
+//
+// Scores.  A key value is scaled by 2^7 whatever lies beside it, a query row by a power of two of its own.  Both
+// halves together keep half an F32 last place of a value, but no less than 2^-25 of the scaled scale: 2^-32
+// of a key value, 2^(x-39) of a query value where the row's largest lies in [2^x, 2^(x+1)).  What that can move
+// a score by, in log2 units, is at most
+//     2^-32 unit sum |q|  +  2^(x-39) unit 2^9 (query values below 2^(x-16)),    unit = scale log2(e),
+// as a finite key value is below 2^9 (a larger one becomes infinite, hi and lo of opposite signs, and every
+// score of it NaN).  A row for which either could exceed 2^-23 gets scores that are NaN.  N(0,1) rows stay
+// below by 2^5.  A row of NaNs is walked in fp32.  So a score depends on its own query and key only, and a weight is
+// off by 1e-7 of itself at most beside the roundings that a sum of F32 products has as well.
 // The splits are made once by a launch of their own (halve_rows) that leaves every tile of 32 keys as the walk wants
 // it in LDS: the walk's tiles are filled by loads that write LDS directly, its registers
 // hold no rows on their way, and a trip is bound by its MFMAs.  Items, packed rows and runs of keys are those of
@@ -59,14 +69,13 @@ struct GqaHalved {
     uint32_t first_tile, tiles;      // of this workgroup's run
     int visible;                     // last key the lane's row sees, from the run's first on
     i32x4 rsrc;                      // the kv head's tiles
-    const uint32_t *factors;         // and their factors
+    const uint32_t *factors;         // and the exponents of their values
     uint32_t lds_base, k_unit, v_unit[2];
     halfx8 q_hi[kSteps], q_lo[kSteps];
-    float q_factor;
+    float q_factor;                  // of the lane's row: scores in log2 units per product as the MFMAs sum them
     floatx16 out[kBlocks];
     float top, neg_top, sum;         // the maximum that weights are relative to (log2 units), this half's denominator
     int reference;                   // the exponent that the accumulators are relative to
-    floatx4 next_factor;             // of the keys of the tile after the next, on their way
     u32x4 next_exponent;             // of the values of the next tile
     uint32_t key_buffer;             // the K tile that the last trip left: free for the next load
 
@@ -94,14 +103,13 @@ struct GqaHalved {
         stage(tile, (uint32_t)((kKeyBuffers + buf) * kTensor), (uint32_t)kTensor, j);
     }
 
-    __device__ __forceinline__ void fetch_factors(uint32_t k_tile, uint32_t v_tile)
+    __device__ __forceinline__ void fetch_exponents(uint32_t tile)
     {
         // (through the vector memory path: a scalar load would make every LDS wait a full one)
         uint32_t zero = 0u;
         __asm__ volatile("" : "+v"(zero));
         const uint32_t *at = factors + zero;
-        next_factor = *reinterpret_cast<const floatx4 *>(at + (first_tile + min(k_tile, tiles - 1u)) * 8u);
-        next_exponent = *reinterpret_cast<const u32x4 *>(at + (first_tile + min(v_tile, tiles - 1u)) * 8u + 4u);
+        next_exponent = *reinterpret_cast<const u32x4 *>(at + (first_tile + min(tile, tiles - 1u)) * 8u + 4u);
     }
 
     // `unit`: of the lane, in the tile's buffer
@@ -125,27 +133,22 @@ struct GqaHalved {
         for (int i = 0; i < 16; ++i) s[i] = 8 * (i / 4) + i % 4 <= seen ? s[i] : -INFINITY;
     }
 
-    // the largest of four scores in log2 units, with what came before
-    __device__ static __forceinline__ float peak_of(const floatx16 &s, const floatx4 &factor, int g, float peak)
+    // the largest score
+    __device__ static __forceinline__ float peak_of(const floatx16 &s)
     {
-        const float m = fmaxf(fmaxf(fmaxf(s[4 * g], s[4 * g + 1]), s[4 * g + 2]), s[4 * g + 3]);
-        return fmaxf(peak, m * factor[g]);
+        float peak = s[0];
+#pragma unroll
+        for (int i = 1; i < 16; ++i) peak = fmaxf(peak, s[i]);
+        return peak;
     }
-    __device__ static __forceinline__ float peak_of(const floatx16 &s, const floatx4 &factor)
+    // The largest of four and what came before, without fmaxf's canonical forms.  The compiler sees no
+    // instructions here: the scores must have been complete for some MFMAs.
+    __device__ static __forceinline__ void peak_step(const floatx16 &s, int g, float &peak)
     {
-        return peak_of(s, factor, 3, peak_of(s, factor, 2, peak_of(s, factor, 1, peak_of(s, factor, 0, -INFINITY))));
-    }
-    // The same without fmaxf's canonical forms.  The compiler sees no instructions here: the scores must
-    // have been complete for some MFMAs.
-    __device__ static __forceinline__ void peak_step(const floatx16 &s, const floatx4 &factor, int g, float &peak)
-    {
-        float m;
-        __asm__ volatile("v_max3_f32 %0, %2, %3, %4\n\t"
-                         "v_max_f32 %0, %0, %5\n\t"
-                         "v_mul_f32 %0, %0, %6\n\t"
-                         "v_max_f32 %1, %1, %0"
-                         : "=&v"(m), "+v"(peak)
-                         : "v"(s[4 * g]), "v"(s[4 * g + 1]), "v"(s[4 * g + 2]), "v"(s[4 * g + 3]), "v"(factor[g]));
+        __asm__ volatile("v_max3_f32 %0, %0, %1, %2\n\t"
+                         "v_max3_f32 %0, %0, %3, %4"
+                         : "+v"(peak)
+                         : "v"(s[4 * g]), "v"(s[4 * g + 1]), "v"(s[4 * g + 2]), "v"(s[4 * g + 3]));
     }
 
     // Brings the maximum to the peak of a tile (over both halves of a row) that exceeds it by more than
@@ -171,7 +174,7 @@ struct GqaHalved {
     }
 
     // What goes from trip to trip beside the scores: the operands of the first slots, the peak of the
-    // tile in this lane's half of its row.
+    // tile in this lane's half of its row (log2 units).
     struct Carried {
         halfx8 hi[2], lo[2];
         float peak;
@@ -180,17 +183,16 @@ struct GqaHalved {
     // The trip of tile t; kAt = t % 2.
     template <int kAt>
     __device__ __forceinline__ void trip(uint32_t t, uint32_t wave_tiles, uint32_t unmasked, floatx16 &s_cur,
-                                         floatx16 &s_next, floatx4 &f_cur, floatx4 &f_next, Carried &c)
+                                         floatx16 &s_next, Carried &c)
     {
         constexpr int kNext = kAt ^ 1;
         // K(t+2) and V(t) have landed (this wave's loads, then everybody's); every wave is done with
         // K(t) and V(t-1)
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         __syncthreads();
-        f_next = next_factor * q_factor;
         u32x4 exponents = next_exponent;
-        __asm__ volatile("" : "+v"(f_next), "+v"(exponents));
-        fetch_factors(t + 2u, t + 1u);
+        __asm__ volatile("" : "+v"(exponents));
+        fetch_exponents(t + 1u);
         const uint32_t free_keys = key_buffer;
         key_buffer = key_buffer == 2u ? 0u : key_buffer + 1u;  // of t+1, and after that of t+2
         if (t >= wave_tiles) {
@@ -222,7 +224,7 @@ struct GqaHalved {
         auto weigh_step = [&](int k) __attribute__((always_inline)) {
             const int w = k / 4 * 2 + k % 4;
             if (k % 4 < 2) {
-                s_cur[w] = fast_exp2(fmaf(s_cur[w], f_cur[w / 4], neg_top));
+                s_cur[w] = fast_exp2(fmaf(s_cur[w], q_factor, neg_top));
                 part_sum += s_cur[w];
                 // (behind the sum: the exponential's result has been read once)
                 __asm__ volatile("" : "+v"(s_cur[w]), "+v"(part_sum));
@@ -267,7 +269,7 @@ struct GqaHalved {
             ride<i, 16, kHalfSlots - 1, 3 * kHalfSlots / 2 - 1>(
                 [&](int k) __attribute__((always_inline)) { weigh_step(16 + k); });
             ride<i, 4, 3 * kHalfSlots / 2, kSlots>(
-                [&](int g) __attribute__((always_inline)) { peak_step(s_next, f_next, g, peak); });
+                [&](int g) __attribute__((always_inline)) { peak_step(s_next, g, peak); });
             __builtin_amdgcn_sched_barrier(0);
         };
         __builtin_amdgcn_sched_barrier(0);
@@ -281,9 +283,9 @@ struct GqaHalved {
         sum += part_sum;
         if (t + 1u >= unmasked && t + 1u < wave_tiles) {
             mask(s_next, t + 1u);
-            peak = peak_of(s_next, f_next);
+            peak = peak_of(s_next);
         }
-        c.peak = peak;
+        c.peak = peak * q_factor;
     }
 
     // Steps of a kind, spread over slots [kFrom, kTo).
@@ -307,8 +309,24 @@ struct GqaHalved {
         for (int s = 0; s < kSteps; ++s)
 #pragma unroll
             for (int j = 0; j < 8; ++j) most = fmaxf(most, fabsf(x[s][j / 4][j % 4]));
-        const uint32_t bits = __builtin_bit_cast(uint32_t, max_xor32(most)), e = group_exponent(bits);
-        q_factor = bits >> 23 > kExponentMost ? __builtin_nanf("") : up_factor(e) * (p.scale * YVEX_LOG2E);
+        // (a row below 2^-62 as one of that size: q_factor stays a normal number)
+        const uint32_t e = max(group_exponent(__builtin_bit_cast(uint32_t, max_xor32(most))), 64u);
+        const float up = up_factor(e), unit = p.scale * YVEX_LOG2E;  // 2^x / 2^14, a score's log2 units
+        // (NaN where the halves' floors could move a score: the row is then not finite, and is walked in fp32)
+        q_factor = up * (unit * (1.f / Tile::kKeyFactor));
+        if (__builtin_amdgcn_ballot_w64(!(up * unit * (float)(kDim << 14) <= 128.f)) != 0ull) {
+            float l1 = 0.f, tiny = 0.f;
+#pragma unroll
+            for (int s = 0; s < kSteps; ++s)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const float v = fabsf(x[s][j / 4][j % 4]);
+                    l1 += v;
+                    tiny += v != 0.f && v < 0.25f * up ? 1.f : 0.f;
+                }
+            if (!(sum_xor32(l1) * unit <= 512.f && sum_xor32(tiny) * up * unit <= 0x1p-7f))
+                q_factor = __builtin_nanf("");
+        }
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) {
             uint32_t hi[4], lo[4];
@@ -479,12 +497,10 @@ struct GqaHalved {
         for (int j = 0; j < kLoads; ++j) stage_keys(1u, 1u, j);
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) stage_values(0u, 0, j);
-        fetch_factors(0u, 0u);
+        fetch_exponents(0u);
         load_queries(query);
-        floatx4 f_even = next_factor * q_factor, f_odd;
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         __syncthreads();
-        fetch_factors(1u, 0u);
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) stage_keys(2u, 2u, j);
         floatx16 s_even, s_odd;
@@ -504,22 +520,22 @@ struct GqaHalved {
             c.hi[k] = key_operand(k_unit + kTensor, k, 0);
         }
         if (unmasked == 0u) mask(s_even, 0u);
-        c.peak = peak_of(s_even, f_even);
+        c.peak = peak_of(s_even) * q_factor;
         key_buffer = 0u;
         // (two copies of a trip instead of three take less time to fetch: 1777 tokens 122 -> 118.5 us; at 256 the
         // compiler moves more registers about in that form: 1000 tokens 102 -> 116)
         uint32_t t = 0u;
         if constexpr (kDim == 256) {
             for (; t + 1u < tiles; t += 2u) {
-                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, f_even, f_odd, c);
-                trip<1>(t + 1u, wave_tiles, unmasked, s_odd, s_even, f_odd, f_even, c);
+                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, c);
+                trip<1>(t + 1u, wave_tiles, unmasked, s_odd, s_even, c);
             }
-            if (t < tiles) trip<0>(t, wave_tiles, unmasked, s_even, s_odd, f_even, f_odd, c);
+            if (t < tiles) trip<0>(t, wave_tiles, unmasked, s_even, s_odd, c);
         } else {
             for (;;) {
-                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, f_even, f_odd, c);
+                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, c);
                 if (++t == tiles) break;
-                trip<1>(t, wave_tiles, unmasked, s_odd, s_even, f_odd, f_even, c);
+                trip<1>(t, wave_tiles, unmasked, s_odd, s_even, c);
                 if (++t == tiles) break;
             }
         }
