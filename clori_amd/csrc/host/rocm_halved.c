@@ -1,10 +1,10 @@
-/* Prefill-shaped EXACT_F32 requests over keys and values split into halves beforehand: the plan of a
+/* Prefill-shaped EXACT_F32 requests over keys and values split into 16-bit parts beforehand: the plan of a
  * request, the bytes it wants attached, and its launches.
  *
- * One launch splits the visible key and value rows (kernels/gqa_f32_halved.h), the second walks them
+ * One launch splits the visible key and value rows (kernels/gqa_f32_halve_rows.h), the second walks them
  * with the query heads of a kv head packed into the rows of its tiles and, where the launch would leave
  * units idle, in runs of keys (the plan of the bf16 prefill, rocm_prefill.c, with steps of 32 keys), and
- * a third merges the runs.  Halves and partials live in the attached workspace; without one
+ * a third merges the runs.  Parts and partials live in the attached workspace; without one
  * that holds them a request runs in one launch with fp32 products (kernels/gqa_f32_walk.h).
  * Everything here is a function of the request's geometry only, so that the planner's
  * workspace_required and the execution agree. */
@@ -15,14 +15,13 @@
 
 enum {
     HALVED_STEP_KEYS = 32,
-    HALVED_GROUP_MAX = 16, /* query heads packed into the rows of a tile */
-    HALVED_FACTOR_WORDS = 8 /* of a tile */
+    HALVED_GROUP_MAX = 16 /* query heads packed into the rows of a tile */
 };
-#define HALVED_TILES_MAX (512ull << 20) /* bytes of halves a request may ask for */
+#define HALVED_TILES_MAX (640ull << 20) /* bytes of parts a request may ask for */
 
 typedef struct {
     yvex_rocm_walk_plan walk;
-    unsigned long long kv_tiles, tile_bytes, factor_bytes; /* of all kv heads */
+    unsigned long long kv_tiles, tile_bytes; /* of all kv heads */
     unsigned long long total;
 } halved_plan;
 
@@ -51,14 +50,12 @@ static int halved_plan_make(const yvex_transformer_attention_requirement *r, hal
         return 0;
     if (visible_keys(r) < d + 192ull) return 0;
     plan->kv_tiles = (visible_keys(r) + HALVED_STEP_KEYS - 1ull) / HALVED_STEP_KEYS;
-    plan->tile_bytes = r->key_value_heads * plan->kv_tiles * 256ull * d;
-    plan->factor_bytes = r->key_value_heads * plan->kv_tiles * HALVED_FACTOR_WORDS * sizeof(uint32_t);
-    plan->factor_bytes = (plan->factor_bytes + 255ull) & ~255ull;
+    plan->tile_bytes = r->key_value_heads * plan->kv_tiles * 320ull * d;
     if (plan->tile_bytes > HALVED_TILES_MAX) return 0;
     yvex_rocm_walk_plan_whole(r, group, HALVED_STEP_KEYS, &plan->walk);
     if (plan->walk.whole_items > 0x7fffffffull) return 0;
     yvex_rocm_walk_plan_cut(r, &plan->walk);
-    plan->total = plan->tile_bytes + plan->factor_bytes + plan->walk.acc_bytes + plan->walk.ml_bytes;
+    plan->total = plan->tile_bytes + plan->walk.acc_bytes + plan->walk.ml_bytes;
     return 1;
 }
 
@@ -117,9 +114,8 @@ int yvex_rocm_halved_launch(yvex_backend *backend, const yvex_transformer_attent
     w->splits = (uint32_t)plan.walk.splits;
     w->merge_groups = plan.walk.splits > 8ull ? 4u : 1u;
     params.tiles = (unsigned char *)(uintptr_t)work;
-    params.factors = (uint32_t *)(uintptr_t)(work + plan.tile_bytes);
-    w->part_acc = (float *)(uintptr_t)(work + plan.tile_bytes + plan.factor_bytes);
-    w->part_ml = (float *)(uintptr_t)(work + plan.tile_bytes + plan.factor_bytes + plan.walk.acc_bytes);
+    w->part_acc = (float *)(uintptr_t)(work + plan.tile_bytes);
+    w->part_ml = (float *)(uintptr_t)(work + plan.tile_bytes + plan.walk.acc_bytes);
     params.scale = f->scale;
     params.kv_tiles = (uint32_t)plan.kv_tiles;
     /* two workgroups of a unit: the second tier of items in reverse, equal sums for causal walks */

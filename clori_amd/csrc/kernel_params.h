@@ -220,19 +220,17 @@ typedef struct {
     uint32_t merge_groups; /* groups of threads that the merge deals a row's runs to: 1 or 4 */
 } yvex_rocm_prefill_params;
 
-/* EXACT_F32 attention over keys and values split into halves (gqa_f32_halved.h).
+/* EXACT_F32 attention over keys and values split into 16-bit parts (gqa_f32_halved.h).
  * yvex_rocm_gqa_f32_halve_* splits kv_tiles tiles of 32 keys of every kv head (grid = (kv_tiles,
  * kv_heads), block 256), yvex_rocm_gqa_f32_halved_* walks them (grid = whole_items + tail_items * splits,
  * block 256), yvex_rocm_gqa_f32_merge_* merges the runs of cut items as yvex_rocm_prefill_merge* does.
  *   walk:    the request as for the bf16 prefill, but q, k, v and out are F32, gate is unused, and a step
  *            is 32 keys
- *   tiles:   [kv_heads][kv_tiles][256 * head_dim] bytes
- *   factors: [kv_heads][kv_tiles][8]: four words unused, then per eight values their exponent
+ *   tiles:   [kv_heads][kv_tiles][320 * head_dim] bytes
  *   pair_units: as in yvex_rocm_gqa_f32_params */
 typedef struct {
     yvex_rocm_prefill_params walk;
     unsigned char *tiles;
-    uint32_t *factors;
     float scale;
     uint32_t kv_tiles, pair_units, reserved;
 } yvex_rocm_gqa_f32_halved_params;

@@ -7,27 +7,18 @@
 namespace {
 
 typedef _Float16 halfx8 __attribute__((ext_vector_type(8)));
-typedef _Float16 halfx2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ floatx16 mfma_32x32x16_f16(halfx8 a, halfx8 b, floatx16 c)
 {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-// Magnitudes compare as whole numbers; a NaN is larger than all of them.
-template <int kControl>
-__device__ __forceinline__ uint32_t dpp_max(uint32_t v)
-{
-    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kControl, 0xf, 0xf, true));
-}
+// Biased exponent that a query row whose largest magnitude has these bits is scaled by: 2^(141 - e)
+// brings it to [2^14, 2^15).  A row below 2^-62 is scaled as one of that size (so that 2^(e - 141) times a
+// score's unit stays a normal number), one of 2^51 and more as one of that.
+constexpr uint32_t kExponentLeast = 64u, kExponentMost = 177u;
 
-// Biased exponent that a group whose largest magnitude has these bits is scaled by: 2^(141 - e)
-// brings it to [2^14, 2^15).  Both that factor and its inverse 2^(e - 141) are normal numbers for
-// e in [kExponentLeast, kExponentMost]; a group below the range is scaled as its least, one above
-// it (2^51 and more, infinities) is left to the fp32 walk.
-constexpr uint32_t kExponentLeast = 15u, kExponentMost = 177u;
-
-__device__ __forceinline__ uint32_t group_exponent(uint32_t max_bits)
+__device__ __forceinline__ uint32_t row_exponent(uint32_t max_bits)
 {
     return min(max(max_bits >> 23, kExponentLeast), kExponentMost);
 }
@@ -63,21 +54,6 @@ __device__ __forceinline__ void split_pair_by_lane(float a, float b, float facto
                      "v_fma_mixhi_f16 %1, %3, %4, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
                      : "=&v"(hi), "=&v"(lo)
                      : "v"(a), "v"(b), "v"(factor));
-}
-
-// The same in two steps.
-__device__ __forceinline__ void split_hi(float a, float b, float factor, uint32_t &hi)
-{
-    __asm__ volatile("v_fma_mixlo_f16 %0, %1, %3, 0\n\tv_fma_mixhi_f16 %0, %2, %3, 0"
-                     : "=&v"(hi)
-                     : "v"(a), "v"(b), "s"(factor));
-}
-__device__ __forceinline__ void split_lo(float a, float b, float factor, uint32_t hi, uint32_t &lo)
-{
-    __asm__ volatile("v_fma_mixlo_f16 %0, %1, %3, -%4 op_sel_hi:[0,0,1]\n\t"
-                     "v_fma_mixhi_f16 %0, %2, %3, -%4 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
-                     : "=&v"(lo)
-                     : "v"(a), "v"(b), "s"(factor), "v"(hi));
 }
 
 // x / y given r = 1 / y: one step of Newton's method from x r, which leaves the nearest value but for rare

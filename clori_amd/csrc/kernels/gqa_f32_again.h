@@ -1,4 +1,4 @@
-// The fp32 walk of an item whose f16 halves left the range: what gqa_f32_halved.h falls back to.
+// The fp32 walk of an item whose parts left the range: what gqa_f32_halved.h falls back to.
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
 #define YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
 

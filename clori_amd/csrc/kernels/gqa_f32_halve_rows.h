@@ -1,4 +1,4 @@
-// Key and value rows of EXACT_F32 attention split into halves, tile by tile (f16_split.h), for the walk of
+// Key and value rows of EXACT_F32 attention split into 16-bit parts, tile by tile, for the walk of
 // gqa_f32_halved.h.
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVE_ROWS_H
 #define YVEX_ROCM_KERNELS_GQA_F32_HALVE_ROWS_H
@@ -9,14 +9,15 @@
 
 namespace {
 
-// A tile in memory and in LDS: [K hi | K lo] and [V hi | V lo].
+// A tile in memory and in LDS: [K hi | K lo], f16, and [V 1 | V 2 | V 3], bf16.
 //   K: 16-byte units (octet of dims, key);  V: units (16 keys u, lane half, dim) of eight keys in the order of the
 //   score registers: keys 16 u + 4 half + 0..3, then 16 u + 8 + 4 half + 0..3
 template <int kDim>
 struct HalvedTile {
     static constexpr int kKeys = 32;
     static constexpr float kKeyFactor = 128.f;  // of every key value (gqa_f32_halved.h)
-    static constexpr int kPlane = kKeys * kDim * 2, kTensor = 2 * kPlane, kBytes = 2 * kTensor;
+    static constexpr int kPlane = kKeys * kDim * 2;
+    static constexpr int kKeyBytes = 2 * kPlane, kValueBytes = 3 * kPlane, kBytes = kKeyBytes + kValueBytes;
 
     // Where the unit of `dim` lies among those of its keys: lanes that write units four dims apart,
     // and lanes that read neighbouring ones, meet every bank once.
@@ -24,8 +25,7 @@ struct HalvedTile {
 };
 
 // Splits the rows of one tile of one kv head: a workgroup of four waves, eight rows of K and eight of V each.
-// Beside the tile it leaves the exponent of each eight values (past kExponentMost where one lies past the range).
-// Bound by memory: 14.6 MB of rows in and as much out, 1777 tokens of 8 kv heads of 128.
+// Bound by memory: 14.6 MB of rows in and 18.2 out, 1777 tokens of 8 kv heads of 128.
 template <int kDim>
 struct HalveRows {
     typedef HalvedTile<kDim> Tile;
@@ -46,23 +46,27 @@ struct HalveRows {
                                                  (int)(uint32_t)min(bytes, (uint64_t)0xffffffffu), 0x00027000);
     }
 
-    static __device__ __forceinline__ uint32_t wave_max(uint32_t v)
-    {
-        v = dpp_max<0x112>(dpp_max<0x111>(v));  // row_shr 1, 2, 4, 8: the last lane of a row has its largest
-        v = dpp_max<0x118>(dpp_max<0x114>(v));
-        v = dpp_max<0x143>(dpp_max<0x142>(v));  // row_bcast 15, 31
-        return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
-    }
-
-    static __device__ __forceinline__ uint32_t bits_of(float v)
-    {
-        return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
-    }
-
     static __device__ __forceinline__ void halves(float x, float factor, _Float16 &hi, _Float16 &lo)
     {
         hi = (_Float16)(x * factor);
         lo = (_Float16)fmaf(x, factor, -(float)hi);
+    }
+
+    // A value as the sum of three bf16 values, each the nearest of what is left: all 24 bits, and F32's range of
+    // exponents.  The last bits of a value below 2^-102 would lie below bf16's normal numbers: it is a NaN
+    // here, and so is every row that meets it.  Two values at a time.
+    static __device__ __forceinline__ void thirds(float a, float b, uint32_t (&part)[3])
+    {
+        float left[2] = {a, b};
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (left[i] != 0.f && fabsf(left[i]) < 0x1p-102f) left[i] = __builtin_nanf("");
+#pragma unroll
+        for (int n = 0; n < 3; ++n) {
+            part[n] = pack_bf16x2(left[0], left[1]);
+            left[0] -= __builtin_bit_cast(float, part[n] << 16);
+            left[1] -= __builtin_bit_cast(float, part[n] & 0xffff0000u);
+        }
     }
 
     static __device__ void run(const yvex_rocm_gqa_f32_halved_params &p, unsigned char *lds)
@@ -84,18 +88,6 @@ struct HalveRows {
         for (int j = 0; j < kPieces; ++j) k[j] = load(keys, k_offset + 256 * (j / 2) + 16 * (j % 2));
 #pragma unroll
         for (int j = 0; j < kPieces; ++j) v[j] = load(values, v_offset + (uint32_t)j * v_row);
-        uint32_t v_most = 0u;
-#pragma unroll
-        for (int j = 0; j < kPieces; ++j)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v_most = max(v_most, bits_of(v[j][i]));
-        v_most = wave_max(v_most);
-        const uint32_t v_exponent = group_exponent(v_most);
-        if (lane == 0) {
-            uint32_t *words = p.factors + ((uint64_t)kv_head * p.kv_tiles + tile) * 8u;
-            words[4 + quarter] = v_most >> 23 > kExponentMost ? kExponentMost + 1u : v_exponent;
-        }
-        const float v_factor = down_factor(v_exponent);
         unsigned char *k_unit = lds + ((lane >> 3) * 32 + 8 * quarter + (lane & 7)) * 16;
 #pragma unroll
         for (int r = 0; r < kOctets; ++r) {
@@ -119,14 +111,14 @@ struct HalveRows {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int at = ((quarter >> 1) * 2 + ((from + j0) >> 2)) * kDim + Tile::value_unit(dim + i);
-                unsigned char *unit = lds + Tile::kTensor + at * 16 + (quarter & 1) * 8 + ((from + j0) & 3) * 2;
+                unsigned char *unit = lds + Tile::kKeyBytes + at * 16 + (quarter & 1) * 8 + ((from + j0) & 3) * 2;
 #pragma unroll
                 for (int j = 0; j < kRun; j += 2) {
-                    _Float16 h[2], l[2];
-                    halves(v[j0 + j][i], v_factor, h[0], l[0]);
-                    halves(v[j0 + j + 1][i], v_factor, h[1], l[1]);
-                    *reinterpret_cast<halfx2 *>(unit + 2 * j) = (halfx2){h[0], h[1]};
-                    *reinterpret_cast<halfx2 *>(unit + 2 * j + Tile::kPlane) = (halfx2){l[0], l[1]};
+                    uint32_t part[3];
+                    thirds(v[j0 + j][i], v[j0 + j + 1][i], part);
+#pragma unroll
+                    for (int n = 0; n < 3; ++n)
+                        *reinterpret_cast<uint32_t *>(unit + 2 * j + n * Tile::kPlane) = part[n];
                 }
             }
         __syncthreads();

@@ -1,18 +1,30 @@
-// EXACT_F32 attention over keys and values that were split into halves beforehand.
+// EXACT_F32 attention over keys and values that were split into parts of 16 bits beforehand.
 //
-// An F32 value times a power of two is written as the sum of two f16 values, hi = its nearest and
-// lo = the nearest of what hi leaves, and a product as hi hi + hi lo + lo hi.  The f16 matrix
-// instruction does 16 times the fp32 one's work per cycle, so three of them take 3/16 of its time.
+// The 16-bit matrix instructions do 16 times the fp32 one's work per cycle.  A product of two F32 values is three of
+// f16 parts in the scores and six of bf16 parts in the update (the splitting of an operand into parts of fewer
+// bits with F32 accumulation is a published method, Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial
+// Intelligence Datatype For Higher-Precision Computations", 2019).
 //
-// Scores.  A key value is scaled by 2^7 whatever lies beside it, a query row by a power of two of its own.  Both
-// halves together keep half an F32 last place of a value, but no less than 2^-25 of the scaled scale: 2^-32
-// of a key value, 2^(x-39) of a query value where the row's largest lies in [2^x, 2^(x+1)).  What that can move
-// a score by, in log2 units, is at most
+// Scores.  An F32 value times a power of two as the sum of two f16 values, hi = its nearest and lo = the nearest of
+// what hi leaves, a product as hi hi + hi lo + lo hi.  A key value is scaled by 2^7 whatever lies beside it, a query
+// row by a power of two of its own.  Both halves together keep half an F32 last place of a value, but
+// no less than 2^-25 after scaling: 2^-32 of a key value, 2^(x-39) of a query value where the row's largest lies in
+// [2^x, 2^(x+1)).  What that can move a score by, in log2 units, is at most
 //     2^-32 unit sum |q|  +  2^(x-39) unit 2^9 (query values below 2^(x-16)),    unit = scale log2(e),
 // as a finite key value is below 2^9 (a larger one becomes infinite, hi and lo of opposite signs, and every
 // score of it NaN).  A row for which either could exceed 2^-23 gets scores that are NaN.  N(0,1) rows stay
 // below by 2^5.  A row of NaNs is walked in fp32.  So a score depends on its own query and key only, and a weight is
 // off by 1e-7 of itself at most beside the roundings that a sum of F32 products has as well.
+//
+// Update.  A weight and a value as the sum of three bf16 values each, 24 bits at F32's range of exponents, and
+// the six products of 2^-16 and more: off by 2^-23 of a product at most, however small or large its factors are
+// (a weight below 2^-102 keeps 2^-126 of the row's largest).  With f16 halves here (three products, 122 us instead
+// of 147 for 1777 tokens of 40/8 heads of 128) the weights had to carry the exponents of the values: beside a value
+// of 2^30, or behind a sink of a weight of 1 and a value near zero, the other weights lost their bits.
+//
+// Against 64 bits, per element relative to sum w |v|, the largest error is 2e-7 to 4e-7 on N(0,1) rows (fp32 walk
+// 4e-7 to 6e-7), and at most the fp32 walk's with rows, channels or components of 2^16 to 2^50 and with sinks.
+//
 // The splits are made once by a launch of their own (halve_rows) that leaves every tile of 32 keys as the walk wants
 // it in LDS: the walk's tiles are filled by loads that write LDS directly, its registers
 // hold no rows on their way, and a trip is bound by its MFMAs.  Items, packed rows and runs of keys are those of
@@ -44,23 +56,21 @@ namespace {
 // with tile t; behind the MFMAs ride the loads of K(t+2) and V(t+1), the exponentials of tile t and their
 // split, and the maximum of tile t+1.  An MFMA leaves room for about 24 cycles of vector work (whole
 // instructions take 4 to 5, the exponential and the conversions 8 to 9), so a pair of weights is
-// four steps of less than that.
+// five steps of less than that.
 template <int kDim>
 struct GqaHalved {
     typedef HalvedTile<kDim> Tile;
     static constexpr int kBlocks = kDim / 32, kSteps = kDim / 16, kKeys = Tile::kKeys;
-    static constexpr int kRows = YVEX_ROCM_PREFILL_ROWS, kPlane = Tile::kPlane, kTensor = Tile::kTensor;
-    static constexpr int kLoads = kTensor / 4096;  // 1 KB loads per wave and K or V tile
-    static constexpr int kHalfSlots = 3 * kSteps, kSlots = 2 * kHalfSlots;
-    // weights are at most 2^kLazy (a maximum is raised when it is exceeded by that), so times
-    // 2^kWeightShift they stay inside f16
-    static constexpr int kLazy = 6, kWeightShift = 15 - kLazy;
-
-    static constexpr int kKeyBuffers = 3;
+    static constexpr int kRows = YVEX_ROCM_PREFILL_ROWS, kPlane = Tile::kPlane;
+    static constexpr int kKeyLoads = Tile::kKeyBytes / 4096;  // 1 KB loads per wave and K tile
+    static constexpr int kValueLoads = Tile::kValueBytes / 4096;
+    static constexpr int kScoreSlots = 3 * kSteps, kSlots = kScoreSlots + 6 * 2 * kBlocks;
+    static constexpr int kLazy = 6;  // weights are at most 2^kLazy: a maximum is raised when it is exceeded by that
+    static constexpr int kRing = 4;  // operands on their way from LDS
 
     struct Shared {
-        __attribute__((aligned(16))) unsigned char k[kKeyBuffers][kTensor];
-        __attribute__((aligned(16))) unsigned char v[2][kTensor];
+        __attribute__((aligned(16))) unsigned char k[2][Tile::kKeyBytes];
+        __attribute__((aligned(16))) unsigned char v[2][Tile::kValueBytes];
     };
 
     const yvex_rocm_gqa_f32_halved_params &p;
@@ -69,15 +79,11 @@ struct GqaHalved {
     uint32_t first_tile, tiles;      // of this workgroup's run
     int visible;                     // last key the lane's row sees, from the run's first on
     i32x4 rsrc;                      // the kv head's tiles
-    const uint32_t *factors;         // and the exponents of their values
     uint32_t lds_base, k_unit, v_unit[2];
     halfx8 q_hi[kSteps], q_lo[kSteps];
     float q_factor;                  // of the lane's row: scores in log2 units per product as the MFMAs sum them
     floatx16 out[kBlocks];
     float top, neg_top, sum;         // the maximum that weights are relative to (log2 units), this half's denominator
-    int reference;                   // the exponent that the accumulators are relative to
-    u32x4 next_exponent;             // of the values of the next tile
-    uint32_t key_buffer;             // the K tile that the last trip left: free for the next load
 
     __device__ GqaHalved(const yvex_rocm_gqa_f32_halved_params &params, Shared &shared, int thread)
         : p(params), lds(shared), lane(thread & 63), wave(__builtin_amdgcn_readfirstlane(thread >> 6)),
@@ -87,42 +93,53 @@ struct GqaHalved {
 
     // 1 KB load j of this wave for the K or V tile `tile` into buffer `buf`; tiles past the last are the
     // last once more, so that a trip has no branches.
-    __device__ __forceinline__ void stage(uint32_t tile, uint32_t to, uint32_t at, int j) const
+    __device__ __forceinline__ void stage(uint32_t tile, uint32_t to, uint32_t at, uint32_t mine) const
     {
-        const uint32_t mine = (uint32_t)(wave * (kTensor / 4) + j * 1024);
         lds_dma_b128(lds_base + to + mine, rsrc, (uint32_t)lane * 16u,
                      (uint32_t)__builtin_amdgcn_readfirstlane(
                          (int)((first_tile + min(tile, tiles - 1u)) * (uint32_t)Tile::kBytes + at + mine)));
     }
-    __device__ __forceinline__ void stage_keys(uint32_t tile, uint32_t buf, int j) const
+    __device__ __forceinline__ void stage_keys(uint32_t tile, int buf, int j) const
     {
-        stage(tile, buf * (uint32_t)kTensor, 0u, j);
+        stage(tile, (uint32_t)(buf * Tile::kKeyBytes), 0u, (uint32_t)((wave * kKeyLoads + j) * 1024));
     }
     __device__ __forceinline__ void stage_values(uint32_t tile, int buf, int j) const
     {
-        stage(tile, (uint32_t)((kKeyBuffers + buf) * kTensor), (uint32_t)kTensor, j);
+        stage(tile, (uint32_t)(2 * Tile::kKeyBytes + buf * Tile::kValueBytes), (uint32_t)Tile::kKeyBytes,
+              (uint32_t)((wave * kValueLoads + j) * 1024));
     }
 
-    __device__ __forceinline__ void fetch_exponents(uint32_t tile)
+    __device__ __forceinline__ u32x4 key_operand(int buf, int step, int plane) const
     {
-        // (through the vector memory path: a scalar load would make every LDS wait a full one)
-        uint32_t zero = 0u;
-        __asm__ volatile("" : "+v"(zero));
-        const uint32_t *at = factors + zero;
-        next_exponent = *reinterpret_cast<const u32x4 *>(at + (first_tile + min(tile, tiles - 1u)) * 8u + 4u);
-    }
-
-    // `unit`: of the lane, in the tile's buffer
-    __device__ __forceinline__ halfx8 key_operand(uint32_t unit, int step, int plane) const
-    {
-        return *reinterpret_cast<const halfx8 *>(lds.k[0] + unit + step * 1024 + plane * kPlane);
+        return *reinterpret_cast<const u32x4 *>(lds.k[buf] + k_unit + step * 1024 + plane * kPlane);
     }
     // operand m = u * kBlocks + block
-    __device__ __forceinline__ halfx8 value_operand(int buf, int m, int plane) const
+    __device__ __forceinline__ u32x4 value_operand(int buf, int m, int plane) const
     {
         const int u = m / kBlocks, b = m % kBlocks;
-        return *reinterpret_cast<const halfx8 *>(lds.v[buf] + v_unit[b & 1] + u * kDim * 32 + b * 512 +
-                                                 plane * kPlane);
+        return *reinterpret_cast<const u32x4 *>(lds.v[buf] + v_unit[b & 1] + u * kDim * 32 + b * 512 +
+                                                plane * kPlane);
+    }
+    // Operand n of a trip: lo and hi of a step of S^T from the last plane on, then the three planes of a step of the
+    // update, likewise.
+    template <int n>
+    __device__ __forceinline__ u32x4 operand(int k_buf, int v_buf) const
+    {
+        if constexpr (n < 2 * kSteps) return key_operand(k_buf, n / 2, 1 - n % 2);
+        else return value_operand(v_buf, (n - 2 * kSteps) / 3, 2 - (n - 2 * kSteps) % 3);
+    }
+    static constexpr int kOperands = 2 * kSteps + 3 * 2 * kBlocks;
+
+    // Step `part` (0, 1, 2) of the split of two F32 values into three bf16 values each: the nearest of what is left.
+    __device__ static __forceinline__ uint32_t third(int part, float &a, float &b)
+    {
+        uint32_t pair = pack_bf16x2(a, b);
+        if (part < 2) {
+            a -= __builtin_bit_cast(float, pair << 16);
+            b -= __builtin_bit_cast(float, pair & 0xffff0000u);
+        }
+        __asm__ volatile("" : "+v"(pair), "+v"(a), "+v"(b));
+        return pair;
     }
 
     __device__ __forceinline__ void mask(floatx16 &s, uint32_t tile) const
@@ -152,19 +169,13 @@ struct GqaHalved {
     }
 
     // Brings the maximum to the peak of a tile (over both halves of a row) that exceeds it by more than
-    // 2^kLazy in some row, and what is accumulated to the exponents of the tile's values.
-    __device__ __forceinline__ void adjust(float peak, int most)
+    // 2^kLazy in some row.
+    __device__ __forceinline__ void adjust(float peak)
     {
         const float raised = fmaxf(top, peak);
         // a row that has seen nothing yet keeps the maximum -inf
-        float keep = raised == -INFINITY ? 1.f : fast_exp2(top - raised);
+        const float keep = raised == -INFINITY ? 1.f : fast_exp2(top - raised);
         sum *= keep;
-        if (most > reference) {
-            // one power of two of room, so that the accumulators seldom move
-            keep = __builtin_amdgcn_ldexpf(keep, reference - most - 1);
-            reference = most + 1;
-            if (most > (int)kExponentMost) sum = __builtin_nanf("");  // values past the range
-        }
 #pragma unroll
         for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
@@ -173,119 +184,94 @@ struct GqaHalved {
         neg_top = raised == -INFINITY ? 0.f : -raised;
     }
 
-    // What goes from trip to trip beside the scores: the operands of the first slots, the peak of the
-    // tile in this lane's half of its row (log2 units).
-    struct Carried {
-        halfx8 hi[2], lo[2];
-        float peak;
-    };
-
-    // The trip of tile t; kAt = t % 2.
+    // The trip of tile t; kAt = t % 2; `peak`: of tile t in this lane's half of its row (log2 units).
     template <int kAt>
     __device__ __forceinline__ void trip(uint32_t t, uint32_t wave_tiles, uint32_t unmasked, floatx16 &s_cur,
-                                         floatx16 &s_next, Carried &c)
+                                         floatx16 &s_next, float &peak)
     {
         constexpr int kNext = kAt ^ 1;
-        // K(t+2) and V(t) have landed (this wave's loads, then everybody's); every wave is done with
+        // K(t+1) and V(t) have landed (this wave's loads, then everybody's); every wave is done with
         // K(t) and V(t-1)
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         __syncthreads();
-        u32x4 exponents = next_exponent;
-        __asm__ volatile("" : "+v"(exponents));
-        fetch_exponents(t + 1u);
-        const uint32_t free_keys = key_buffer;
-        key_buffer = key_buffer == 2u ? 0u : key_buffer + 1u;  // of t+1, and after that of t+2
         if (t >= wave_tiles) {
             // nothing of this tile is visible to the wave: it only keeps staging
 #pragma unroll
-            for (int j = 0; j < kLoads; ++j) stage_keys(t + 3u, free_keys, j);
+            for (int j = 0; j < kKeyLoads; ++j) stage_keys(t + 2u, kAt, j);
 #pragma unroll
-            for (int j = 0; j < kLoads; ++j) stage_values(t + 1u, kNext, j);
+            for (int j = 0; j < kValueLoads; ++j) stage_values(t + 1u, kNext, j);
             return;
         }
-        const uint32_t k_now = k_unit + key_buffer * (uint32_t)kTensor;
-        const uint32_t k_then = k_unit + (key_buffer == 2u ? 0u : key_buffer + 1u) * (uint32_t)kTensor;
-        halfx8(&hi)[2] = c.hi, (&lo)[2] = c.lo;
-        float weight_factor[4];
-        uint32_t p_hi[8], p_lo[8];
-        float part_sum = 0.f, peak = -INFINITY;
-        int e[4], most = 0;
+        u32x4 ring[kRing];
+        for_each<kRing>([&](auto n) __attribute__((always_inline)) {
+            ring[decltype(n)::value] = operand<decltype(n)::value>(kNext, kAt);
+        });
+        uint32_t weights[3][8];
+        float part_sum = 0.f, next_peak = -INFINITY;
         bool raise = false;
-        // the maximum of this tile's rows and the exponents of its values
+        // the maximum of this tile's rows
         auto settle_step = [&](int k) __attribute__((always_inline)) {
-            if (k < 4) {
-                e[k] = __builtin_amdgcn_readfirstlane((int)exponents[k]);
-                most = max(most, e[k]);
-            }
-            if (k == 0) c.peak = max_xor32(c.peak);
-            if (k == 2) raise = __builtin_amdgcn_ballot_w64(c.peak > top + (float)kLazy) != 0ull;
+            if (k == 0) peak = max_xor32(peak);
+            if (k == 1) raise = __builtin_amdgcn_ballot_w64(peak > top + (float)kLazy) != 0ull;
         };
-        // pair k / 4 of the weights: the two exponentials, then their hi and their lo halves
+        // pair k / 5 of the weights: the two exponentials, then their parts
         auto weigh_step = [&](int k) __attribute__((always_inline)) {
-            const int w = k / 4 * 2 + k % 4;
-            if (k % 4 < 2) {
-                s_cur[w] = fast_exp2(fmaf(s_cur[w], q_factor, neg_top));
-                part_sum += s_cur[w];
-                // (behind the sum: the exponential's result has been read once)
-                __asm__ volatile("" : "+v"(s_cur[w]), "+v"(part_sum));
-            } else if (k % 4 == 2) {
-                split_hi(s_cur[w - 2], s_cur[w - 1], weight_factor[k / 8], p_hi[k / 4]);
+            const int w = k / 5 * 2;
+            if (k % 5 < 2) {
+                float weight = fast_exp2(fmaf(s_cur[w + k % 5], q_factor, neg_top));
+                part_sum += weight;
+                __asm__ volatile("" : "+v"(weight), "+v"(part_sum));
+                s_cur[w + k % 5] = weight;
             } else {
-                split_lo(s_cur[w - 3], s_cur[w - 2], weight_factor[k / 8], p_hi[k / 4], p_lo[k / 4]);
+                float a = s_cur[w], b = s_cur[w + 1];
+                weights[k % 5 - 2][k / 5] = third(k % 5 - 2, a, b);
+                s_cur[w] = a;
+                s_cur[w + 1] = b;
             }
         };
-        constexpr int kSettled = 4;  // slots before the weights can be formed
+        constexpr int kSettled = 3;  // slots before the weights can be formed
         auto slot = [&](auto index) __attribute__((always_inline)) {
             constexpr int i = decltype(index)::value;
-            constexpr int m = (i % kHalfSlots) / 3, term = i % 3;
-            if constexpr (i < kHalfSlots) {
+            if constexpr (i < kScoreSlots) {
+                constexpr int m = i / 3, term = i % 3, n = 2 * m + (term != 0);
                 const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                s_next = mfma_32x32x16_f16(term == 0 ? lo[m % 2] : hi[m % 2], term == 1 ? q_lo[m] : q_hi[m],
+                s_next = mfma_32x32x16_f16(__builtin_bit_cast(halfx8, ring[n % kRing]), term == 1 ? q_lo[m] : q_hi[m],
                                            i == 0 ? zero : s_next);
+                if constexpr (term != 1) ring[n % kRing] = operand<n + kRing>(kNext, kAt);
             } else {
-                constexpr int first = m / kBlocks * 4;
-                u32x4 words;
-                if constexpr (term == 1)
-                    words = (u32x4){p_lo[first], p_lo[first + 1], p_lo[first + 2], p_lo[first + 3]};
-                else
-                    words = (u32x4){p_hi[first], p_hi[first + 1], p_hi[first + 2], p_hi[first + 3]};
-                out[m % kBlocks] = mfma_32x32x16_f16(term == 0 ? lo[m % 2] : hi[m % 2],
-                                                     __builtin_bit_cast(halfx8, words), out[m % kBlocks]);
+                // value and weight parts 3 1, 2 2, 2 1, 1 3, 1 2, 1 1
+                constexpr int m = (i - kScoreSlots) / 6, term = (i - kScoreSlots) % 6, first = m / kBlocks * 4;
+                constexpr int plane = term == 0 ? 0 : term < 3 ? 1 : 2, n = 2 * kSteps + 3 * m + plane;
+                constexpr int part = term == 0 ? 0 : term < 3 ? 2 - term : 5 - term;
+                const uint32_t(&w)[8] = weights[part];
+                out[m % kBlocks] = mfma_32x32x16(as_bf16x8(ring[n % kRing]),
+                                                 as_bf16x8((u32x4){w[first], w[first + 1], w[first + 2], w[first + 3]}),
+                                                 out[m % kBlocks]);
+                if constexpr ((term == 0 || term == 2 || term == 5) && n + kRing < kOperands)
+                    ring[n % kRing] = operand<n + kRing>(kNext, kAt);
             }
-            // the operands two steps on: of K(t+1), of V(t), and of K(t+2) for the next trip
-            if constexpr (term != 1) {
-                constexpr int n = m + 2 + (i < kHalfSlots ? 0 : kSteps);
-                halfx8 &into = (term == 0 ? lo : hi)[m % 2];
-                if constexpr (n < kSteps) into = key_operand(k_now, n, term == 0);
-                else if constexpr (n < 2 * kSteps) into = value_operand(kAt, n - kSteps, term == 0);
-                else into = key_operand(k_then, n - 2 * kSteps, term == 0);
-            }
-            if constexpr (i < kLoads) stage_keys(t + 3u, free_keys, i);
-            else if constexpr (i < 2 * kLoads) stage_values(t + 1u, kNext, i - kLoads);
-            ride<i, 4, 0, kSettled>(settle_step);
-            // the first eight weights before the update's first MFMA, the others before its second half, with
-            // two slots between a split and the MFMA that reads it
-            ride<i, 16, kSettled, kHalfSlots - 1>(weigh_step);
-            ride<i, 16, kHalfSlots - 1, 3 * kHalfSlots / 2 - 1>(
-                [&](int k) __attribute__((always_inline)) { weigh_step(16 + k); });
-            ride<i, 4, 3 * kHalfSlots / 2, kSlots>(
-                [&](int g) __attribute__((always_inline)) { peak_step(s_next, g, peak); });
+            if constexpr (i < kKeyLoads) stage_keys(t + 2u, kAt, i);
+            else if constexpr (i < kKeyLoads + kValueLoads) stage_values(t + 1u, kNext, i - kKeyLoads);
+            ride<i, 2, 0, 2>(settle_step);
+            // the first eight weights before the update's first MFMA, the others before its second half
+            ride<i, 20, kSettled, kScoreSlots>(weigh_step);
+            ride<i, 20, kScoreSlots, kScoreSlots + 6 * kBlocks - 1>(
+                [&](int k) __attribute__((always_inline)) { weigh_step(20 + k); });
+            ride<i, 4, kScoreSlots + 6 * kBlocks, kSlots>(
+                [&](int g) __attribute__((always_inline)) { peak_step(s_next, g, next_peak); });
             __builtin_amdgcn_sched_barrier(0);
         };
         __builtin_amdgcn_sched_barrier(0);
         for_each<kSettled>(slot);
-        if (raise || most > reference) adjust(c.peak, most);
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-            weight_factor[g] = power_of_two((uint32_t)max(127 + kWeightShift + e[g] - reference, 0));
+        if (raise) adjust(peak);
         __builtin_amdgcn_sched_barrier(0);
         for_each<kSlots, kSettled>(slot);
         sum += part_sum;
         if (t + 1u >= unmasked && t + 1u < wave_tiles) {
             mask(s_next, t + 1u);
-            peak = peak_of(s_next);
+            next_peak = peak_of(s_next);
         }
-        c.peak = peak * q_factor;
+        peak = next_peak * q_factor;
     }
 
     // Steps of a kind, spread over slots [kFrom, kTo).
@@ -309,8 +295,7 @@ struct GqaHalved {
         for (int s = 0; s < kSteps; ++s)
 #pragma unroll
             for (int j = 0; j < 8; ++j) most = fmaxf(most, fabsf(x[s][j / 4][j % 4]));
-        // (a row below 2^-62 as one of that size: q_factor stays a normal number)
-        const uint32_t e = max(group_exponent(__builtin_bit_cast(uint32_t, max_xor32(most))), 64u);
+        const uint32_t e = row_exponent(__builtin_bit_cast(uint32_t, max_xor32(most)));
         const float up = up_factor(e), unit = p.scale * YVEX_LOG2E;  // 2^x / 2^14, a score's log2 units
         // (NaN where the halves' floors could move a score: the row is then not finite, and is walked in fp32)
         q_factor = up * (unit * (1.f / Tile::kKeyFactor));
@@ -379,13 +364,11 @@ struct GqaHalved {
 
         const uint64_t head_bytes = (uint64_t)p.kv_tiles * Tile::kBytes;
         rsrc = raw_buffer(p.tiles + kv_head * head_bytes, (uint32_t)head_bytes);
-        factors = p.factors + (uint64_t)kv_head * p.kv_tiles * 8u;
         lds_base = (uint32_t)__builtin_amdgcn_readfirstlane((int)lds_address_of(lds.k[0]));
         k_unit = (uint32_t)(half * 32 + column) * 16u;
 #pragma unroll
         for (int b = 0; b < 2; ++b)
             v_unit[b] = (uint32_t)((half * kDim + Tile::value_unit(32 * b + column)) * 16 - b * 512);
-        reference = 0;
         top = -INFINITY;
         neg_top = 0.f;
         sum = 0.f;
@@ -401,8 +384,6 @@ struct GqaHalved {
         sum = sum_xor32(sum);
         // (a run none of whose keys the row sees leaves a maximum of -inf and nothing)
         bool good = isfinite(sum) && (partial && top == -INFINITY ? sum == 0.f : sum > 0.f && isfinite(top));
-        // the accumulators are relative to 2^(reference - 127), weights to 2^kWeightShift and values to 2^14
-        const int shift = reference - (141 + kWeightShift);
         const float inverse = 1.0f / sum;
         if (!partial) {
 #pragma unroll
@@ -413,11 +394,8 @@ struct GqaHalved {
 #pragma unroll
         for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                out[b][i] = __builtin_amdgcn_ldexpf(out[b][i], shift);
-                good &= isfinite(out[b][i]);
-            }
-        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.v[1]);  // a word of each wave, behind the rows
+            for (int i = 0; i < 16; ++i) good &= isfinite(out[b][i]);
+        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.v[2]) - 4;  // a word of each wave, behind the rows
         __syncthreads();  // the tiles in LDS are done with
         lay_rows_down();
         if (lane == 0) verdict[wave] = 0u;
@@ -464,7 +442,7 @@ struct GqaHalved {
     static constexpr uint32_t kUnits = kDim / 4;
     __device__ __forceinline__ floatx4 *laid_rows() const
     {
-        static_assert(4 * 32 * kDim * 4 <= offsetof(Shared, v[1]), "rows end before the verdicts");
+        static_assert(4 * 32 * kDim * 4 <= sizeof(Shared) - 16, "rows end before the verdicts");
         return reinterpret_cast<floatx4 *>(lds.k[0]) + (uint32_t)wave * 32u * kUnits;
     }
     __device__ __forceinline__ void lay_rows_down() const
@@ -492,50 +470,41 @@ struct GqaHalved {
     __device__ __forceinline__ void walk_tiles(uint32_t wave_tiles, uint32_t unmasked, const float *query)
     {
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) stage_keys(0u, 0u, j);
+        for (int j = 0; j < kKeyLoads; ++j) stage_keys(0u, 0, j);
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) stage_keys(1u, 1u, j);
+        for (int j = 0; j < kKeyLoads; ++j) stage_keys(1u, 1, j);
 #pragma unroll
-        for (int j = 0; j < kLoads; ++j) stage_values(0u, 0, j);
-        fetch_exponents(0u);
+        for (int j = 0; j < kValueLoads; ++j) stage_values(0u, 0, j);
         load_queries(query);
         __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < kLoads; ++j) stage_keys(2u, 2u, j);
         floatx16 s_even, s_odd;
 #pragma unroll
         for (int i = 0; i < 16; ++i) s_even[i] = 0.f;
 #pragma unroll
         for (int m = 0; m < kSteps; ++m) {
-            const halfx8 lo = key_operand(k_unit, m, 1), hi = key_operand(k_unit, m, 0);
+            const halfx8 lo = __builtin_bit_cast(halfx8, key_operand(0, m, 1));
+            const halfx8 hi = __builtin_bit_cast(halfx8, key_operand(0, m, 0));
             s_even = mfma_32x32x16_f16(lo, q_hi[m], s_even);
             s_even = mfma_32x32x16_f16(hi, q_lo[m], s_even);
             s_even = mfma_32x32x16_f16(hi, q_hi[m], s_even);
         }
-        Carried c;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            c.lo[k] = key_operand(k_unit + kTensor, k, 1);
-            c.hi[k] = key_operand(k_unit + kTensor, k, 0);
-        }
         if (unmasked == 0u) mask(s_even, 0u);
-        c.peak = peak_of(s_even) * q_factor;
-        key_buffer = 0u;
+        float peak = peak_of(s_even) * q_factor;
         // (two copies of a trip instead of three take less time to fetch: 1777 tokens 122 -> 118.5 us; at 256 the
         // compiler moves more registers about in that form: 1000 tokens 102 -> 116)
         uint32_t t = 0u;
         if constexpr (kDim == 256) {
             for (; t + 1u < tiles; t += 2u) {
-                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, c);
-                trip<1>(t + 1u, wave_tiles, unmasked, s_odd, s_even, c);
+                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
+                trip<1>(t + 1u, wave_tiles, unmasked, s_odd, s_even, peak);
             }
-            if (t < tiles) trip<0>(t, wave_tiles, unmasked, s_even, s_odd, c);
+            if (t < tiles) trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
         } else {
             for (;;) {
-                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, c);
+                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
                 if (++t == tiles) break;
-                trip<1>(t, wave_tiles, unmasked, s_odd, s_even, c);
+                trip<1>(t, wave_tiles, unmasked, s_odd, s_even, peak);
                 if (++t == tiles) break;
             }
         }

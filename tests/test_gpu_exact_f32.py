@@ -611,19 +611,13 @@ def test_gqa_split_beforehand_follows_magnitudes_and_views(backend, d):
         assert e.value.code == B.YVEX_ERR_FORMAT
 
 
-KEY_SPREADS = ("key-octet", "key-tile", "key-later", "key-later-tile", "excluded-early", "excluded-late",
-               "query-channel", "key-channel")
-
-
 @pytest.mark.parametrize("d", [64, 128, 256])
 @pytest.mark.parametrize("power", [8, 16, 24, 32, 40, 50])
 @pytest.mark.parametrize("tk", [500, 1500])
-def test_gqa_split_beforehand_holds_the_spread_of_keys_and_queries(backend, d, power, tk):
-    """A key or query row, or one dimension of them, of 2^8 to 2^50 among N(0,1) ones, seen, unseen or of weight zero:
-    as test_gqa_matrix_core_kernel_holds_the_spread, with the workspace, cut walks among them."""
+def test_gqa_split_beforehand_holds_the_spread(backend, d, power, tk):
+    """One row, channel or component of 2^8 to 2^50 among N(0,1) ones, seen, unseen or of weight zero, and sinks: as
+    test_gqa_matrix_core_kernel_holds_the_spread, with the workspace, cut walks among them."""
     for label, q, k, v, start in spread_cases(d, power, tk=tk):
-        if label not in KEY_SPREADS:
-            continue
         out, lse, facts, need = run_attached(backend, q, k, v, query_start=start)
         assert facts.kernel_launches == 3 and facts.temporary_bytes == need
         worst = relative_to_weighted_magnitudes(out, q, k, v, start)

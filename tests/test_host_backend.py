@@ -682,7 +682,7 @@ def test_exact_prefill_workspace_is_planned_and_offered(fake_runtime):
                 req = b.attention_requirement(tokens, keys, 4, 2, d, query_start=keys - tokens)
                 need = b.attention_workspace_required(req)
                 tiles = 2 * ((keys + 31) // 32)
-                halves = tiles * 256 * d + (tiles * 32 + 255) // 256 * 256
+                halves = tiles * 320 * d
                 assert need >= halves
                 launches = launches or (3 if need > halves else 2)
                 assert (launches == 3) == (need > halves)
