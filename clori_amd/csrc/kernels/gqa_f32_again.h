@@ -1,4 +1,4 @@
-// The fp32 walk of an item whose parts left the range: what gqa_f32_halved.h falls back to.
+// The fp32 walk of the rows of an item whose parts left the range: what gqa_f32_halved.h falls back to.
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
 #define YVEX_ROCM_KERNELS_GQA_F32_AGAIN_H
 
@@ -29,15 +29,23 @@ __device__ __forceinline__ void leave_partial(float *part_acc, float *part_ml, u
                 (floatx4){o[b][g * 4], o[b][g * 4 + 1], o[b][g * 4 + 2], o[b][g * 4 + 3]};
 }
 
-// The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  It takes
+// Row `row` of a tile, of which the bits of lower (rows 0 to 63) and upper (64 to 127) failed.
+__device__ __forceinline__ bool row_failed(uint64_t lower, uint64_t upper, uint32_t row)
+{
+    return ((row < 64u ? lower : upper) >> (row & 63u) & 1ull) != 0ull;
+}
+
+// The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  Only the rows
+// that failed (bits of `failed`, 32 rows to a word) are left: the others have been, and what a row gives does
+// not depend on whether another one fails.  It takes
 // the kernel's arguments from where they lie; `arguments` is the kernel's to find, a function that is called
 // is not given the place.
 typedef __attribute__((address_space(3))) unsigned char local_bytes;
 typedef __attribute__((address_space(4))) const yvex_rocm_gqa_f32_halved_params constant_params;
 template <int kDim>
-__device__ __forceinline__ void walk_again(constant_params *arguments, local_bytes *shared, bool cut, uint32_t slot_,
-                                           uint32_t row_head_, uint32_t tile_row_, uint32_t tile_end_,
-                                           uint32_t first_tile_, uint32_t tiles_)
+__device__ __forceinline__ void walk_again(constant_params *arguments, local_bytes *shared, u32x4 failed, bool cut,
+                                           uint32_t slot_, uint32_t row_head_, uint32_t tile_row_,
+                                           uint32_t tile_end_, uint32_t first_tile_, uint32_t tiles_)
 {
     auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
     const uint64_t at = (uint64_t)arguments;
@@ -46,6 +54,8 @@ __device__ __forceinline__ void walk_again(constant_params *arguments, local_byt
     const uint32_t tile_end = uniform(tile_end_), first_tile = uniform(first_tile_), tiles = uniform(tiles_);
     const bool partial = uniform(cut) != 0u;
     const uint32_t pack = p.walk.pack;
+    const uint64_t lower = (uint64_t)uniform(failed[1]) << 32 | uniform(failed[0]);
+    const uint64_t upper = (uint64_t)uniform(failed[3]) << 32 | uniform(failed[2]);
     yvex_rocm_gqa_f32_params f = {};
     f.q = (const float *)p.walk.q;
     f.k = (const float *)p.walk.k;
@@ -68,12 +78,16 @@ __device__ __forceinline__ void walk_again(constant_params *arguments, local_byt
     for (uint32_t h = 0u; h < pack; ++h) {
         // rows token * pack + h in [tile_row, tile_end)
         const uint32_t first = (tile_row + pack - 1u - h) / pack, end = (tile_end + pack - 1u - h) / pack;
-        if (first >= end) continue;
+        bool some = false;  // of the rows with this head (the same in every wave)
+        for (uint32_t row = threadIdx.x & 63u; row < (uint32_t)YVEX_ROCM_PREFILL_ROWS; row += 64u)
+            some |= row_failed(lower, upper, row) && (tile_row + row) % pack == h;
+        if (first >= end || __builtin_amdgcn_ballot_w64(some) == 0ull) continue;
         tile.walk(row_head * pack + h, first, end, first_tile, partial ? first_tile + tiles : ~0ull >> 8,
                   [&](uint64_t head, uint64_t token, floatx16(&o)[kDim / 32], float m, float l) {
+                      const uint32_t row = (uint32_t)token * pack + h - tile_row;
+                      if (!row_failed(lower, upper, row)) return;
                       if (partial)
-                          leave_partial(part_acc, part_ml, slot, (uint32_t)token * pack + h - tile_row, tile.half, o,
-                                        m * YVEX_LOG2E, l);
+                          leave_partial(part_acc, part_ml, slot, row, tile.half, o, m * YVEX_LOG2E, l);
                       else
                           tile.publish(head, token, o, m, l);
                   });
@@ -84,11 +98,11 @@ __device__ __forceinline__ void walk_again(constant_params *arguments, local_byt
 // The same as a function of its own: inlined, its registers are found by spilling the walk's (24/4 heads of 256,
 // 700 tokens 100 -> 85 us, 1000 112 -> 108; at 64, where they are there, the call costs 2 %).
 template <int kDim>
-__device__ __attribute__((noinline)) void walk_again_apart(constant_params *arguments, local_bytes *shared, bool cut,
-                                                           uint32_t slot, uint32_t row_head, uint32_t tile_row,
-                                                           uint32_t tile_end, uint32_t first_tile, uint32_t tiles)
+__device__ __attribute__((noinline)) void
+walk_again_apart(constant_params *arguments, local_bytes *shared, u32x4 failed, bool cut, uint32_t slot,
+                 uint32_t row_head, uint32_t tile_row, uint32_t tile_end, uint32_t first_tile, uint32_t tiles)
 {
-    walk_again<kDim>(arguments, shared, cut, slot, row_head, tile_row, tile_end, first_tile, tiles);
+    walk_again<kDim>(arguments, shared, failed, cut, slot, row_head, tile_row, tile_end, first_tile, tiles);
 }
 
 }  // namespace

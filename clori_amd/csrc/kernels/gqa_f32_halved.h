@@ -168,11 +168,12 @@ struct GqaHalved {
                          : "v"(s[4 * g]), "v"(s[4 * g + 1]), "v"(s[4 * g + 2]), "v"(s[4 * g + 3]));
     }
 
-    // Brings the maximum to the peak of a tile (over both halves of a row) that exceeds it by more than
-    // 2^kLazy in some row.
+    // Brings the maximum of the rows where a tile's peak (over both halves of a row) exceeds it by more than
+    // 2^kLazy to that peak.  The other rows of the wave keep theirs, bit for bit: what a row gives
+    // does not depend on the rows beside it.
     __device__ __forceinline__ void adjust(float peak)
     {
-        const float raised = fmaxf(top, peak);
+        const float raised = peak > top + (float)kLazy ? peak : top;
         // a row that has seen nothing yet keeps the maximum -inf
         const float keep = raised == -INFINITY ? 1.f : fast_exp2(top - raised);
         sum *= keep;
@@ -395,44 +396,44 @@ struct GqaHalved {
         for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
             for (int i = 0; i < 16; ++i) good &= isfinite(out[b][i]);
-        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.v[2]) - 4;  // a word of each wave, behind the rows
+        // the rows of every wave that are left to the fp32 walk, as bits: a word of each wave, behind the rows
+        uint32_t *verdict = reinterpret_cast<uint32_t *>(lds.v[2]) - 4;
+        const uint64_t bad = __builtin_amdgcn_ballot_w64(own && !good);
+        const uint32_t failed = (uint32_t)bad | (uint32_t)(bad >> 32);
         __syncthreads();  // the tiles in LDS are done with
         lay_rows_down();
-        if (lane == 0) verdict[wave] = 0u;
-        if (own && !good) verdict[wave] = 1u;
+        if (lane == 0) verdict[wave] = failed;
         __syncthreads();
         const u32x4 verdicts = *reinterpret_cast<u32x4 *>(verdict);
-        const bool failed = (verdicts[0] | verdicts[1] | verdicts[2] | verdicts[3]) != 0u;
         const uint32_t slot = partial ? (item - w.whole_items) * w.splits + split : 0u;
-        if (failed) {
-            __syncthreads();  // every wave has read the verdict
-            local_bytes *shared = (local_bytes *)(void *)&lds;
-            constant_params *arguments = (constant_params *)__builtin_amdgcn_kernarg_segment_ptr();
-            if constexpr (kDim == 64)
-                walk_again<kDim>(arguments, shared, partial, slot, row_head, tile_row, tile_end, first_tile, tiles);
-            else
-                walk_again_apart<kDim>(arguments, shared, partial, slot, row_head, tile_row, tile_end, first_tile,
-                                       tiles);
-            return;
-        }
-        if (row0 >= w.rows) return;
-        if (partial) {
+        const bool leave = own && half == 0 && (failed >> column & 1u) == 0u;
+        if (row0 < w.rows && partial) {
             const uint64_t first = (uint64_t)slot * kRows + (row0 - tile_row);
-            publish_rows(row0, [&](uint32_t, uint32_t r) { return w.part_acc + (first + r) * kDim; });
-            if (own && half == 0) {
+            publish_rows(row0, failed, [&](uint32_t, uint32_t r) { return w.part_acc + (first + r) * kDim; });
+            if (leave) {
                 float *ml = w.part_ml + 2u * (first + (uint32_t)column);
                 ml[0] = top;
                 ml[1] = sum;
             }
-            return;
+        } else if (row0 < w.rows) {
+            publish_rows(row0, failed, [&](uint32_t row_, uint32_t) {
+                const uint32_t token_ = token_of(w, row_);
+                return (float *)w.out +
+                       ((uint64_t)token_ * w.query_heads + (row_head * w.pack + (row_ - token_ * w.pack))) * kDim;
+            });
+            if (leave && w.lse) w.lse[(uint64_t)token * w.query_heads + head] = top * YVEX_LN2 + logf(sum);
         }
-        publish_rows(row0, [&](uint32_t row_, uint32_t) {
-            const uint32_t token_ = token_of(w, row_);
-            return (float *)w.out +
-                   ((uint64_t)token_ * w.query_heads + (row_head * w.pack + (row_ - token_ * w.pack))) * kDim;
-        });
-        if (own && w.lse && half == 0)
-            w.lse[(uint64_t)token * w.query_heads + head] = top * YVEX_LN2 + logf(sum);
+        if ((verdicts[0] | verdicts[1] | verdicts[2] | verdicts[3]) != 0u) {
+            __syncthreads();  // every wave is done with the rows and the verdicts
+            local_bytes *shared = (local_bytes *)(void *)&lds;
+            constant_params *arguments = (constant_params *)__builtin_amdgcn_kernarg_segment_ptr();
+            if constexpr (kDim == 64)
+                walk_again<kDim>(arguments, shared, verdicts, partial, slot, row_head, tile_row, tile_end, first_tile,
+                                 tiles);
+            else
+                walk_again_apart<kDim>(arguments, shared, verdicts, partial, slot, row_head, tile_row, tile_end,
+                                       first_tile, tiles);
+        }
     }
 
     // The wave's 32 rows go through its part of LDS, 16-byte units of a row dealt by its number so that
@@ -456,14 +457,15 @@ struct GqaHalved {
                     (floatx4){out[b][4 * g], out[b][4 * g + 1], out[b][4 * g + 2], out[b][4 * g + 3]};
     }
     template <typename To>
-    __device__ __forceinline__ void publish_rows(uint32_t row0, const To &to) const
+    __device__ __forceinline__ void publish_rows(uint32_t row0, uint32_t failed, const To &to) const
     {
         const floatx4 *rows = laid_rows();
 #pragma unroll
         for (uint32_t i = 0; i < kUnits / 2u; ++i) {
             const uint32_t r = (i * 64u + (uint32_t)lane) / kUnits, unit = (i * 64u + (uint32_t)lane) % kUnits;
             const floatx4 x = rows[r * kUnits + (unit ^ (r & 15u))];
-            if (row0 + r < p.walk.rows) *reinterpret_cast<floatx4 *>(to(row0 + r, r) + 4u * unit) = x;
+            if (row0 + r < p.walk.rows && (failed >> r & 1u) == 0u)
+                *reinterpret_cast<floatx4 *>(to(row0 + r, r) + 4u * unit) = x;
         }
     }
 
