@@ -15,9 +15,14 @@
 
 enum {
     HALVED_STEP_KEYS = 32,
+    HALVED_KEYS_MIN = 64,
     HALVED_GROUP_MAX = 16 /* query heads packed into the rows of a tile */
 };
-#define HALVED_TILES_MAX (640ull << 20) /* bytes of parts a request may ask for */
+/* Bytes of parts a request may ask for: a quarter more than the F32 rows that they are made from.  The offsets of a
+ * kv head's tiles are 32-bit ones; 2 GiB, 209715 keys of 8 kv heads of 128, keeps them below 2^31.  A request past it
+ * runs in one launch, which takes 6 (300 tokens behind 60000: 8.5 ms, with the workspace 1.4) to 17 times
+ * as long (64 tokens: 8.4 ms, 0.50). */
+#define HALVED_TILES_MAX (2ull << 30)
 
 typedef struct {
     yvex_rocm_walk_plan walk;
@@ -31,13 +36,13 @@ static unsigned long long visible_keys(const yvex_transformer_attention_requirem
                                                              : r->key_value_tokens;
 }
 
-/* Returns 0 when the request is not for these kernels.  Walks of fewer than d + 192 keys stay with the one
- * launch: the launch that splits, and a workgroup's longer start, cost more than they save.  With the
- * workspace / without, us: 40/8 heads of 128, 200 tokens 24.2 / 23.7, 330 26.5 / 31.5, 400 28 / 35, 1777
- * 116 / 142, 4096 461 / 640, 32 behind 200 24.9 / 23.8, 32 behind 290 20.8 / 28.6, 32 behind 4000 45 / 271, 300
- * behind 5000 125 / 316; 16/4 of 64, 100 12.2 / 12.5, 200 14.7 / 15.6, 32 behind 100 13.6 / 12.2, 32 behind 230
- * 16.1 / 17.0, 1000 35.4 / 44.8; 24/4 of 256, 300 53 / 47, 450 57 / 64, 500 61 / 74, 32 behind 420 33 / 60,
- * 1000 101 / 130, 64 behind 20000 175 / 2003. */
+/* Returns 0 when the request is not for these kernels.  Walks of fewer than 64 keys stay with the one launch: the
+ * launch that splits, and a workgroup's longer start, cost more than they save.  With the workspace / without,
+ * us: 40/8 heads of 128, 32 tokens 13.2 / 10.9, 64 15.1 / 16.1, 32 behind 32 14.8 / 15.5, 100 17.7 / 25.7, 200 22.3 /
+ * 39.4, 330 28.8 / 58.0, 1777 142 / 310, 4096 596 / 1418, 32 behind 200 23.1 / 42.7, 32 behind 4000 42 / 573, 300
+ * behind 5000 146 / 764; 16/4 of 64, 32 9.1 / 7.4, 64 10.4 / 10.3, 32 behind 32 10.2 / 9.9, 32 behind 64 11.1 / 12.4,
+ * 200 13.9 / 23.3, 1000 37.0 / 88.3; 24/4 of 256, 32 22.0 / 16.4, 64 25.3 / 25.9, 32 behind 32 25.2 / 25.1, 32 behind 64
+ * 28.0 / 33.6, 200 38 / 69, 1000 120 / 289, 64 behind 20000 206 / 5288. */
 static int halved_plan_make(const yvex_transformer_attention_requirement *r, halved_plan *plan)
 {
     const unsigned long long d = r->head_dimension, group = r->query_heads / r->key_value_heads;
@@ -48,7 +53,7 @@ static int halved_plan_make(const yvex_transformer_attention_requirement *r, hal
         r->key_value_tokens > (1ull << 30) || ((r->key_token_stride | r->value_token_stride) >> 24) != 0ull ||
         (r->key_value_heads * d >> 24) != 0ull)
         return 0;
-    if (visible_keys(r) < d + 192ull) return 0;
+    if (visible_keys(r) < HALVED_KEYS_MIN) return 0;
     plan->kv_tiles = (visible_keys(r) + HALVED_STEP_KEYS - 1ull) / HALVED_STEP_KEYS;
     plan->tile_bytes = r->key_value_heads * plan->kv_tiles * 320ull * d;
     if (plan->tile_bytes > HALVED_TILES_MAX) return 0;

@@ -529,6 +529,8 @@ def run_attached(backend, q, k, v, short=0, **kw):
 
 
 @pytest.mark.parametrize("tq,tk,hq,hkv,d,start,causal", [
+    (32, 64, 4, 2, 128, 32, True), (64, 64, 3, 1, 64, 0, True), (33, 65, 2, 1, 256, 32, True),
+    (95, 96, 5, 1, 64, 0, False),
     (33, 320, 4, 1, 128, 287, True), (129, 385, 10, 2, 128, 256, True), (1000, 1000, 5, 1, 128, 0, True),
     (40, 3001, 10, 2, 128, 2950, True), (64, 799, 3, 3, 128, 0, False), (520, 1040, 40, 8, 128, 520, True),
     (32, 256, 6, 2, 64, 224, True), (1300, 1300, 16, 4, 64, 0, True), (77, 9000, 7, 1, 64, 8923, True),

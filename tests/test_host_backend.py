@@ -675,7 +675,7 @@ def test_exact_prefill_workspace_is_planned_and_offered(fake_runtime):
     three launches, one byte short, or absent, in one that allocates nothing."""
     with Backend() as b:
         for d in (64, 128, 256):
-            shortest = d + 192
+            shortest = 64
             assert b.attention_workspace_required(
                 b.attention_requirement(32, shortest - 1, 4, 2, d, query_start=shortest - 33)) == 0
             for tokens, keys, launches in ((32, shortest, None), (32, 6000, 3), (8192, 8192, 2)):
