@@ -41,8 +41,8 @@ static unsigned long long visible_keys(const yvex_transformer_attention_requirem
  * us: 40/8 heads of 128, 32 tokens 13.2 / 10.9, 64 15.1 / 16.1, 32 behind 32 14.8 / 15.5, 100 17.7 / 25.7, 200 22.3 /
  * 39.4, 330 28.8 / 58.0, 1777 142 / 310, 4096 596 / 1418, 32 behind 200 23.1 / 42.7, 32 behind 4000 42 / 573, 300
  * behind 5000 146 / 764; 16/4 of 64, 32 9.1 / 7.4, 64 10.4 / 10.3, 32 behind 32 10.2 / 9.9, 32 behind 64 11.1 / 12.4,
- * 200 13.9 / 23.3, 1000 37.0 / 88.3; 24/4 of 256, 32 22.0 / 16.4, 64 25.3 / 25.9, 32 behind 32 25.2 / 25.1, 32 behind 64
- * 28.0 / 33.6, 200 38 / 69, 1000 120 / 289, 64 behind 20000 206 / 5288. */
+ * 200 13.9 / 23.3, 1000 37.0 / 88.3; 24/4 of 256, 32 22.0 / 16.4, 64 25.3 / 25.9, 32 behind 32 25.2 / 25.1, 32 behind
+ * 64 28.0 / 33.6, 200 38 / 69, 1000 120 / 289, 64 behind 20000 206 / 5288. */
 static int halved_plan_make(const yvex_transformer_attention_requirement *r, halved_plan *plan)
 {
     const unsigned long long d = r->head_dimension, group = r->query_heads / r->key_value_heads;
