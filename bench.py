@@ -41,7 +41,8 @@ from clori_amd.backend import Backend, kv_pack_pages, q8_0_encode_rows  # noqa: 
 
 HBM_PEAK_GBS = 8000.0        # MI355X HBM3E, published
 MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16, published
-MFMA_F32_SPLIT_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 3    # an F32 product is three f16 products
+# an F32 product is three f16 products in the scores and six bf16 ones in the update, half of the products each
+MFMA_F32_SPLIT_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 4.5
 
 
 def bf16_bits(x):
@@ -264,7 +265,7 @@ def workload_prefill2(backend, rng, steps, warmup, hq=40, hkv=8, d=128, name="pr
 
 
 def workload_exact2(backend, rng, steps, warmup, hq=40, hkv=8, d=128, name="exact2"):
-    """Configuration 2 under the EXACT_F32 contract (F32 tensors, F32 products): the request
+    """Configuration 2 under the EXACT_F32 contract (F32 tensors, F32 precision): the request
     the reference's engine makes.  Not one of the metric's configurations: run by name."""
     t = 2048
     q = backend.tensor("q", B.DTYPE_F32, (t, hq, d), rng.standard_normal((t, hq, d), dtype=np.float32))
@@ -276,7 +277,7 @@ def workload_exact2(backend, rng, steps, warmup, hq=40, hkv=8, d=128, name="exac
     backend.workspace_attach(work)
     run = lambda: backend.attention_execute(req, q, k, v, out)  # noqa: E731
     facts = run()
-    # keys and values split into f16 halves, the walk, and for items that were cut the merge
+    # keys and values split into 16-bit parts, the walk, and for items that were cut the merge
     kernels = ["yvex_rocm_gqa_f32_%s_%d" % (part, d) for part in
                ("halved", "halve", "merge")[:int(facts.kernel_launches)]]
     timed = time_steps(backend, run, steps, warmup, kernels)
