@@ -51,7 +51,7 @@ static unsigned long long item_steps(const yvex_transformer_attention_requiremen
 static unsigned long long tail_cost(const yvex_transformer_attention_requirement *r, const yvex_rocm_walk_plan *plan,
                                     unsigned long long steps, unsigned long long splits)
 {
-    /* 0.9 us for a 128-row step at 128, of 64 keys in bf16 and of 32 with F32 products as three */
+    /* 0.9 us for a 128-row step of 64 keys at 128 in bf16; walks over F32 parts (32 keys) are cut alike */
     const unsigned long long step_ns = 7ull * r->head_dimension;
     const unsigned long long turns = (plan->tail_items * splits + PREFILL_UNITS - 1ull) / PREFILL_UNITS;
     const unsigned long long live = plan->rows < YVEX_ROCM_PREFILL_ROWS ? plan->rows : YVEX_ROCM_PREFILL_ROWS;

@@ -37,15 +37,16 @@ __device__ __forceinline__ bool row_failed(uint64_t lower, uint64_t upper, uint3
 
 // The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  Only the rows
 // that failed (bits of `failed`, 32 rows to a word) are left: the others have been, and what a row gives does
-// not depend on whether another one fails.  It takes
-// the kernel's arguments from where they lie; `arguments` is the kernel's to find, a function that is called
-// is not given the place.
+// not depend on whether another one fails.  A function of its own, whose registers are not found by spilling
+// the walk's (64 tokens behind 20000 at 24/4 heads of 256 209 us, inlined 211 to 215; the others alike).  It takes the
+// kernel's arguments from where they lie; `arguments` is the kernel's to find, a function that is called is not
+// given the place.
 typedef __attribute__((address_space(3))) unsigned char local_bytes;
 typedef __attribute__((address_space(4))) const yvex_rocm_gqa_f32_halved_params constant_params;
 template <int kDim>
-__device__ __forceinline__ void walk_again(constant_params *arguments, local_bytes *shared, u32x4 failed, bool cut,
-                                           uint32_t slot_, uint32_t row_head_, uint32_t tile_row_,
-                                           uint32_t tile_end_, uint32_t first_tile_, uint32_t tiles_)
+__device__ __attribute__((noinline)) void
+walk_again(constant_params *arguments, local_bytes *shared, u32x4 failed, bool cut, uint32_t slot_, uint32_t row_head_,
+           uint32_t tile_row_, uint32_t tile_end_, uint32_t first_tile_, uint32_t tiles_)
 {
     auto uniform = [](uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); };
     const uint64_t at = (uint64_t)arguments;
@@ -93,16 +94,6 @@ __device__ __forceinline__ void walk_again(constant_params *arguments, local_byt
                   });
         __syncthreads();  // every wave is done with the tiles in LDS
     }
-}
-
-// The same as a function of its own: inlined, its registers are found by spilling the walk's (24/4 heads of 256,
-// 700 tokens 100 -> 85 us, 1000 112 -> 108; at 64, where they are there, the call costs 2 %).
-template <int kDim>
-__device__ __attribute__((noinline)) void
-walk_again_apart(constant_params *arguments, local_bytes *shared, u32x4 failed, bool cut, uint32_t slot,
-                 uint32_t row_head, uint32_t tile_row, uint32_t tile_end, uint32_t first_tile, uint32_t tiles)
-{
-    walk_again<kDim>(arguments, shared, failed, cut, slot, row_head, tile_row, tile_end, first_tile, tiles);
 }
 
 }  // namespace

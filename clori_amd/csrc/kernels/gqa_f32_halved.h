@@ -30,11 +30,10 @@
 // hold no rows on their way, and a trip is bound by its MFMAs.  Items, packed rows and runs of keys are those of
 // the bf16 prefill (kernel_params.h), with steps of 32 keys.
 //
-// What bounds the walk is power: 4096 tokens of 40/8 heads of 128 run at 1.66 GHz with the matrix cores busy
-// 62 % of the cycles, 1.1 PFLOP/s of f16 products (a large bf16 product reaches 1.29 on this part), 373
-// TFLOP/s of F32 ones; 1777 tokens 108 of 116 us.  Trips that prefetch their first operands across the barrier, and
-// peaks without canonical forms, made no difference there (122 against 121 us), which is why no more is
-// hidden: at 256, one wave per SIMD, they did (1000 tokens 120 -> 112 us, now 101).
+// What bounds the walk is power.  At 128 it runs at 1.55 to 1.57 GHz with the matrix cores busy 72 to 74 % of the
+// cycles: 1777 tokens of 40/8 heads 129 of 140 us, 2048 tokens 162 of 171, 265 TFLOP/s of F32 products, 1.19 PFLOP/s
+// of 16-bit ones, where a large bf16 product reaches 1.29 on this part.  At 256, one wave per SIMD, 1.95 GHz and
+// 51 %: the first operands of a trip come behind its barrier (2048 tokens of 24/4 heads 227 of 236 us).
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 #define YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 
@@ -427,12 +426,8 @@ struct GqaHalved {
             __syncthreads();  // every wave is done with the rows and the verdicts
             local_bytes *shared = (local_bytes *)(void *)&lds;
             constant_params *arguments = (constant_params *)__builtin_amdgcn_kernarg_segment_ptr();
-            if constexpr (kDim == 64)
-                walk_again<kDim>(arguments, shared, verdicts, partial, slot, row_head, tile_row, tile_end, first_tile,
-                                 tiles);
-            else
-                walk_again_apart<kDim>(arguments, shared, verdicts, partial, slot, row_head, tile_row, tile_end,
-                                       first_tile, tiles);
+            walk_again<kDim>(arguments, shared, verdicts, partial, slot, row_head, tile_row, tile_end, first_tile,
+                             tiles);
         }
     }
 
@@ -493,22 +488,13 @@ struct GqaHalved {
         }
         if (unmasked == 0u) mask(s_even, 0u);
         float peak = peak_of(s_even) * q_factor;
-        // (two copies of a trip instead of three take less time to fetch: 1777 tokens 122 -> 118.5 us; at 256 the
-        // compiler moves more registers about in that form: 1000 tokens 102 -> 116)
-        uint32_t t = 0u;
-        if constexpr (kDim == 256) {
-            for (; t + 1u < tiles; t += 2u) {
-                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
-                trip<1>(t + 1u, wave_tiles, unmasked, s_odd, s_even, peak);
-            }
-            if (t < tiles) trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
-        } else {
-            for (;;) {
-                trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
-                if (++t == tiles) break;
-                trip<1>(t, wave_tiles, unmasked, s_odd, s_even, peak);
-                if (++t == tiles) break;
-            }
+        // (two copies of a trip; a third for an odd last tile takes as long: 139 to 142 us at 1777 tokens of 128, 119
+        // at 1000 of 256)
+        for (uint32_t t = 0u;;) {
+            trip<0>(t, wave_tiles, unmasked, s_even, s_odd, peak);
+            if (++t == tiles) break;
+            trip<1>(t, wave_tiles, unmasked, s_odd, s_even, peak);
+            if (++t == tiles) break;
         }
         // nothing may still be in flight into LDS
         __builtin_amdgcn_s_waitcnt(0x0f70);
