@@ -119,15 +119,16 @@ struct GqaHalved {
         return *reinterpret_cast<const u32x4 *>(lds.v[buf] + v_unit[b & 1] + u * kDim * 32 + b * 512 +
                                                 plane * kPlane);
     }
-    // Operand n of a trip: lo and hi of a step of S^T from the last plane on, then the three planes of a step of the
-    // update, likewise.
+    // Operand n of a trip: lo and hi of the steps of S^T, hi of them once more, then the three planes of a step of the
+    // update from the last on.
     template <int n>
     __device__ __forceinline__ u32x4 operand(int k_buf, int v_buf) const
     {
         if constexpr (n < 2 * kSteps) return key_operand(k_buf, n / 2, 1 - n % 2);
-        else return value_operand(v_buf, (n - 2 * kSteps) / 3, 2 - (n - 2 * kSteps) % 3);
+        else if constexpr (n < kScoreSlots) return key_operand(k_buf, n - 2 * kSteps, 0);
+        else return value_operand(v_buf, (n - kScoreSlots) / 3, 2 - (n - kScoreSlots) % 3);
     }
-    static constexpr int kOperands = 2 * kSteps + 3 * 2 * kBlocks;
+    static constexpr int kOperands = kScoreSlots + 3 * 2 * kBlocks;
 
     // Step `part` (0, 1, 2) of the split of two F32 values into three bf16 values each: the nearest of what is left.
     __device__ static __forceinline__ uint32_t third(int part, float &a, float &b)
@@ -233,15 +234,18 @@ struct GqaHalved {
         auto slot = [&](auto index) __attribute__((always_inline)) {
             constexpr int i = decltype(index)::value;
             if constexpr (i < kScoreSlots) {
-                constexpr int m = i / 3, term = i % 3, n = 2 * m + (term != 0);
+                // lo hi and hi lo of all steps while the sum is small, then hi hi: a third of the roundings that count
+                // (2-norm from 64 bits, 24/4 heads of 256: 100 tokens 2.9e-7 -> 2.0e-7, fp32 walk 2.7e-7; 1000 tokens
+                // 4.4e-7 -> 3.3e-7, 4.6e-7; for an operand more to read a step, 119 -> 120 us)
+                constexpr int m = i < 2 * kSteps ? i / 2 : i - 2 * kSteps;
                 const floatx16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                s_next = mfma_32x32x16_f16(__builtin_bit_cast(halfx8, ring[n % kRing]), term == 1 ? q_lo[m] : q_hi[m],
-                                           i == 0 ? zero : s_next);
-                if constexpr (term != 1) ring[n % kRing] = operand<n + kRing>(kNext, kAt);
+                s_next = mfma_32x32x16_f16(__builtin_bit_cast(halfx8, ring[i % kRing]),
+                                           i < 2 * kSteps && i % 2 != 0 ? q_lo[m] : q_hi[m], i == 0 ? zero : s_next);
+                ring[i % kRing] = operand<i + kRing>(kNext, kAt);
             } else {
                 // value and weight parts 3 1, 2 2, 2 1, 1 3, 1 2, 1 1
                 constexpr int m = (i - kScoreSlots) / 6, term = (i - kScoreSlots) % 6, first = m / kBlocks * 4;
-                constexpr int plane = term == 0 ? 0 : term < 3 ? 1 : 2, n = 2 * kSteps + 3 * m + plane;
+                constexpr int plane = term == 0 ? 0 : term < 3 ? 1 : 2, n = kScoreSlots + 3 * m + plane;
                 constexpr int part = term == 0 ? 0 : term < 3 ? 2 - term : 5 - term;
                 const uint32_t(&w)[8] = weights[part];
                 out[m % kBlocks] = mfma_32x32x16(as_bf16x8(ring[n % kRing]),
@@ -480,12 +484,12 @@ struct GqaHalved {
         for (int i = 0; i < 16; ++i) s_even[i] = 0.f;
 #pragma unroll
         for (int m = 0; m < kSteps; ++m) {
-            const halfx8 lo = __builtin_bit_cast(halfx8, key_operand(0, m, 1));
-            const halfx8 hi = __builtin_bit_cast(halfx8, key_operand(0, m, 0));
-            s_even = mfma_32x32x16_f16(lo, q_hi[m], s_even);
-            s_even = mfma_32x32x16_f16(hi, q_lo[m], s_even);
-            s_even = mfma_32x32x16_f16(hi, q_hi[m], s_even);
+            s_even = mfma_32x32x16_f16(__builtin_bit_cast(halfx8, key_operand(0, m, 1)), q_hi[m], s_even);
+            s_even = mfma_32x32x16_f16(__builtin_bit_cast(halfx8, key_operand(0, m, 0)), q_lo[m], s_even);
         }
+#pragma unroll
+        for (int m = 0; m < kSteps; ++m)
+            s_even = mfma_32x32x16_f16(__builtin_bit_cast(halfx8, key_operand(0, m, 0)), q_hi[m], s_even);
         if (unmasked == 0u) mask(s_even, 0u);
         float peak = peak_of(s_even) * q_factor;
         // (two copies of a trip; a third for an odd last tile takes as long: 139 to 142 us at 1777 tokens of 128, 119

@@ -638,6 +638,29 @@ def test_gqa_split_beforehand_holds_the_spread_in_whole_walks(backend, d, hq, hk
         assert worst < spread_bound(label, d), (label, worst)
 
 
+@pytest.mark.parametrize("tq,start,hq,hkv,d", [
+    (100, 0, 24, 4, 256), (500, 0, 12, 2, 256), (70, 1500, 12, 2, 256), (100, 0, 10, 2, 128), (500, 0, 10, 2, 128),
+    (70, 1500, 10, 2, 128), (100, 0, 8, 2, 64), (500, 0, 8, 2, 64), (70, 1500, 8, 2, 64)])
+def test_gqa_split_beforehand_is_no_further_from_64_bits(backend, tq, start, hq, hkv, d):
+    """The distance from 64 bits, in the 2-norm, of the walk over parts is smaller than that of the fp32 walk: its sums
+    take fewer roundings (seen: 0.3 to 0.75 of it)."""
+    rng = np.random.default_rng(tq + start + d)
+    tk = start + tq
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((tq, hq, d), (tk, hkv, d), (tk, hkv, d)))
+    q *= rng.uniform(0.5, 1.5, hq).astype(np.float32)[None, :, None]
+    attached = run_attached(backend, q, k, v, query_start=start)[0]
+    one = run_exact(backend, q, k, v, query_start=start)[0]
+    apart = []
+    for head in range(hq):
+        scores = q[:, head].astype(np.float64) @ k[:, head // (hq // hkv)].astype(np.float64).T / math.sqrt(d)
+        scores[np.arange(tk)[None, :] > (start + np.arange(tq))[:, None]] = -np.inf
+        weights = np.exp(scores - scores.max(axis=1, keepdims=True))
+        want = weights / weights.sum(axis=1, keepdims=True) @ v[:, head // (hq // hkv)].astype(np.float64)
+        apart.append([((got[:, head] - want) ** 2).sum() for got in (attached, one)])
+    of_parts, of_fp32 = np.sqrt(np.sum(apart, axis=0))
+    assert of_parts <= 0.9 * of_fp32, (of_parts, of_fp32)
+
+
 @pytest.mark.parametrize("d,hq,hkv", [(64, 5, 1), (128, 6, 2), (256, 4, 2)])
 @pytest.mark.parametrize("tq,start", [(600, 0), (70, 2000)])
 @pytest.mark.parametrize("form", ["attached", "one launch"])
