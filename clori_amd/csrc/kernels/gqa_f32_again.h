@@ -35,9 +35,11 @@ __device__ __forceinline__ bool row_failed(uint64_t lower, uint64_t upper, uint3
     return ((row < 64u ? lower : upper) >> (row & 63u) & 1ull) != 0ull;
 }
 
-// The item, or the run, once more in fp32: head by head, the tokens whose rows lie in the tile.  Only the rows
-// that failed (bits of `failed`, 32 rows to a word) are left: the others have been, and what a row gives does
-// not depend on whether another one fails.  A function of its own, whose registers are not found by spilling
+// The item, or the run, once more in fp32, its rows packed as they are.  Only the rows that failed (bits of
+// `failed`, 32 rows to a word) are left: the others have been, and what a row gives does
+// not depend on whether another one fails.  Head by head, with the tokens of a head in its tiles, it took
+// as many walks as heads share a tile (every row failed, 1777 tokens of 40/8 heads of 128 1420 us, 1000 of 24/4 of 256
+// 2260; now 424 and 447, in one launch 313 and 291).  A function of its own, whose registers are not found by spilling
 // the walk's (64 tokens behind 20000 at 24/4 heads of 256 209 us, inlined 211 to 215; the others alike).  It takes the
 // kernel's arguments from where they lie; `arguments` is the kernel's to find, a function that is called is not
 // given the place.
@@ -76,24 +78,23 @@ walk_again(constant_params *arguments, local_bytes *shared, u32x4 failed, bool c
     f.causal = (int32_t)p.walk.causal;
     float *const part_acc = p.walk.part_acc, *const part_ml = p.walk.part_ml;
     const GqaTile<kDim / 32> tile(f, (float *)(unsigned char *)shared, (int)threadIdx.x);
-    for (uint32_t h = 0u; h < pack; ++h) {
-        // rows token * pack + h in [tile_row, tile_end)
-        const uint32_t first = (tile_row + pack - 1u - h) / pack, end = (tile_end + pack - 1u - h) / pack;
-        bool some = false;  // of the rows with this head (the same in every wave)
-        for (uint32_t row = threadIdx.x & 63u; row < (uint32_t)YVEX_ROCM_PREFILL_ROWS; row += 64u)
-            some |= row_failed(lower, upper, row) && (tile_row + row) % pack == h;
-        if (first >= end || __builtin_amdgcn_ballot_w64(some) == 0ull) continue;
-        tile.walk(row_head * pack + h, first, end, first_tile, partial ? first_tile + tiles : ~0ull >> 8,
-                  [&](uint64_t head, uint64_t token, floatx16(&o)[kDim / 32], float m, float l) {
-                      const uint32_t row = (uint32_t)token * pack + h - tile_row;
-                      if (!row_failed(lower, upper, row)) return;
-                      if (partial)
-                          leave_partial(part_acc, part_ml, slot, row, tile.half, o, m * YVEX_LOG2E, l);
-                      else
-                          tile.publish(head, token, o, m, l);
-                  });
-        __syncthreads();  // every wave is done with the tiles in LDS
-    }
+    // the rows as they are packed; a wave without one that failed only stages (its lanes' words are the same)
+    const uint64_t word = tile.wave < 2 ? lower : upper;
+    const bool idle = (uint32_t)(tile.wave % 2 == 0 ? word : word >> 32) == 0u;
+    typedef typename GqaTile<kDim / 32>::Place Place;
+    tile.walk(row_head * pack / (p.walk.query_heads / p.walk.kv_heads), tile_end - tile_row, idle,
+              [&](uint32_t row) {
+                  const uint32_t token = (tile_row + row) / pack;
+                  return Place{token, row_head * pack + (tile_row + row - token * pack)};
+              },
+              first_tile, partial ? first_tile + tiles : ~0ull >> 8,
+              [&](const Place &place, uint32_t row, floatx16(&o)[kDim / 32], float m, float l) {
+                  if (!row_failed(lower, upper, row)) return;
+                  if (partial)
+                      leave_partial(part_acc, part_ml, slot, row, tile.half, o, m * YVEX_LOG2E, l);
+                  else
+                      tile.publish(place.head, place.token, o, m, l);
+              });
 }
 
 }  // namespace

@@ -138,37 +138,45 @@ struct GqaTile {
     __device__ void item(const uint64_t id) const
     {
         const uint64_t tiles_q = (p.query_tokens + kQueries - 1) / kQueries;
-        const uint64_t first = (tiles_q - 1 - id / p.query_heads) * kQueries;
-        walk(id % p.query_heads, first, min(first + kQueries, p.query_tokens), 0, ~0ull >> 8,
-             [&](uint64_t head, uint64_t token, floatx16(&out)[kBlocks], float top, float sum) {
-                 publish(head, token, out, top, sum);
+        const uint64_t first = (tiles_q - 1 - id / p.query_heads) * kQueries, head = id % p.query_heads;
+        walk(head / (p.query_heads / p.kv_heads), (uint32_t)min((uint64_t)kQueries, p.query_tokens - first), false,
+             [&](uint32_t row) { return Place{first + row, head}; }, 0, ~0ull >> 8,
+             [&](const Place &at, uint32_t, floatx16(&out)[kBlocks], float top, float sum) {
+                 publish(at.head, at.token, out, top, sum);
              });
     }
 
-    // Queries [first, end) of a head, at most kQueries, over key tiles [from, to) as far as they see
-    // them.  finish(head, token, accumulators, maximum, denominator) is called for every query by the two
-    // lanes that hold its halves; the maximum is -inf where a query sees none of the keys.
-    template <class Finish>
-    __device__ __forceinline__ void walk(const uint64_t head, const uint64_t first, const uint64_t end,
-                                         const uint64_t from, const uint64_t to, const Finish &finish) const
+    // A query: its token and its head.
+    struct Place {
+        uint64_t token, head;
+    };
+
+    // `rows` queries of the query heads of a kv head, at most kQueries, over key tiles [from, to) as far as they see
+    // them: place(row) tells where row `row` lies, tokens do not fall from row to row.  finish(place, row,
+    // accumulators, maximum, denominator) is called for every query by the two lanes that hold its halves; the maximum
+    // is -inf where a query sees none of the keys.  An idle wave computes nothing and only stages.
+    template <class Locate, class Finish>
+    __device__ __forceinline__ void walk(const uint64_t kv_head, const uint32_t rows, const bool idle,
+                                         const Locate &place, const uint64_t from, const uint64_t to,
+                                         const Finish &finish) const
     {
-        const uint64_t kv_head = head / (p.query_heads / p.kv_heads);
-        const uint64_t q0 = first + (uint64_t)wave * 32u;
+        const uint32_t row0 = (uint32_t)wave * 32u;
         // rows past the last query repeat it: they compute, they are not stored
-        const uint64_t token = min(q0 + (uint64_t)column, end - 1);
+        const Place at = place(min(row0 + (uint32_t)column, rows - 1u));
+        const uint64_t wave_end = place(min(row0 + 31u, rows - 1u)).token + 1, end = place(rows - 1u).token + 1;
         // last key of this lane's query, and the keys that every query of the wave sees
-        const uint32_t last = last_visible(p, p.query_start + token);
-        const uint32_t seen_by_all = last_visible(p, p.query_start + min(q0, end - 1)) + 1u;
+        const uint32_t last = last_visible(p, p.query_start + at.token);
+        const uint32_t seen_by_all = last_visible(p, p.query_start + place(min(row0, rows - 1u)).token) + 1u;
         // last key any query of the workgroup, and of this wave, may see
         const uint64_t group_last = p.causal ? min(p.kv_tokens, p.query_start + end) : p.kv_tokens;
-        const uint64_t wave_last = p.causal ? min(p.kv_tokens, p.query_start + min(q0 + 32u, end)) : p.kv_tokens;
+        const uint64_t wave_last = p.causal ? min(p.kv_tokens, p.query_start + wave_end) : p.kv_tokens;
         const uint64_t tiles = min((group_last + kKeys - 1) / kKeys, to);
-        const uint64_t wave_tiles = q0 < end ? min((wave_last + kKeys - 1) / kKeys, to) : 0;
+        const uint64_t wave_tiles = row0 < rows && !idle ? min((wave_last + kKeys - 1) / kKeys, to) : 0;
 
         // this lane's half of its query row: Q[token][half * kHalf + s], s = 0 .. kHalf-1
         float q[kHalf];
         {
-            const float *row = p.q + token * p.q_stride + head * kDim + half * kHalf;
+            const float *row = p.q + at.token * p.q_stride + at.head * kDim + half * kHalf;
 #pragma unroll
             for (int s = 0; s < kHalf; s += 4) {
                 const floatx4 piece = *reinterpret_cast<const floatx4 *>(row + s);
@@ -239,7 +247,7 @@ struct GqaTile {
         }
 
         // (no early exit above this point: every wave of the workgroup keeps the barriers)
-        if (q0 + (uint64_t)column < end) finish(head, token, out, top, sum_xor32(sum));
+        if (row0 + (uint32_t)column < rows) finish(at, row0 + (uint32_t)column, out, top, sum_xor32(sum));
     }
 
     // Normalises and publishes one query's row, and its LSE.

@@ -438,6 +438,7 @@ def spread_cases(d, power, tq=64, tk=500, hq=4, hkv=2):
     yield "value-row-small", q, k, changed(v, np.s_[40:48], lambda x: x / big), start
     quiet_k, quiet_q = changed(k, np.s_[..., 9], np.zeros_like), changed(q, np.s_[..., 9], np.zeros_like)
     yield "query-channel", changed(q, np.s_[..., 9], grow), quiet_k, v, start
+    yield "query-one", changed(q, np.s_[tq // 2, 1], grow), k, v, start
     yield "key-channel", quiet_q, changed(k, np.s_[..., 9], grow), v, start
     # a first key that takes all but 2^-5 to 2^-17 of the weight, with a value near zero, or zero
     for label, extra, factor in (("", 8.0, 1e-4), ("-deep", 16.0, 1e-6), ("-zero", 16.0, 0.0)):
@@ -622,8 +623,8 @@ def test_gqa_split_beforehand_holds_the_spread(backend, d, power, tk):
         out, lse, facts, need = run_attached(backend, q, k, v, query_start=start)
         assert facts.kernel_launches == 3 and facts.temporary_bytes == need
         worst = relative_to_weighted_magnitudes(out, q, k, v, start)
-        # (scores of a key of 2^8, up to 1000, are rounded to 2^-25 of that; in one launch it is 9e-6 as well)
-        large = power == 8 and label.startswith("key-later")
+        # (scores of a key or query of 2^8, up to 1000, are rounded to 2^-25 of that; in one launch it is 9e-6 as well)
+        large = power == 8 and label.startswith(("key-later", "query-one"))
         assert worst < (3e-5 if large else spread_bound(label, d)), (label, worst)
 
 
