@@ -22,18 +22,20 @@
 // of 147 for 1777 tokens of 40/8 heads of 128) the weights had to carry the exponents of the values: beside a value
 // of 2^30, or behind a sink of a weight of 1 and a value near zero, the other weights lost their bits.
 //
-// Against 64 bits, per element relative to sum w |v|, the largest error is 2e-7 to 4e-7 on N(0,1) rows (fp32 walk
-// 4e-7 to 6e-7), and at most the fp32 walk's with rows, channels or components of 2^16 to 2^50 and with sinks.
+// Against 64 bits, largest error of an element relative to sum w |v| of it, head dimensions 64 / 128 / 256 (fp32 walk):
+// N(0,1) rows, other rows of 2^20 and 2^40 beside them unseen, 5.0e-7 / 6.4e-7 / 5.6e-7 (8.3e-7 / 1.1e-6 / 7.6e-7);
+// such rows, channels and components seen 1.4e-6 / 1.4e-6 / 1.7e-6 (3.0e-6 / 2.4e-6 / 2.7e-6); behind sinks of 2^11
+// to 2^23 times the other weights 3.9e-6 / 3.8e-6 / 6.5e-6 (7.4e-6 / 1.0e-5 / 1.2e-5).
 //
 // The splits are made once by a launch of their own (halve_rows) that leaves every tile of 32 keys as the walk wants
 // it in LDS: the walk's tiles are filled by loads that write LDS directly, its registers
 // hold no rows on their way, and a trip is bound by its MFMAs.  Items, packed rows and runs of keys are those of
 // the bf16 prefill (kernel_params.h), with steps of 32 keys.
 //
-// What bounds the walk is power.  At 128 it runs at 1.55 to 1.57 GHz with the matrix cores busy 72 to 74 % of the
-// cycles: 1777 tokens of 40/8 heads 129 of 140 us, 2048 tokens 162 of 171, 265 TFLOP/s of F32 products, 1.19 PFLOP/s
-// of 16-bit ones, where a large bf16 product reaches 1.29 on this part.  At 256, one wave per SIMD, 1.95 GHz and
-// 51 %: the first operands of a trip come behind its barrier (2048 tokens of 24/4 heads 227 of 236 us).
+// What bounds the walk is power.  At 128 it runs at 1.52 to 1.57 GHz with the matrix cores busy 71 to 75 % of the
+// cycles: 1777 tokens of 40/8 heads 131 of 140 us, 2048 tokens 165 of 175, 260 TFLOP/s of F32 products, 1.17 PFLOP/s
+// of 16-bit ones, where a large bf16 product reaches 1.29 on this part.  At 256, one wave per SIMD, 1.91 GHz and
+// 51 %: the first operands of a trip come behind its barrier (2048 tokens of 24/4 heads 231 of 240 us).
 #ifndef YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 #define YVEX_ROCM_KERNELS_GQA_F32_HALVED_H
 
