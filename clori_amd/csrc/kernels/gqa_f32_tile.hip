@@ -2,7 +2,7 @@
 // tokens of one query head (gqa_f32_walk.h), which needs no workspace, and the walk over keys and values split
 // beforehand (gqa_f32_halved.h).
 //
-// The one-launch form stays with fp32 products.  Split products in it take 150 us instead of 314 (1777 tokens of
+// The one-launch form stays with fp32 products.  Split products in it take 150 us instead of 310 (1777 tokens of
 // 40/8 heads of 128), but with one power of two to eight rows they lost what lay 2^20 and more below the largest of
 // the eight, and split as the walk over halves splits them every workgroup would make the splits for itself again.
 //

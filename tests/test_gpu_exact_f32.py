@@ -686,6 +686,28 @@ def test_gqa_prefill_rows_do_not_depend_on_later_rows(backend, d, hq, hkv, tq, s
         assert np.abs(out2[keep:] - out[keep:]).max() > 0.0
 
 
+def test_gqa_split_beforehand_reaches_the_last_of_its_parts(backend):
+    """The most keys whose parts a request may ask for (2 GiB less a tile or two, one kv head of 256): every head's one
+    key of weight 1 lies elsewhere, the last in the last tile, and the head's rows are that key's values."""
+    tq, tk, hq, d = 32, 838800, 4, 256
+    places = [5, 400000, 700001, tk - tq - 3]
+    q, k = np.zeros((tq, hq, d), np.float32), np.zeros((tk, 1, d), np.float32)
+    v = (np.arange(tk, dtype=np.float32) % 1021.0 + 1.0)[:, None, None] * \
+        np.linspace(0.5, 1.5, d, dtype=np.float32)[None, None, :]
+    for head, key in enumerate(places):
+        q[:, head, head] = 8.0
+        k[key, 0, head] = 400.0                     # a score of 200, the others' is 0
+    need = backend.attention_workspace_required(backend.attention_requirement(tq, tk, hq, 1, d, query_start=tk - tq))
+    assert (1 << 31) - (4 << 20) < need < (1 << 31) + (96 << 20)
+    out, lse, facts, _ = run_attached(backend, q, k, v, query_start=tk - tq)
+    assert facts.kernel_launches == 3 and facts.temporary_bytes == need
+    for head, key in enumerate(places):
+        assert np.allclose(out[:, head], v[key, 0], rtol=1e-6, atol=0.0), head
+    assert np.abs(lse - 200.0).max() < 1e-4
+    assert backend.attention_workspace_required(
+        backend.attention_requirement(tq, tk + 96, hq, 1, d, query_start=tk + 96 - tq)) == 0
+
+
 # ------------------------------------------------ decode-shaped requests over long contexts ----
 
 @pytest.mark.parametrize("tq,tk,hq,hkv,d,causal", [
